@@ -342,3 +342,101 @@ def run(state):
     else:
         _issue(state["calls"])
     return state["out"]
+
+
+def _f32(t):
+    """A 64-bit value rounded once to float32, kept in 64 bits."""
+    return t.float().double()
+
+
+def _quantized_activations(x, block):
+    """The values that an int8 activation quantizer with blocks of `block` leaves of x, in 64 bits: scale max|x| / 127, a
+    reciprocal, a product and a rounding half away from zero, each as float32 defines it."""
+    v = x.double().reshape(-1, block)
+    peak = v.abs().amax(dim=1, keepdim=True)
+    scale = torch.where(peak == 0, 1.0, _f32(peak / 127.0))
+    t = _f32(v * _f32(1.0 / scale))
+    return (torch.sign(t) * torch.floor(t.abs() + 0.5).clamp(max=127.0) * scale).reshape(x.shape)
+
+
+def _dequantized(fmt, raw, out_dim, in_dim):
+    """The values of GGUF blocks in 64 bits."""
+    values, size = BLOCK[fmt]
+    blocks = raw.reshape(-1, size)
+    halves = blocks[:, : 4 if fmt == "q4_k" else 2].contiguous().view(torch.float16).double()
+    if fmt == "q8_0":
+        dense = blocks[:, 2:].contiguous().view(torch.int8).double() * halves
+    elif fmt == "q4_0":
+        quants = blocks[:, 2:]
+        dense = (torch.cat([quants & 15, quants >> 4], dim=1).double() - 8.0) * halves
+    else:
+        packed, quants = blocks[:, 4:16], blocks[:, 16:].reshape(-1, 4, 32)
+        low, mid, high = packed[:, 0:4], packed[:, 4:8], packed[:, 8:12]
+        scales = torch.cat([low & 63, (high & 15) | (low >> 6 << 4)], dim=1).double() * halves[:, 0:1]
+        minima = torch.cat([mid & 63, (high >> 4) | (mid >> 6 << 4)], dim=1).double() * halves[:, 1:2]
+        nibbles = torch.stack([quants & 15, quants >> 4], dim=2).reshape(-1, 8, 32).double()
+        dense = nibbles * scales[:, :, None] - minima[:, :, None]
+    return dense.reshape(out_dim, in_dim)
+
+
+def _product(fmt, x, raw, out_dim):
+    """x times the transposed weight in 64 bits, on the activations that the library's definition of the op takes."""
+    rows, in_dim = x.shape
+    if fmt == "q4_k":  # 8-bit activations on a set of short inner sizes and row counts, float32 elsewhere
+        counts = (1, 2, 4, 9, 50, 64, 77, 154, 197, 231, 257, 308, 514)
+        quantized = 256 if out_dim >= 512 and in_dim in (512, 768, 1536, 2048, 3072) and rows in counts else 0
+    else:
+        quantized = 32 if out_dim >= 512 and in_dim >= 96 else 0
+    values = _quantized_activations(x, quantized) if quantized else x.double()
+    return values @ _dequantized(fmt, raw, out_dim, in_dim).T
+
+
+def exact(case, seed):
+    """What run() returns for the inputs of prepare(case, seed), by plain torch in 64 bits."""
+    src, fmt, m = _Source(seed), case["fmt"], case["rows"]
+
+    def linear(x, n):
+        return _product(fmt, x, src.raw_weight(fmt, n, x.shape[1]), n)
+
+    if case["kind"] == "linear":
+        return {"y": linear(src.hidden(m, case["in_dim"]), case["out_dim"])}
+    if case["kind"] == "rows":
+        src.normal(m, case["dim"])  # the rows to quantize; the bytes have no 64-bit value
+        table = _dequantized(fmt, src.raw_weight(fmt, m, case["dim"]), m, case["dim"])
+        ids = torch.randint(0, m, (case["lookups"],), generator=src.gen, device=DEVICE)
+        return {"quantized": None, "dense": table, "looked_up": table[ids]}
+    h, f = case["hidden"], case["ffn"]
+    if case["kind"] == "encoder":
+        out = {}
+        for i in range(case["layers"]):
+            made = {name: (src.raw_weight(fmt, n, k), n, (src.normal(n) * 0.1).double())
+                    for name, n, k in (("q", h, h), ("k", h, h), ("v", h, h), ("o", h, h), ("fc1", f, h), ("fc2", h, f))}
+            x, context, residual, mid = src.hidden(m, h), src.normal(m, h), src.normal(m, h), src.hidden(m, h)
+            wide = torch.nn.functional.gelu(src.normal(m, f))
+
+            def biased(a, name, made=made):
+                raw, n, bias = made[name]
+                return _product(fmt, a, raw, n) + bias
+
+            out.update({f"{i}.q": biased(x, "q"), f"{i}.k": biased(x, "k"), f"{i}.v": biased(x, "v")})
+            out[f"{i}.attn"] = biased(context, "o") + residual.double()
+            out[f"{i}.up"] = torch.nn.functional.gelu(biased(mid, "fc1"), approximate="tanh")
+            out[f"{i}.down"] = biased(wide, "fc2") + out[f"{i}.attn"]
+        return out
+    layers = {name: [] for name in ("qkv", "attn", "gate", "up", "down") + (("key", "value") if case["kv"] else ())}
+    for _ in range(case["layers"]):
+        x = src.hidden(m, h)
+        layers["qkv"].append(linear(x, case["qkv"]))
+        if case["kv"]:
+            layers["key"].append(linear(x, case["kv"]))
+            layers["value"].append(linear(x, case["kv"]))
+        layers["attn"].append(linear(src.normal(m, h), h))
+        x = src.hidden(m, h)
+        layers["gate"].append(linear(x, f))
+        layers["up"].append(linear(x, f))
+        layers["down"].append(linear(src.gated(m, f), h))
+    out = {name: torch.stack(values) for name, values in layers.items()}
+    if case["vocab"]:
+        logits = linear(src.hidden(m, h)[-1:], case["vocab"])
+        out["token"] = logits.argmax(dim=1).to(torch.int32)
+    return out
