@@ -77,6 +77,10 @@ static WorkspaceView workspace_view(uint64_t base, size_t rows, size_t in_dim) {
 // two rows of any length, and for three or four rows of Q4_0 up to this many 32-value
 // blocks of X; beyond, a separate kernel quantizes X once.
 constexpr size_t kGemvFusedQuantBlocks = 512;
+// Fewest outputs of a matrix that the f32 route takes to the matrix cores (PREPARED layout).  Below, a wavefront per output
+// is the shorter chain: a pair of 256 columns at K = 2048, eight rows 6.1 us against 8.1, sixteen rows 9.9 against 9.4, 77
+// rows 39.0 against 9.6, 2048 rows 961 against 74; on a short K three rows of 5000 columns (K = 64) 10.6 against 3.1.
+constexpr size_t kF32RouteMfmaMinOutputs = 4096;
 // fewest rows served by the single-shot MFMA kernel (batch_mfma_kernels.hip)
 constexpr size_t kBatchMfmaMinRows = 5;
 
@@ -408,14 +412,15 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
     // The block dots only exist on the activation-quantized route.
     const bool route_a = want_dots || afhip_uses_activation_quant(rows, in_dim, out_dim);
     if (!route_a) {
-        if (counters) counters->f32_route++;
-        hipError_t e = launch_linear_generic(stream, tensor_type, layout, false, y, nullptr, x, nullptr, nullptr, w,
-                                             static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), ep);
-        if (e == hipSuccess && pair) {
-            if (counters) counters->f32_route++;
-            e = launch_linear_generic(stream, tensor_type, layout, false, y_b, nullptr, x, nullptr, nullptr, w_b,
-                                      static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), ep_b);
+        if (counters) counters->f32_route += pair ? 2 : 1;
+        const int m = static_cast<int>(rows), k = static_cast<int>(in_dim), n = static_cast<int>(out_dim);
+        if (layout == AFHIP_LAYOUT_PREPARED && out_count >= kF32RouteMfmaMinOutputs) {
+            const hipError_t e = launch_linear_f32_rows(stream, tensor_type, y, x, w, m, k, n, ep, pair ? y_b : nullptr,
+                                                        pair ? w_b : nullptr, ep_b);
+            return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
         }
+        const hipError_t e = launch_linear_generic(stream, tensor_type, layout, false, y, nullptr, x, nullptr, nullptr, w, m, k, n, ep,
+                                                   pair ? y_b : nullptr, pair ? w_b : nullptr, ep_b);
         return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
     }
 

@@ -1,0 +1,186 @@
+// The f32 route (fewer than 512 columns, or K below 96: narrow key / value projections) on the matrix cores, PREPARED
+// layout: y[r][o] = sum over blocks of d[o][b] * sum_i x[r][32 b + i] * q[o][32 b + i], f32 activations.
+//
+// What bounded the one-wavefront-per-output kernel (linear_f32_route_kernel, still used for a few rows and the raw layout):
+// every output read its whole row of X and row of W again and converted every weight again -- one convert and one
+// multiply-add per weight and row on the vector ALU.  Here an activation is split once per workgroup column group into
+// three bf16 numbers hi + mid + lo, each the leading eight bits of what the previous ones left over: together all 24 bits
+// of the f32, so the products q * x (q is exact in bf16) are exact in the accumulator and nothing is lost against f32.
+// Three v_mfma_f32_16x16x32_bf16 per 16 rows x 16 columns x block then leave the block's dots, and one multiply-add per
+// element applies the scale, as before.
+//
+// A workgroup owns 16 rows x 16 * kTiles columns and all of K; its wavefronts take the blocks round robin (sixteen of them
+// where K allows) and their sums meet in LDS in wavefront order.  kTiles column tiles share one split of X: the split is
+// about 70 of 100 vector instructions at one tile, but a short prompt has too few tiles to give up workgroups for it.
+// Bound by the vector ALU (the split) on many rows, by latency on few.  A pair of 256 columns at K = 2048: 77 rows 39.0 us
+// (two launches of a wavefront per output: 46) -> 9.6, 2048 rows 961 -> 74.  Relative error against 64 bits 1.0e-7 (1.3e-7).
+#include <hip/hip_runtime.h>
+
+#include "device_common.h"
+#include "qmatmul_launch.h"
+
+namespace afhip {
+
+namespace {
+
+typedef float r_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 r_bf16x8 __attribute__((ext_vector_type(8)));
+union Bf16x8 {
+    r_bf16x8 v;
+    uint32_t u[4];
+};
+
+constexpr int kRouteRows = 16;   // rows of a workgroup, and columns of a tile
+constexpr int kRouteDepth = 4;   // blocks a wavefront requests ahead of its arithmetic
+
+__device__ __forceinline__ uint32_t upper_halves(float a, float b) {  // bf16 bits of a, b (already exact in bf16): a low, b high
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+__device__ __forceinline__ float leading8(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u); }
+
+// x = hi + mid + lo exactly (truncation: no rounding can overflow).  An infinity is its own hi with nothing left over, so that
+// it reaches the sum as an infinity; a NaN leaves a NaN behind even where its payload lies in the low bits.
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t* hi, uint32_t* mid, uint32_t* lo) {
+    const float h0 = leading8(x0), h1 = leading8(x1);
+    const float r0 = __builtin_isinf(x0) ? 0.0f : x0 - h0, r1 = __builtin_isinf(x1) ? 0.0f : x1 - h1;
+    const float m0 = leading8(r0), m1 = leading8(r1);
+    *hi = upper_halves(h0, h1);
+    *mid = upper_halves(m0, m1);
+    *lo = upper_halves(r0 - m0, r1 - m1);
+}
+
+}  // namespace
+
+// A second matrix of the same shape on the same X: grid.z = 2.
+struct RouteSecond {
+    float* dst;
+    const uint8_t* weight;
+    Epilogue ep;
+};
+
+template <int kType, int kTiles>
+__global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
+                                                               const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
+                                                               Epilogue ep_a, RouteSecond second) {
+    extern __shared__ __align__(16) float route_sums[];  // [wavefront][tile][4][64]
+    const bool is_b = blockIdx.z != 0;
+    float* dst = is_b ? second.dst : dst_a;
+    const uint8_t* weight = is_b ? second.weight : weight_a;
+    const Epilogue ep = is_b ? second.ep : ep_a;
+    constexpr int kQuantBytes = kType == 2 ? 16 : 32;
+    const int kb = in_dim >> 5;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+    const int c = lane & 15, g = lane >> 4;  // operand row / column, and the eight values 8 g .. 8 g + 7 of a block
+    const int m0 = blockIdx.y * kRouteRows, n0 = blockIdx.x * (16 * kTiles);
+    // rows and columns past the end repeat the last one; their results are not stored
+    const float* xrow = x + static_cast<size_t>(min(m0 + c, rows - 1)) * in_dim + 8 * g;
+    const size_t blocks = static_cast<size_t>(out_dim) * kb;
+    const uint16_t* scales = reinterpret_cast<const uint16_t*>(weight + blocks * kQuantBytes);
+    size_t first[kTiles];  // first block of this lane's column in each tile
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) first[t] = static_cast<size_t>(min(n0 + 16 * t + c, out_dim - 1)) * kb;
+
+    r_f32x4 acc[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) acc[t] = r_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    for (int b0 = wave; b0 < kb; b0 += waves * kRouteDepth) {
+        float4 xv[kRouteDepth][2];
+        uint2 wq[kRouteDepth][kTiles];
+        uint16_t ws[kRouteDepth][kTiles];
+#pragma unroll
+        for (int u = 0; u < kRouteDepth; ++u) {
+            const int b = min(b0 + u * waves, kb - 1);  // past the end: the last block again, not used
+            xv[u][0] = reinterpret_cast<const float4*>(xrow + b * 32)[0];
+            xv[u][1] = reinterpret_cast<const float4*>(xrow + b * 32)[1];
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) {
+                // Q4_0: values 0..15 are the low nibbles of the 16 bytes, 16..31 the high ones
+                const uint8_t* at = weight + (first[t] + b) * kQuantBytes + 8 * (kType == 2 ? g & 1 : g);
+                wq[u][t] = *reinterpret_cast<const uint2*>(at);
+                ws[u][t] = scales[first[t] + b];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRouteDepth; ++u) {
+            if (b0 + u * waves >= kb) break;  // wavefront-uniform
+            Bf16x8 part[3];
+            const float v[8] = {xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w, xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) split_pair(v[2 * i], v[2 * i + 1], &part[0].u[i], &part[1].u[i], &part[2].u[i]);
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) {
+                // bytes biased to unsigned (nibbles are so already), converted, the bias taken off: integers below 2^8, exact
+                const uint32_t p[2] = {wq[u][t].x, wq[u][t].y};
+                Bf16x8 w;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t biased = kType == 2 ? (p[i] >> (4 * (g >> 1))) & 0x0F0F0F0Fu : p[i] ^ 0x80808080u;
+                    constexpr float kBias = kType == 2 ? 8.0f : 128.0f;
+                    const float f0 = static_cast<float>(biased & 0xFFu) - kBias, f1 = static_cast<float>((biased >> 8) & 0xFFu) - kBias;
+                    const float f2 = static_cast<float>((biased >> 16) & 0xFFu) - kBias, f3 = static_cast<float>(biased >> 24) - kBias;
+                    w.u[2 * i] = upper_halves(f0, f1);
+                    w.u[2 * i + 1] = upper_halves(f2, f3);
+                }
+                r_f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int q = 2; q >= 0; --q) dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[q].v, w.v, dot, 0, 0, 0);
+                const float d = half_bits_to_f32(ws[u][t]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fmaf(d, dot[i], acc[t][i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) route_sums[((wave * kTiles + t) * 4 + i) * 64 + lane] = acc[t][i];
+    __syncthreads();
+    for (int at = tid; at < kTiles * 256; at += blockDim.x) {
+        float total = 0.0f;
+        for (int w = 0; w < waves; ++w) total += route_sums[w * (kTiles * 256) + at];
+        const int l = at & 63, i = (at >> 6) & 3, t = at >> 8;
+        const int m = m0 + 4 * (l >> 4) + i, n = n0 + 16 * t + (l & 15);
+        if (m < rows && n < out_dim) {
+            const size_t to = static_cast<size_t>(m) * out_dim + n;
+            dst[to] = finish_output(ep, n, to, total);
+        }
+    }
+}
+
+hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* dst, const float* x, const uint8_t* weight_prepared,
+                                  int rows, int in_dim, int out_dim, const Epilogue& ep0, float* dst_b, const uint8_t* weight_b,
+                                  const Epilogue& ep_b0) {
+    if (rows <= 0 || out_dim <= 0) return hipSuccess;
+    const int kb = in_dim / 32, matrices = weight_b != nullptr ? 2 : 1;
+    int waves = 16;
+    while (waves > 1 && waves > kb) waves /= 2;
+    constexpr int kRowsPerLaunch = 16 * 65535;  // grid.y
+    for (int r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
+        const int nr = rows - r0 < kRowsPerLaunch ? rows - r0 : kRowsPerLaunch;
+        const unsigned groups = static_cast<unsigned>((nr + 15) / 16);
+        // one column tile while four of them a workgroup would leave compute units without one
+        const long wide = static_cast<long>(groups) * ((out_dim + 63) / 64) * matrices;
+        const int tiles = wide >= gemv_compute_units() ? 4 : 1;
+        const dim3 grid(static_cast<unsigned>((out_dim + 16 * tiles - 1) / (16 * tiles)), groups, matrices), block(64 * waves);
+        const size_t lds = static_cast<size_t>(waves) * tiles * 1024;  // at most 64 KiB
+        Epilogue ep = ep0, ep_b = ep_b0;
+        if (ep.residual) ep.residual += static_cast<size_t>(r0) * out_dim;
+        if (ep_b.residual) ep_b.residual += static_cast<size_t>(r0) * out_dim;
+        float* d = dst + static_cast<size_t>(r0) * out_dim;
+        const float* in = x + static_cast<size_t>(r0) * in_dim;
+        const RouteSecond second{dst_b ? dst_b + static_cast<size_t>(r0) * out_dim : nullptr, weight_b, ep_b};
+        if (tensor_type == 2) {
+            if (tiles == 4) hipLaunchKernelGGL((linear_f32_rows_kernel<2, 4>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+            else hipLaunchKernelGGL((linear_f32_rows_kernel<2, 1>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+        } else {
+            if (tiles == 4) hipLaunchKernelGGL((linear_f32_rows_kernel<8, 4>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+            else hipLaunchKernelGGL((linear_f32_rows_kernel<8, 1>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+        }
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+}  // namespace afhip

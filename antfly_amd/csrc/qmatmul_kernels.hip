@@ -50,12 +50,16 @@ __device__ __forceinline__ void linear_f32_route_body(float* __restrict__ dst, c
     if (lane == 0) dst[static_cast<size_t>(r) * out_dim + o] = finish_output(ep, o, static_cast<size_t>(r) * out_dim + o, acc);
 }
 
+// grid.z = 2: a second matrix of the same shape on the same X (the key and value projections of a decode step are 256
+// wavefronts each, one per compute unit: as two launches each cost a launch).
 template <typename Weights>
 __global__ __launch_bounds__(64) void linear_f32_route_kernel(float* __restrict__ dst,
                                                               const float* __restrict__ input, Weights w,
                                                               int rows, int in_dim, int out_dim,
-                                                              Epilogue ep) {
-    linear_f32_route_body(dst, input, w, rows, in_dim, out_dim, ep);
+                                                              Epilogue ep, float* __restrict__ dst_b, Weights w_b,
+                                                              Epilogue ep_b) {
+    if (blockIdx.z != 0) linear_f32_route_body(dst_b, input, w_b, rows, in_dim, out_dim, ep_b);
+    else linear_f32_route_body(dst, input, w, rows, in_dim, out_dim, ep);
 }
 
 // Route A from pre-quantized activations.  grid = (out_dim, rows), block = 64.
@@ -483,21 +487,23 @@ hipError_t launch_quantize_activations(hipStream_t stream, const float* x, int r
 template <typename Weights>
 static hipError_t launch_generic(hipStream_t stream, bool route_a, float* dst, int* dots, const float* input,
                                  const int8_t* qx, const float* sx, Weights w, int rows, int in_dim, int out_dim,
-                                 const Epilogue& ep) {
-    dim3 grid(out_dim, rows);
+                                 const Epilogue& ep, float* dst_b, Weights w_b, const Epilogue& ep_b) {
+    dim3 grid(out_dim, rows, dst_b != nullptr ? 2 : 1);
     if (route_a) {
         hipLaunchKernelGGL(linear_act_generic_kernel<Weights>, grid, dim3(64), 0, stream, dst, dots, qx, sx, w, rows,
                            in_dim, out_dim, ep);
     } else {
         hipLaunchKernelGGL(linear_f32_route_kernel<Weights>, grid, dim3(64), 0, stream, dst, input, w, rows, in_dim,
-                           out_dim, ep);
+                           out_dim, ep, dst_b, w_b, ep_b);
     }
     return launch_status();
 }
 
 hipError_t launch_linear_generic(hipStream_t stream, int tensor_type, int layout, bool route_a, float* dst, int* dots,
                                  const float* input, const int8_t* qx, const float* sx, const uint8_t* weight,
-                                 int rows, int in_dim, int out_dim, const Epilogue& ep0) {
+                                 int rows, int in_dim, int out_dim, const Epilogue& ep0, float* dst_b, const uint8_t* weight_b,
+                                 const Epilogue& ep_b0) {
+    if (route_a && weight_b != nullptr) return hipErrorInvalidValue;
     const size_t blocks = static_cast<size_t>(out_dim) * (in_dim / 32);
     // grid.y is limited to 65535 rows per launch
     for (int r0 = 0; r0 < rows; r0 += 32768) {
@@ -509,18 +515,24 @@ hipError_t launch_linear_generic(hipStream_t stream, int tensor_type, int layout
         const float* s = sx ? sx + static_cast<size_t>(r0) * (in_dim / 32) : nullptr;
         Epilogue ep = ep0;
         if (ep.residual) ep.residual += static_cast<size_t>(r0) * out_dim;
+        Epilogue ep_b = ep_b0;
+        if (ep_b.residual) ep_b.residual += static_cast<size_t>(r0) * out_dim;
+        float* d_b = weight_b ? dst_b + static_cast<size_t>(r0) * out_dim : nullptr;
+        const uint8_t* second = weight_b ? weight_b : weight;
         hipError_t e;
         if (layout == 0) {
-            if (tensor_type == 2) e = launch_generic(stream, route_a, d, dd, in, q, s, RawWeights<2>{weight}, nr, in_dim, out_dim, ep);
-            else e = launch_generic(stream, route_a, d, dd, in, q, s, RawWeights<8>{weight}, nr, in_dim, out_dim, ep);
+            if (tensor_type == 2) e = launch_generic(stream, route_a, d, dd, in, q, s, RawWeights<2>{weight}, nr, in_dim, out_dim, ep, d_b, RawWeights<2>{second}, ep_b);
+            else e = launch_generic(stream, route_a, d, dd, in, q, s, RawWeights<8>{weight}, nr, in_dim, out_dim, ep, d_b, RawWeights<8>{second}, ep_b);
         } else {
-            const uint4* qs = reinterpret_cast<const uint4*>(weight);
+            const uint4 *qs = reinterpret_cast<const uint4*>(weight), *qs_b = reinterpret_cast<const uint4*>(second);
             if (tensor_type == 2) {
-                PreparedWeights<2> w{qs, reinterpret_cast<const uint16_t*>(weight + blocks * 16)};
-                e = launch_generic(stream, route_a, d, dd, in, q, s, w, nr, in_dim, out_dim, ep);
+                const PreparedWeights<2> w{qs, reinterpret_cast<const uint16_t*>(weight + blocks * 16)};
+                const PreparedWeights<2> w_b{qs_b, reinterpret_cast<const uint16_t*>(second + blocks * 16)};
+                e = launch_generic(stream, route_a, d, dd, in, q, s, w, nr, in_dim, out_dim, ep, d_b, w_b, ep_b);
             } else {
-                PreparedWeights<8> w{qs, reinterpret_cast<const uint16_t*>(weight + blocks * 32)};
-                e = launch_generic(stream, route_a, d, dd, in, q, s, w, nr, in_dim, out_dim, ep);
+                const PreparedWeights<8> w{qs, reinterpret_cast<const uint16_t*>(weight + blocks * 32)};
+                const PreparedWeights<8> w_b{qs_b, reinterpret_cast<const uint16_t*>(second + blocks * 32)};
+                e = launch_generic(stream, route_a, d, dd, in, q, s, w, nr, in_dim, out_dim, ep, d_b, w_b, ep_b);
             }
         }
         if (e != hipSuccess) return e;

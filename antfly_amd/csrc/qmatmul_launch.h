@@ -128,10 +128,17 @@ hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* par
 hipError_t launch_quantize_activations(hipStream_t stream, const float* x, int rows, int in_dim, int8_t* q,
                                        float* scale, int* sum);
 
-// Any layout / shape.  route_a: uses qx/sx (pre-quantized), else f32 `input`.
+// Any layout / shape.  route_a: uses qx/sx (pre-quantized), else f32 `input`.  dst_b / weight_b (f32 `input` only): a second
+// matrix of the same shape in the same launch.
 hipError_t launch_linear_generic(hipStream_t stream, int tensor_type, int layout, bool route_a, float* dst, int* dots,
                                  const float* input, const int8_t* qx, const float* sx, const uint8_t* weight,
-                                 int rows, int in_dim, int out_dim, const Epilogue& ep = Epilogue{});
+                                 int rows, int in_dim, int out_dim, const Epilogue& ep = Epilogue{}, float* dst_b = nullptr,
+                                 const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{});
+// The f32 route on the matrix cores: PREPARED weights, any rows, no scratch; dst_b / weight_b: a second matrix of the same
+// shape on the same X in the same launch.
+hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* dst, const float* x, const uint8_t* weight_prepared,
+                                  int rows, int in_dim, int out_dim, const Epilogue& ep, float* dst_b = nullptr,
+                                  const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{});
 
 hipError_t launch_prepare_weight(hipStream_t stream, int tensor_type, uint8_t* dst, const uint8_t* src,
                                  size_t out_dim, size_t kb);

@@ -203,6 +203,35 @@ def test_f32_route_matches_oracle(fmt, layout, rows, in_dim, out_dim):
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(16, 2048, 256), (77, 544, 256), (17, 96, 511), (8, 512, 511), (9, 512, 457), (3, 64, 5000),
+                                                 (1, 32, 4096), (300, 2048, 511), (2100, 64, 70)])
+def test_f32_route_on_many_outputs(fmt, rows, in_dim, out_dim):
+    """From 4096 outputs on the f32 route runs on the matrix cores: row and column remainders, K shorter than and not a multiple
+    of what its wavefronts take together, one and four column tiles a workgroup; a pair is one launch with the bits of two calls.
+    Activations are split exactly and summed in f32, so the error is that of f32 sums (TIGHT), also next to 10^6 times larger
+    ones; an infinity stays in its row and reaches it as the reference's does."""
+    print(f"case: f32 route rows={rows} in={in_dim} out={out_dim} fmt={fmt}", flush=True)
+    assert not O.uses_activation_quant(rows, in_dim, out_dim)
+    x = synth.activations(5 * rows + in_dim, rows, in_dim)
+    x[rows // 2, ::7] *= 1e6
+    x[0, :3] = [1e36, 1e-38, 0.0]  # (times a quant of 127 still finite in f32)
+    wa, wb = synth.weights(fmt, 3 * out_dim, out_dim, in_dim), synth.weights(fmt, 3 * out_dim + 1, out_dim, in_dim)
+    da, db = G.prepare(fmt, wa, out_dim, in_dim), G.prepare(fmt, wb, out_dim, in_dim)
+    ya, yb = G.linear_pair(fmt, PREP, x, da, db, rows, in_dim, out_dim)
+    for w, y in ((wa, ya), (wb, yb)):
+        y64 = x.astype(np.float64) @ O.dequantize(fmt, w).reshape(out_dim, in_dim).astype(np.float64).T
+        assert G.max_rel_err(y, y64) <= TIGHT
+    assert np.array_equal(G.linear(fmt, PREP, x, da, rows, in_dim, out_dim), ya)
+    assert np.array_equal(G.linear(fmt, PREP, x, db, rows, in_dim, out_dim), yb)
+    x[rows - 1, 5] = np.inf
+    y = G.linear(fmt, PREP, x, da, rows, in_dim, out_dim)
+    with np.errstate(invalid="ignore"):
+        want = x[-1].astype(np.float64) @ O.dequantize(fmt, wa).reshape(out_dim, in_dim).astype(np.float64).T
+    assert np.array_equal(np.isnan(y[-1]), np.isnan(want)) and np.array_equal(np.isposinf(y[-1]), np.isposinf(want))
+    assert np.array_equal(y[:-1], ya[:-1])
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
 @pytest.mark.parametrize("rows", [6, 12])  # 12 rows forced onto the GEMV kernels: activations quantized by their own kernel
 def test_forced_dispatch_kinds_agree(fmt, rows):
     """A plan may force any kernel family; all of them compute the same op."""
