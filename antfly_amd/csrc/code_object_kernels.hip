@@ -27,7 +27,7 @@
 //       multiple of slices, grid ceil(groups / (w / slices)); dynamic LDS = rows * (in_dim + 8 kb) + 256 * max(rows, 4)
 //   termite_hip_gemm_q4_0_f32 / _q8_0_f32(dst, input, weight_prepared, rows, in_dim, out_dim, q, scales, m_tiles, n_tiles)
 //       the mm bucket on int8 MFMA, 64 x 128 tiles (`input` is not read): m_tiles = ceil(rows / 64), n_tiles =
-//       ceil(out_dim / 128), grid ceil(n_tiles / 8) * m_tiles * 8, block 1024, dynamic LDS 110592 (Q8_0) / 143360 (Q4_0)
+//       ceil(out_dim / 128), grid ceil(n_tiles / 8) * m_tiles * 8, block 1024, dynamic LDS 110592 (Q8_0) / 77824 (Q4_0; more is allowed)
 //   termite_hip_gemm_q4_0_f32_small / _q8_0_f32_small(...)  the same on 32 x 64 tiles for launches whose 64 x 128
 //       tiles would leave units idle: m_tiles = ceil(rows / 32), n_tiles = ceil(out_dim / 64), block 512,
 //       the same dynamic LDS

@@ -19,7 +19,13 @@
 // tile that share the K loop: a stage holds 2*kSplit blocks and wavefront ks of a
 // tile takes pair ks of every stage.  The kSplit partial sums of a tile are added
 // in LDS at the end, in ks order (so y is a fixed-order sum of kSplit block-ascending
-// partial sums).  Sixteen wavefronts per workgroup put four on every SIMD.
+// partial sums).  Four wavefronts on every SIMD, where LDS allows as two workgroups of
+// eight: they wait at barriers of their own, so one computes while the other meets (a
+// workgroup of sixteen spent a quarter of its K loop at barriers).  A wavefront with two
+// tiles (kPerM = 2) reads one weight fragment for both.  Bound by the vector ALU beside the
+// MFMA: about 230 SIMD cycles per 32 x 32 outputs and block (300 before, Q4_0), of which
+// the arithmetic alone takes 140.  2048 rows, K = 4096, N = 14336: Q4_0 513 -> 393 us
+// (612 TOP/s), Q8_0 434 -> 400 us.
 //
 // Operands reach LDS without passing through registers: activations and Q8_0 weight
 // bytes are fetched with global_load_lds_dwordx4 into a ring of kRing stages (4, or
@@ -30,8 +36,9 @@
 // the row, so that the MFMA fragment reads (one row per lane, same chunk column) of 16
 // consecutive lanes hit 16 different bank groups.  Block scales arrive the same way
 // (f32 activation scales as they are, fp16 weight scales zero-extended to 32 bits
-// and converted when read).  Q4_0 nibble chunks land in a staging area of the slot
-// and are expanded to int8 fragments by the wavefront that fetched them.
+// and converted when read).  Q4_0 nibble chunks stay packed in LDS: a lane half of an
+// MFMA operand is one nibble of every byte, shifted to the top of its byte and so
+// sixteen times its value (two instructions a word), and the scale is a sixteenth.
 //
 // MFMA operands: A = activations (row = lane % 32 -> m), B = weights (column =
 // lane % 32 -> n); lane / 32 selects bytes [16*(lane/32), +16) of the block.
@@ -54,17 +61,18 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-template <int kWavesM, int kWavesN, int kSplit, bool kQ4>
+// A wavefront owns kPerM x kPerN tiles of 32 x 32.
+template <int kWavesM, int kWavesN, int kSplit, bool kQ4, int kPerM = 1, int kPerN = 1>
 struct GemmShape {
     static constexpr int kTiles = kWavesM * kWavesN;
     static constexpr int kWaves = kTiles * kSplit;
     static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kTM = 32 * kWavesM, kTN = 32 * kWavesN;
+    static constexpr int kTM = 32 * kWavesM * kPerM, kTN = 32 * kWavesN * kPerN;
     static constexpr int kStageBlocks = 2 * kSplit;              // one pair per wavefront and stage
     static constexpr int kChunksPerRow = 2 * kStageBlocks;       // 16-byte chunks of int8 per row and stage
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;      // rows one 64-lane LDS load covers
     static constexpr int kGroupsA = kTM / kRowsPerLoad, kGroupsB = kTN / kRowsPerLoad;
-    static constexpr int kABytes = kTM * kChunksPerRow * 16, kBBytes = kTN * kChunksPerRow * 16;
+    static constexpr int kABytes = kTM * kChunksPerRow * 16, kBBytes = kTN * kStageBlocks * (kQ4 ? 16 : 32);
     // LDS keeps a stage of an operand row-major, [row][chunk], with the chunk index
     // XOR-swizzled by the row so that 16 consecutive rows reading the same chunk
     // column hit 16 different 16-byte bank groups (a row is 16 * kChunksPerRow bytes,
@@ -75,8 +83,7 @@ struct GemmShape {
     }
     static_assert(kChunksPerRow == 4 || kChunksPerRow == 8 || kChunksPerRow == 16, "swizzle covers rows of 64..256 bytes");
     static constexpr int kSxBytes = kTM * kStageBlocks * 4, kSwBytes = kTN * kStageBlocks * 4;
-    static constexpr int kRawBytes = kQ4 ? kTN * kStageBlocks * 16 : 0;  // Q4_0 nibble chunks as fetched
-    static constexpr int kStageBytes = kABytes + kBBytes + kSxBytes + kSwBytes + kRawBytes;
+    static constexpr int kStageBytes = kABytes + kBBytes + kSxBytes + kSwBytes;
     static constexpr int kReduceBytes = kSplit > 1 ? kSplit * kTM * kTN * 4 : 0;
     // LDS stages: loads run kRing - 1 stages ahead of the consumer
     static constexpr int kRing = 4 * kStageBytes <= 160 * 1024 ? 4 : 3;
@@ -131,19 +138,21 @@ extern __shared__ __align__(16) unsigned char gemm_lds[];
 // 32-bit counts over the start of dst, [8 * (workgroup * wavefronts + wavefront)]: shader-clock cycles before
 // the K loop, in it, waiting for its own loads, waiting at the workgroup barrier, 100 MHz reference ticks
 // spent in the loop (cycles / ticks = the clock the chip held), cycles after the loop, 0, and the HW_ID register.
-template <int kType, int kWavesM, int kWavesN, int kSplit, bool kWriteDots, bool kShareK = false, bool kStamps = false>
+template <int kType, int kWavesM, int kWavesN, int kSplit, bool kWriteDots, bool kShareK = false, bool kStamps = false, int kPerM = 1,
+          int kPerN = 1>
 __device__ __forceinline__ void gemm_i8_body(
     float* __restrict__ dst, int* __restrict__ dots, const int8_t* __restrict__ qx, const float* __restrict__ sx,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_tiles, int n_tiles,
     int share_blocks, float* __restrict__ partial, const Epilogue& ep) {
-    using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2>;
+    using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2, kPerM, kPerN>;
+    static_assert(kPerM * kPerN == 1 || (!kWriteDots && !kStamps), "block dots and clock readings: one tile a wavefront");
     constexpr int kWaves = S::kWaves, kSB = S::kStageBlocks, kRPL = S::kRowsPerLoad, kCPR = S::kChunksPerRow;
     constexpr int kTM = S::kTM, kTN = S::kTN, kRing = S::kRing;
     constexpr int kQuantBytes = kType == 2 ? 16 : 32;
     constexpr bool kQ4 = kType == 2;
     // units of 64 lanes per stage, by kind
     constexpr int kUnitsA = S::kGroupsA;                          // LDS loads of activation bytes
-    constexpr int kUnitsB = kQ4 ? kTN * kSB / 64 : S::kGroupsB;   // Q8_0: LDS loads; Q4_0: register loads of 16-byte nibble chunks
+    constexpr int kUnitsB = kQ4 ? kTN * kSB / 64 : S::kGroupsB;   // Q4_0: of 16-byte nibble chunks
     constexpr int kUnitsSx = kTM * kSB / 64, kUnitsSw = kTN * kSB / 64;
     constexpr int kPerA = (kUnitsA + kWaves - 1) / kWaves, kPerB = (kUnitsB + kWaves - 1) / kWaves;
     constexpr int kPerSx = (kUnitsSx + kWaves - 1) / kWaves, kPerSw = (kUnitsSw + kWaves - 1) / kWaves;
@@ -197,140 +206,130 @@ __device__ __forceinline__ void gemm_i8_body(
 #pragma unroll
     for (int i = 0; i < kPerSw; ++i) loads_per_stage += usw0 + i * kWaves < kUnitsSw;
 
-    // Per-lane byte offsets of the loads, for a full stage ([0]) and for the last
-    // stage ([1], block indices clamped to the last valid block: nothing is read past
-    // a row's end; the scales of the clamped blocks are written as zero).
-    // LDS position p = lane of a 64-lane load is chunk slot p % kCPR of row p / kCPR:
-    // eight (or more) consecutive lanes read one 128-byte line, in swizzled order.
-    const int dma_r = lane / kCPR, dma_slot = lane % kCPR;
-    uint32_t off_a[kPerA][2], off_b[kPerB][2], off_sx[kPerSx][2], off_sw[kPerSw][2];
-    int lds_b4[kPerB][2];  // Q4_0: LDS chunk positions of the low- and high-nibble halves
-    auto dma_chunk_last = [&](int c) { return min(c >> 1, last_blocks - 1) * 2 + (c & 1); };
+    // Per-lane byte offsets of the loads of a stage whose blocks from `blocks_here` on are clamped to the one before (the last
+    // stage: nothing is read past a row's end; the scales of the clamped blocks are taken as zero).
+    // LDS position p = lane of a 64-lane load is chunk slot p % kCPR of row p / kCPR: eight (or more) consecutive lanes
+    // read one 128-byte line, in swizzled order.
+    auto chunk_offset = [&](int unit, int l, int tile_rows, int first_row, int last_row, int blocks_here) {
+        const int r = min(unit * kRPL + l / kCPR, tile_rows - 1);
+        const int c = (l % kCPR) ^ ((r / S::kRowsPerWrap) % kCPR);
+        return static_cast<uint32_t>(min(first_row + r, last_row) - first_row) * static_cast<uint32_t>(kb_full) * 32u +
+               (min(c >> 1, blocks_here - 1) * 2 + (c & 1)) * 16;
+    };
+    auto offset_a = [&](int i, int l, int blocks_here) { return chunk_offset(ua0 + i * kWaves, l, kTM, m0, rows - 1, blocks_here); };
+    // Q4_0: LDS position of a row's nibble chunk, [row][block] with the block XOR-swizzled by the row like the chunks
+    auto nibble_slot = [](int r, int blk) { return blk ^ ((r / (16 / kSB)) % kSB); };
+    auto offset_b = [&](int i, int l, int blocks_here) {
+        if (!kQ4) return chunk_offset(ub0 + i * kWaves, l, kTN, n0, out_dim - 1, blocks_here);
+        const int q = min((ub0 + i * kWaves) * 64 + l, kTN * kSB - 1), r = q / kSB;
+        return static_cast<uint32_t>(min(n0 + r, out_dim - 1) - n0) * static_cast<uint32_t>(kb_full) * 16u +
+               min(nibble_slot(r, q % kSB), blocks_here - 1) * 16;
+    };
+    auto scale_offset = [&](int unit, int l, int values, int first_row, int last_row, int blocks_here) {
+        const int q = min(unit * 64 + l, values - 1);
+        return static_cast<uint32_t>(min(first_row + q / kSB, last_row) - first_row) * static_cast<uint32_t>(kb_full) +
+               min(q % kSB, blocks_here - 1);
+    };
+    auto offset_sx = [&](int i, int l, int blocks_here) { return 4 * scale_offset(usx0 + i * kWaves, l, kTM * kSB, m0, rows - 1, blocks_here); };
+    auto offset_sw = [&](int i, int l, int blocks_here) { return 2 * scale_offset(usw0 + i * kWaves, l, kTN * kSB, n0, out_dim - 1, blocks_here); };
+    uint32_t off_a[kPerA], off_b[kPerB], off_sx[kPerSx], off_sw[kPerSw];  // of a full stage
 #pragma unroll
-    for (int i = 0; i < kPerA; ++i) {
-        const int r = min((ua0 + i * kWaves) * kRPL + dma_r, kTM - 1);
-        const int c = dma_slot ^ ((r / S::kRowsPerWrap) % kCPR);
-        const uint32_t rowoff = static_cast<uint32_t>(min(m0 + r, rows - 1) - m0) * static_cast<uint32_t>(in_dim);
-        off_a[i][0] = rowoff + c * 16;
-        off_a[i][1] = rowoff + dma_chunk_last(c) * 16;
-    }
+    for (int i = 0; i < kPerA; ++i) off_a[i] = offset_a(i, lane, kSB);
 #pragma unroll
-    for (int i = 0; i < kPerB; ++i) {
-        if (kQ4) {
-            const int q = min((ub0 + i * kWaves) * 64 + lane, kTN * kSB - 1);
-            const int r = q / kSB, blk = q % kSB;
-            const uint32_t rowoff = static_cast<uint32_t>(min(n0 + r, out_dim - 1) - n0) * static_cast<uint32_t>(kb_full) * 16u;
-            off_b[i][0] = rowoff + blk * 16;
-            off_b[i][1] = rowoff + min(blk, last_blocks - 1) * 16;
-            lds_b4[i][0] = S::chunk_pos(r, 2 * blk);
-            lds_b4[i][1] = S::chunk_pos(r, 2 * blk + 1);
-        } else {
-            const int r = min((ub0 + i * kWaves) * kRPL + dma_r, kTN - 1);
-            const int c = dma_slot ^ ((r / S::kRowsPerWrap) % kCPR);
-            const uint32_t rowoff = static_cast<uint32_t>(min(n0 + r, out_dim - 1) - n0) * static_cast<uint32_t>(kb_full) * 32u;
-            off_b[i][0] = rowoff + c * 16;
-            off_b[i][1] = rowoff + dma_chunk_last(c) * 16;
-            lds_b4[i][0] = lds_b4[i][1] = 0;
-        }
-    }
+    for (int i = 0; i < kPerB; ++i) off_b[i] = offset_b(i, lane, kSB);
 #pragma unroll
-    for (int i = 0; i < kPerSx; ++i) {
-        const int q = min((usx0 + i * kWaves) * 64 + lane, kTM * kSB - 1);
-        const int r = q / kSB, blk = q % kSB;
-        const uint32_t rowoff = static_cast<uint32_t>(min(m0 + r, rows - 1) - m0) * static_cast<uint32_t>(kb_full);
-        off_sx[i][0] = (rowoff + blk) * 4;
-        off_sx[i][1] = (rowoff + min(blk, last_blocks - 1)) * 4;
-    }
+    for (int i = 0; i < kPerSx; ++i) off_sx[i] = offset_sx(i, lane, kSB);
 #pragma unroll
-    for (int i = 0; i < kPerSw; ++i) {
-        const int q = min((usw0 + i * kWaves) * 64 + lane, kTN * kSB - 1);
-        const int r = q / kSB, blk = q % kSB;
-        const uint32_t rowoff = static_cast<uint32_t>(min(n0 + r, out_dim - 1) - n0) * static_cast<uint32_t>(kb_full);
-        off_sw[i][0] = (rowoff + blk) * 2;
-        off_sw[i][1] = (rowoff + min(blk, last_blocks - 1)) * 2;
-    }
+    for (int i = 0; i < kPerSw; ++i) off_sw[i] = offset_sw(i, lane, kSB);
 
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(gemm_lds)));
-    constexpr int kOffB = S::kABytes, kOffSx = kOffB + S::kBBytes, kOffSw = kOffSx + S::kSxBytes, kOffRaw = kOffSw + S::kSwBytes;
+    constexpr int kOffB = S::kABytes, kOffSx = kOffB + S::kBBytes, kOffSw = kOffSx + S::kSxBytes;
     auto stage_ptr = [&](int slot) { return gemm_lds + slot * S::kStageBytes; };
 
     // Issues every load of stage `st` (clamped to the last stage) towards ring slot `slot`.
     auto issue_loads = [&](int slot, int st) {
         const int se = min(st, stages - 1);
-        const int sel = se == stages - 1 ? 1 : 0;
         const uint32_t sp = lds_base + slot * S::kStageBytes;
+        auto issue = [&](auto&& at_a, auto&& at_b, auto&& at_sx, auto&& at_sw) {
 #pragma unroll
-        for (int i = 0; i < kPerA; ++i) {
-            const int u = ua0 + i * kWaves;
-            if (u < kUnitsA) lds_load16(a_base + static_cast<size_t>(se) * (kSB * 32), off_a[i][sel], sp + u * 1024);
-        }
-#pragma unroll
-        for (int i = 0; i < kPerB; ++i) {
-            const int u = ub0 + i * kWaves;
-            if (u < kUnitsB)
-                lds_load16(b_base + static_cast<size_t>(se) * (kSB * kQuantBytes), off_b[i][sel],
-                           sp + (kQ4 ? kOffRaw + u * 1024 : kOffB + u * 1024));
-        }
-#pragma unroll
-        for (int i = 0; i < kPerSx; ++i) {
-            const int u = usx0 + i * kWaves;
-            if (u < kUnitsSx) lds_load4(sx_base + static_cast<size_t>(se) * (kSB * 4), off_sx[i][sel], sp + kOffSx + u * 256);
-        }
-#pragma unroll
-        for (int i = 0; i < kPerSw; ++i) {
-            const int u = usw0 + i * kWaves;
-            if (u < kUnitsSw) lds_load2(sw_base + static_cast<size_t>(se) * (kSB * 2), off_sw[i][sel], sp + kOffSw + u * 256);
-        }
-    };
-
-    // Q4_0: expands the nibble chunks this wavefront fetched for ring slot `slot` into
-    // int8 fragments (its own loads have landed: no other wavefront is involved).
-    auto expand_q4 = [&](int slot) {
-        if (!kQ4) return;
-        unsigned char* sp = stage_ptr(slot);
-        const int4* raw = reinterpret_cast<const int4*>(sp + kOffRaw);
-        int4* bs = reinterpret_cast<int4*>(sp + kOffB);
-#pragma unroll
-        for (int i = 0; i < kPerB; ++i) {
-            const int u = ub0 + i * kWaves;
-            if (u < kUnitsB) {
-                const int4 r = raw[u * 64 + lane];
-                const uint32_t p[4] = {static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y), static_cast<uint32_t>(r.z), static_cast<uint32_t>(r.w)};
-                int v[8];
-                unpack_q4(p, v);  // low nibbles = values 0..15 (half 0), high nibbles = 16..31 (half 1)
-                bs[lds_b4[i][0]] = make_int4(v[0], v[1], v[2], v[3]);
-                bs[lds_b4[i][1]] = make_int4(v[4], v[5], v[6], v[7]);
+            for (int i = 0; i < kPerA; ++i) {
+                const int u = ua0 + i * kWaves;
+                if (u < kUnitsA) lds_load16(a_base + static_cast<size_t>(se) * (kSB * 32), at_a(i), sp + u * 1024);
             }
+#pragma unroll
+            for (int i = 0; i < kPerB; ++i) {
+                const int u = ub0 + i * kWaves;
+                if (u < kUnitsB) lds_load16(b_base + static_cast<size_t>(se) * (kSB * kQuantBytes), at_b(i), sp + kOffB + u * 1024);
+            }
+#pragma unroll
+            for (int i = 0; i < kPerSx; ++i) {
+                const int u = usx0 + i * kWaves;
+                if (u < kUnitsSx) lds_load4(sx_base + static_cast<size_t>(se) * (kSB * 4), at_sx(i), sp + kOffSx + u * 256);
+            }
+#pragma unroll
+            for (int i = 0; i < kPerSw; ++i) {
+                const int u = usw0 + i * kWaves;
+                if (u < kUnitsSw) lds_load2(sw_base + static_cast<size_t>(se) * (kSB * 2), at_sw(i), sp + kOffSw + u * 256);
+            }
+        };
+        if (se == stages - 1 && last_blocks < kSB) {  // the last stage's own offsets: kept beside the others, they cost registers
+            int l = lane;
+            asm volatile("" : "+v"(l));
+            issue([&](int i) { return offset_a(i, l, last_blocks); }, [&](int i) { return offset_b(i, l, last_blocks); },
+                  [&](int i) { return offset_sx(i, l, last_blocks); }, [&](int i) { return offset_sw(i, l, last_blocks); });
+        } else {
+            issue([&](int i) { return off_a[i]; }, [&](int i) { return off_b[i]; }, [&](int i) { return off_sx[i]; },
+                  [&](int i) { return off_sw[i]; });
         }
     };
 
-    // this lane's fragment positions (loop-invariant; only the ring slot changes)
-    const int row = wm * 32 + lj;  // activation row (A operand) inside the tile
-    const int col = wn * 32 + lj;  // weight column (B operand) inside the tile
-    const int b0 = 2 * ks;         // first block of this wavefront's pair inside a stage
+    // this lane's fragment positions (loop-invariant; only the ring slot changes).  Tile (i, j) of the wavefront lies 32 i rows
+    // and 32 j columns on, a whole number of swizzle periods.
+    const int row = wm * (32 * kPerM) + lj;  // activation row (A operand) inside the tile
+    const int col = wn * (32 * kPerN) + lj;  // weight column (B operand) inside the tile
+    const int b0 = 2 * ks;                   // first block of this wavefront's pair inside a stage
     const int frag_a0 = S::chunk_pos(row, 2 * b0 + lh), frag_a1 = S::chunk_pos(row, 2 * b0 + 2 + lh);
-    const int frag_b0 = S::chunk_pos(col, 2 * b0 + lh), frag_b1 = S::chunk_pos(col, 2 * b0 + 2 + lh);
+    const int frag_b0 = kQ4 ? col * kSB + nibble_slot(col, b0) : S::chunk_pos(col, 2 * b0 + lh);
+    const int frag_b1 = kQ4 ? col * kSB + nibble_slot(col, b0 + 1) : S::chunk_pos(col, 2 * b0 + 2 + lh);
     const int frag_sx = row * kSB + b0 + lh;  // lanes 0-31 carry block b0, lanes 32-63 block b0 + 1
     const int frag_sw = col * kSB + b0 + lh;
+    const int nibble_shift = lh ? 0 : 4;  // Q4_0: values 0..15 of a block are the low nibbles
 
-    v16f acc = {};
+    v16f acc[kPerM][kPerN] = {};
 
     // MFMA operands of one stage as read from LDS (scales still raw)
     struct Frag {
-        int4 a0, a1, w0, w1;
-        float ta;
-        uint32_t tb;  // fp16 bits
+        int4 a0[kPerM], a1[kPerM], w0[kPerN], w1[kPerN];
+        float ta[kPerM];
+        uint32_t tb[kPerN];  // fp16 bits
     };
     auto read_frag = [&](int slot, Frag& f) {
         const unsigned char* sp = stage_ptr(slot);
         const int4* as = reinterpret_cast<const int4*>(sp);
         const int4* bs = reinterpret_cast<const int4*>(sp + kOffB);
-        f.a0 = as[frag_a0];
-        f.a1 = as[frag_a1];
-        f.w0 = bs[frag_b0];
-        f.w1 = bs[frag_b1];
-        f.ta = reinterpret_cast<const float*>(sp + kOffSx)[frag_sx];
-        f.tb = reinterpret_cast<const uint32_t*>(sp + kOffSw)[frag_sw];
+        constexpr int kStepA = 32 * kCPR, kStepB = 32 * (kQ4 ? kSB : kCPR);
+#pragma unroll
+        for (int i = 0; i < kPerM; ++i) {
+            f.a0[i] = as[frag_a0 + i * kStepA];
+            f.a1[i] = as[frag_a1 + i * kStepA];
+            f.ta[i] = reinterpret_cast<const float*>(sp + kOffSx)[frag_sx + i * 32 * kSB];
+        }
+#pragma unroll
+        for (int j = 0; j < kPerN; ++j) {
+            f.w0[j] = bs[frag_b0 + j * kStepB];
+            f.w1[j] = bs[frag_b1 + j * kStepB];
+            f.tb[j] = reinterpret_cast<const uint32_t*>(sp + kOffSw)[frag_sw + j * 32 * kSB];
+        }
+    };
+    // Q4_0: sixteen times the value, nibble n as the byte 16 (n - 8); the scale takes the sixteenth back, so that every
+    // product with the scale is the one of the plain value
+    auto weight_bytes = [&](const int4& w) {
+        if (!kQ4) return v4i{w.x, w.y, w.z, w.w};
+        v4i v = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            v[i] = static_cast<int>(((static_cast<uint32_t>(v[i]) << nibble_shift) & 0xF0F0F0F0u) ^ 0x80808080u);
+        return v;
     };
     // One pair of blocks, first block `blk` (absolute index): MFMAs of block blk and of
     // the scale products, vector-ALU work of block blk, then the same for block blk + 1 in
@@ -340,40 +339,55 @@ __device__ __forceinline__ void gemm_i8_body(
     auto pair_step = [&](const Frag& f, int blk, auto&& between) {
         // blocks past the end of K (clamped re-reads of the last block) get scale 0
         const bool live = blk + lh < kb;
-        const float ta = live ? f.ta : 0.0f;
-        const float tb = live ? half_bits_to_f32(static_cast<uint16_t>(f.tb)) : 0.0f;
-        const v4i a0 = {f.a0.x, f.a0.y, f.a0.z, f.a0.w}, a1 = {f.a1.x, f.a1.y, f.a1.z, f.a1.w};
-        const v4i w0 = {f.w0.x, f.w0.y, f.w0.z, f.w0.w}, w1 = {f.w1.x, f.w1.y, f.w1.z, f.w1.w};
         const v16i zi = {};
         const v32f zf = {};
-        const int n = n0 + col;
-        v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, w0, zi, 0, 0, 0);
-        v32f t = __builtin_amdgcn_mfma_f32_32x32x1f32(ta, tb, zf, 0, 0, 0);
+        v4i w0[kPerN], w1[kPerN], a0[kPerM], a1[kPerM];
+        float tb[kPerN], ta[kPerM];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (kWriteDots && blk + h < kb) {
+        for (int j = 0; j < kPerN; ++j) {
+            w0[j] = weight_bytes(f.w0[j]);
+            w1[j] = weight_bytes(f.w1[j]);
+            tb[j] = live ? half_bits_to_f32(static_cast<uint16_t>(f.tb[j])) * (kQ4 ? 0.0625f : 1.0f) : 0.0f;
+        }
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int m = m0 + wm * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                    if (m < rows && n < out_dim) dots[(static_cast<size_t>(m) * out_dim + n) * kb_full + blk_begin + blk + h] = c[v];
+        for (int i = 0; i < kPerM; ++i) {
+            if (i == 0) {
+#pragma unroll
+                for (int i2 = 0; i2 < kPerM; ++i2) {
+                    ta[i2] = live ? f.ta[i2] : 0.0f;
+                    a0[i2] = v4i{f.a0[i2].x, f.a0[i2].y, f.a0[i2].z, f.a0[i2].w};
+                    a1[i2] = v4i{f.a1[i2].x, f.a1[i2].y, f.a1[i2].z, f.a1[i2].w};
                 }
             }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] = __builtin_fmaf(t[16 * h + v], static_cast<float>(c[v]), acc[v]);
-            if (h == 0) {
-                // compiler fence (no instruction): block blk is finished before block blk + 1 starts
-                asm volatile("" : "+v"(acc), "+v"(t) : : "memory");
-                c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zi, 0, 0, 0);
-                between();
+            for (int j = 0; j < kPerN; ++j) {
+                const int n = n0 + col + 32 * j;
+                v16f& sum = acc[i][j];
+                v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[i], w0[j], zi, 0, 0, 0);
+                v32f t = __builtin_amdgcn_mfma_f32_32x32x1f32(ta[i], tb[j], zf, 0, 0, 0);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (kWriteDots && blk + h < kb) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const int m = m0 + row - lj + 32 * i + 8 * (v >> 2) + 4 * lh + (v & 3);
+                            if (m < rows && n < out_dim) dots[(static_cast<size_t>(m) * out_dim + n) * kb_full + blk_begin + blk + h] = kQ4 ? c[v] >> 4 : c[v];
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sum[v] = __builtin_fmaf(t[16 * h + v], static_cast<float>(c[v]), sum[v]);
+                    if (h == 0) {
+                        // compiler fence (no instruction): block blk is finished before block blk + 1 starts
+                        asm volatile("" : "+v"(sum), "+v"(t) : : "memory");
+                        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[i], w1[j], zi, 0, 0, 0);
+                        if (i == kPerM - 1 && j == kPerN - 1) between();
+                    }
+                }
+                asm volatile("" : "+v"(sum) : : "memory");
             }
         }
     };
-    // Program-order fence for the compiler (it emits no instruction): a stage's arithmetic
-    // is emitted before it.  Without it the optimizer gathers the MFMAs of several stages
-    // in one place and spills their results.
-    auto pin_acc = [&]() { asm volatile("" : "+v"(acc) : : "memory"); };
-
-    uint64_t stamp_begin = 0, stamp_loop = 0, stamp_tail = 0, ref_loop = 0, ref_tail = 0, stamp_wait = 0, stamp_barrier = 0;
+    uint64_t stamp_begin = 0, stamp_loop = 0, stamp_tail = 0, ref_loop = 0, retail = 0, stamp_wait = 0, stamp_barrier = 0;
     if (kStamps) stamp_begin = __builtin_readcyclecounter();
     // ---- prologue: stages 0 .. kRing-2 in flight, stages 0 and 1 landed, stage 0 in registers
     static_assert(kRing == 4, "the loop reads stage st + 1 while stage st + 2 lands and stage st + 3 is issued");
@@ -382,8 +396,6 @@ __device__ __forceinline__ void gemm_i8_body(
     // Loads complete in order: a stage has landed for this wavefront once at most the
     // loads of the stages issued after it are outstanding.
     wait_vm_outstanding(loads_per_stage);
-    expand_q4(0);
-    expand_q4(1);
     __syncthreads();
     {
         // The next stage's operands are read from LDS while this stage's arithmetic runs.
@@ -401,13 +413,11 @@ __device__ __forceinline__ void gemm_i8_body(
                 issue_loads((d + kRing - 1) % kRing, st + kRing - 1);
                 // the next stage's operands landed before the last barrier
                 pair_step(frag[d & 1], st * kSB + b0, [&]() { read_frag((d + 1) % kRing, frag[(d + 1) & 1]); });
-                pin_acc();
                 // stage st + 2 (issued two stages ago) has to be complete before the barrier:
                 // the next stage reads its operands
                 uint64_t s0 = 0, s1 = 0;
                 if (kStamps) s0 = __builtin_readcyclecounter();
                 wait_vm_outstanding(loads_per_stage);
-                expand_q4((d + 2) % kRing);
                 if (kStamps) s1 = __builtin_readcyclecounter();
                 __syncthreads();
                 if (kStamps) {
@@ -419,29 +429,32 @@ __device__ __forceinline__ void gemm_i8_body(
     }
     if (kStamps) {
         stamp_tail = __builtin_readcyclecounter();
-        ref_tail = __builtin_amdgcn_s_memrealtime();
+        retail = __builtin_amdgcn_s_memrealtime();
     }
 
     // Loads still in flight target ring slots nobody reads again; they must land before
     // the ring is reused for the reduction (and before the workgroup ends).
     wait_vm_outstanding(0);
-    const int n = n0 + col;
+    constexpr int kPerWave = kPerM * kPerN;
     if (kSplit > 1) {
         // ---- the kSplit partial sums of a tile meet in LDS
         __syncthreads();
-        float* red = reinterpret_cast<float*>(gemm_lds);  // [ks][tile][v][lane]
+        float* red = reinterpret_cast<float*>(gemm_lds);  // [ks][tile][tile of the wavefront][v][lane]
 #pragma unroll
-        for (int v = 0; v < 16; ++v) red[((ks * S::kTiles + tile) * 16 + v) * 64 + lane] = acc[v];
+        for (int p = 0; p < kPerWave; ++p)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                red[(((ks * S::kTiles + tile) * kPerWave + p) * 16 + v) * 64 + lane] = acc[p / kPerN][p % kPerN][v];
         __syncthreads();
         if (dst == nullptr) return;
         constexpr int kPer = 16 / kSplit;
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int v = ks * kPer + j;
-            float sum = red[(tile * 16 + v) * 64 + lane];
+        for (int j = 0; j < kPer * kPerWave; ++j) {
+            const int p = j / kPer, v = ks * kPer + j % kPer;
+            float sum = red[((tile * kPerWave + p) * 16 + v) * 64 + lane];
 #pragma unroll
-            for (int k2 = 1; k2 < kSplit; ++k2) sum += red[((k2 * S::kTiles + tile) * 16 + v) * 64 + lane];
-            const int m = m0 + wm * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+            for (int k2 = 1; k2 < kSplit; ++k2) sum += red[(((k2 * S::kTiles + tile) * kPerWave + p) * 16 + v) * 64 + lane];
+            const int m = m0 + row - lj + 32 * (p / kPerN) + 8 * (v >> 2) + 4 * lh + (v & 3), n = n0 + col + 32 * (p % kPerN);
             if (kStamps) {
                 asm volatile("" : : "v"(sum));  // the sum is formed, not stored
             } else if (m < rows && n < out_dim) {
@@ -457,7 +470,7 @@ __device__ __forceinline__ void gemm_i8_body(
             out[1] = static_cast<int>(stamp_tail - stamp_loop);
             out[2] = static_cast<int>(stamp_wait);
             out[3] = static_cast<int>(stamp_barrier);
-            out[4] = static_cast<int>(ref_tail - ref_loop);
+            out[4] = static_cast<int>(retail - ref_loop);
             out[5] = static_cast<int>(stamp_end - stamp_tail);
             out[6] = 0;
             out[7] = static_cast<int>(__builtin_amdgcn_s_getreg((31 << 11) | 4));
@@ -465,27 +478,54 @@ __device__ __forceinline__ void gemm_i8_body(
     } else {
         if (dst == nullptr) return;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int m = m0 + wm * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+        for (int j = 0; j < 16 * kPerWave; ++j) {
+            const int p = j / 16, v = j % 16;
+            const int m = m0 + row - lj + 32 * (p / kPerN) + 8 * (v >> 2) + 4 * lh + (v & 3), n = n0 + col + 32 * (p % kPerN);
             if (m < rows && n < out_dim) {
                 const size_t at = static_cast<size_t>(m) * out_dim + n;
-                if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = acc[v];
-                else dst[at] = finish_output(ep, n, at, acc[v]);
+                const float sum = acc[p / kPerN][p % kPerN][v];
+                if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
+                else dst[at] = finish_output(ep, n, at, sum);
             }
         }
     }
 }
 
-template <int kType, int kWavesM, int kWavesN, int kSplit, bool kWriteDots, bool kShareK = false, bool kStamps = false>
+template <int kType, int kWavesM, int kWavesN, int kSplit, bool kWriteDots, bool kShareK = false, bool kStamps = false, int kPerM = 1,
+          int kPerN = 1>
 __global__ __launch_bounds__(64 * kWavesM * kWavesN * kSplit) void gemm_i8_kernel(
     float* __restrict__ dst, int* __restrict__ dots, const int8_t* __restrict__ qx, const float* __restrict__ sx,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_tiles, int n_tiles,
     int share_blocks, float* __restrict__ partial, Epilogue ep) {
-    gemm_i8_body<kType, kWavesM, kWavesN, kSplit, kWriteDots, kShareK, kStamps>(dst, dots, qx, sx, weight, rows, in_dim, out_dim,
-                                                                                 m_tiles, n_tiles, share_blocks, partial, ep);
+    gemm_i8_body<kType, kWavesM, kWavesN, kSplit, kWriteDots, kShareK, kStamps, kPerM, kPerN>(
+        dst, dots, qx, sx, weight, rows, in_dim, out_dim, m_tiles, n_tiles, share_blocks, partial, ep);
 }
 
 namespace {
+
+// Grids that fill the compute units: f32 results of whole K only (no shares, no block dots).
+template <int kType, int kWavesM, int kWavesN, int kSplit, int kPerM, int kPerN>
+hipError_t launch_wide_tile(hipStream_t stream, float* dst, const int8_t* qx, const float* sx, const uint8_t* weight, int rows,
+                            int in_dim, int out_dim, const Epilogue& ep) {
+    using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2, kPerM, kPerN>;
+    const int m_tiles = (rows + S::kTM - 1) / S::kTM, n_tiles = (out_dim + S::kTN - 1) / S::kTN;
+    const long long grid = static_cast<long long>((n_tiles + 7) / 8) * m_tiles * 8;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    // per-lane load offsets are 32-bit, relative to the workgroup's first row
+    if (static_cast<long long>(S::kTM > S::kTN ? S::kTM : S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
+    auto kernel = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false, false, false, kPerM, kPerN>;
+    static std::atomic<bool> attr_done{false};
+    if (!attr_done.load(std::memory_order_acquire)) {
+        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               S::kLdsBytes);
+            e != hipSuccess)
+            return e;
+        attr_done.store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(S::kThreads), S::kLdsBytes, stream, dst, nullptr, qx, sx, weight,
+                       rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, ep);
+    return hipGetLastError();
+}
 
 template <int kType, int kWavesM, int kWavesN, int kSplit>
 hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
@@ -539,11 +579,38 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
 template <int kType>
 hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
                        const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial) {
-    // 64 x 128 tiles while they still give every CU a workgroup, 32 x 64 with a deeper K split otherwise
-    const long long big = static_cast<long long>((rows + 63) / 64) * ((out_dim + 127) / 128);
-    static const char* force = std::getenv("AFHIP_GEMM_TILE");  // tuning: "L" = 64x128, "S" = 32x64
-    const bool use_big = force ? force[0] != 'S' : big >= 256;
-    if (use_big) return launch_tile<kType, 2, 4, 2>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial);
+    // us of the whole op, M x K x N; "before" is the 64 x 128 tile by sixteen wavefronts that served these grids.
+    static const char* env_tile = std::getenv("AFHIP_GEMM_TILE");  // tuning: "S", "Y", "X" or "V", see below
+    const char force = dots == nullptr && env_tile ? env_tile[0] : '\0';
+    const long long units = gemv_compute_units();
+    const long long grid = static_cast<long long>((rows + 63) / 64) * ((out_dim + 127) / 128);
+    char tile = 'S';  // 32 x 64 outputs, K in four
+    if (kType == 2) {
+        // Q4_0.  "S" and "X" (64 x 128 outputs, two tiles a wavefront) both leave room for a second workgroup on a compute
+        // unit.  "X" moves less per output but its few workgroups leave units idle on a small grid: 333 x 2048 x 5632
+        // 26.9 / 35.0 (44.4 before), 333 x 4096 x 6144 51.5 / 60.4 (77.7), even at 11/8 of the units (512 x 2048 x 5632 37.4 / 37.0,
+        // 45.7), 777 x 4096 x 4096 74 / 67 (84), 2048 x 4096 x 14336 498 / 398 (513).
+        if (grid * 8 >= units * 11) tile = 'X';
+    } else if (grid >= units) {
+        // Q8_0, whose 64 x 128 stage does not fit twice: "Y" (64 x 64 outputs, two workgroups a unit) or "V" (128 x 128, two tiles
+        // a wavefront, one workgroup a unit), whichever the grid's rounds make shorter.  A round takes about (K = 4096, us) "V" 62,
+        // "Y" 37 with two workgroups on a unit and 27 with one: 333 x 4096 x 6144 52 / 56 (65 before), 512 x 4096 x 4096 40 / 57 (40),
+        // 512 x 4096 x 14336 121 / 122 (136), 777 x 4096 x 14336 201 / 224 (200), 2048 x 4096 x 14336 459 / 389 (434).
+        const long long wide = static_cast<long long>((rows + 127) / 128) * ((out_dim + 127) / 128);
+        const long long square = static_cast<long long>((rows + 63) / 64) * ((out_dim + 63) / 64);
+        const long long rest = square % (2 * units);
+        const long long square_us = square / (2 * units) * 37 + (rest == 0 ? 0 : rest <= units ? 27 : 37);
+        tile = (wide + units - 1) / units * 62 < square_us ? 'V' : 'Y';
+    }
+    if (force != '\0') tile = force;
+    if (dots == nullptr) {
+        if constexpr (kType == 2) {
+            if (tile == 'X') return launch_wide_tile<2, 1, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
+        } else {
+            if (tile == 'V') return launch_wide_tile<8, 2, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
+            if (tile == 'Y') return launch_wide_tile<8, 2, 2, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
+        }
+    }
     return launch_tile<kType, 1, 2, 4>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial);
 }
 
@@ -586,16 +653,16 @@ hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* par
     return hipGetLastError();
 }
 
-// Diagnostic: the Q8_0 64 x 128 tile kernel with its clock readings in place of results (see kStamps); dst has to
+// Diagnostic: the Q8_0 64 x 64 tile kernel with its clock readings in place of results (see kStamps); dst has to
 // hold 8 ints per wavefront of the grid, which it does whenever it holds the rows x out_dim results.
 hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* qx, const float* sx, const uint8_t* weight,
                                  int rows, int in_dim, int out_dim) {
-    using S = GemmShape<2, 4, 2, false>;
+    using S = GemmShape<2, 2, 2, false>;
     const int m_tiles = (rows + S::kTM - 1) / S::kTM, n_tiles = (out_dim + S::kTN - 1) / S::kTN;
     const long long grid = static_cast<long long>((n_tiles + 7) / 8) * m_tiles * 8;
     if (grid > 0x7fffffffLL || static_cast<long long>(S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
     if (static_cast<long long>(rows) * out_dim < grid * S::kWaves * 8) return hipErrorInvalidValue;
-    auto kernel = gemm_i8_kernel<8, 2, 4, 2, false, false, true>;
+    auto kernel = gemm_i8_kernel<8, 2, 2, 2, false, false, true>;
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            S::kLdsBytes);
         e != hipSuccess)

@@ -377,7 +377,7 @@ def main() -> int:
         ops = 2.0 * m * k * n
         return {"bound": "int8_mfma", "achieved": round(ops / t_op / 1e12, 2), "peak": INT8_MFMA_PEAK_OPS / 1e12,
                 "unit": "TOP/s", "frac": round(ops / t_op / INT8_MFMA_PEAK_OPS, 4),
-                "kernel": "quantize_activations_kernel + gemm_i8_kernel<Q8_0> (64 x 128 tiles)",
+                "kernel": "quantize_activations_kernel + gemm_i8_kernel<Q8_0> (64 x 64 tiles)",
                 "workload": f"Q8_0 prefill GEMM, x f32 [{m}x{k}] quantized on the GPU, W [{n}x{k}] 34-byte blocks",
                 "ops_per_launch": ops, "us_per_op": round(t_op * 1e6, 3), "us_quantizer": round(t_quant * 1e6, 3),
                 "us_kernel_by_subtraction": round(t_kernel * 1e6, 3),
@@ -560,10 +560,10 @@ def main() -> int:
             if rc != 0:
                 raise RuntimeError(f"gemm stamps failed: {rc}")
         torch.cuda.synchronize()
-        groups = ((n + 127) // 128 + 7) // 8 * ((m + 63) // 64) * 8
-        st = y.cpu().numpy().reshape(-1).view(np.int32)[: groups * 16 * 8].reshape(groups, 16, 8).astype(np.int64)
+        groups = ((n + 63) // 64 + 7) // 8 * ((m + 63) // 64) * 8
+        st = y.cpu().numpy().reshape(-1).view(np.int32)[: groups * 8 * 8].reshape(groups, 8, 8).astype(np.int64)
         ghz = float(np.median(st[:, :, 1] / (st[:, :, 4] / 100e6))) / 1e9
-        print(f"Q8_0 prefill kernel, M={m}, K={k}, N={n}: {groups} workgroups x 16 wavefronts, launch {launches} of {launches} back to back")
+        print(f"Q8_0 prefill kernel, M={m}, K={k}, N={n}: {groups} workgroups x 8 wavefronts, launch {launches} of {launches} back to back")
         print(f"clock held in the K loop: {ghz:.3f} GHz (loop cycles / 100 MHz reference ticks, median over wavefronts)")
         print("| per wavefront, shader-clock cycles | median | min | max |")
         print("|---|---|---|---|")
@@ -573,7 +573,7 @@ def main() -> int:
             print(f"| {name} | {int(np.median(v))} | {v.min()} | {v.max()} |")
         print("| wavefront of the workgroup (launch order = age on its SIMD) | K loop | waiting at barriers |")
         print("|---|---|---|")
-        for wv in range(16):
+        for wv in range(8):
             print(f"| {wv} | {int(np.median(st[:, wv, 1]))} | {int(np.median(st[:, wv, 3]))} |")
         tile_blocks = (m // 32) * (n // 32) * (k // 32) / (groups * 4)  # per SIMD
         print(f"tile-blocks (32 x 32 outputs x one 32-value block) per SIMD: {tile_blocks:.0f}; loop cycles per tile-block and SIMD: "

@@ -652,10 +652,10 @@ afhip_status afhip_launch_rows8_timeline(void *stream, size_t rows, afhip_buffer
  * wide matrix take the 32-row MFMA kernel on 64-column tiles; negative restores the default (one workgroup per
  * compute unit), 0 switches that kernel off.  Tests lift the bound to reach the kernel's K shares and pair launches. */
 afhip_status afhip_tune_batch32_max_workgroups(long bound);
-/* Diagnostic with no counterpart in the reference: the Q8_0 prefill kernel (64 x 128 tiles) on activations
+/* Diagnostic with no counterpart in the reference: the Q8_0 prefill kernel (64 x 64 tiles) on activations
  * already quantized by afhip_launch_quantize_activations, computing as usual but storing, instead of results,
  * eight 32-bit counts per wavefront over the start of `stamps` (which has to hold rows x out_dim floats):
- * [8 * (workgroup * 16 + wavefront)] = shader-clock cycles before the K loop, in it, waiting for the wavefront's
+ * [8 * (workgroup * 8 + wavefront)] = shader-clock cycles before the K loop, in it, waiting for the wavefront's
  * own loads, waiting at the workgroup barrier, 100 MHz reference ticks in the loop, cycles after the loop, 0, HW_ID.
  * `bench.py --probe gemm` prints them. */
 afhip_status afhip_launch_gemm_stamps(void *stream, afhip_buffer stamps, afhip_buffer q, afhip_buffer scales,

@@ -182,6 +182,18 @@ def test_block_dots_bit_exact_and_outputs_within_tolerance(fmt, layout, rows, in
     assert G.max_rel_err(y, y64) <= TIGHT
 
 
+@pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(700, 96, 4097), (1100, 544, 3800), (129, 160, 16385), (257, 672, 10921)])
+def test_prefill_grids_past_the_compute_units(fmt, rows, in_dim, out_dim):
+    """Grids that take the 64 x 128 (Q4_0), 64 x 64 and 128 x 128 (Q8_0) tiles: row and column remainders, K shorter than a stage
+    of four blocks' ring and ending one to three blocks into a stage; f32 sums in another order (TIGHT)."""
+    print(f"case: large prefill fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(rows + in_dim, rows, in_dim)
+    w = synth.weights(fmt, out_dim + 1, out_dim, in_dim)
+    y = G.linear(fmt, PREP, x, G.prepare(fmt, w, out_dim, in_dim), rows, in_dim, out_dim)
+    assert G.max_rel_err(y, O.linear_act_f64(fmt, x, w, rows, in_dim, out_dim)) <= TIGHT
+
+
 SHAPES_B = [(1, 32, 3), (2, 64, 600), (3, 96, 11), (4, 4096, 100), (1, 64, 4096), (12, 128, 40)]
 
 

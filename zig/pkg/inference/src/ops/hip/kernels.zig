@@ -316,7 +316,7 @@ pub const KernelModule = struct {
         const n_tiles = (out_dim + tile_n - 1) / tile_n;
         const grid = try checkedMul(try checkedMul((n_tiles + 7) / 8, m_tiles), 8);
         // four stages of operands: 27648 bytes each, and 8192 more for Q4_0's nibble chunks
-        const lds: usize = if (tensor_type == .q4_0) 143360 else 110592;
+        const lds: usize = if (tensor_type == .q4_0) 77824 else 110592;
         var dst_ptr = dst.ptr;
         var input_ptr = input.ptr;
         var weight_ptr = weight_prepared.ptr;
