@@ -110,22 +110,20 @@ static int env_int(const char* name) {
 // Whether the single-shot MFMA kernel serves this shape (measured against the kernels it replaces;
 // AFHIP_BATCH_MFMA_MIN_ROWS overrides the lower row bound for tuning runs, 0 switches the kernel off):
 // from five rows on (six on a K longer than 4096, where the split-K GEMV still wins at five) up to 64
-// (128 on wide Q4_0 matrices), and for Q8_0, whose K shares are half as long, only while all workgroups
+// (96 on some Q4_0 matrices), and for Q8_0, whose K shares are half as long, only while all workgroups
 // of the launch are resident at once.  Five to eight rows (Q8_0: sixteen) on a K of whole 256-value runs always:
 // the eight-row kernel requests weights as it goes and needs neither condition.  Two to four rows where measured
 // faster than the decode kernels (the rules below).
 static bool batch_mfma_preferred(int tensor_type, size_t rows, size_t in_dim, size_t out_dim, bool pair) {
     static const char* v = std::getenv("AFHIP_BATCH_MFMA_MIN_ROWS");
     static const long forced = v && *v ? std::atol(v) : -1;
-    // up to 64 rows everywhere; up to 128 on a Q4_0 matrix wide enough to give every compute unit a
-    // column tile (there the tiled GEMM, whose 64 x 128 workgroup tiles re-read X per tile, is slower)
-    // ... and where the tiled GEMM's grid of 32 x 64 tiles would not fit the compute units in one round while its
-    // 64 x 128 tiles leave most of them idle (65 .. 128 rows on 4608 .. 8160 columns: 128 rows x 4608 columns 31.5 -> 24.1 us,
-    // 65 rows x 6144 columns 31.0 -> 19.9, 100 rows of K = 8192 x 6144 columns 56.6 -> 43.8; one round of the GEMM stays
-    // faster: 128 rows x 4096 columns 17.8 against 21.2, 96 rows x 5120 columns 17.7 against 20.1)
+    // up to 64 rows everywhere; 65 .. 96 of Q4_0 on a K around 4096 where the GEMM's grid of 32 x 64 tiles just passes one
+    // workgroup a compute unit while this kernel's 32-column tiles still fit them in one round (96 rows x 6144 columns 20.6
+    // against 22.0 us, x 8192 21.7 / 22.9; the GEMM wins on 10240 columns 36.2 / 23.8, with K = 2048 x 7168 16.9 / 14.8,
+    // K = 8192 x 8192 41.0 / 38.4, and from 97 rows on: 128 x 6144 25.5 / 23.0, x 14336 47.6 / 41.3)
     const size_t units = static_cast<size_t>(gemv_compute_units());
-    const bool wide = (out_dim + 31) / 32 >= units || (rows + 31) / 32 * ((out_dim + 63) / 64) > units;
-    const size_t max_rows = tensor_type == AFHIP_TYPE_Q4_0 && wide ? 128 : 64;
+    const bool one_round = (out_dim + 31) / 32 <= units && (rows + 31) / 32 * ((out_dim + 63) / 64) > units;
+    const size_t max_rows = tensor_type == AFHIP_TYPE_Q4_0 && one_round && in_dim >= 3072 && in_dim <= 6144 ? 96 : 64;
     if (forced == 0 || rows > max_rows || !batch_mfma_supports(tensor_type, rows, in_dim, out_dim)) return false;
     if (forced > 0) return rows >= static_cast<size_t>(forced);
     if (rows >= kBatchMfmaMinRows && batch_mfma_eight_rows(tensor_type, rows, in_dim, out_dim)) return true;
