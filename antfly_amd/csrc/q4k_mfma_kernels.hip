@@ -744,22 +744,27 @@ __global__ __launch_bounds__(256) void q4k_split_rows_kernel(const float* __rest
     }
 }
 
-// Y[32 rows][256 columns] per workgroup, K walked one super-block at a time: the X chunk of the
-// next super-block travels global -> registers while the current one is computed from LDS,
-// then registers -> the other LDS buffer, one barrier per super-block.  A wavefront owns a
+// Y[32 rows][256 columns] per workgroup, K walked half a super-block at a time: the X chunk of the
+// next half travels global -> registers while the current one is computed from LDS,
+// then registers -> the other LDS buffer, one barrier per half.  A wavefront owns a
 // 32-column tile for all of K (no K split: nothing to combine).  Here the three parts of X lie
 // along K instead of along the MFMA rows: a sub-block is six chained MFMAs (part x half) into
 // one D of 32 real rows -- lane (row c, half g) supplies the same K values as in the GEMV
 // kernel, from part 0, 1, 2 in turn against the same B -- so a row costs two multiply-adds per
 // sub-block and the weights are converted once per 32 rows.  (A first version with the parts
 // along the rows, ten rows per MFMA pass and four passes, measured 12-28 % slower.)
+// Half super-blocks keep a workgroup at 55 KiB of LDS and 118 registers, so two of them share a compute unit: a SIMD has
+// four wavefronts to fill the matrix pipe (200 cycles per 32 x 32 outputs and sub-block) while others convert, accumulate or
+// wait at the other workgroup's barrier.  Whole super-blocks with the next sub-block's operands requested by hand took 105 KiB
+// and 186 registers, two wavefronts a SIMD, 520 cycles where this takes 440: 333 x 4096 x 14336 187 -> 158 us, 1024 x 4096 x 14336
+// 426 -> 369, 333 x 14336 x 4096 201 -> 181.
 constexpr int kG32Rows = 32;
-constexpr int kG32PartStride = 512 + 16;
+constexpr int kG32PartStride = 256 + 16;
 constexpr int kG32PartsBytes = kG32Rows * 3 * kG32PartStride;
 constexpr int kG32ChunkBytes = kG32PartsBytes + kG32Rows * 64;  // parts, then the parts of the sums: [row][part 0..3][sub-block] bf16
-constexpr int kG32Units = kG32Rows * 3 * 32;
+constexpr int kG32Units = kG32Rows * 3 * 16;
 
-__global__ __launch_bounds__(512) void gemm_q4k_rows32_kernel(float* __restrict__ dst, const uint32_t* __restrict__ parts,
+__global__ __launch_bounds__(512, 4) void gemm_q4k_rows32_kernel(float* __restrict__ dst, const uint32_t* __restrict__ parts,
                                                               const uint16_t* __restrict__ sum_parts, const uint8_t* __restrict__ weight,
                                                               int rows, int in_dim, int out_dim, int sb_per_split,
                                                               float* __restrict__ partial, Epilogue ep) {
@@ -779,42 +784,35 @@ __global__ __launch_bounds__(512) void gemm_q4k_rows32_kernel(float* __restrict_
     const uint8_t* tile_base = weight + static_cast<size_t>(tile) * kb * kTileBytes;
     const int groups_per_row = in_dim >> 3;
 
-    static_assert(kG32Units == 6 * 512, "six 16-byte units of the X chunk per thread");
-    // (six named registers, not an array: the array stayed in scratch memory across the two
-    // branches that fill and drain it)
-    uint4 stage0, stage1, stage2, stage3, stage4, stage5;
+    static_assert(kG32Units == 3 * 512, "three 16-byte units of the X chunk per thread");
+    // (named registers, not an array: an array stayed in scratch memory across the two branches that fill and drain it)
+    uint4 stage0, stage1, stage2;
     uint4 stage_sum = make_uint4(0u, 0u, 0u, 0u);
-    auto fetch_unit = [&](int i, int sb) {
+    auto fetch_unit = [&](int i, int h) {
         const int u = tid + i * 512;
-        const int rp = u >> 5, k16 = u & 31;
+        const int rp = u >> 4, k16 = u & 15;
         const int r = min(rp / 3, rows_here - 1), part = rp - (rp / 3) * 3;  // rows past the end repeat the last one
-        return reinterpret_cast<const uint4*>(parts)[(static_cast<size_t>(row0 + r) * 3 + part) * groups_per_row + sb * 32 + k16];
+        return reinterpret_cast<const uint4*>(parts)[(static_cast<size_t>(row0 + r) * 3 + part) * groups_per_row + h * 16 + k16];
     };
-    auto fetch = [&](int sb) {
-        stage0 = fetch_unit(0, sb);
-        stage1 = fetch_unit(1, sb);
-        stage2 = fetch_unit(2, sb);
-        stage3 = fetch_unit(3, sb);
-        stage4 = fetch_unit(4, sb);
-        stage5 = fetch_unit(5, sb);
-        if (tid < kG32Rows * 4) {  // 64 bytes of sum parts per row
+    auto fetch = [&](int h) {  // half super-block h; the sum parts (64 bytes per row) come with the second half
+        stage0 = fetch_unit(0, h);
+        stage1 = fetch_unit(1, h);
+        stage2 = fetch_unit(2, h);
+        if ((h & 1) && tid < kG32Rows * 4) {
             const int r = min(tid >> 2, rows_here - 1);
-            stage_sum = reinterpret_cast<const uint4*>(sum_parts)[(static_cast<size_t>(row0 + r) * kb + sb) * 4 + (tid & 3)];
+            stage_sum = reinterpret_cast<const uint4*>(sum_parts)[(static_cast<size_t>(row0 + r) * kb + (h >> 1)) * 4 + (tid & 3)];
         }
     };
     auto deposit_unit = [&](unsigned char* chunk, int i, const uint4& v) {
         const int u = tid + i * 512;
-        *reinterpret_cast<uint4*>(chunk + (u >> 5) * kG32PartStride + (u & 31) * 16) = v;
+        *reinterpret_cast<uint4*>(chunk + (u >> 4) * kG32PartStride + (u & 15) * 16) = v;
     };
-    auto deposit = [&](int buffer) {
-        unsigned char* chunk = q4k_mfma_lds + buffer * kG32ChunkBytes;
+    auto deposit = [&](int h) {
+        unsigned char* chunk = q4k_mfma_lds + (h & 1) * kG32ChunkBytes;
         deposit_unit(chunk, 0, stage0);
         deposit_unit(chunk, 1, stage1);
         deposit_unit(chunk, 2, stage2);
-        deposit_unit(chunk, 3, stage3);
-        deposit_unit(chunk, 4, stage4);
-        deposit_unit(chunk, 5, stage5);
-        if (tid < kG32Rows * 4) reinterpret_cast<uint4*>(chunk + kG32PartsBytes)[tid] = stage_sum;
+        if ((h & 1) && tid < kG32Rows * 4) reinterpret_cast<uint4*>(chunk + kG32PartsBytes)[tid] = stage_sum;
     };
 
     const int c = lane & 31, g = lane >> 5;
@@ -823,121 +821,98 @@ __global__ __launch_bounds__(512) void gemm_q4k_rows32_kernel(float* __restrict_
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
-    t_u32x4 hdr, qv[4], hdr_next, qv_next[4];
-    auto request = [&](int sb, t_u32x4& h, t_u32x4 (&q)[4]) {
-        const uint8_t* base = tile_base + static_cast<size_t>(sb) * kTileBytes;
-        h = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(base + 16 * (lane & 31)));
+    t_u32x4 hdr, qv[2], hdr_next, qv_next[2];
+    auto request = [&](int h, t_u32x4& header, t_u32x4 (&q)[2]) {
+        const uint8_t* base = tile_base + static_cast<size_t>(h >> 1) * kTileBytes;
+        if ((h & 1) == 0) header = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(base + 16 * (lane & 31)));
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-            q[t] = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(base + 512 + t * 1024 + 16 * lane));
+        for (int t = 0; t < 2; ++t)
+            q[t] = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(base + 512 + (2 * (h & 1) + t) * 1024 + 16 * lane));
     };
 
     if (sb_begin >= sb_end) return;  // workgroup-uniform (the host sends no empty shares)
-    fetch(sb_begin);
-    request(sb_begin, hdr, qv);
-    deposit(sb_begin & 1);
+    fetch(2 * sb_begin);
+    request(2 * sb_begin, hdr, qv);
+    hdr_next = hdr;
+    deposit(2 * sb_begin);
     __syncthreads();
     for (int sb = sb_begin; sb < sb_end; ++sb) {
-        const bool more = sb + 1 < sb_end;  // uniform
-        if (more) {
-            fetch(sb + 1);
-            request(sb + 1, hdr_next, qv_next);
-        }
-        const unsigned char* chunk = q4k_mfma_lds + (sb & 1) * kG32ChunkBytes;
-        const unsigned char* sums = chunk + kG32PartsBytes + c * 64 + 16 * g;
         const float d = half_bits_to_f32(static_cast<uint16_t>(hdr.x & 0xFFFFu));
-        const float dmin = half_bits_to_f32(static_cast<uint16_t>(hdr.x >> 16));
-        const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, mn_lo = hdr.z & 0x3F3F3F3Fu;
-        const uint32_t sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
-        const uint32_t mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
-        // Software pipeline over the eight sub-blocks, written out because the compiler on its own
-        // waits for every LDS read right in front of the MFMA that uses it: the A fragments of
-        // sub-block s + 1 are requested before the MFMAs of s are issued, and the accumulation
-        // of s - 1 (vector ALU) runs while those MFMAs are in the matrix core.  Two D sets.
-        uint4 afrag[2][3];  // the three parts of one K half of a sub-block, current and next
-        t_f32x16 D[2];
-        auto load_a = [&](int half, uint4 (&a)[3]) {  // half = 2 * sub-block + m
 #pragma unroll
-            for (int part = 0; part < 3; ++part)
-                a[part] = *reinterpret_cast<const uint4*>(chunk + a_offset + part * kG32PartStride + (32 * (half >> 1) + 8 * (half & 1)) * 2);
-        };
-        auto accumulate = [&](int sub, const t_f32x16& Dv) {
-            const float sc = ubyte_to_f32(sub < 4 ? sc_lo : sc_hi, sub & 3);
-            const float dsc = d * sc;
+        for (int half = 0; half < 2; ++half) {
+            const bool more = half == 0 || sb + 1 < sb_end;  // uniform
+            if (more) {
+                fetch(2 * sb + half + 1);
+                request(2 * sb + half + 1, hdr_next, qv_next);
+            }
+            const unsigned char* chunk = q4k_mfma_lds + half * kG32ChunkBytes;
+            // scales of sub-blocks 0..3 (first half) or 4..7
+            const uint32_t scales = half == 0 ? hdr.y & 0x3F3F3F3Fu : (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(dsc, Dv[i], acc[i]);
-        };
-        union {
-            t_bf16x8 v;
-            t_bf16x2 pair[4];
-        } b[2];
-        load_a(0, afrag[0]);
-#pragma unroll
-        for (int half = 0; half < 16; ++half) {
-            const int sub = half >> 1, m = half & 1;
-            const int t = sub >> 1, hi = sub & 1;  // low nibbles of chunk t: sub-block 2 t, high nibbles: 2 t + 1
-            if (half + 1 < 16) load_a(half + 1, afrag[(half + 1) & 1]);
-            if (m == 0) {
+            for (int sub = 0; sub < 4; ++sub) {
+                t_f32x16 D = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                const int t = sub >> 1, hi = sub & 1;  // low nibbles of chunk t: sub-block 2 t, high nibbles: 2 t + 1
                 const uint32_t w[4] = {qv[t].x, qv[t].y, qv[t].z, qv[t].w};
 #pragma unroll
-                for (int mm = 0; mm < 2; ++mm)
+                for (int m = 0; m < 2; ++m) {
+                    union {
+                        t_bf16x8 v;
+                        t_bf16x2 pair[4];
+                    } b;
 #pragma unroll
                     for (int k = 0; k < 2; ++k) {
-                        const uint32_t nib = hi ? (w[2 * mm + k] >> 4) & 0x0F0F0F0Fu : w[2 * mm + k] & 0x0F0F0F0Fu;
-                        b[mm].pair[2 * k] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(static_cast<int>(nib), 512.0f, false);
-                        b[mm].pair[2 * k + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(static_cast<int>(nib), 512.0f, true);
+                        const uint32_t nib = hi ? (w[2 * m + k] >> 4) & 0x0F0F0F0Fu : w[2 * m + k] & 0x0F0F0F0Fu;
+                        b.pair[2 * k] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(static_cast<int>(nib), 512.0f, false);
+                        b.pair[2 * k + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(static_cast<int>(nib), 512.0f, true);
                     }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            t_f32x16 Dv;
-            if (m == 0) Dv = t_f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            else Dv = D[sub & 1];
 #pragma unroll
-            for (int part = 0; part < 3; ++part) {
-                union {
-                    t_bf16x8 v;
-                    uint4 u;
-                } a;
-                a.u = afrag[half & 1][part];
-                Dv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b[m].v, Dv, 0, 0, 0);
-            }
-            D[sub & 1] = Dv;
-            __builtin_amdgcn_sched_barrier(0);
-            if (m == 0 && sub > 0) {
-                accumulate(sub - 1, D[(sub - 1) & 1]);
-                // pin the accumulation here: left to itself the compiler keeps every D set and its
-                // operands alive and accumulates at the end (spills)
+                    for (int part = 0; part < 3; ++part) {
+                        union {
+                            t_bf16x8 v;
+                            uint4 u;
+                        } a;
+                        a.u = *reinterpret_cast<const uint4*>(chunk + a_offset + part * kG32PartStride + (32 * sub + 8 * m) * 2);
+                        D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, D, 0, 0, 0);
+                    }
+                }
+                const float dsc = d * ubyte_to_f32(scales, sub);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(dsc, D[i], acc[i]);
+                // pin the accumulation here: left to itself the compiler keeps every D and its operands alive (spills)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(acc[i]));
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // The min term of the whole super-block, sum over sub-blocks of m[column][sub] * X[row][sub],
-        // is one more small product: A = the three bf16 parts of the eight sub-block sums of each
-        // row (K = part * 8 + sub, padded with zeros to 32), B = the eight 6-bit mins of each column.
-        union {
-            t_bf16x8 v;
-            uint4 u;
-        } sa0, sa1, mb;
-        sa0.u = *reinterpret_cast<const uint4*>(sums);       // parts 0 (g = 0) and 1 (g = 1)
-        sa1.u = *reinterpret_cast<const uint4*>(sums + 32);  // part 2 (g = 0) and the zeros (g = 1)
-        mb.u = make_uint4(bf16_pair(ubyte_to_f32(mn_lo, 0), ubyte_to_f32(mn_lo, 1)),
-                          bf16_pair(ubyte_to_f32(mn_lo, 2), ubyte_to_f32(mn_lo, 3)),
-                          bf16_pair(ubyte_to_f32(mn_hi, 0), ubyte_to_f32(mn_hi, 1)),
-                          bf16_pair(ubyte_to_f32(mn_hi, 2), ubyte_to_f32(mn_hi, 3)));
-        t_f32x16 T = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa0.v, mb.v, T, 0, 0, 0);
-        T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa1.v, mb.v, T, 0, 0, 0);
-        accumulate(7, D[1]);
+            if (half == 1) {
+                // The min term of the whole super-block, sum over sub-blocks of m[column][sub] * X[row][sub],
+                // is one more small product: A = the three bf16 parts of the eight sub-block sums of each
+                // row (K = part * 8 + sub, padded with zeros to 32), B = the eight 6-bit mins of each column.
+                const unsigned char* sums = chunk + kG32PartsBytes + c * 64 + 16 * g;
+                const float dmin = half_bits_to_f32(static_cast<uint16_t>(hdr.x >> 16));
+                const uint32_t mn_lo = hdr.z & 0x3F3F3F3Fu, mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+                union {
+                    t_bf16x8 v;
+                    uint4 u;
+                } sa0, sa1, mb;
+                sa0.u = *reinterpret_cast<const uint4*>(sums);       // parts 0 (g = 0) and 1 (g = 1)
+                sa1.u = *reinterpret_cast<const uint4*>(sums + 32);  // part 2 (g = 0) and the zeros (g = 1)
+                mb.u = make_uint4(bf16_pair(ubyte_to_f32(mn_lo, 0), ubyte_to_f32(mn_lo, 1)),
+                                  bf16_pair(ubyte_to_f32(mn_lo, 2), ubyte_to_f32(mn_lo, 3)),
+                                  bf16_pair(ubyte_to_f32(mn_hi, 0), ubyte_to_f32(mn_hi, 1)),
+                                  bf16_pair(ubyte_to_f32(mn_hi, 2), ubyte_to_f32(mn_hi, 3)));
+                t_f32x16 T = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa0.v, mb.v, T, 0, 0, 0);
+                T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa1.v, mb.v, T, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(-dmin, T[i], acc[i]);
-        if (more) {
-            deposit((sb + 1) & 1);
-            hdr = hdr_next;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) qv[t] = qv_next[t];
+                for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(-dmin, T[i], acc[i]);
+                hdr = hdr_next;
+            }
+            if (more) {
+                deposit(2 * sb + half + 1);
+                qv[0] = qv_next[0];
+                qv[1] = qv_next[1];
+            }
+            __syncthreads();  // the next chunk is in place, and nobody still reads the one about to be replaced
         }
-        __syncthreads();  // the next chunk is in place, and nobody still reads the one about to be replaced
     }
 
     if (!tile_ok) return;
@@ -1183,14 +1158,7 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
     const unsigned grid_y = static_cast<unsigned>((rows + kG32Rows - 1) / kG32Rows);
     if (grid_y > 65535) return hipErrorInvalidValue;
     const unsigned grid_x = static_cast<unsigned>((n_tiles + 7) / 8);
-    static std::atomic<bool> large_lds{false};  // raising the limit is sticky per kernel: once, outside any stream capture opened later
-    if (!large_lds) {
-        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_q4k_rows32_kernel),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            e != hipSuccess)
-            return e;
-        large_lds = true;
-    }
+    static_assert(2 * kG32ChunkBytes <= 64 * 1024, "no raised LDS limit");
     hipLaunchKernelGGL(gemm_q4k_rows32_kernel, dim3(grid_x, grid_y, shares), dim3(512), 2 * kG32ChunkBytes, stream, dst, parts,
                        xsum, weight, rows, in_dim, out_dim, sb_per_split, partial, ep);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || shares == 1) return e;
