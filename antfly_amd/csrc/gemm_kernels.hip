@@ -241,6 +241,20 @@ __device__ __forceinline__ void gemm_i8_body(
     for (int i = 0; i < kPerSx; ++i) off_sx[i] = offset_sx(i, lane, kSB);
 #pragma unroll
     for (int i = 0; i < kPerSw; ++i) off_sw[i] = offset_sw(i, lane, kSB);
+    // ... and of the last stage, kept where registers allow: the three issues past the end repeat it, and on a short share of K
+    // that is most of them
+    constexpr bool kKeepLast = kPerM * kPerN == 1;
+    uint32_t last_a[kPerA], last_b[kPerB], last_sx[kPerSx], last_sw[kPerSw];
+    if constexpr (kKeepLast) {
+#pragma unroll
+        for (int i = 0; i < kPerA; ++i) last_a[i] = offset_a(i, lane, last_blocks);
+#pragma unroll
+        for (int i = 0; i < kPerB; ++i) last_b[i] = offset_b(i, lane, last_blocks);
+#pragma unroll
+        for (int i = 0; i < kPerSx; ++i) last_sx[i] = offset_sx(i, lane, last_blocks);
+#pragma unroll
+        for (int i = 0; i < kPerSw; ++i) last_sw[i] = offset_sw(i, lane, last_blocks);
+    }
 
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(gemm_lds)));
     constexpr int kOffB = S::kABytes, kOffSx = kOffB + S::kBBytes, kOffSw = kOffSx + S::kSxBytes;
@@ -272,11 +286,16 @@ __device__ __forceinline__ void gemm_i8_body(
                 if (u < kUnitsSw) lds_load2(sw_base + static_cast<size_t>(se) * (kSB * 2), at_sw(i), sp + kOffSw + u * 256);
             }
         };
-        if (se == stages - 1 && last_blocks < kSB) {  // the last stage's own offsets: kept beside the others, they cost registers
-            int l = lane;
-            asm volatile("" : "+v"(l));
-            issue([&](int i) { return offset_a(i, l, last_blocks); }, [&](int i) { return offset_b(i, l, last_blocks); },
-                  [&](int i) { return offset_sx(i, l, last_blocks); }, [&](int i) { return offset_sw(i, l, last_blocks); });
+        if (se == stages - 1 && last_blocks < kSB) {
+            if constexpr (kKeepLast) {
+                issue([&](int i) { return last_a[i]; }, [&](int i) { return last_b[i]; }, [&](int i) { return last_sx[i]; },
+                      [&](int i) { return last_sw[i]; });
+            } else {
+                int l = lane;
+                asm volatile("" : "+v"(l));
+                issue([&](int i) { return offset_a(i, l, last_blocks); }, [&](int i) { return offset_b(i, l, last_blocks); },
+                      [&](int i) { return offset_sx(i, l, last_blocks); }, [&](int i) { return offset_sw(i, l, last_blocks); });
+            }
         } else {
             issue([&](int i) { return off_a[i]; }, [&](int i) { return off_b[i]; }, [&](int i) { return off_sx[i]; },
                   [&](int i) { return off_sw[i]; });
