@@ -6,6 +6,9 @@
 // multiply-add per weight and row on the vector ALU.  Here an activation is split once per workgroup column group into
 // three bf16 numbers hi + mid + lo, each the leading eight bits of what the previous ones left over: together all 24 bits
 // of the f32, so the products q * x (q is exact in bf16) are exact in the accumulator and nothing is lost against f32.
+// (Below about 2^-110 the last part is a subnormal, which holds fewer than eight bits: a wavefront that met such a value goes
+// over its blocks once more for what was left.  Without that the error at 2^-116 was 6e-6 of the row's largest output, at 2^-124
+// 1.8e-3; now 2.4e-7 and 3.1e-7.)
 // Three v_mfma_f32_16x16x32_bf16 per 16 rows x 16 columns x block then leave the block's dots, and one multiply-add per
 // element applies the scale, as before.
 //
@@ -40,13 +43,55 @@ __device__ __forceinline__ float leading8(float v) { return __builtin_bit_cast(f
 
 // x = hi + mid + lo exactly (truncation: no rounding can overflow).  An infinity is its own hi with nothing left over, so that
 // it reaches the sum as an infinity; a NaN leaves a NaN behind even where its payload lies in the low bits.
-__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t* hi, uint32_t* mid, uint32_t* lo) {
+// `left` collects the lanes whose lo has bits in the half that a bf16 does not hold: values below about 2^-110 only.
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t* hi, uint32_t* mid, uint32_t* lo, uint64_t* left) {
     const float h0 = leading8(x0), h1 = leading8(x1);
     const float r0 = __builtin_isinf(x0) ? 0.0f : x0 - h0, r1 = __builtin_isinf(x1) ? 0.0f : x1 - h1;
     const float m0 = leading8(r0), m1 = leading8(r1);
     *hi = upper_halves(h0, h1);
     *mid = upper_halves(m0, m1);
-    *lo = upper_halves(r0 - m0, r1 - m1);
+    const float l0 = r0 - m0, l1 = r1 - m1;
+    *lo = upper_halves(l0, l1);
+    *left |= __ballot(static_cast<uint16_t>(__builtin_bit_cast(uint32_t, l0) | __builtin_bit_cast(uint32_t, l1)) != 0);
+}
+
+// What hi + mid + lo leave of x, at most sixteen bits of a subnormal, times 2^100: a normal number, in two bf16 parts.
+__device__ __forceinline__ void left_pair(float x0, float x1, uint32_t* hi, uint32_t* lo) {
+    const float x[2] = {x0, x1};
+    float h[2], l[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float r = __builtin_isinf(x[i]) ? 0.0f : x[i] - leading8(x[i]);
+        const float lo_part = r - leading8(r);
+        const float e = (lo_part - leading8(lo_part)) * 0x1p100f;
+        h[i] = leading8(e);
+        l[i] = e - h[i];
+    }
+    *hi = upper_halves(h[0], h[1]);
+    *lo = upper_halves(l[0], l[1]);
+}
+
+// Where in a block's bytes the eight values 8 g .. 8 g + 7 lie; Q4_0: values 0..15 are the low nibbles of the 16 bytes, 16..31
+// the high ones.
+template <int kType>
+__device__ __forceinline__ int quant_offset(int g) { return 8 * (kType == 2 ? g & 1 : g); }
+
+// Eight weights of a lane as bf16: bytes biased to unsigned (nibbles are so already), converted, the bias taken off: integers
+// below 2^8, exact.
+template <int kType>
+__device__ __forceinline__ r_bf16x8 weights_bf16(uint2 packed, int g) {
+    const uint32_t p[2] = {packed.x, packed.y};
+    Bf16x8 w;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t biased = kType == 2 ? (p[i] >> (4 * (g >> 1))) & 0x0F0F0F0Fu : p[i] ^ 0x80808080u;
+        constexpr float kBias = kType == 2 ? 8.0f : 128.0f;
+        const float f0 = static_cast<float>(biased & 0xFFu) - kBias, f1 = static_cast<float>((biased >> 8) & 0xFFu) - kBias;
+        const float f2 = static_cast<float>((biased >> 16) & 0xFFu) - kBias, f3 = static_cast<float>(biased >> 24) - kBias;
+        w.u[2 * i] = upper_halves(f0, f1);
+        w.u[2 * i + 1] = upper_halves(f2, f3);
+    }
+    return w.v;
 }
 
 }  // namespace
@@ -59,7 +104,7 @@ struct RouteSecond {
 };
 
 template <int kType, int kTiles>
-__global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
+__global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
                                                                const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
                                                                Epilogue ep_a, RouteSecond second) {
     extern __shared__ __align__(16) float route_sums[];  // [wavefront][tile][4][64]
@@ -85,6 +130,7 @@ __global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) acc[t] = r_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
+    uint64_t left_behind = 0;  // lanes that met a value below about 2^-110
     for (int b0 = wave; b0 < kb; b0 += waves * kRouteDepth) {
         float4 xv[kRouteDepth][2];
         uint2 wq[kRouteDepth][kTiles];
@@ -96,9 +142,7 @@ __global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict
             xv[u][1] = reinterpret_cast<const float4*>(xrow + b * 32)[1];
 #pragma unroll
             for (int t = 0; t < kTiles; ++t) {
-                // Q4_0: values 0..15 are the low nibbles of the 16 bytes, 16..31 the high ones
-                const uint8_t* at = weight + (first[t] + b) * kQuantBytes + 8 * (kType == 2 ? g & 1 : g);
-                wq[u][t] = *reinterpret_cast<const uint2*>(at);
+                wq[u][t] = *reinterpret_cast<const uint2*>(weight + (first[t] + b) * kQuantBytes + quant_offset<kType>(g));
                 ws[u][t] = scales[first[t] + b];
             }
         }
@@ -108,24 +152,13 @@ __global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict
             Bf16x8 part[3];
             const float v[8] = {xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w, xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) split_pair(v[2 * i], v[2 * i + 1], &part[0].u[i], &part[1].u[i], &part[2].u[i]);
+            for (int i = 0; i < 4; ++i) split_pair(v[2 * i], v[2 * i + 1], &part[0].u[i], &part[1].u[i], &part[2].u[i], &left_behind);
 #pragma unroll
             for (int t = 0; t < kTiles; ++t) {
-                // bytes biased to unsigned (nibbles are so already), converted, the bias taken off: integers below 2^8, exact
-                const uint32_t p[2] = {wq[u][t].x, wq[u][t].y};
-                Bf16x8 w;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t biased = kType == 2 ? (p[i] >> (4 * (g >> 1))) & 0x0F0F0F0Fu : p[i] ^ 0x80808080u;
-                    constexpr float kBias = kType == 2 ? 8.0f : 128.0f;
-                    const float f0 = static_cast<float>(biased & 0xFFu) - kBias, f1 = static_cast<float>((biased >> 8) & 0xFFu) - kBias;
-                    const float f2 = static_cast<float>((biased >> 16) & 0xFFu) - kBias, f3 = static_cast<float>(biased >> 24) - kBias;
-                    w.u[2 * i] = upper_halves(f0, f1);
-                    w.u[2 * i + 1] = upper_halves(f2, f3);
-                }
+                const r_bf16x8 w = weights_bf16<kType>(wq[u][t], g);
                 r_f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int q = 2; q >= 0; --q) dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[q].v, w.v, dot, 0, 0, 0);
+                for (int q = 2; q >= 0; --q) dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[q].v, w, dot, 0, 0, 0);
                 const float d = half_bits_to_f32(ws[u][t]);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fmaf(d, dot[i], acc[t][i]);
@@ -136,6 +169,37 @@ __global__ __launch_bounds__(1024) void linear_f32_rows_kernel(float* __restrict
     for (int t = 0; t < kTiles; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) route_sums[((wave * kTiles + t) * 4 + i) * 64 + lane] = acc[t][i];
+    // A second pass over the wavefront's blocks where a value left something behind, added to its own sums in LDS: no activation
+    // of a model does, and nothing of this may take registers in the loop above: four tiles keep to the 64 that give a compute
+    // unit two workgroups (as a branch in the loop 128; one workgroup: 4096 rows of K = 288 x 288 columns 11.0 -> 12.1 us).
+    if (left_behind != 0) {
+        int again = lane;
+        asm volatile("" : "+v"(again));  // addresses are formed anew
+        const int c2 = again & 15, g2 = again >> 4;
+        const float* row = x + static_cast<size_t>(min(m0 + c2, rows - 1)) * in_dim + 8 * g2;
+#pragma unroll 1
+        for (int b = wave; b < kb; b += waves) {
+            const float4 x0 = reinterpret_cast<const float4*>(row + b * 32)[0], x1 = reinterpret_cast<const float4*>(row + b * 32)[1];
+            Bf16x8 rest[2];
+            left_pair(x0.x, x0.y, &rest[0].u[0], &rest[1].u[0]);
+            left_pair(x0.z, x0.w, &rest[0].u[1], &rest[1].u[1]);
+            left_pair(x1.x, x1.y, &rest[0].u[2], &rest[1].u[2]);
+            left_pair(x1.z, x1.w, &rest[0].u[3], &rest[1].u[3]);
+#pragma unroll 1
+            for (int t = 0; t < kTiles; ++t) {
+                const size_t at = static_cast<size_t>(min(n0 + 16 * t + c2, out_dim - 1)) * kb + b;
+                const r_bf16x8 w = weights_bf16<kType>(*reinterpret_cast<const uint2*>(weight + at * kQuantBytes + quant_offset<kType>(g2)), g2);
+                r_f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int q = 1; q >= 0; --q) dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rest[q].v, w, dot, 0, 0, 0);
+                const float d = half_bits_to_f32(scales[at]);
+                float* sums = route_sums + (wave * kTiles + t) * 256 + again;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (dot[i] != 0.0f) sums[64 * i] += d * dot[i] * 0x1p-100f;  // (d may be an infinity)
+            }
+        }
+    }
     __syncthreads();
     for (int at = tid; at < kTiles * 256; at += blockDim.x) {
         float total = 0.0f;

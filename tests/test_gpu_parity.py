@@ -244,6 +244,23 @@ def test_f32_route_on_many_outputs(fmt, rows, in_dim, out_dim):
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(48, 544, 256), (2100, 64, 70)])  # one and four column tiles a workgroup
+def test_f32_route_keeps_small_activations(fmt, rows, in_dim, out_dim):
+    """Activations near the bottom of f32's range, next to rows of ordinary size: below 2^-110 the last of an activation's three
+    bf16 parts is a subnormal and leaves bits behind.  Largest outputs are about 2^-123 (2^-124 activations): subnormal roundings
+    of 2^-150, one a block and sum, are 2^-26 of that each, 4e-7 for 17 blocks and 16 wavefront sums -- under TIGHT."""
+    print(f"case: small activations rows={rows} in={in_dim} out={out_dim} fmt={fmt}", flush=True)
+    x = synth.activations(9 * rows + in_dim, rows, in_dim)
+    x[::3] *= np.float32(2.0 ** -116)
+    x[1::3] = (x[1::3].astype(np.float64) * 2.0 ** -124).astype(np.float32)
+    x[2, 3] = np.float32(1e-40)  # a lone one among ordinary values
+    w = synth.weights(fmt, 3 * out_dim, out_dim, in_dim)
+    y = G.linear(fmt, PREP, x, G.prepare(fmt, w, out_dim, in_dim), rows, in_dim, out_dim)
+    y64 = x.astype(np.float64) @ O.dequantize(fmt, w).reshape(out_dim, in_dim).astype(np.float64).T
+    assert G.max_rel_err(y, y64) <= TIGHT
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
 @pytest.mark.parametrize("rows", [6, 12])  # 12 rows forced onto the GEMV kernels: activations quantized by their own kernel
 def test_forced_dispatch_kinds_agree(fmt, rows):
     """A plan may force any kernel family; all of them compute the same op."""
