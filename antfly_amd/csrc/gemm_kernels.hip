@@ -612,14 +612,20 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
         if (grid * 8 >= units * 11) tile = 'X';
     } else if (grid >= units) {
         // Q8_0, whose 64 x 128 stage does not fit twice: "Y" (64 x 64 outputs, two workgroups a unit) or "V" (128 x 128, two tiles
-        // a wavefront, one workgroup a unit), whichever the grid's rounds make shorter.  A round takes about (K = 4096, us) "V" 62,
-        // "Y" 37 with two workgroups on a unit and 27 with one: 333 x 4096 x 6144 52 / 56 (65 before), 512 x 4096 x 4096 40 / 57 (40),
-        // 512 x 4096 x 14336 121 / 122 (136), 777 x 4096 x 14336 201 / 224 (200), 2048 x 4096 x 14336 459 / 389 (434).
-        const long long wide = static_cast<long long>((rows + 127) / 128) * ((out_dim + 127) / 128);
-        const long long square = static_cast<long long>((rows + 63) / 64) * ((out_dim + 63) / 64);
-        const long long rest = square % (2 * units);
-        const long long square_us = square / (2 * units) * 37 + (rest == 0 ? 0 : rest <= units ? 27 : 37);
-        tile = (wide + units - 1) / units * 62 < square_us ? 'V' : 'Y';
+        // a wavefront, one workgroup a unit), whichever the rounds make shorter.  An XCD (an eighth of the units) serves every
+        // eighth column of tiles, so it is the XCD with most columns whose rounds count.  K = 4096: a round of "V" takes about
+        // 50 us, one workgroup more on every unit about 15 of "Y".  Y / V (64 x 128 by sixteen wavefronts before):
+        // 333 x 4096 x 6144 49 / 52 (60), 512 x 4096 x 4096 36 / 53 (35), 512 x 4096 x 14336 106 / 101 (118), 777 x 4096 x 14336
+        // 170 / 192 (175), 1300 x 4096 x 5632 115 / 145 (121; six columns of tiles on four of the XCDs: three rounds of "V"),
+        // 2048 x 4096 x 14336 435 / 362 (425).  Over 349 sizes (96 .. 2048 rows, K 1024 .. 14336, N 2048 .. 14336) 0.2 % above the
+        // better of the two on the mean; counted over the whole chip instead 2.6 %, at worst 28 %.
+        constexpr long long kXcds = 8;
+        auto rounds = [&](long long tile_rows, long long tile_cols) {
+            const long long cols_of_xcd = ((out_dim + tile_cols - 1) / tile_cols + kXcds - 1) / kXcds;
+            const long long units_of_xcd = units >= kXcds ? units / kXcds : 1;
+            return (cols_of_xcd * ((rows + tile_rows - 1) / tile_rows) + units_of_xcd - 1) / units_of_xcd;
+        };
+        tile = 7 * rounds(128, 128) <= 2 * rounds(64, 64) ? 'V' : 'Y';
     }
     if (force != '\0') tile = force;
     if (dots == nullptr) {

@@ -121,6 +121,8 @@ def linear_epilogue(fmt, layout, x, w_dev, rows, in_dim, out_dim, bias=None, res
 
 EPILOGUE_SHAPES = [(1, 4096, 1024), (1, 8224, 513), (3, 1024, 600), (6, 2048, 640), (40, 512, 640), (300, 512, 1024), (20, 2048, 300),
                    (3, 64, 100), (6, 512, 8200)]
+# the prefill GEMM's larger tiles, odd rows and columns: Q4_0 64 x 128 both, Q8_0 64 x 64 (257 rows) and 128 x 128 (700)
+EPILOGUE_SHAPES += [(257, 160, 10921), (700, 160, 4097)]
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4, Q4K])

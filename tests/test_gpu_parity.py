@@ -183,10 +183,14 @@ def test_block_dots_bit_exact_and_outputs_within_tolerance(fmt, layout, rows, in
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
-@pytest.mark.parametrize("rows,in_dim,out_dim", [(700, 96, 4097), (1100, 544, 3800), (129, 160, 16385), (257, 672, 10921)])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [
+    # Q8_0 on 256 units: 128 x 128 tiles ...
+    (700, 96, 4097), (700, 544, 4097), (700, 576, 4097), (700, 608, 4097),
+    # ... and 64 x 64; the last has fewer 128 x 128 tiles a unit, but six columns of them on four of the eight XCDs
+    (1100, 544, 3800), (129, 160, 16385), (257, 672, 10921), (1300, 192, 5630)])
 def test_prefill_grids_past_the_compute_units(fmt, rows, in_dim, out_dim):
-    """Grids that take the 64 x 128 (Q4_0), 64 x 64 and 128 x 128 (Q8_0) tiles: row and column remainders, K shorter than a stage
-    of four blocks' ring and ending one to three blocks into a stage; f32 sums in another order (TIGHT)."""
+    """Grids that take the 64 x 128 (Q4_0: all of these), 64 x 64 and 128 x 128 (Q8_0) tiles: row and column remainders, K shorter
+    than the ring of four-block stages and ending one, two and three blocks into a stage; f32 sums in another order (TIGHT)."""
     print(f"case: large prefill fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
     x = synth.activations(rows + in_dim, rows, in_dim)
     w = synth.weights(fmt, out_dim + 1, out_dim, in_dim)
