@@ -77,10 +77,16 @@ static WorkspaceView workspace_view(uint64_t base, size_t rows, size_t in_dim) {
 // two rows of any length, and for three or four rows of Q4_0 up to this many 32-value
 // blocks of X; beyond, a separate kernel quantizes X once.
 constexpr size_t kGemvFusedQuantBlocks = 512;
-// Fewest outputs of a matrix that the f32 route takes to the matrix cores (PREPARED layout).  Below, a wavefront per output
-// is the shorter chain: a pair of 256 columns at K = 2048, eight rows 6.1 us against 8.1, sixteen rows 9.9 against 9.4, 77
-// rows 39.0 against 9.6, 2048 rows 961 against 74; on a short K three rows of 5000 columns (K = 64) 10.6 against 3.1.
-constexpr size_t kF32RouteMfmaMinOutputs = 4096;
+// Fewest outputs of a matrix that the f32 route takes to the matrix cores (PREPARED layout).  That kernel has one workgroup
+// for 16 x 16 outputs and, on so few, the same time whatever their number; a wavefront per output grows with them and with K.
+// One call, wavefront per output / matrix cores, us: K = 512, 4096 outputs 3.7 / 3.9; K = 1024, 4096 4.3 / 5.7, 6144 5.5 / 5.7;
+// K = 4096, 4096 9.2 / 16.0, 4608 10.2 / 14.7, 6144 12.8 / 16.2, 8192 16.5 / 16.2.  A pair, one launch either way and its halves
+// the bits of single calls, so one line for both: K = 4096, 4096 16.6 / 16.0, 4608 19.1 / 14.7, 6144 24.0 / 16.2, 8192 32.8 / 16.2.
+// From K = 1024 on the line lies where what a single call loses is what a pair gains.
+static size_t f32_route_mfma_min_outputs(size_t in_dim) {
+    if (in_dim <= 512) return 4096;
+    return in_dim >= 1024 ? 6144 : 4096 + 4 * (in_dim - 512);
+}
 // fewest rows served by the single-shot MFMA kernel (batch_mfma_kernels.hip)
 constexpr size_t kBatchMfmaMinRows = 5;
 
@@ -412,7 +418,7 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
     if (!route_a) {
         if (counters) counters->f32_route += pair ? 2 : 1;
         const int m = static_cast<int>(rows), k = static_cast<int>(in_dim), n = static_cast<int>(out_dim);
-        if (layout == AFHIP_LAYOUT_PREPARED && out_count >= kF32RouteMfmaMinOutputs) {
+        if (layout == AFHIP_LAYOUT_PREPARED && out_count >= f32_route_mfma_min_outputs(in_dim)) {
             const hipError_t e = launch_linear_f32_rows(stream, tensor_type, y, x, w, m, k, n, ep, pair ? y_b : nullptr,
                                                         pair ? w_b : nullptr, ep_b);
             return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);

@@ -220,12 +220,15 @@ def test_f32_route_matches_oracle(fmt, layout, rows, in_dim, out_dim):
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
 @pytest.mark.parametrize("rows,in_dim,out_dim", [(16, 2048, 256), (77, 544, 256), (17, 96, 511), (8, 512, 511), (9, 512, 457), (3, 64, 5000),
-                                                 (1, 32, 4096), (300, 2048, 511), (2100, 64, 70)])
+                                                 (1, 32, 4096), (300, 2048, 511), (2100, 64, 70),
+                                                 # either side of the lines: 4096 outputs up to K = 512, 4864 at 704, 6144 from 1024 on
+                                                 (16, 512, 256), (39, 512, 105), (19, 704, 256), (16, 704, 304), (24, 1024, 256),
+                                                 (24, 4096, 256), (23, 4096, 267)])
 def test_f32_route_on_many_outputs(fmt, rows, in_dim, out_dim):
-    """From 4096 outputs on the f32 route runs on the matrix cores: row and column remainders, K shorter than and not a multiple
-    of what its wavefronts take together, one and four column tiles a workgroup; a pair is one launch with the bits of two calls.
-    Activations are split exactly and summed in f32, so the error is that of f32 sums (TIGHT), also next to 10^6 times larger
-    ones; an infinity stays in its row and reaches it as the reference's does."""
+    """From 4096 outputs on (6144 from K = 1024 on) the f32 route runs on the matrix cores: row and column remainders, K shorter than
+    and not a multiple of what its wavefronts take together, one and four column tiles a workgroup; a pair is one launch with the
+    bits of two calls.  Activations are split exactly and summed in f32, so the error is that of f32 sums (TIGHT), also next to
+    10^6 times larger ones; an infinity stays in its row and reaches it as the reference's does."""
     print(f"case: f32 route rows={rows} in={in_dim} out={out_dim} fmt={fmt}", flush=True)
     assert not O.uses_activation_quant(rows, in_dim, out_dim)
     x = synth.activations(5 * rows + in_dim, rows, in_dim)
