@@ -116,20 +116,29 @@ static int env_int(const char* name) {
 // Whether the single-shot MFMA kernel serves this shape (measured against the kernels it replaces;
 // AFHIP_BATCH_MFMA_MIN_ROWS overrides the lower row bound for tuning runs, 0 switches the kernel off):
 // from five rows on (six on a K longer than 4096, where the split-K GEMV still wins at five) up to 64
-// (96 on some Q4_0 matrices), and for Q8_0, whose K shares are half as long, only while all workgroups
+// (96 on some Q4_0 matrices, below), and for Q8_0, whose K shares are half as long, only while all workgroups
 // of the launch are resident at once.  Five to eight rows (Q8_0: sixteen) on a K of whole 256-value runs always:
 // the eight-row kernel requests weights as it goes and needs neither condition.  Two to four rows where measured
 // faster than the decode kernels (the rules below).
 static bool batch_mfma_preferred(int tensor_type, size_t rows, size_t in_dim, size_t out_dim, bool pair) {
     static const char* v = std::getenv("AFHIP_BATCH_MFMA_MIN_ROWS");
     static const long forced = v && *v ? std::atol(v) : -1;
-    // up to 64 rows everywhere; 65 .. 96 of Q4_0 on a K around 4096 where the GEMM's grid of 32 x 64 tiles just passes one
-    // workgroup a compute unit while this kernel's 32-column tiles still fit them in one round (96 rows x 6144 columns 20.6
-    // against 22.0 us, x 8192 21.7 / 22.9; the GEMM wins on 10240 columns 36.2 / 23.8, with K = 2048 x 7168 16.9 / 14.8,
-    // K = 8192 x 8192 41.0 / 38.4, and from 97 rows on: 128 x 6144 25.5 / 23.0, x 14336 47.6 / 41.3)
-    const size_t units = static_cast<size_t>(gemv_compute_units());
-    const bool one_round = (out_dim + 31) / 32 <= units && (rows + 31) / 32 * ((out_dim + 63) / 64) > units;
-    const size_t max_rows = tensor_type == AFHIP_TYPE_Q4_0 && one_round && in_dim >= 3072 && in_dim <= 6144 ? 96 : 64;
+    // Up to 64 rows everywhere; 65 .. 96 of Q4_0 where the GEMM's grid of 32 x 64 tiles passes one workgroup a compute unit (on
+    // one it takes 15.5 us at K = 4096 x 4608 columns) and this kernel's 32-column tiles need few rounds.  It takes 17 us for every
+    // unit's worth of workgroups whatever K up to a share of 128 blocks, so K has to be near that (this kernel / the GEMM, 65 rows):
+    //  * one share and one round, K over 3072: 3104 x 6144 columns 19.2 / 20.2, 4096 x 8192 19.5 / 20.7; 3072 x 6144 18.1 / 17.0
+    //    and, with a second share, 4352 x 6144 29.1 / 23.6, 6144 x 6144 33.4 / 27.0 go to the GEMM
+    //  * a pair, one launch here and two of the GEMM, also in three rounds: 4096 x 11008 50.2 / 56.1, 4096 x 12288 50.8 / 56.5
+    //    where the GEMM needs a second round itself (10240 50.1 / 40.1 does not; 10880 50.2 / 55.8 does, an XCD having every eighth
+    //    column of tiles and a round of two workgroups a unit); on two shares 6656 x 6144 49.9 / 58.3,
+    //    8192 x 6144 51.8 / 65.0, 5632 x 5632 48.0 / 50.3, but 5120 x 5632 47.8 / 43.8.  One matrix of those shapes is better on
+    //    the GEMM (4096 x 11008 33.2 / 29.3, 6656 x 6144 33.6 / 30.3), so there a pair's sums have another order than a call's.
+    const size_t units = static_cast<size_t>(gemv_compute_units()), tiles = (out_dim + 31) / 32;
+    const size_t gemm_rows = (rows + 31) / 32, gemm_cols = (out_dim + 63) / 64, gemm_grid = gemm_rows * gemm_cols;
+    bool few_rounds = false;
+    if (in_dim > 3072 && in_dim <= 4096) few_rounds = tiles <= units || (pair && 2 * tiles <= 3 * units && gemm_rows * ((gemm_cols + 7) / 8) * 8 > 2 * units);
+    else if (in_dim > 5376 && in_dim <= 8192) few_rounds = pair && 4 * tiles <= 3 * units;
+    const size_t max_rows = tensor_type == AFHIP_TYPE_Q4_0 && few_rounds && gemm_grid > units ? 96 : 64;
     if (forced == 0 || rows > max_rows || !batch_mfma_supports(tensor_type, rows, in_dim, out_dim)) return false;
     if (forced > 0) return rows >= static_cast<size_t>(forced);
     if (rows >= kBatchMfmaMinRows && batch_mfma_eight_rows(tensor_type, rows, in_dim, out_dim)) return true;

@@ -188,7 +188,9 @@ afhip_status afhip_launch_linear_f32_static(void *stream, int tensor_type, int l
  * bit for bit what afhip_launch_linear_f32 gives for that matrix wherever the pair and the
  * single call take the same kernel -- everywhere but three and four rows of Q4_0 with
  * in_dim <= 4096 whose two matrices together exceed two (four rows of fewer than 4096 values: one) rounds of the decode
- * kernel's workgroups while one of them does not: there the same block dots are summed in
+ * kernel's workgroups while one of them does not, and 65 to 96 rows of Q4_0 on some shapes that
+ * one matrix takes to the tiled GEMM and two together to a single launch (on 256 compute units in_dim 3104 to 4096
+ * with 10753 to 12288 columns, in_dim 5408 to 8192 with 5441 to 6144): there the same block dots are summed in
  * another order (equal within the op's tolerance).  X is quantized once, and up to 8 rows
  * (Q8_0: 16) both matrices are served by one kernel launch. */
 afhip_status afhip_launch_linear_pair_f32(void *stream, int tensor_type, int layout, afhip_buffer dst_a,

@@ -136,8 +136,9 @@ SHAPES_A = [  # (rows, in_dim, out_dim): all take the activation-quantized route
     # the single-shot MFMA kernel (5..64 rows): every count of live result registers, two row tiles, a K
     # that ends inside a wavefront's run of blocks, a second K share of one block, ragged columns
     (24, 4096, 544), (25, 2048, 512), (32, 4128, 513), (48, 320, 520), (12, 3072, 1000),
-    (70, 512, 8200), (128, 1056, 8192), (97, 256, 8224),  # three and four row tiles (Q4_0 on a wide matrix)
-    (100, 512, 4700), (66, 1024, 6150),  # ... and on a matrix whose tiled-GEMM grid would take a second round
+    # 65 to 128 rows on the tiled GEMM's 32 x 64 tiles: every row remainder of a tile, ragged columns, K ending inside a stage
+    # (three row tiles of the single-shot kernel: test_sixty_five_to_ninety_six_rows)
+    (70, 512, 8200), (128, 1056, 8192), (97, 256, 8224), (100, 512, 4700), (66, 1024, 6150),
     # the eight-row MFMA kernel (5..8 rows on a grid of at least a workgroup per compute unit): one live
     # wavefront and a ragged last tile; 64-column tiles, ragged; K shares with a short last share; a
     # wavefront with half its blocks
@@ -180,6 +181,33 @@ def test_block_dots_bit_exact_and_outputs_within_tolerance(fmt, layout, rows, in
         err = G.max_rel_err(y, ref.astype(np.float64))
         assert err <= TOL and err <= TIGHT, err
     assert G.max_rel_err(y, y64) <= TIGHT
+
+
+@pytest.mark.parametrize("rows,in_dim,out_dim,same", [
+    # one matrix and a pair on three row tiles of the single-shot kernel: K ending inside a wavefront's run of sixteen blocks,
+    # the last K of one share, row and column remainders, the most columns of one round
+    (96, 3104, 5500, True), (65, 4096, 5442, True), (70, 3328, 8190, True),
+    # a pair there alone: in three rounds, and with a second K share that ends inside a run
+    (66, 3104, 10753, False), (95, 5408, 5500, False),
+    # ... and both on the GEMM: one step of rows, K or columns past each line
+    (97, 3104, 5500, True), (66, 3072, 5500, True), (66, 4128, 5500, True), (66, 5376, 5500, True), (66, 3104, 5440, True),
+    (66, 3104, 10752, True)])
+def test_sixty_five_to_ninety_six_rows(rows, in_dim, out_dim, same):
+    """Q4_0 either side of the lines between the single-shot kernel and the tiled GEMM, against 64-bit sums, with a bias and a
+    residual too; a pair's halves have the bits of single calls but where only the pair takes the single-shot kernel."""
+    print(f"case: 65 to 96 rows rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(71 * rows + in_dim, rows, in_dim)
+    wa, wb = synth.weights(Q4, out_dim, out_dim, in_dim), synth.weights(Q4, out_dim + 1, out_dim, in_dim)
+    da, db = G.prepare(Q4, wa, out_dim, in_dim), G.prepare(Q4, wb, out_dim, in_dim)
+    y64 = [O.linear_act_f64(Q4, x, w, rows, in_dim, out_dim) for w in (wa, wb)]
+    single = [G.linear(Q4, PREP, x, d, rows, in_dim, out_dim) for d in (da, db)]
+    for pair_half, one, want in zip(G.linear_pair(Q4, PREP, x, da, db, rows, in_dim, out_dim), single, y64):
+        assert G.max_rel_err(one, want) <= TIGHT and G.max_rel_err(pair_half, want) <= TIGHT
+        assert np.array_equal(pair_half, one) == same
+    bias = synth.activations(72, 1, out_dim)[0]
+    assert G.max_rel_err(G.linear_bias(Q4, PREP, x, da, bias, rows, in_dim, out_dim), y64[0] + bias) <= TIGHT
+    biased = G.linear_pair_bias(Q4, PREP, x, da, bias, db, -bias, rows, in_dim, out_dim)
+    assert G.max_rel_err(biased[0], y64[0] + bias) <= TIGHT and G.max_rel_err(biased[1], y64[1] - bias) <= TIGHT
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
