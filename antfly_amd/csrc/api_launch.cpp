@@ -442,7 +442,7 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
     const int chunk = gemv_row_chunk(rows, in_dim);
     const bool fused_ok = layout == AFHIP_LAYOUT_PREPARED && chunk > 0 && kind != AFHIP_DISPATCH_SCALAR &&
                           in_dim <= static_cast<size_t>(gemv_fused_max_in_dim());
-    // Five to 64 (128) rows: the weights are read once, so the single-shot MFMA kernel (X quantized into
+    // Five to 64 (96) rows: the weights are read once, so the single-shot MFMA kernel (X quantized into
     // MFMA operand order first) beats both the row-by-row GEMV and the tiled GEMM.
     if (layout == AFHIP_LAYOUT_PREPARED && !want_dots && kind != AFHIP_DISPATCH_SCALAR &&
         batch_mfma_preferred(tensor_type, rows, in_dim, out_dim, pair) &&
@@ -835,8 +835,8 @@ size_t afhip_linear_workspace_bytes(int tensor_type, size_t rows, size_t in_dim,
     const size_t gemm_bytes = partial != 0 ? (base + 255) / 256 * 256 + partial : base;
     // small batches on a long K (also slices of eight rows of a forced plan): the K slices' sums, for a pair of matrices
     const size_t batch_bytes = gemv_batch_partial_bytes(rows < 8 ? rows : 8, in_dim, out_dim, true);
-    // up to 128 rows: X in MFMA operand order and the partial sums of K shares of the single-shot MFMA kernel
-    const size_t mfma_bytes = rows <= 128 ? batch_mfma_workspace_bytes(tensor_type, rows, in_dim, out_dim) : 0;
+    // up to 64 rows (Q4_0 96): X in MFMA operand order and the partial sums of K shares of the single-shot MFMA kernel
+    const size_t mfma_bytes = batch_mfma_workspace_bytes(tensor_type, rows, in_dim, out_dim);
     size_t need = gemm_bytes > batch_bytes ? gemm_bytes : batch_bytes;
     return need > mfma_bytes ? need : mfma_bytes;
 }

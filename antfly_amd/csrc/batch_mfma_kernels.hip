@@ -1,4 +1,4 @@
-// Batched decode (a few to 128 rows) on CDNA4 int8 MFMA, activation-quantized route
+// Batched decode (a few to 64 rows, some Q4_0 matrices to 96) on CDNA4 int8 MFMA, activation-quantized route
 // (ops/native_compute.zig:13304-13478 for Q8_0, :23427-23775 for Q4_0):
 //   dot[m][n][b] = sum_i qx[m][32b+i] * qw[n][32b+i]            (int32, exact)
 //   y[m][n]      = sum_b (sx[m][b] * sw[n][b]) * f32(dot[m][n][b])
@@ -1093,9 +1093,8 @@ hipError_t bm_launch_rows(hipStream_t stream, float* dst, float* partial, const 
     if (rows <= 16) AFHIP_BM(1, 8);
     if (rows <= 24) AFHIP_BM(1, 12);
     if (rows <= 32) AFHIP_BM(1, 16);
-    if (rows <= 64) AFHIP_BM(2, 16);
-    if (rows <= 96) AFHIP_BM(3, 16);
-    AFHIP_BM(4, 16);
+    if (kType == 8 || rows <= 64) AFHIP_BM(2, 16);
+    if constexpr (kType == 2) AFHIP_BM(3, 16);
 #undef AFHIP_BM
 }
 
@@ -1219,7 +1218,7 @@ hipError_t bm_launch32(hipStream_t stream, float* dst, float* partial, const uin
 
 bool batch_mfma_supports(int tensor_type, size_t rows, size_t in_dim, size_t out_dim) {
     if (tensor_type != 2 && tensor_type != 8) return false;
-    if (rows < 1 || rows > 128 || in_dim == 0 || in_dim % 32 != 0 || out_dim == 0) return false;
+    if (rows < 1 || rows > (tensor_type == 2 ? 96 : 64) || in_dim == 0 || in_dim % 32 != 0 || out_dim == 0) return false;
     // 32-bit lane offsets relative to a column tile, grid.y
     if (in_dim > (1u << 22) || out_dim > 0x7fffffff) return false;
     return true;
