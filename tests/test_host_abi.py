@@ -178,7 +178,7 @@ def test_linear_workspace_covers_every_kernel_family():
     assert kernels.workspaceBytes(_lib.TYPE_Q4_0, 95, 4096, 8192) >= mfma(_lib.TYPE_Q4_0, 95, 4096, 8192) == 96 * 4096 + 128 * 96 * 4
     assert kernels.workspaceBytes(_lib.TYPE_Q4_0, 95, 8192, 6144) == mfma(_lib.TYPE_Q4_0, 95, 8192, 6144)  # two K shares of a pair
     for fmt, rows in ((_lib.TYPE_Q4_0, 97), (_lib.TYPE_Q8_0, 65)):  # one row past the kernel: the quantized activations alone
-        assert kernels.workspaceBytes(fmt, rows, 8192, 16384) == quantized(rows, 8192)
+        assert kernels.workspaceBytes(fmt, rows, 4096, 16384) == quantized(rows, 4096)
     assert mfma(_lib.TYPE_Q8_0, 4, 4096, 512) == 32 * 4096 + 128 * 32 * 4 + 2 * 2 * 4 * 512 * 4
 
 
