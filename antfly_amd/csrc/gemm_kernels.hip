@@ -406,7 +406,7 @@ __device__ __forceinline__ void gemm_i8_body(
             }
         }
     };
-    uint64_t stamp_begin = 0, stamp_loop = 0, stamp_tail = 0, ref_loop = 0, retail = 0, stamp_wait = 0, stamp_barrier = 0;
+    uint64_t stamp_begin = 0, stamp_loop = 0, stamp_tail = 0, ref_loop = 0, ref_tail = 0, stamp_wait = 0, stamp_barrier = 0;
     if (kStamps) stamp_begin = __builtin_readcyclecounter();
     // ---- prologue: stages 0 .. kRing-2 in flight, stages 0 and 1 landed, stage 0 in registers
     static_assert(kRing == 4, "the loop reads stage st + 1 while stage st + 2 lands and stage st + 3 is issued");
@@ -448,7 +448,7 @@ __device__ __forceinline__ void gemm_i8_body(
     }
     if (kStamps) {
         stamp_tail = __builtin_readcyclecounter();
-        retail = __builtin_amdgcn_s_memrealtime();
+        ref_tail = __builtin_amdgcn_s_memrealtime();
     }
 
     // Loads still in flight target ring slots nobody reads again; they must land before
@@ -489,7 +489,7 @@ __device__ __forceinline__ void gemm_i8_body(
             out[1] = static_cast<int>(stamp_tail - stamp_loop);
             out[2] = static_cast<int>(stamp_wait);
             out[3] = static_cast<int>(stamp_barrier);
-            out[4] = static_cast<int>(retail - ref_loop);
+            out[4] = static_cast<int>(ref_tail - ref_loop);
             out[5] = static_cast<int>(stamp_end - stamp_tail);
             out[6] = 0;
             out[7] = static_cast<int>(__builtin_amdgcn_s_getreg((31 << 11) | 4));
