@@ -315,7 +315,7 @@ pub const KernelModule = struct {
         const m_tiles = (rows + tile_m - 1) / tile_m;
         const n_tiles = (out_dim + tile_n - 1) / tile_n;
         const grid = try checkedMul(try checkedMul((n_tiles + 7) / 8, m_tiles), 8);
-        // four stages of operands: 27648 bytes each, and 8192 more for Q4_0's nibble chunks
+        // four stages of operands and scales: 19456 bytes each (Q4_0, nibbles packed) or 27648 (Q8_0)
         const lds: usize = if (tensor_type == .q4_0) 77824 else 110592;
         var dst_ptr = dst.ptr;
         var input_ptr = input.ptr;
