@@ -48,6 +48,7 @@
 
 #include <atomic>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device_common.h"
 #include "gemv_common.h"
@@ -355,7 +356,9 @@ __device__ __forceinline__ void gemm_i8_body(
     // the registers block blk's dots have left (the two halves of a wavefront's work do
     // not overlap anyway, and 16 registers fewer are live).  `between` runs after the
     // last MFMA has been issued: the operand registers are free from there on.
-    auto pair_step = [&](const Frag& f, int blk, auto&& between) {
+    // `sixteenth`: the scale takes back the sixteen times of a Q4_0 weight; else the dot does.
+    auto pair_step = [&](const Frag& f, int blk, auto sixteenth, auto&& between) {
+        constexpr bool kSixteenth = kQ4 && decltype(sixteenth)::value;
         // blocks past the end of K (clamped re-reads of the last block) get scale 0
         const bool live = blk + lh < kb;
         const v16i zi = {};
@@ -366,7 +369,7 @@ __device__ __forceinline__ void gemm_i8_body(
         for (int j = 0; j < kPerN; ++j) {
             w0[j] = weight_bytes(f.w0[j]);
             w1[j] = weight_bytes(f.w1[j]);
-            tb[j] = live ? half_bits_to_f32(static_cast<uint16_t>(f.tb[j])) * (kQ4 ? 0.0625f : 1.0f) : 0.0f;
+            tb[j] = live ? half_bits_to_f32(static_cast<uint16_t>(f.tb[j])) * (kSixteenth ? 0.0625f : 1.0f) : 0.0f;
         }
 #pragma unroll
         for (int i = 0; i < kPerM; ++i) {
@@ -394,7 +397,7 @@ __device__ __forceinline__ void gemm_i8_body(
                         }
                     }
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) sum[v] = __builtin_fmaf(t[16 * h + v], static_cast<float>(c[v]), sum[v]);
+                    for (int v = 0; v < 16; ++v) sum[v] = __builtin_fmaf(t[16 * h + v], static_cast<float>(kQ4 && !kSixteenth ? c[v] >> 4 : c[v]), sum[v]);
                     if (h == 0) {
                         // compiler fence (no instruction): block blk is finished before block blk + 1 starts
                         asm volatile("" : "+v"(sum), "+v"(t) : : "memory");
@@ -431,7 +434,7 @@ __device__ __forceinline__ void gemm_i8_body(
                 // the slot of stage st - 1 is free (its fragments were read a stage ago): refill it, kRing - 1 stages ahead
                 issue_loads((d + kRing - 1) % kRing, st + kRing - 1);
                 // the next stage's operands landed before the last barrier
-                pair_step(frag[d & 1], st * kSB + b0, [&]() { read_frag((d + 1) % kRing, frag[(d + 1) & 1]); });
+                pair_step(frag[d & 1], st * kSB + b0, std::true_type{}, [&]() { read_frag((d + 1) % kRing, frag[(d + 1) & 1]); });
                 // stage st + 2 (issued two stages ago) has to be complete before the barrier:
                 // the next stage reads its operands
                 uint64_t s0 = 0, s1 = 0;
@@ -459,11 +462,67 @@ __device__ __forceinline__ void gemm_i8_body(
         // ---- the kSplit partial sums of a tile meet in LDS
         __syncthreads();
         float* red = reinterpret_cast<float*>(gemm_lds);  // [ks][tile][tile of the wavefront][v][lane]
+        auto store_sums = [&]() {
 #pragma unroll
-        for (int p = 0; p < kPerWave; ++p)
+            for (int p = 0; p < kPerWave; ++p)
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                red[(((ks * S::kTiles + tile) * kPerWave + p) * 16 + v) * 64 + lane] = acc[p / kPerN][p % kPerN][v];
+                for (int v = 0; v < 16; ++v)
+                    red[(((ks * S::kTiles + tile) * kPerWave + p) * 16 + v) * 64 + lane] = acc[p / kPerN][p % kPerN][v];
+        };
+        store_sums();
+        // A sixteenth of a product of scales below 2^-122 is subnormal where the product may not be, and loses up to four of its
+        // bits: 2^-150 times a dot of up to 2^19 a block, 2^-122 over 512 blocks, which no sum from 2^-96 on feels (2^-26 of it).
+        // A wavefront with a smaller sum -- a zero is one -- looks its activation scales over and, if one is below 2^-98 (the
+        // smallest fp16 scale is 2^-24; activations below 4e-28), forms its sums again from plain products, operands straight from
+        // memory.  Error at 2^-116, 333 x 512 x 8200: 1.5e-5 without, 8.7e-7 with, as Q4_0 had unpacked.  Looking for such scales in
+        // the K loop cost 1.1 % of all prefills, a branch there 4.5 %; this 0.1 %.
+        if constexpr (kQ4 && !kWriteDots) {
+            float least = __builtin_huge_valf();
+#pragma unroll
+            for (int p = 0; p < kPerWave; ++p)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) least = __builtin_fminf(least, __builtin_fabsf(acc[p / kPerN][p % kPerN][v]));
+            bool again = __ballot(least < 0x1p-96f) != 0;
+            int l = lane;
+            asm volatile("" : "+v"(l));  // addresses are formed anew: nothing of this takes registers in the loop above
+            const int half = l >> 5;
+            if (again) {
+                bool small = false;
+#pragma unroll 1
+                for (int blk = b0; blk < kb; blk += kSB)
+#pragma unroll
+                    for (int i = 0; i < kPerM; ++i) {
+                        const size_t r = min(m0 + wm * (32 * kPerM) + 32 * i + (l & 31), rows - 1) - m0;
+                        small |= reinterpret_cast<const float*>(sx_base)[r * kb_full + min(blk + half, kb - 1)] < 0x1p-98f;
+                    }
+                again = __ballot(small) != 0;
+            }
+            if (again) {
+#pragma unroll
+                for (int p = 0; p < kPerWave; ++p) acc[p / kPerN][p % kPerN] = v16f{};
+#pragma unroll 1
+                for (int blk = b0; blk < kb; blk += kSB) {
+                    const int blk1 = min(blk + 1, kb - 1), blk_h = half ? blk1 : blk;
+                    Frag f;
+#pragma unroll
+                    for (int i = 0; i < kPerM; ++i) {
+                        const size_t r = min(m0 + wm * (32 * kPerM) + 32 * i + (l & 31), rows - 1) - m0;
+                        f.a0[i] = *reinterpret_cast<const int4*>(a_base + r * in_dim + blk * 32 + 16 * half);
+                        f.a1[i] = *reinterpret_cast<const int4*>(a_base + r * in_dim + blk1 * 32 + 16 * half);
+                        f.ta[i] = reinterpret_cast<const float*>(sx_base)[r * kb_full + blk_h];
+                    }
+#pragma unroll
+                    for (int j = 0; j < kPerN; ++j) {
+                        const size_t r = min(n0 + wn * (32 * kPerN) + 32 * j + (l & 31), out_dim - 1) - n0;
+                        f.w0[j] = *reinterpret_cast<const int4*>(b_base + (r * kb_full + blk) * kQuantBytes);
+                        f.w1[j] = *reinterpret_cast<const int4*>(b_base + (r * kb_full + blk1) * kQuantBytes);
+                        f.tb[j] = reinterpret_cast<const uint16_t*>(sw_base)[r * kb_full + blk_h];
+                    }
+                    pair_step(f, blk, std::false_type{}, []() {});
+                }
+                store_sums();
+            }
+        }
         __syncthreads();
         if (dst == nullptr) return;
         constexpr int kPer = 16 / kSplit;

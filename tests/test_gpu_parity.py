@@ -226,6 +226,33 @@ def test_prefill_grids_past_the_compute_units(fmt, rows, in_dim, out_dim):
     assert G.max_rel_err(y, O.linear_act_f64(fmt, x, w, rows, in_dim, out_dim)) <= TIGHT
 
 
+@pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [
+    (700, 160, 4097), (257, 672, 10921), (130, 544, 4100),  # the large tiles and 32 x 64
+    (130, 1056, 520)])                                      # ... with K shared out over workgroups
+def test_prefill_keeps_small_activations(fmt, rows, in_dim, out_dim):
+    """Rows scaled by the power of two that takes the smallest product of two scales just above 2^-126 give the same bits scaled:
+    every product is a normal number and every sum a multiple of 2^-149, so nothing is rounded that is not in the row of ordinary
+    size.  (Packed Q4_0 nibbles are sixteen times their value and the scale products a sixteenth, subnormal here.)"""
+    print(f"case: small prefill activations fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    rng = np.random.default_rng(17 * rows + in_dim)
+    x = rng.uniform(-1.0, 1.0, (rows, in_dim)).astype(np.float32)
+    x[:, ::32] = rng.uniform(1.0, 1.5, x[:, ::32].shape)  # every block's peak: all scales within a factor of three
+    w = synth.weights(fmt, out_dim + 3, out_dim, in_dim)
+    blocks = w.reshape(out_dim * in_dim // 32, -1)
+    blocks[:, :2] = rng.uniform(2.0 ** -8, 2.0 ** -7, len(blocks)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    down = 2.0 ** (-126 + 15)  # the smallest product of two scales is 2^-8 / 127
+    x_small = x.copy()
+    x_small[::3] = (x[::3].astype(np.float64) * down).astype(np.float32)
+    x_small[5] = 0.0
+    wd = G.prepare(fmt, w, out_dim, in_dim)
+    y = G.linear(fmt, PREP, x, wd, rows, in_dim, out_dim)
+    want = y.copy()
+    want[::3] = (y[::3].astype(np.float64) * down).astype(np.float32)
+    want[5] = 0.0
+    assert np.array_equal(G.linear(fmt, PREP, x_small, wd, rows, in_dim, out_dim), want)
+
+
 SHAPES_B = [(1, 32, 3), (2, 64, 600), (3, 96, 11), (4, 4096, 100), (1, 64, 4096), (12, 128, 40)]
 
 
