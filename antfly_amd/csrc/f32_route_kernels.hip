@@ -1,7 +1,7 @@
 // The f32 route (fewer than 512 columns, or K below 96: narrow key / value projections) on the matrix cores, PREPARED
 // layout: y[r][o] = sum over blocks of d[o][b] * sum_i x[r][32 b + i] * q[o][32 b + i], f32 activations.
 //
-// What bounded the one-wavefront-per-output kernel (linear_f32_route_kernel, still used for a few rows and the raw layout):
+// What bounded the one-wavefront-per-output kernel (linear_f32_route_kernel, still used for few outputs and the raw layout):
 // every output read its whole row of X and row of W again and converted every weight again -- one convert and one
 // multiply-add per weight and row on the vector ALU.  Here an activation is split once per workgroup column group into
 // three bf16 numbers hi + mid + lo, each the leading eight bits of what the previous ones left over: together all 24 bits

@@ -686,6 +686,8 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
         };
         tile = 7 * rounds(128, 128) <= 2 * rounds(64, 64) ? 'V' : 'Y';
     }
+    // Block dots, bound by writing them, take "S" on every grid: 512 x 4096 x 4096 Q4_0 4183 -> 3925, Q8_0 4273 -> 3447 from the tile
+    // before, 300 x 2048 x 14336 4461 -> 2465 and 4671 -> 2229.
     if (force != '\0') tile = force;
     if (dots == nullptr) {
         if constexpr (kType == 2) {

@@ -575,7 +575,9 @@ def main() -> int:
         print("|---|---|---|")
         for wv in range(8):
             print(f"| {wv} | {int(np.median(st[:, wv, 1]))} | {int(np.median(st[:, wv, 3]))} |")
-        tile_blocks = (m // 32) * (n // 32) * (k // 32) / (groups * 4)  # per SIMD
+        # two workgroups share a compute unit where there are enough of them: their loops run side by side on its four SIMDs
+        together = min(2, -(-groups // torch.cuda.get_device_properties(0).multi_processor_count))
+        tile_blocks = (m // 32) * (n // 32) * (k // 32) / (groups * 4) * together  # per SIMD
         print(f"tile-blocks (32 x 32 outputs x one 32-value block) per SIMD: {tile_blocks:.0f}; loop cycles per tile-block and SIMD: "
               f"{float(np.median(st[:, :, 1])) / tile_blocks:.0f}")
         print(json.dumps({"probe": "gemm", "clock_ghz": round(ghz, 3), "loop_cycles_median": int(np.median(st[:, :, 1])),

@@ -135,7 +135,9 @@ int afhip_quant_row_bucket(size_t rows);                                        
 int afhip_quant_format_from_tensor_type(int tensor_type); /* graph/backend_contracts.zig:199-236 */
 /* Route gate of the CPU engine (ops/native_compute.zig:3410-3419): 1 when the op
  * quantizes activations to int8 per 32-block, 0 when it multiplies f32
- * activations by dequantized weights. */
+ * activations by dequantized weights.  (Neither route promises a row the same last bits whatever the number of rows
+ * of its call: kernels are chosen by shape and sum in orders of their own.  On the f32 route with PREPARED weights the
+ * line is rows * out_dim = 4096, on in_dim > 512 rising to 6144 at 1024.) */
 int afhip_uses_activation_quant(size_t rows, size_t in_dim, size_t out_dim);
 /* Q4_K only: whether the op quantizes the activations to Q8_K (256-value blocks) and takes
  * integer sub-block dots, as the CPU engine does on a gated set of shapes
