@@ -658,7 +658,7 @@ template <int kType>
 hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
                        const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial) {
     // us of the whole op, M x K x N; "before" is the 64 x 128 tile by sixteen wavefronts that served these grids.
-    static const char* env_tile = std::getenv("AFHIP_GEMM_TILE");  // tuning: "S", "Y", "X" or "V", see below
+    static const char* env_tile = std::getenv("AFHIP_GEMM_TILE");  // tuning: "S", "X", "Y", "V" or "L", see below
     const char force = dots == nullptr && env_tile ? env_tile[0] : '\0';
     const long long units = gemv_compute_units();
     const long long grid = static_cast<long long>((rows + 63) / 64) * ((out_dim + 127) / 128);
@@ -684,7 +684,11 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
             const long long units_of_xcd = units >= kXcds ? units / kXcds : 1;
             return (cols_of_xcd * ((rows + tile_rows - 1) / tile_rows) + units_of_xcd - 1) / units_of_xcd;
         };
-        tile = 7 * rounds(128, 128) <= 2 * rounds(64, 64) ? 'V' : 'Y';
+        // 33 .. 64 rows have one row of tiles and fetch every weight once, so nothing is gained by a second workgroup that shares
+        // them: "L" (64 x 128, one tile for each of sixteen wavefronts), Y / L: 64 x 4096 x 65536 85.4 / 77.9, 64 x 8192 x 32768
+        // 79.5 / 71.3, a pair 180 / 160, 64 x 4096 x 128256 173 / 169, 40 x 4096 x 32768 34.4 / 35.0 (V, half empty, 105 at 8192).
+        if (rows > 32 && rows <= 64) tile = 'L';
+        else tile = 7 * rounds(128, 128) <= 2 * rounds(64, 64) ? 'V' : 'Y';
     }
     // Block dots, bound by writing them, take "S" on every grid: 512 x 4096 x 4096 Q4_0 4183 -> 3925, Q8_0 4273 -> 3447 from the tile
     // before, 300 x 2048 x 14336 4461 -> 2465 and 4671 -> 2229.
@@ -693,6 +697,7 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
         if constexpr (kType == 2) {
             if (tile == 'X') return launch_wide_tile<2, 1, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
         } else {
+            if (tile == 'L') return launch_wide_tile<8, 2, 4, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
             if (tile == 'V') return launch_wide_tile<8, 2, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
             if (tile == 'Y') return launch_wide_tile<8, 2, 2, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
         }

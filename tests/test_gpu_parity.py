@@ -215,9 +215,11 @@ def test_sixty_five_to_ninety_six_rows(rows, in_dim, out_dim, same):
     # Q8_0 on 256 units: 128 x 128 tiles ...
     (700, 96, 4097), (700, 544, 4097), (700, 576, 4097), (700, 608, 4097),
     # ... and 64 x 64; the last has fewer 128 x 128 tiles a unit, but six columns of them on four of the eight XCDs
-    (1100, 544, 3800), (129, 160, 16385), (257, 672, 10921), (1300, 192, 5630)])
+    (1100, 544, 3800), (129, 160, 16385), (257, 672, 10921), (1300, 192, 5630),
+    # ... and 64 x 128: 33 to 64 rows on more columns than the single-shot kernel takes (Q4_0 stays on that)
+    (64, 2080, 32780), (33, 2112, 32780), (49, 2144, 32769)])
 def test_prefill_grids_past_the_compute_units(fmt, rows, in_dim, out_dim):
-    """Grids that take the 64 x 128 (Q4_0: all of these), 64 x 64 and 128 x 128 (Q8_0) tiles: row and column remainders, K shorter
+    """Grids that take the 64 x 128 (Q4_0), 64 x 64, 128 x 128 and 64 x 128 (Q8_0) tiles: row and column remainders, K shorter
     than the ring of four-block stages and ending one, two and three blocks into a stage; f32 sums in another order (TIGHT)."""
     print(f"case: large prefill fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
     x = synth.activations(rows + in_dim, rows, in_dim)
