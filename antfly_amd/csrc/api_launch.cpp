@@ -298,12 +298,13 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
             else if (kind == AFHIP_DISPATCH_SMALL_BATCH) counters->small_batch++;
             else counters->mm++;
         }
-        if (gemm) {
-            hipError_t e = launch_gemm_q4k_tiled(stream, reinterpret_cast<float*>(i ? dst_b.ptr : dst.ptr),
-                                                 reinterpret_cast<const float*>(input.ptr),
-                                                 reinterpret_cast<const uint8_t*>(i ? weight_b.ptr : weight.ptr),
-                                                 reinterpret_cast<void*>(workspace.ptr), static_cast<int>(rows),
-                                                 static_cast<int>(in_dim), static_cast<int>(out_dim), i ? ep_b : ep, i == 0);
+        if (gemm) {  // a pair goes down together: X is split once
+            if (i == 1) continue;
+            hipError_t e = launch_gemm_q4k_tiled(stream, reinterpret_cast<float*>(dst.ptr), reinterpret_cast<const float*>(input.ptr),
+                                                 reinterpret_cast<const uint8_t*>(weight.ptr), reinterpret_cast<void*>(workspace.ptr),
+                                                 static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), ep,
+                                                 pair ? reinterpret_cast<float*>(dst_b.ptr) : nullptr,
+                                                 pair ? reinterpret_cast<const uint8_t*>(weight_b.ptr) : nullptr, ep_b);
             if (e != hipSuccess) return static_cast<afhip_status>(e);
             continue;
         }

@@ -39,6 +39,7 @@
 #include <stdint.h>
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "device_common.h"
 #include "qmatmul_launch.h"
@@ -705,11 +706,11 @@ int tuning_int(const char* name) {
     return v && *v ? std::atoi(v) : 0;
 }
 
-// ------------------------------------------------------------------ prefill
-// Many rows (more than one GEMV launch holds): X is split once by its own kernel --
+// ------------------------------------------------------------------ short prefill
+// More rows than one GEMV launch holds, up to 64 (longer ones: the fp6 GEMM below): X is split once by its own kernel --
 // parts bf16 [rows][3][in_dim], sub-block sums as bf16 parts [rows][in_dim / 256][4][8] -- and the GEMM below
 // converts every weight once per 32 rows instead of once per launch of six.
-__global__ __launch_bounds__(256) void q4k_split_rows_kernel(const float* __restrict__ x, uint32_t* __restrict__ parts,
+__global__ __launch_bounds__(256) void q4k_split_parts_kernel(const float* __restrict__ x, uint32_t* __restrict__ parts,
                                                              uint16_t* __restrict__ sum_parts, size_t groups, int groups_per_row) {
     // one thread per eight consecutive values; whole quads run together (groups is a multiple of four)
     for (size_t grp = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; grp < groups;
@@ -929,6 +930,519 @@ __global__ __launch_bounds__(512, 4) void gemm_q4k_rows32_kernel(float* __restri
     }
 }
 
+// ------------------------------------------------------------------ prefill
+// More than 64 rows: X is split once by its own kernel, then a GEMM on the 6-bit matrix
+// instructions.  v_mfma_scale_f32_32x32x64_f8f6f4 multiplies 64 fp6 (e2m3) numbers a column in the 33 cycles that
+// v_mfma_f32_32x32x16_bf16 needs for 16 bf16 ones, and to it
+//   * the fp6 codes 0 .. 15 are the numbers n / 8, so a weight nibble is its own code (with two zero bits on top);
+//   * an activation is eight 4-bit digits with its sign: |x| = sum over d of digit_d * 2^(e - 4 (d + 1)), with
+//     2^(e - 1) <= max |x| < 2^e over the sub-block.  Rounded to 2^-33 of that maximum (24-bit numbers down to 2^-8 of it are
+//     exact); products with the scales 2^(e - 4 d) that the instruction applies to 32 values at a time are exact.
+// A sub-block of 32 values is four such instructions -- lane half g of number p multiplies digit 2 p + g -- against six bf16
+// ones, and its result needs no conversion: (d sc) * D is added to the sum.  Against 64 bits the four leave 4.4e-8 of a
+// sub-block's sum, the three bf16 parts of the kernel above 6.9e-8 (32 normal values; 3.9e-8 / 6.7e-8 with outliers).
+//
+// The order of the 16 values of a lane half inside its three 32-bit words of codes: the one in which nine instructions spread
+// the nibbles of the tile-major layout (expand_nibbles).
+constexpr int kFp6Order[16] = {0, 12, 5, 10, 3, 15, 4, 9, 2, 14, 7, 8, 1, 13, 6, 11};
+
+// Workspace: the digits, for every 32 rows (the last tile: its rows, rounded up to even) and sub-block the operands of the four
+// instructions, each [half g][row] 16 bytes and then [half g][row] 8 bytes (a lane's six words); behind them, for every row and
+// super-block 64 bytes: the eight sub-block sums as three bf16 parts, [part][sub-block], and the sub-blocks' scale bytes.
+constexpr int kDigitBytes = 192;  // of a row and sub-block
+
+__device__ __forceinline__ int rows_of_tile(int rows, int tile) { return (min(kG32Rows, rows - tile * kG32Rows) + 1) & ~1; }
+
+// One wavefront per 32 rows and sub-block, a lane for 16 values; the image is put together in LDS and written as it lies.
+__global__ __launch_bounds__(64) void q4k_split_digits_kernel(const float* __restrict__ x, uint8_t* __restrict__ digits,
+                                                            uint8_t* __restrict__ sums, int rows, int in_dim) {
+    __shared__ __align__(16) uint32_t image[kG32Rows * kDigitBytes / 4];
+    const int lane = threadIdx.x, tile = blockIdx.y, sub = blockIdx.x;
+    const int tile_rows = rows_of_tile(rows, tile);
+    const int r = lane >> 1, half = lane & 1, row = tile * kG32Rows + r;
+    float v[16];
+    if (row < rows) {
+        const float4* src = reinterpret_cast<const float4*>(x + static_cast<size_t>(row) * in_dim + sub * 32 + half * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 q = src[i];
+            v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = 0.0f;
+    }
+    uint32_t peak = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) peak = max(peak, __float_as_uint(v[i]) & 0x7FFFFFFFu);
+    peak = max(peak, static_cast<uint32_t>(dpp_move<kDppXor1>(static_cast<int>(peak))));
+    // the biased exponent is the scale byte of digit 0; below 4 (2^-122) the digits reach 2^-154, under every f32, and the scales
+    // of the lower ones would leave their range.  255: an infinity or a NaN, which the instruction takes as NaN
+    const int exponent = max(static_cast<int>(peak >> 23), 4);
+    uint32_t u[16], sign[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int f = 0; f < 16; ++f) {
+        const float value = v[kFp6Order[f]];
+        u[f] = static_cast<uint32_t>(__builtin_rintf(__builtin_ldexpf(__builtin_fabsf(value), 158 - exponent)));
+        const int at = 6 * f + 5;
+        sign[at >> 5] |= (__float_as_uint(value) >> 31) << (at & 31);
+    }
+    uint8_t* img = reinterpret_cast<uint8_t*>(image);
+    if (r < tile_rows) {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            uint32_t w[3] = {sign[0], sign[1], sign[2]};
+#pragma unroll
+            for (int f = 0; f < 16; ++f) {
+                const uint32_t digit = (u[f] >> (28 - 4 * d)) & 15u;
+                const int at = 6 * f;
+                w[at >> 5] |= digit << (at & 31);
+                if ((at & 31) > 28) w[(at >> 5) + 1] |= digit >> (32 - (at & 31));
+            }
+            const int p = d >> 1, g = d & 1;
+            uint32_t* wide = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + (g * tile_rows + r) * 16);
+            uint32_t* rest = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + tile_rows * 32 + (g * tile_rows + r) * 8);
+            if (half == 0) {
+                wide[0] = w[0]; wide[1] = w[1]; wide[2] = w[2];
+            } else {
+                wide[3] = w[0]; rest[0] = w[1]; rest[1] = w[2];
+            }
+        }
+    }
+    float s = (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]))) +
+              (((v[8] + v[9]) + (v[10] + v[11])) + ((v[12] + v[13]) + (v[14] + v[15])));
+    s += dpp_move<kDppXor1>(s);
+    if (half == 0 && row < rows) {
+        uint32_t hi, mid, lo;
+        split3_pair(s, 0.0f, &hi, &mid, &lo);
+        uint8_t* cell = sums + (static_cast<size_t>(row) * (in_dim >> 8) + (sub >> 3)) * 64;
+        uint16_t* part = reinterpret_cast<uint16_t*>(cell) + (sub & 7);
+        part[0] = static_cast<uint16_t>(hi);
+        part[8] = static_cast<uint16_t>(mid);
+        part[16] = static_cast<uint16_t>(lo);
+        cell[48 + (sub & 7)] = static_cast<uint8_t>(exponent);
+    }
+    __syncthreads();
+    uint4* out = reinterpret_cast<uint4*>(digits + static_cast<size_t>(tile) * kG32Rows * in_dim * 6 +
+                                          static_cast<size_t>(sub) * tile_rows * kDigitBytes);
+    for (int i = lane; i < tile_rows * (kDigitBytes / 16); i += 64) out[i] = reinterpret_cast<const uint4*>(img)[i];
+}
+
+// (x & mask) | (y & ~mask) and (x & mask) | y in one instruction at the fast rate (v_bitop3_b32 2.4 cycles; v_and_or_b32 and the
+// shifts 4.4, v_permlane32_swap_b32 8.7).
+__device__ __forceinline__ uint32_t blend(uint32_t mask, uint32_t x, uint32_t y) {
+    return __builtin_amdgcn_bitop3_b32(mask, x, y, 0xCA);
+}
+__device__ __forceinline__ uint32_t masked_or(uint32_t mask, uint32_t x, uint32_t y) {
+    return __builtin_amdgcn_bitop3_b32(mask, x, y, 0xEA);
+}
+
+// One 64-lane load of 16 bytes a lane from base + off straight into LDS at lds + at + 16 lane, then off += step (as inline
+// assembly, as in gemm_kernels.hip: the compiler would make every later LDS read wait for all of them).  The addition stands
+// where M0 needs a wait state before it is used; lds, base and step are wave-uniform, `at` a constant.
+__device__ __forceinline__ void q4k_lds_load16(const void* base, uint32_t& off, uint32_t step, uint32_t lds, int at) {
+    uint32_t next;
+    asm volatile("s_add_u32 m0, %1, %5\n\tv_add_u32 %0, %2, %3\n\tglobal_load_lds_dwordx4 %3, %4"
+                 : "=&v"(next)
+                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "s"(step), "v"(off), "s"(base), "i"(at)
+                 : "memory", "m0", "scc");
+    off = next;
+}
+
+typedef int t_i32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t t_u32x2 __attribute__((ext_vector_type(2)));
+typedef int t_i32x6 __attribute__((ext_vector_type(6)));
+
+// s_waitcnt for "at most kLeft vector memory operations outstanding".
+template <int kLeft>
+__device__ __forceinline__ void q4k_wait_vm() {
+    static_assert(kLeft < 16, "the count's low four bits");
+    __builtin_amdgcn_s_waitcnt(kLeft | (7 << 4) | (15 << 8));
+}
+
+template <int kWaves, int kR, int kC>
+struct G6Shape {
+    static constexpr int kThreads = 64 * kWaves;
+    static constexpr int kRows = kG32Rows * kR, kTiles = kC * kWaves, kCols = kTileCols * kTiles;
+    static constexpr int kDigits = kR * kG32Rows * kDigitBytes;  // of a sub-block: ring of four
+    static constexpr int kChunk = kTiles * 1024;                 // nibbles of two sub-blocks: two
+    static constexpr int kHeaders = kTiles * 512;                // of a super-block: one
+    static constexpr int kSums = kR * kG32Rows * 64;             // of a super-block: two
+    static constexpr int kChunkAt = 4 * kDigits, kHeadersAt = kChunkAt + 2 * kChunk, kSumsAt = kHeadersAt + kHeaders;
+    static constexpr int kLdsBytes = kSumsAt + 2 * kSums;
+    // 1 KiB loads of a stage, dealt out to the wavefronts in turn
+    static constexpr int kUnitsDigits = 6 * kR, kUnitsChunk = kTiles, kUnitsHeaders = kTiles / 2, kUnitsSums = 2 * kR;
+    static_assert(kTiles % 2 == 0, "headers are loaded for two column tiles at a time");
+};
+
+// Y[32 kR rows][32 kC kWaves columns] per workgroup; a wavefront owns kC column tiles for all rows of the workgroup and the
+// whole K of the launch.  A stage is a sub-block: digits and weights travel global -> LDS three stages ahead, and what a stage
+// computes with is read from LDS one stage (or row tile) ahead.
+// Bound by instruction issue beside the MFMAs and, on a full chip, by its power (1.7 GHz): four MFMAs of 33 cycles, 45 other
+// instructions (16 of them the multiply-adds) and about 210 SIMD cycles per 32 x 32 outputs and sub-block, where the bf16 kernel took
+// 440.  Against it: 2048 x 4096 x 14336 685 -> 501 us, 333 x 4096 x 14336 twice 290 -> 212, 333 x 14336 x 4096 166 -> 121.
+template <int kWaves, int kR, int kC, int kOcc>
+__global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
+    float* __restrict__ dst, const uint8_t* __restrict__ digits, const uint8_t* __restrict__ sums,
+    const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_groups, int n_groups, int band, int sb_per_split,
+    float* __restrict__ partial, Epilogue ep, Q4kSecond second) {
+    using S = G6Shape<kWaves, kR, kC>;
+    if (blockIdx.z != 0) {  // a second matrix on the same X
+        dst = second.dst;
+        weight = second.weight;
+        ep = second.ep;
+    }
+    const int kb = in_dim >> 8;
+    // K range of this workgroup: all of it, or share blockIdx.y, whose sums go to partial[share][rows][out_dim]
+    const int sb_begin = blockIdx.y * sb_per_split;
+    const int sb_end = min(kb, sb_begin + sb_per_split);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    // An XCD (consecutive ids go round-robin over the eight) takes an eighth of the list of tiles, in which `band` row groups of a
+    // column group follow each other, then the next column group's: what is resident on an XCD shares both operands in its L2.
+    const int id = blockIdx.x, index = (id & 7) * (gridDim.x >> 3) + (id >> 3);
+    const int band_at = index / (band * n_groups) * band, band_rows = min(band, m_groups - band_at), in_band = index - band_at * n_groups;
+    if (index >= m_groups * n_groups || sb_begin >= sb_end) return;  // workgroup-uniform
+    const int m_group = band_at + in_band % band_rows, n_group = in_band / band_rows;
+    const int n_tiles = (out_dim + kTileCols - 1) >> 5, m_tiles = (rows + kG32Rows - 1) / kG32Rows;
+    const int tile0 = n_group * S::kTiles;
+    const uint32_t tile_stride = static_cast<uint32_t>(kb) * kTileBytes;
+    auto tile_at = [&](int tile) { return weight + static_cast<size_t>(min(tile0 + tile, n_tiles - 1)) * tile_stride; };  // spare ones repeat the last
+
+    // ---- loads: units of each kind, dealt out in turn; where they do not go round, some wavefronts repeat another's, so that all
+    // count the same loads and no branch stands between them (branches on the counts cost a wavefront 400 cycles a stage)
+    constexpr int kPerDigits = (S::kUnitsDigits + kWaves - 1) / kWaves, kPerChunk = (S::kUnitsChunk + kWaves - 1) / kWaves;
+    constexpr int kPerHeaders = (S::kUnitsHeaders + kWaves - 1) / kWaves, kPerSums = (S::kUnitsSums + kWaves - 1) / kWaves;
+    const uint32_t lds_base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(q4k_mfma_lds)));
+    // bases stay, this lane's offsets move on with every load
+    const uint8_t *digit_base[kPerDigits], *chunk_base[kPerChunk], *header_base[kPerHeaders], *sum_base[kPerSums];
+    uint32_t digit_off[kPerDigits], chunk_off[kPerChunk], header_off[kPerHeaders], sum_off[kPerSums], digit_step[kPerDigits];
+    uint32_t digit_lds[kPerDigits], chunk_lds[kPerChunk], header_lds[kPerHeaders], sum_lds[kPerSums];
+#pragma unroll
+    for (int k = 0; k < kPerDigits; ++k) {
+        const int u = (wave + k * kWaves) % S::kUnitsDigits, q = u % 6;
+        const int mt = min(m_group * kR + u / 6, m_tiles - 1), n = rows_of_tile(rows, mt);
+        digit_step[k] = n * kDigitBytes;
+        digit_base[k] = digits + static_cast<size_t>(mt) * kG32Rows * in_dim * 6 + static_cast<size_t>(sb_begin) * 8 * digit_step[k];
+        digit_lds[k] = lds_base + u * 1024;
+        const int o = q * 1024 + lane * 16, p = o / 1536, w = o - p * 1536;  // image offset of this lane's bytes
+        int at;
+        if (w < 1024) at = ((w >> 9) * n + min((w >> 4) & 31, n - 1)) * 16;
+        else at = n * 32 + (((w - 1024) >> 8) * n + min(((w - 1024) >> 3) & 31, n - 2)) * 8;
+        digit_off[k] = static_cast<uint32_t>(p * n * 48 + at);
+    }
+#pragma unroll
+    for (int k = 0; k < kPerChunk; ++k) {
+        const int u = (wave + k * kWaves) % S::kUnitsChunk;
+        chunk_base[k] = tile_at(u) + static_cast<size_t>(sb_begin) * kTileBytes + 512;
+        chunk_off[k] = 16 * lane;
+        chunk_lds[k] = lds_base + S::kChunkAt + u * 1024;
+    }
+#pragma unroll
+    for (int k = 0; k < kPerHeaders; ++k) {
+        const int u = (wave + k * kWaves) % S::kUnitsHeaders;
+        header_base[k] = tile_at(2 * u) + static_cast<size_t>(sb_begin) * kTileBytes;
+        header_off[k] = (g != 0 && tile0 + 2 * u + 1 < n_tiles ? tile_stride : 0u) + 16 * c;
+        header_lds[k] = lds_base + S::kHeadersAt + u * 1024;
+    }
+#pragma unroll
+    for (int k = 0; k < kPerSums; ++k) {
+        const int u = (wave + k * kWaves) % S::kUnitsSums, mt = min(m_group * kR + (u >> 1), m_tiles - 1);
+        sum_base[k] = sums + (static_cast<size_t>(mt) * kG32Rows * kb + sb_begin) * 64;
+        sum_off[k] = static_cast<uint32_t>(min(c, rows - 1 - mt * kG32Rows)) * static_cast<uint32_t>(kb * 64) + (2 * (u & 1) + g) * 16;
+        sum_lds[k] = lds_base + S::kSumsAt + u * 1024;
+    }
+    // load l of stage s (0 .. 7)
+    constexpr int kLoadsOdd = kPerDigits, kLoadsEven = kPerDigits + kPerChunk, kLoadsFirst = kLoadsEven + kPerHeaders + kPerSums;
+    auto loads_of = [](int s) constexpr { return s == 0 ? kLoadsFirst : ((s & 1) ? kLoadsOdd : kLoadsEven); };
+    auto issue_one = [&](int s, int l, int parity) {
+        if (l < kPerDigits) {
+            const int k = l;
+            q4k_lds_load16(digit_base[k], digit_off[k], digit_step[k], digit_lds[k], (s & 3) * S::kDigits);
+        } else if (l < kLoadsEven) {
+            const int k = l - kPerDigits;
+            q4k_lds_load16(chunk_base[k], chunk_off[k], s < 6 ? 1024 : kTileBytes - 3072, chunk_lds[k], ((s >> 1) & 1) * S::kChunk);
+        } else if (l < kLoadsEven + kPerHeaders) {
+            const int k = l - kLoadsEven;
+            q4k_lds_load16(header_base[k], header_off[k], kTileBytes, header_lds[k], 0);
+        } else {
+            const int k = l - kLoadsEven - kPerHeaders;
+            q4k_lds_load16(sum_base[k], sum_off[k], 64, sum_lds[k] + parity * S::kSums, 0);  // [row tile][16-byte chunk][row]
+        }
+    };
+    auto issue = [&](int s, int parity) {
+#pragma unroll
+        for (int l = 0; l < loads_of(s); ++l) issue_one(s, l, parity);
+    };
+    auto past_the_end = [&](bool last) {  // the loads that run past the end of K repeat its last super-block: nobody uses them
+        const uint32_t back = last ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < kPerDigits; ++k) digit_off[k] -= 8 * back * digit_step[k];
+#pragma unroll
+        for (int k = 0; k < kPerChunk; ++k) chunk_off[k] -= back * kTileBytes;
+#pragma unroll
+        for (int k = 0; k < kPerHeaders; ++k) header_off[k] -= back * kTileBytes;
+#pragma unroll
+        for (int k = 0; k < kPerSums; ++k) sum_off[k] -= back * 64;
+    };
+
+    t_f32x16 acc[kR][kC];
+#pragma unroll
+    for (int i = 0; i < kR; ++i)
+#pragma unroll
+        for (int j = 0; j < kC; ++j) acc[i][j] = t_f32x16{};
+
+    // Statements below that only name registers ("+v") hold what follows, or what made them, in its place.
+    typedef const __attribute__((address_space(3))) t_u32x4* lds16_ptr;
+    typedef const __attribute__((address_space(3))) t_u32x2* lds8_ptr;
+    uint32_t lane16 = lds_base + 16 * lane, lane8 = lds_base + 1024 + 8 * lane;
+    const uint32_t own_tiles = 1024 * wave * kC;
+    t_u32x4 qv[kC];
+    uint32_t nib[kC][2], e[kC][3];
+    t_i32x6 a[4], b[2][kC];
+    auto read_digits = [&](int s, int i, int p) {
+        asm volatile("" : "+v"(lane16), "+v"(lane8));
+        const int at = (s & 3) * S::kDigits + i * 6144 + p * 1536;
+        const t_u32x4 wide = *reinterpret_cast<lds16_ptr>(lane16 + at);
+        const t_u32x2 rest = *reinterpret_cast<lds8_ptr>(lane8 + at);
+        a[p] = t_i32x6{static_cast<int>(wide.x), static_cast<int>(wide.y), static_cast<int>(wide.z), static_cast<int>(wide.w),
+                       static_cast<int>(rest.x), static_cast<int>(rest.y)};
+    };
+    auto read_chunk = [&](int s) {  // nibbles of sub-blocks s and s + 1, s even
+        asm volatile("" : "+v"(lane16));
+#pragma unroll
+        for (int j = 0; j < kC; ++j)
+            qv[j] = *reinterpret_cast<lds16_ptr>(lane16 + own_tiles + (S::kChunkAt + ((s >> 1) & 1) * S::kChunk + j * 1024));
+    };
+    // The weights of sub-block s in three parts: nibbles of the sub-block alone, sixteen 6-bit codes in three words, all 32 values
+    // in both lane halves.
+    auto convert = [&](int s, int j, int piece) {
+        constexpr uint32_t kLow = 0x0F0F0F0Fu;
+        if (piece == 0) {
+            t_u32x4 w = qv[j];
+            asm volatile("" : "+v"(w));
+            if ((s & 1) == 0) {
+                nib[j][0] = blend(kLow, w.x, w.y << 4);
+                nib[j][1] = blend(kLow, w.z, w.w << 4);
+            } else {
+                nib[j][0] = blend(kLow, w.x >> 4, w.y);
+                nib[j][1] = blend(kLow, w.z >> 4, w.w);
+            }
+            asm volatile("" : "+v"(nib[j][0]), "+v"(nib[j][1]));
+        } else if (piece == 1) {
+            const uint32_t n = nib[j][0], x = nib[j][1] << 2;
+            e[j][0] = masked_or(0xC03C03C0u, x, n & 0x0F00F00Fu);
+            e[j][1] = masked_or(0x03C03C00u, x, n & 0xF00F00F0u) | (nib[j][1] >> 30);
+            e[j][2] = masked_or(0x3C03C03Cu, x, n & 0x00F00F00u);
+            asm volatile("" : "+v"(e[j][0]), "+v"(e[j][1]), "+v"(e[j][2]));
+        } else {
+            t_i32x6& to = b[s & 1][j];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const auto both = __builtin_amdgcn_permlane32_swap(e[j][k], e[j][k], false, false);
+                to[k] = static_cast<int>(both[0]);
+                to[k + 3] = static_cast<int>(both[1]);
+            }
+            asm volatile("" : "+v"(to));
+        }
+    };
+
+    const int b_scale = 130 | 122 << 8 | 114 << 16 | 106 << 24;  // 2^(3 - 8 p): codes are eighths, digit pair p weighs 2^(-8 p)
+    issue(0, sb_begin & 1);
+    issue(1, 0);
+    issue(2, 0);
+    q4k_wait_vm<kLoadsEven>();  // loads complete in order: stages 0 and 1 have landed
+    __syncthreads();
+    read_chunk(0);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) read_digits(0, 0, p);
+#pragma unroll
+    for (int j = 0; j < kC; ++j)
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece) convert(0, j, piece);
+
+    // A step is one row tile and sub-block: kC times four chained MFMAs into D.  A slot is one MFMA and what stands behind it: the
+    // matrix pipe takes 33 cycles an instruction and only what is issued in between overlaps it.  That is a share of the
+    // multiply-adds of the step before (its D times its factor), the reads of the next step's digits, the conversion of the next
+    // sub-block's weights and the loads of the stage three ahead.  Eight sub-blocks are followed by the min term, a step of two bf16
+    // MFMAs per row tile.
+    t_f32x16 D[2][kC];
+    float factor[2][kC];
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+        D[1][j] = t_f32x16{};
+        factor[1][j] = 0.0f;
+    }
+    int a_scale[kR], a_scale_next[kR];
+    uint32_t first_half = g == 0 ? 0xFFFFFFFFu : 0u;
+    asm volatile("" : "+v"(first_half));  // (a select here would become a branch around an MFMA)
+    auto read_scales = [&](int sb, int half) {
+#pragma unroll
+        for (int i = 0; i < kR; ++i)
+            a_scale_next[i] = *reinterpret_cast<const int*>(q4k_mfma_lds + S::kSumsAt + (sb & 1) * S::kSums + i * 2048 + 1536 + 16 * c + 4 * half);
+    };
+    auto accumulate = [&](int before, int i, int j, int first, int last) {
+#pragma unroll
+        for (int v = first; v < last; ++v) acc[i][j][v] = __builtin_fmaf(factor[before][j], D[before][j][v], acc[i][j][v]);
+        asm volatile("" : "+v"(acc[i][j]));
+    };
+    read_scales(sb_begin, 0);
+    for (int sb = sb_begin; sb < sb_end; ++sb) {
+        const unsigned char* cell = q4k_mfma_lds + S::kSumsAt + (sb & 1) * S::kSums;
+        t_u32x4 hdr[kC];
+        uint4 mins[kC], sum_parts[2];
+        float d[kC];
+#pragma unroll
+        for (int j = 0; j < kC; ++j) hdr[j] = *reinterpret_cast<const t_u32x4*>(q4k_mfma_lds + S::kHeadersAt + (wave * kC + j) * 512 + 16 * c);
+        auto read_sums = [&](int i) {
+            sum_parts[0] = *reinterpret_cast<const uint4*>(cell + i * 2048 + g * 512 + 16 * c);  // parts 0 (g = 0) and 1 (g = 1)
+            sum_parts[1] = *reinterpret_cast<const uint4*>(cell + i * 2048 + 1024 + 16 * c);     // part 2
+        };
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (s == 5) past_the_end(sb + 1 == sb_end);
+            constexpr int kSlots = 4 * kR * kC;
+            const int to_issue = loads_of((s + 3) & 7);
+            if ((s & 3) == 0) {
+#pragma unroll
+                for (int i = 0; i < kR; ++i) a_scale[i] = a_scale_next[i] - 0x04040404 * g;
+            }
+#pragma unroll
+            for (int i = 0; i < kR; ++i) {
+                const int step = s * kR + i, now = step & 1, before = now ^ 1, i_before = (i + kR - 1) % kR;
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const t_i32x8 a8 = __builtin_shufflevector(a[p], a[p], 0, 1, 2, 3, 4, 5, -1, -1);
+#pragma unroll
+                    for (int j = 0; j < kC; ++j) {
+                        const t_i32x8 b8 = __builtin_shufflevector(b[s & 1][j], b[s & 1][j], 0, 1, 2, 3, 4, 5, -1, -1);
+                        const t_f32x16 from = p == 0 ? t_f32x16{} : D[now][j];
+                        // Highest digits first: added to a smaller sum, the large products always round the same way, 2.9e-8 of a
+                        // sub-block but with a mean of -8.8e-8 that grows with K (333 x 14336 x 4096: 6.3e-7 against 4.5e-7).
+#define AFHIP_STEP(P, W) \
+    if (p == P && (s & 3) == W) D[now][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a8, b8, from, 2, 2, W, a_scale[i], P, b_scale)
+                        AFHIP_STEP(0, 0); AFHIP_STEP(0, 1); AFHIP_STEP(0, 2); AFHIP_STEP(0, 3);
+                        AFHIP_STEP(1, 0); AFHIP_STEP(1, 1); AFHIP_STEP(1, 2); AFHIP_STEP(1, 3);
+                        AFHIP_STEP(2, 0); AFHIP_STEP(2, 1); AFHIP_STEP(2, 2); AFHIP_STEP(2, 3);
+                        AFHIP_STEP(3, 0); AFHIP_STEP(3, 1); AFHIP_STEP(3, 2); AFHIP_STEP(3, 3);
+#undef AFHIP_STEP
+                        __builtin_amdgcn_sched_barrier(0);
+                        const int at = (i * 4 + p) * kC + j;  // slot of the stage
+#pragma unroll
+                        for (int l = 0; l < to_issue; ++l)
+                            if (l * kSlots / to_issue == at) issue_one((s + 3) & 7, l, (sb + 1) & 1);
+                        if (j == kC - 1) read_digits(i + 1 < kR ? s : s + 1, (i + 1) % kR, p);
+                        if (at == 0 && (s & 1)) read_chunk((s + 1) & 7);
+                        if (at == kC && (s & 3) == 3) read_scales(s == 3 ? sb : sb + 1, s == 3);
+                        if (s == 7 && at == kSlots - 1) read_sums(0);
+                        accumulate(before, i_before, j, 4 * p, 4 * p + 4);
+                        if (s == 0 && i == 0 && p == 2) asm volatile("" : "+v"(hdr[j]));
+                        if (s == 0 && i == 0 && p == 2) d[j] = half_bits_to_f32(static_cast<uint16_t>(hdr[j].x & 0xFFFFu));
+                        if (p == 3) {
+                            const uint32_t scales = s < 4 ? hdr[j].y & 0x3F3F3F3Fu : (hdr[j].w & 0x0F0F0F0Fu) | ((hdr[j].y >> 2) & 0x30303030u);
+                            factor[now][j] = d[j] * ubyte_to_f32(scales, s & 3);
+                        }
+                        if (i == kR - 1 && p > 0) convert((s + 1) & 7, j, p - 1);
+                        if (s == 6 && i == 0 && p == 0) {
+                            asm volatile("" : "+v"(hdr[j]));
+                            const uint32_t mn_lo = hdr[j].z & 0x3F3F3F3Fu, mn_hi = ((hdr[j].w >> 4) & 0x0F0F0F0Fu) | ((hdr[j].z >> 2) & 0x30303030u);
+                            mins[j] = make_uint4(bf16_pair(ubyte_to_f32(mn_lo, 0), ubyte_to_f32(mn_lo, 1)),
+                                                 bf16_pair(ubyte_to_f32(mn_lo, 2), ubyte_to_f32(mn_lo, 3)),
+                                                 bf16_pair(ubyte_to_f32(mn_hi, 0), ubyte_to_f32(mn_hi, 1)),
+                                                 bf16_pair(ubyte_to_f32(mn_hi, 2), ubyte_to_f32(mn_hi, 3)));
+                            asm volatile("" : "+v"(mins[j].x), "+v"(mins[j].y), "+v"(mins[j].z), "+v"(mins[j].w));
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            if (s == 7) {
+                // The min term of the whole super-block, sum over sub-blocks of m[column][sub] * X[row][sub]: A = the three bf16
+                // parts of the eight sub-block sums of each row (K = part * 8 + sub), B = the eight 6-bit mins of each column
+                // (nothing for the last eight K).
+#pragma unroll
+                for (int i = 0; i < kR; ++i) {
+                    const int now = i & 1, before = now ^ 1, i_before = (i + kR - 1) % kR;  // (step 8 kR + i)
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        union {
+                            t_bf16x8 v;
+                            uint4 u;
+                        } sa, mb;
+                        sa.u = sum_parts[m];
+#pragma unroll
+                        for (int j = 0; j < kC; ++j) {
+                            mb.u = mins[j];
+                            if (m == 1) mb.u = make_uint4(mb.u.x & first_half, mb.u.y & first_half, mb.u.z & first_half, mb.u.w & first_half);
+                            D[now][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa.v, mb.v, m == 0 ? t_f32x16{} : D[now][j], 0, 0, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (m == 1 && j == kC - 1 && i + 1 < kR) read_sums(i + 1);
+                            accumulate(before, i_before, j, 8 * m, 8 * (m + 1));
+                            if (m == 1) factor[now][j] = -half_bits_to_f32(static_cast<uint16_t>(hdr[j].x >> 16));
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                }
+                if (kR & 1) {  // an odd number of steps: the next super-block expects the last one in the second set
+#pragma unroll
+                    for (int j = 0; j < kC; ++j) {
+                        D[1][j] = D[0][j];
+                        factor[1][j] = factor[0][j];
+                    }
+                }
+            }
+            // stage s + 2 has landed for every wavefront: the next stage reads its operands ahead
+            if (s == 5) q4k_wait_vm<kLoadsFirst>();
+            else if (s & 1) q4k_wait_vm<kLoadsEven>();
+            else q4k_wait_vm<kLoadsOdd>();
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kC; ++j) accumulate(1, kR - 1, j, 0, 16);
+    q4k_wait_vm<0>();  // what is still on its way to LDS lands before the workgroup ends
+
+    // Results.  Plain ones go straight out of the registers; an epilogue is a loop over a copy in LDS, not 64 copies of its code
+    // in a row (45 KB of them: 333 x 4096 x 4096 79 -> 76 us without).
+    const int row0 = m_group * S::kRows + 4 * g, col0 = (tile0 + wave * kC) * kTileCols + c;
+    if (partial != nullptr || (ep.bias == nullptr && ep.residual == nullptr && ep.activation == kActNone)) {
+        float* out = partial != nullptr ? partial + static_cast<size_t>(blockIdx.y) * rows * out_dim : dst;
+#pragma unroll
+        for (int j = 0; j < kC; ++j) {
+            if (col0 + j * kTileCols >= out_dim) continue;
+#pragma unroll
+            for (int i = 0; i < kR; ++i) {
+                float* to = out + static_cast<size_t>(row0 + i * kG32Rows) * out_dim + col0 + j * kTileCols;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int r = 8 * (v >> 2) + (v & 3);
+                    if (row0 + i * kG32Rows + r < rows) to[static_cast<size_t>(r) * out_dim] = acc[i][j][v];
+                }
+            }
+        }
+        return;
+    }
+    __syncthreads();  // every wavefront's loads have landed: the ring is free
+    static_assert(kR * kC * kWaves * 4096 <= S::kLdsBytes, "a tile of results is 4 KB");
+    float* copy = reinterpret_cast<float*>(q4k_mfma_lds) + wave * (kR * kC * 1024) + lane;
+#pragma unroll
+    for (int i = 0; i < kR; ++i)
+#pragma unroll
+        for (int j = 0; j < kC; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) copy[((i * kC + j) * 16 + v) * 64] = acc[i][j][v];
+#pragma unroll 1
+    for (int n = 0; n < kR * kC * 16; ++n) {  // a lane reads back what it wrote
+        const int v = n & 15, j = (n >> 4) % kC, i = (n >> 4) / kC;
+        const int r = row0 + i * kG32Rows + 8 * (v >> 2) + (v & 3), o = col0 + j * kTileCols;
+        if (r < rows && o < out_dim) {
+            const size_t at = static_cast<size_t>(r) * out_dim + o;
+            dst[at] = finish_output(ep, o, at, copy[n * 64]);
+        }
+    }
+}
+
 size_t q4k_mfma_lds_bytes(int rows, int in_dim, int waves, int groups) {
     return static_cast<size_t>(rows) * 3 * (static_cast<size_t>(in_dim) * 2 + kRowPadBytes) +
            static_cast<size_t>(rows) * (in_dim / 32) * 4 + static_cast<size_t>(waves) * groups * 64 * 4;
@@ -1118,51 +1632,168 @@ int device_units() {
     return cus;
 }
 
-// K shares of the GEMM: one when its workgroups fill the compute units anyway, else as many
-// (a power of two, at most eight, at least two super-blocks each) as spread it over them.
-int gemm_q4k_splits(size_t rows, size_t in_dim, size_t out_dim) {
-    const long workgroups = static_cast<long>((out_dim + 255) / 256) * static_cast<long>((rows + kG32Rows - 1) / kG32Rows);
+// What serves a GEMM call: the bf16 kernel (kParts), or the fp6 kernel with one of its tiles; and over how many workgroups K is
+// shared out (a power of two, at most eight, at least two super-blocks each).
+enum Q4kGemmKind { kParts, kFp6Tile64x256, kFp6Tile64x128, kFp6Tile32x128 };
+struct Q4kGemmPlan {
+    Q4kGemmKind kind;
+    int splits;
+};
+
+// Time of a call in us, from the rounds of the busiest XCD's compute units.  `steps[n]`: a sub-block of a wavefront's tiles with n + 1
+// workgroups on the unit; `round`: start and drain of a workgroup; `shares`, `share_mb`: the reduce launch and its MB; `split`: per
+// million values of X; `out`: per MB of Y.  Fitted to 1600 timed calls (65 .. 2048 rows, K 1024 .. 14336, N 1536 .. 14336; 5 % rms);
+// over these the choice is 3 % from the best tile and share count on the mean.
+struct Q4kGemmCost {
+    int rows, cols, tiles, resident;
+    double steps[4], round, base, shares, share_mb, split, out;
+    double us(double m, double k, double n, int s) const {
+        const long long groups = static_cast<long long>((m + rows - 1) / rows) * static_cast<long long>((n + cols - 1) / cols);
+        const long long units = device_units() >= 8 ? device_units() / 8 : 1;
+        const long long per_unit = ((groups + 7) / 8 * s + units - 1) / units, kb = static_cast<long long>(k / kQ4kBlockValues);
+        const double work = static_cast<double>(tiles * 8 * ((kb + s - 1) / s)), mb = m * n * 4e-6;
+        const long long full = per_unit / resident, rest = per_unit % resident;
+        double t = static_cast<double>(full) * work * steps[resident - 1] + static_cast<double>(full + (rest > 0)) * round + base;
+        if (rest > 0) t += work * steps[rest - 1];
+        if (s > 1) t += shares + share_mb * (s + 1) * mb;
+        return t + split * m * k * 1e-6 + out * mb;
+    }
+};
+constexpr Q4kGemmCost kQ4kGemmCosts[4] = {
+    {32, 256, 1, 2, {0.351, 0.609, 0, 0}, 3.2, 3.2, 0.0, 0.40, 3.3, 0.32},
+    {64, 256, 4, 2, {0.108, 0.213, 0, 0}, 3.2, 5.7, 3.2, 0.16, 3.7, 0.31},
+    {64, 128, 2, 2, {0.138, 0.258, 0, 0}, 1.2, 6.3, 2.8, 0.20, 3.5, 0.26},
+    {32, 128, 1, 4, {0.219, 0.329, 0.490, 0.627}, 0.0, 7.2, 2.5, 0.21, 3.1, 0.25},
+};
+
+// `pair`: for both matrices of a pair in one launch (one share); its tile may be another than the single call's, as a result's bits
+// depend on the shares alone (333 x 4096 x 14336 twice: 64 x 256 tiles 212 us, 64 x 128 231; once 124 / 119).
+// Up to 64 rows the bf16 kernel is the faster one (64 x 4096 x 4096 17.5 against 19.4 us, 32 x 4096 x 14336 21.4 / 22.4) and keeps its
+// own shares: one when its workgroups fill the compute units anyway, else as many as spread it over them.  Above, the tile and
+// share count that cost least -- one share where that costs at most 3 % more, since a pair is one launch then -- unless the bf16
+// kernel is expected within 3 % of it (small matrices: 200 x 2048 x 2048 17.3 against 20.4; 333 x 2048 x 5632 36.9 / 40.6, a grid that
+// just fills its rounds).
+Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, bool pair = false) {
     const int kb = static_cast<int>(in_dim / kQ4kBlockValues);
-    int splits = 1;
-    while (splits < 8 && workgroups * splits * 2 <= device_units() && kb / (splits * 2) >= 2) splits *= 2;
-    return splits;
+    const double m = static_cast<double>(rows), k = static_cast<double>(in_dim), n = static_cast<double>(out_dim);
+    auto allowed = [&](int s) { return s == 1 || (s <= 8 && kb / s >= 2); };
+    Q4kGemmPlan parts{kParts, 1};
+    const long long workgroups = static_cast<long long>((out_dim + 255) / 256) * static_cast<long long>((rows + kG32Rows - 1) / kG32Rows);
+    while (workgroups * parts.splits * 2 <= device_units() && allowed(parts.splits * 2)) parts.splits *= 2;
+    if (rows <= 64) return parts;
+    Q4kGemmPlan best{kFp6Tile64x256, 1};
+    double best_us = 1e30;
+    for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
+        for (int s = 1; allowed(s); s *= 2) {
+            const double us = kQ4kGemmCosts[kind].us(m, k, n, s) * (s == 1 ? 1.0 : 1.03);
+            if (us < best_us) {
+                best_us = us;
+                best = {static_cast<Q4kGemmKind>(kind), s};
+            }
+        }
+    if (kQ4kGemmCosts[kParts].us(m, k, n, parts.splits) * 0.97 < best_us) return parts;
+    if (pair && best.splits == 1) {
+        best_us = 1e30;
+        for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
+            if (const double us = kQ4kGemmCosts[kind].us(m, k, 2 * n, 1); us < best_us) {
+                best_us = us;
+                best.kind = static_cast<Q4kGemmKind>(kind);
+            }
+    }
+    return best;
 }
 
-size_t gemm_q4k_split_bytes(size_t rows, size_t in_dim) { return (rows * in_dim * 6 + rows * (in_dim / 32) * 8 + 255) / 256 * 256; }
+// The parts or digits of X; the fp6 kernel's rows are padded to even.
+size_t gemm_q4k_digit_bytes(size_t rows, size_t in_dim) { return (rows + 1) / 2 * 2 * in_dim * 6; }
+size_t gemm_q4k_split_bytes(const Q4kGemmPlan& plan, size_t rows, size_t in_dim) {
+    const size_t values = plan.kind == kParts ? rows * in_dim * 6 : gemm_q4k_digit_bytes(rows, in_dim);
+    return (values + rows * (in_dim / 32) * 8 + 255) / 256 * 256;
+}
+
+struct Q4kGemmCall {
+    hipStream_t stream;
+    float* dst;
+    const uint8_t *digits, *sums, *weight;
+    int rows, in_dim, out_dim, sb_per_split, shares;
+    float* partial;
+    const Epilogue& ep;
+    const Q4kSecond* second;
+};
+
+template <int kWaves, int kR, int kC, int kOcc>
+hipError_t launch_fp6_tile(const Q4kGemmCall& q) {
+    using S = G6Shape<kWaves, kR, kC>;
+    const int m_groups = (q.rows + S::kRows - 1) / S::kRows, n_groups = (q.out_dim + S::kCols - 1) / S::kCols;
+    const long long grid = (static_cast<long long>(n_groups) * m_groups + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    auto kernel = gemm_q4k_fp6_kernel<kWaves, kR, kC, kOcc>;
+    static std::atomic<bool> attr_done{false};
+    if (S::kLdsBytes > 64 * 1024 && !attr_done.load(std::memory_order_acquire)) {
+        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLdsBytes);
+            e != hipSuccess)
+            return e;
+        attr_done.store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), q.shares, q.second ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, q.stream, q.dst,
+                       q.digits, q.sums, q.weight, q.rows, q.in_dim, q.out_dim, m_groups, n_groups, 8, q.sb_per_split, q.partial, q.ep,
+                       q.second ? *q.second : Q4kSecond{nullptr, nullptr, Epilogue{}});
+    return hipGetLastError();
+}
 }  // namespace
 
 size_t gemm_q4k_workspace_bytes(size_t rows, size_t in_dim, size_t out_dim) {
-    const int splits = gemm_q4k_splits(rows, in_dim, out_dim);
-    return gemm_q4k_split_bytes(rows, in_dim) + (splits > 1 ? static_cast<size_t>(splits) * rows * out_dim * 4 : 0);
+    const Q4kGemmPlan plan = gemm_q4k_plan(rows, in_dim, out_dim);
+    return gemm_q4k_split_bytes(plan, rows, in_dim) + (plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * out_dim * 4 : 0);
 }
 
 hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, void* workspace,
-                                 int rows, int in_dim, int out_dim, const Epilogue& ep, bool split) {
+                                 int rows, int in_dim, int out_dim, const Epilogue& ep, float* dst_b, const uint8_t* weight_b,
+                                 const Epilogue& ep_b) {
     if (in_dim % kQ4kBlockValues != 0 || rows < 1 || workspace == nullptr) return hipErrorInvalidValue;
-    uint32_t* parts = static_cast<uint32_t*>(workspace);
-    uint16_t* xsum = reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(workspace) + static_cast<size_t>(rows) * in_dim * 6);
-    const int splits = gemm_q4k_splits(rows, in_dim, out_dim);
+    const Q4kGemmPlan plan = gemm_q4k_plan(static_cast<size_t>(rows), static_cast<size_t>(in_dim), static_cast<size_t>(out_dim),
+                                           dst_b != nullptr);
     const int kb = in_dim / kQ4kBlockValues;
-    const int sb_per_split = (kb + splits - 1) / splits;
+    const int sb_per_split = (kb + plan.splits - 1) / plan.splits;
     const int shares = (kb + sb_per_split - 1) / sb_per_split;  // no empty share
-    float* partial = shares > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + gemm_q4k_split_bytes(rows, in_dim)) : nullptr;
-    if (split) {
+    uint8_t* const space = static_cast<uint8_t*>(workspace);
+    float* partial = shares > 1 ? reinterpret_cast<float*>(space + gemm_q4k_split_bytes(plan, rows, in_dim)) : nullptr;
+    const int m_tiles = (rows + kG32Rows - 1) / kG32Rows;
+    if (m_tiles > 65535) return hipErrorInvalidValue;
+    uint32_t* parts = static_cast<uint32_t*>(workspace);
+    uint16_t* part_sums = reinterpret_cast<uint16_t*>(space + static_cast<size_t>(rows) * in_dim * 6);
+    uint8_t* digit_sums = space + gemm_q4k_digit_bytes(rows, in_dim);
+    if (plan.kind == kParts) {
         const size_t groups = static_cast<size_t>(rows) * (in_dim >> 3);
         size_t split_grid = (groups + 255) / 256;
         if (split_grid > 65536) split_grid = 65536;
-        hipLaunchKernelGGL(q4k_split_rows_kernel, dim3(static_cast<unsigned>(split_grid)), dim3(256), 0, stream, x, parts, xsum,
+        hipLaunchKernelGGL(q4k_split_parts_kernel, dim3(static_cast<unsigned>(split_grid)), dim3(256), 0, stream, x, parts, part_sums,
                            groups, in_dim >> 3);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    } else {
+        hipLaunchKernelGGL(q4k_split_digits_kernel, dim3(in_dim / 32, m_tiles), dim3(64), 0, stream, x, space, digit_sums, rows, in_dim);
     }
-    const int n_tiles = (out_dim + kTileCols - 1) / kTileCols;
-    const unsigned grid_y = static_cast<unsigned>((rows + kG32Rows - 1) / kG32Rows);
-    if (grid_y > 65535) return hipErrorInvalidValue;
-    const unsigned grid_x = static_cast<unsigned>((n_tiles + 7) / 8);
-    static_assert(2 * kG32ChunkBytes <= 64 * 1024, "no raised LDS limit");
-    hipLaunchKernelGGL(gemm_q4k_rows32_kernel, dim3(grid_x, grid_y, shares), dim3(512), 2 * kG32ChunkBytes, stream, dst, parts,
-                       xsum, weight, rows, in_dim, out_dim, sb_per_split, partial, ep);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess || shares == 1) return e;
-    return launch_splitk_reduce(stream, dst, partial, static_cast<size_t>(rows) * out_dim, out_dim, shares, ep);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    const Q4kSecond second{dst_b, weight_b, ep_b};
+    auto multiply = [&](float* y, const uint8_t* w, const Epilogue& epilogue, const Q4kSecond* with) {
+        const Q4kGemmCall q{stream, y, space, digit_sums, w, rows, in_dim, out_dim, sb_per_split, shares, partial, epilogue, with};
+        hipError_t e;
+        if (plan.kind == kFp6Tile64x256) e = launch_fp6_tile<4, 2, 2, 2>(q);
+        else if (plan.kind == kFp6Tile64x128) e = launch_fp6_tile<4, 2, 1, 2>(q);
+        else if (plan.kind == kFp6Tile32x128) e = launch_fp6_tile<4, 1, 1, 3>(q);
+        else {
+            static_assert(2 * kG32ChunkBytes <= 64 * 1024, "no raised LDS limit");
+            const unsigned grid_x = static_cast<unsigned>((out_dim + 255) / 256);
+            hipLaunchKernelGGL(gemm_q4k_rows32_kernel, dim3(grid_x, m_tiles, shares), dim3(512), 2 * kG32ChunkBytes, stream, y, parts,
+                               part_sums, w, rows, in_dim, out_dim, sb_per_split, partial, epilogue);
+            e = hipGetLastError();
+        }
+        if (e != hipSuccess || shares == 1) return e;
+        return launch_splitk_reduce(stream, y, partial, static_cast<size_t>(rows) * out_dim, out_dim, shares, epilogue);
+    };
+    if (dst_b == nullptr) return multiply(dst, weight, ep, nullptr);
+    if (shares == 1 && plan.kind != kParts) return multiply(dst, weight, ep, &second);
+    // (the partial sums have room for one matrix)
+    if (hipError_t e = multiply(dst, weight, ep, nullptr); e != hipSuccess) return e;
+    return multiply(dst_b, weight_b, ep_b, nullptr);
 }
 
 // Three to eight rows with the caller's scratch: the digit planes of X made once by their own kernel

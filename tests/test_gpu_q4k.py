@@ -401,6 +401,62 @@ def test_prefill_full_size_with_epilogue():
     assert np.array_equal(yb, y + b[None, :])
 
 
+# rows, K, N.  Part tiles of rows (1 .. 31 past a multiple of 32 or 64) and columns; the fp6 kernel's tiles 32 x 128 (single calls of the
+# first five), 64 x 128 and 64 x 256; two, four and eight K shares of even and uneven length; pairs on another tile than the single
+# call; shapes that stay on the bf16 kernel (the last two)
+FP6_SHAPES = [(66, 512, 1000), (95, 768, 97), (127, 1280, 4097), (513, 512, 1025), (67, 14336, 1000), (140, 6144, 5000), (66, 14336, 4096),
+              (200, 1536, 8192), (333, 4096, 6144), (1025, 2048, 4096), (65, 256, 33), (97, 4096, 513)]
+
+@pytest.mark.parametrize("rows,in_dim,out_dim", FP6_SHAPES)
+def test_prefill_past_64_rows(rows, in_dim, out_dim):
+    """Six-bit digits of X on the matrix cores: against the float64 oracle on sampled rows (the f32 sums' own error: 2^-24 per
+    addition, K / 32 additions, as for the other kernels of the format); a pair is two single calls, bit for bit; biases."""
+    print(f"case: q4_k fp6 prefill rows={rows} in={in_dim} out={out_dim}", flush=True)
+    assert not O.uses_q4k_q8k_activation(rows, in_dim, out_dim)
+    wa, wb = synth.weights(Q4K, 81, out_dim, in_dim), synth.weights(Q4K, 82, out_dim, in_dim)
+    x = synth.activations(83, rows, in_dim)
+    x[:, ::97] *= 20.0   # large channels
+    x[rows // 2] = 0.0   # a row of zeros
+    da, db = device_weight(PREP, wa, out_dim, in_dim), device_weight(PREP, wb, out_dim, in_dim)
+    y = G.linear(Q4K, PREP, x, da, rows, in_dim, out_dim)
+    sample = np.unique(np.r_[0, 1, 30:34, rows // 2, 62:67, rows - 2, rows - 1] % rows)
+    assert G.max_rel_err(y[sample], O.linear_q4_k(x[sample], wa, len(sample), in_dim, out_dim, f64=True)) <= TIGHT
+    assert not y[rows // 2].any()
+    ya, yb = G.linear_pair(Q4K, PREP, x, da, db, rows, in_dim, out_dim)
+    assert np.array_equal(ya, y) and np.array_equal(yb, G.linear(Q4K, PREP, x, db, rows, in_dim, out_dim))
+    b = synth.activations(84, 1, out_dim)[0]
+    assert np.array_equal(G.linear_bias(Q4K, PREP, x, da, b, rows, in_dim, out_dim), y + b[None, :])
+
+
+def test_prefill_past_64_rows_on_extreme_activations():
+    """The digits' range: X scaled by powers of two scales Y exactly down to 2^-100 (and at 2^-120, where sub-blocks lie below the
+    digits' lowest scale, to the f32 sums' precision); a sub-block may hold values 2^120 apart; an infinity or a NaN
+    makes its own row NaN and no other."""
+    rows, in_dim, out_dim = 66, 512, 1000
+    print("case: q4_k fp6 prefill on extreme activations", flush=True)
+    w = synth.weights(Q4K, 85, out_dim, in_dim)
+    wd = device_weight(PREP, w, out_dim, in_dim)
+    x = synth.activations(86, rows, in_dim)
+    y = G.linear(Q4K, PREP, x, wd, rows, in_dim, out_dim)
+    for e in (-100, -60, 60, 100):
+        s = np.float32(2.0) ** e
+        assert np.array_equal(G.linear(Q4K, PREP, x * s, wd, rows, in_dim, out_dim), y * s), e
+    tiny = x * np.float32(2.0) ** -120
+    ref = O.linear_q4_k(tiny, w, rows, in_dim, out_dim, f64=True)
+    got = G.linear(Q4K, PREP, tiny, wd, rows, in_dim, out_dim)
+    # results near 2^-120 carry 2^-149 of absolute error per addition: 2^-29 of them, below the sums' own
+    assert G.max_rel_err(got, ref) <= TIGHT
+    mixed = x.copy()
+    mixed[:, 1::2] *= np.float32(2.0) ** -120
+    assert G.max_rel_err(G.linear(Q4K, PREP, mixed, wd, rows, in_dim, out_dim), O.linear_q4_k(mixed, w, rows, in_dim, out_dim, f64=True)) <= TIGHT
+    bad = x.copy()
+    bad[3, 5], bad[40, 300], bad[65, 511] = np.inf, np.nan, -np.inf
+    got = G.linear(Q4K, PREP, bad, wd, rows, in_dim, out_dim)
+    hit = np.isin(np.arange(rows), (3, 40, 65))
+    assert np.isnan(got[hit]).all()
+    assert np.array_equal(got[~hit], y[~hit])
+
+
 def test_linear_argument_checks():
     w = G.to_dev(synth.weights(Q4K, 1, 4, 256))
     x = G.to_dev(synth.activations(2, 1, 256))
