@@ -37,6 +37,12 @@ afhip_status linear_impl(void* stream, int tensor_type, int layout, afhip_buffer
                          afhip_buffer dst_b = afhip_buffer{0, 0}, afhip_buffer weight_b = afhip_buffer{0, 0},
                          const LinearExtras& extras = LinearExtras{});
 
+// Three matrices on the same X in one launch, where linear_triple_shares_launch says so (biases on all of them).
+bool linear_triple_shares_launch(int tensor_type, int layout, size_t rows, size_t in_dim, size_t out_dim);
+afhip_status linear_triple_impl(void* stream, const afhip_buffer (&dst)[3], afhip_buffer input, const afhip_buffer (&weight)[3],
+                                const afhip_buffer (&bias)[3], size_t rows, size_t in_dim, size_t out_dim, afhip_buffer workspace,
+                                LaunchCounters* counters);
+
 // argmax over the last row of f32 [rows, dim]; `workspace` (optional) lets several workgroups scan a long row.
 afhip_status argmax_last_row_impl(void* stream, afhip_buffer token_u32, afhip_buffer token_f32, afhip_buffer input,
                                   size_t rows, size_t dim, afhip_buffer workspace);

@@ -248,19 +248,17 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
                 else if (kind == AFHIP_DISPATCH_SMALL_BATCH) counters->small_batch++;
                 else counters->mm++;
             }
-            if (fused) {  // a pair: both matrices in one launch
-                if (i == 0)
-                    e = launch_linear_q4k_q8k_fused(stream, reinterpret_cast<float*>(dst.ptr), reinterpret_cast<const float*>(input.ptr),
-                                                    reinterpret_cast<const uint8_t*>(weight.ptr), static_cast<int>(rows),
-                                                    static_cast<int>(in_dim), static_cast<int>(out_dim), ep,
-                                                    pair ? reinterpret_cast<float*>(dst_b.ptr) : nullptr,
-                                                    pair ? reinterpret_cast<const uint8_t*>(weight_b.ptr) : nullptr, ep_b);
-                continue;
-            }
-            e = launch_linear_q4k_q8k(stream, reinterpret_cast<float*>(i ? dst_b.ptr : dst.ptr),
-                                      reinterpret_cast<const void*>(workspace.ptr),
-                                      reinterpret_cast<const uint8_t*>(i ? weight_b.ptr : weight.ptr), tiled,
-                                      static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), i ? ep_b : ep);
+            if (i == 1) continue;  // a pair goes down together
+            float* y = reinterpret_cast<float*>(dst.ptr);
+            float* y_b = pair ? reinterpret_cast<float*>(dst_b.ptr) : nullptr;
+            const uint8_t* w = reinterpret_cast<const uint8_t*>(weight.ptr);
+            const uint8_t* w_b = pair ? reinterpret_cast<const uint8_t*>(weight_b.ptr) : nullptr;
+            if (fused)
+                e = launch_linear_q4k_q8k_fused(stream, y, reinterpret_cast<const float*>(input.ptr), w, static_cast<int>(rows),
+                                                static_cast<int>(in_dim), static_cast<int>(out_dim), ep, y_b, w_b, ep_b);
+            else
+                e = launch_linear_q4k_q8k(stream, y, reinterpret_cast<const void*>(workspace.ptr), w, tiled, static_cast<int>(rows),
+                                          static_cast<int>(in_dim), static_cast<int>(out_dim), ep, y_b, w_b, ep_b);
         }
         return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
     }
@@ -323,6 +321,44 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
         if (e != hipSuccess) return static_cast<afhip_status>(e);
     }
     return AFHIP_OK;
+}
+
+// Three matrices of one shape on the same X as one quantizer and one matmul launch, for the gated shapes whose kernel takes
+// them together (linear_triple_shares_launch); the caller has checked every tensor's size and type.
+bool linear_triple_shares_launch(int tensor_type, int layout, size_t rows, size_t in_dim, size_t out_dim) {
+    return tensor_type == AFHIP_TYPE_Q4_K && layout == AFHIP_LAYOUT_PREPARED && rows <= 0x7fffffff && out_dim <= 0x7fffffff &&
+           afhip_uses_q8k_activation_quant(tensor_type, rows, in_dim, out_dim) && linear_q4k_q8k_shares_launch(true, rows, in_dim);
+}
+
+afhip_status linear_triple_impl(void* stream_v, const afhip_buffer (&dst)[3], afhip_buffer input, const afhip_buffer (&weight)[3],
+                                const afhip_buffer (&bias)[3], size_t rows, size_t in_dim, size_t out_dim, afhip_buffer workspace,
+                                LaunchCounters* counters) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_v);
+    if (!linear_triple_shares_launch(AFHIP_TYPE_Q4_K, AFHIP_LAYOUT_PREPARED, rows, in_dim, out_dim)) return AFHIP_ERR_INVALID_ARGUMENT;
+    const size_t y_bytes = rows * out_dim * 4;  // (the gate bounds every dimension but out_dim, which is an int)
+    if (input.ptr == 0 || input.ptr % 16 != 0 || input.len < rows * in_dim * 4 || workspace.ptr == 0 || workspace.ptr % 16 != 0 ||
+        workspace.len < q4k_q8k_workspace_bytes(rows, in_dim))
+        return AFHIP_ERR_INVALID_STATE;
+    for (int i = 0; i < 3; ++i)
+        if (dst[i].ptr == 0 || dst[i].ptr % 4 != 0 || dst[i].len < y_bytes || weight[i].ptr == 0 || weight[i].ptr % 16 != 0 ||
+            weight[i].len < q4k_tiled_bytes(out_dim, in_dim) || bias[i].ptr == 0 || bias[i].ptr % 4 != 0 || bias[i].len < out_dim * 4)
+            return AFHIP_ERR_INVALID_STATE;
+    if (counters) {
+        counters->activation_quant++;
+        const int kind = afhip_quant_matmul_select(rows, in_dim, out_dim, AFHIP_FORMAT_Q4_K);
+        (kind == AFHIP_DISPATCH_MMV ? counters->mmv : kind == AFHIP_DISPATCH_SMALL_BATCH ? counters->small_batch : counters->mm) += 3;
+    }
+    hipError_t e = launch_quantize_q8k(stream, reinterpret_cast<const float*>(input.ptr), static_cast<int>(rows), static_cast<int>(in_dim),
+                                       reinterpret_cast<void*>(workspace.ptr));
+    if (e != hipSuccess) return static_cast<afhip_status>(e);
+    Epilogue ep[3];
+    for (int i = 0; i < 3; ++i) ep[i].bias = reinterpret_cast<const float*>(bias[i].ptr);
+    e = launch_linear_q4k_q8k(stream, reinterpret_cast<float*>(dst[0].ptr), reinterpret_cast<const void*>(workspace.ptr),
+                              reinterpret_cast<const uint8_t*>(weight[0].ptr), true, static_cast<int>(rows), static_cast<int>(in_dim),
+                              static_cast<int>(out_dim), ep[0], reinterpret_cast<float*>(dst[1].ptr),
+                              reinterpret_cast<const uint8_t*>(weight[1].ptr), ep[1], reinterpret_cast<float*>(dst[2].ptr),
+                              reinterpret_cast<const uint8_t*>(weight[2].ptr), ep[2]);
+    return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
 }
 
 static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout, afhip_buffer dst, afhip_buffer input,

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cmath>
+#include <array>
 #include <cstring>
 #include <new>
 #include <string>
@@ -269,6 +270,50 @@ afhip_status linear_no_bias_impl(afhip_compute* self, const afhip_tensor* input,
             delete *out;
             *out = nullptr;
         }
+    }
+    return s;
+}
+
+// The three results of a triple whose weights one launch takes; *shared says whether this was such a call (nothing was done if not).
+afhip_status linear_triple_shared(afhip_compute* self, const afhip_tensor* input, const std::array<const afhip_tensor*, 3>& weights,
+                                  const std::array<const afhip_tensor*, 3>& biases, size_t rows, size_t in_dim, size_t out_dim,
+                                  const std::array<afhip_tensor**, 3>& out, bool* shared) {
+    *shared = false;
+    if (!self || !input || !is_f32(input) || self->phase_timing || self->q4k_f32_activations) return AFHIP_OK;
+    size_t in_count, w_count, out_count, out_bytes;
+    if (!checked_mul(rows, in_dim, &in_count) || !checked_mul(out_dim, in_dim, &w_count) || !checked_mul(rows, out_dim, &out_count) ||
+        !checked_mul(out_count, 4, &out_bytes) || input->elem_count != in_count)
+        return AFHIP_OK;
+    for (int i = 0; i < 3; ++i) {
+        const afhip_tensor *w = weights[i], *b = biases[i];
+        if (!w || !b || !out[i] || w->elem_count != w_count || !is_f32(b) || b->elem_count != out_dim ||
+            !linear_triple_shares_launch(w->quant_type, w->layout, rows, in_dim, out_dim))
+            return AFHIP_OK;
+    }
+    *shared = true;
+    for (afhip_tensor** t : out) *t = nullptr;
+    afhip_status s = make_current(self);
+    if (s != AFHIP_OK) return s;
+    afhip_buffer device[3] = {};
+    for (int i = 0; i < 3 && s == AFHIP_OK; ++i) s = alloc_device_buffer(self, out_bytes, &device[i]);
+    afhip_buffer scratch{0, 0};
+    if (s == AFHIP_OK) s = acquire_scratch(self, afhip_linear_workspace_bytes(AFHIP_TYPE_Q4_K, rows, in_dim, out_dim), &scratch);
+    if (s == AFHIP_OK)
+        s = linear_triple_impl(self->stream, device, input->buffer, {weights[0]->buffer, weights[1]->buffer, weights[2]->buffer},
+                               {biases[0]->buffer, biases[1]->buffer, biases[2]->buffer}, rows, in_dim, out_dim, scratch, &self->counters);
+    for (int i = 0; i < 3; ++i) {
+        if (s == AFHIP_OK) {
+            s = make_f32_result(self, device[i], rows, out_dim, out_count, out[i]);  // (gives the buffer back if it fails)
+            if (s == AFHIP_OK) continue;
+        } else if (device[i].ptr != 0) {
+            release_device_buffer(self, &device[i]);
+        }
+        for (int k = 0; k < i; ++k)
+            if (*out[k]) {
+                free_tensor_storage(self, *out[k]);
+                delete *out[k];
+                *out[k] = nullptr;
+            }
     }
     return s;
 }
@@ -623,9 +668,15 @@ afhip_status afhip_compute_linear_triple(afhip_compute* self, const afhip_tensor
                                          const afhip_tensor* bias_c, size_t rows, size_t in_dim, size_t out_dim,
                                          afhip_tensor** out_first, afhip_tensor** out_second,
                                          afhip_tensor** out_third) {
-    // Q/K/V with separate weights: the first two share one launch where a pair does, the third follows
+    // Q/K/V with separate weights: one launch where a kernel takes all three; else the first two share one where a pair does and
+    // the third follows (as does every call that is not in order: the ops below say what is wrong with it)
     if (!out_third || !weight_c || !bias_c) return AFHIP_ERR_INVALID_ARGUMENT;
     *out_third = nullptr;
+    bool shared = false;
+    if (const afhip_status s = linear_triple_shared(self, input, {weight_a, weight_b, weight_c}, {bias_a, bias_b, bias_c}, rows, in_dim,
+                                                    out_dim, {out_first, out_second, out_third}, &shared);
+        shared || s != AFHIP_OK)
+        return s;
     afhip_status s = afhip_compute_linear_pair(self, input, weight_a, bias_a, weight_b, bias_b, rows, in_dim, out_dim,
                                                out_first, out_second);
     if (s != AFHIP_OK) return s;

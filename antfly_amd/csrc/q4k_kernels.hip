@@ -733,6 +733,100 @@ __global__ __launch_bounds__(768) void linear_q4k_q8k_tiled_kernel(float* __rest
     }
 }
 
+// More rows than nine: the sub-block dots on v_mfma_i32_32x32x32_i8.  A workgroup owns 32 rows x 32 columns, wavefront w
+// super-block w of them (blockDim.x = 64 * in_dim / 256, at most 12): lane (column c, half g) holds values 16 g .. 16 g + 15 of the
+// column's sub-blocks -- the tile-major layout's 16 bytes, masked -- and lane (row c, half g) the same values of its row, read
+// from where the quantizer left them.  D register v is row 8 (v / 4) + 4 g + v % 4, column c: the whole sub-block's dot, exact.  The
+// min terms, (dmin m) * f32(sum q_x), come off two sub-blocks at a time by a v_mfma_f32_32x32x2_f32 (exact products, f32 sums)
+// before their (d sc) * f32(dot) are added; times the row's scale, the super-blocks' results meet in LDS in ascending order.
+// Up to three matrices of one shape on the same X (grid.z; Q, K and V).
+// Bound by the launch and the first loads' latency.  77 rows, kernel time by rocprofv3 against the dot4 kernel above, which walks its
+// rows one after the other: 3072 x 768 12.4 -> 8.7 us, 768 x 3072 8.7 -> 7.5, Q, K and V of 768 x 768 three launches of 5.8 -> one of
+// 7.4; error against 64 bits 3.3e-7 -> 1.5e-7 (an encoder's layers).
+typedef int q8k_v4i __attribute__((ext_vector_type(4)));
+typedef int q8k_v4i_any __attribute__((ext_vector_type(4), aligned(4)));  // (the sums start behind rows * in_dim / 256 scales)
+typedef int q8k_v16i __attribute__((ext_vector_type(16)));
+typedef float q8k_v16f __attribute__((ext_vector_type(16)));
+constexpr int kQ8kMfmaRows = 32;
+
+__global__ __launch_bounds__(768) void linear_q4k_q8k_mfma_kernel(float* __restrict__ dst, const int8_t* __restrict__ q,
+                                                                 const float* __restrict__ xd, const int* __restrict__ sums,
+                                                                 const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim,
+                                                                 Epilogue ep, Q8kSecond second, Q8kSecond third) {
+    if (blockIdx.z != 0) {
+        dst = blockIdx.z == 1 ? second.dst : third.dst;
+        weight = blockIdx.z == 1 ? second.weight : third.weight;
+        ep = blockIdx.z == 1 ? second.ep : third.ep;
+    }
+    extern __shared__ __align__(16) unsigned char q8k_lds[];
+    const int kb = in_dim / kQ4kBlockValues;
+    const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int tile = blockIdx.x, row0 = blockIdx.y * kQ8kMfmaRows;
+    float* red = reinterpret_cast<float*>(q8k_lds);    // [kb][16][64]
+    float* xd_s = red + kb * 1024;                     // [kb][32]
+    const size_t row = min(row0 + c, rows - 1);        // rows past the end repeat the last one and are not stored
+    const uint8_t* tbase = weight + (static_cast<size_t>(tile) * kb + wave) * (32 * kQ4kBlockBytes);
+    const q4k_u32x4 header = *reinterpret_cast<const q4k_u32x4*>(tbase + c * 16);
+    q4k_u32x4 nib[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) nib[t] = *reinterpret_cast<const q4k_u32x4*>(tbase + 512 + t * 1024 + lane * 16);
+    q8k_v4i a[8];
+    const int8_t* xrow = q + row * in_dim + wave * kQ4kBlockValues + 16 * g;
+#pragma unroll
+    for (int sub = 0; sub < 8; ++sub) a[sub] = *reinterpret_cast<const q8k_v4i*>(xrow + sub * 32);
+    const q8k_v4i_any* srow = reinterpret_cast<const q8k_v4i_any*>(sums + (row * kb + wave) * 8);
+    const q8k_v4i s_lo = srow[0], s_hi = srow[1];
+    if (lane < 32) xd_s[wave * 32 + lane] = xd[row * kb + wave];
+
+    float dsc[8], dmn[8];
+    {
+        const float d = half_bits_to_f32(static_cast<uint16_t>(header.x & 0xFFFFu));
+        const float dmin = half_bits_to_f32(static_cast<uint16_t>(header.x >> 16));
+#pragma unroll
+        for (int sub = 0; sub < 8; ++sub) {
+            float sc, mn;
+            q4k_scale_min(header, sub, &sc, &mn);
+            dsc[sub] = d * sc;
+            dmn[sub] = dmin * mn;
+        }
+    }
+    const int s[8] = {s_lo.x, s_lo.y, s_lo.z, s_lo.w, s_hi.x, s_hi.y, s_hi.z, s_hi.w};
+    // (two sub-blocks at a time: the two terms mostly cancel, and a sum that holds only one of them loses more bits)
+    q8k_v16f part = {};
+#pragma unroll
+    for (int sub = 0; sub < 8; ++sub) {
+        if ((sub & 1) == 0)  // K = 2 an instruction: lane half g supplies sub-block sub + g
+            part = __builtin_amdgcn_mfma_f32_32x32x2f32(static_cast<float>(g ? s[sub + 1] : s[sub]), g ? -dmn[sub + 1] : -dmn[sub], part, 0, 0, 0);
+        const q4k_u32x4 p = nib[sub >> 1];
+        const int sh = (sub & 1) * 4;  // low nibbles = sub-block 2t, high nibbles = 2t + 1
+        const q8k_v4i b = {static_cast<int>((p.x >> sh) & 0x0F0F0F0Fu), static_cast<int>((p.y >> sh) & 0x0F0F0F0Fu),
+                           static_cast<int>((p.z >> sh) & 0x0F0F0F0Fu), static_cast<int>((p.w >> sh) & 0x0F0F0F0Fu)};
+        const q8k_v16i zero = {};
+        const q8k_v16i dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[sub], b, zero, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) part[v] = __builtin_fmaf(dsc[sub], static_cast<float>(dot[v]), part[v]);
+    }
+    // (a wavefront reads back the scales that its own lanes wrote: LDS operations of a wavefront complete in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int v = 0; v < 16; ++v) red[(wave * 16 + v) * 64 + lane] = xd_s[wave * 32 + 8 * (v >> 2) + 4 * g + (v & 3)] * part[v];
+    __syncthreads();
+    for (int i = tid; i < 1024; i += threads) {
+        float total = 0.0f;
+        for (int w = 0; w < kb; ++w) total += red[w * 1024 + i];
+        const int v = i >> 6, l = i & 63;
+        const int r = row0 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3), n = tile * 32 + (l & 31);
+        if (r < rows && n < out_dim) {
+            const size_t at = static_cast<size_t>(r) * out_dim + n;
+            dst[at] = finish_output(ep, n, at, total);
+        }
+    }
+}
+
 // int8 [rows][in_dim] (padded to 256 bytes), f32 d [rows][in_dim / 256], int32 sums [rows][in_dim / 32]
 size_t q4k_q8k_workspace_bytes(size_t rows, size_t in_dim) {
     return (rows * in_dim + 255) / 256 * 256 + rows * (in_dim / 256) * 4 + rows * (in_dim / 32) * 4;
@@ -751,16 +845,34 @@ hipError_t launch_quantize_q8k(hipStream_t stream, const float* x, int rows, int
     return hipGetLastError();
 }
 
+bool linear_q4k_q8k_shares_launch(bool tiled, size_t rows, size_t in_dim) {
+    return tiled && rows > 9 && in_dim / kQ4kBlockValues <= 12 && (rows + kQ8kMfmaRows - 1) / kQ8kMfmaRows <= 65535;
+}
+
 hipError_t launch_linear_q4k_q8k(hipStream_t stream, float* dst, const void* workspace, const uint8_t* weight, bool tiled, int rows,
-                                 int in_dim, int out_dim, const Epilogue& ep) {
+                                 int in_dim, int out_dim, const Epilogue& ep, float* dst_b, const uint8_t* weight_b,
+                                 const Epilogue& ep_b, float* dst_c, const uint8_t* weight_c, const Epilogue& ep_c) {
     if (rows == 0 || out_dim == 0) return hipSuccess;
+    const bool shares = linear_q4k_q8k_shares_launch(tiled, static_cast<size_t>(rows), static_cast<size_t>(in_dim));
+    if (dst_b != nullptr && !shares) {  // one launch after the other
+        hipError_t e = launch_linear_q4k_q8k(stream, dst, workspace, weight, tiled, rows, in_dim, out_dim, ep);
+        if (e == hipSuccess) e = launch_linear_q4k_q8k(stream, dst_b, workspace, weight_b, tiled, rows, in_dim, out_dim, ep_b);
+        if (e == hipSuccess && dst_c != nullptr) e = launch_linear_q4k_q8k(stream, dst_c, workspace, weight_c, tiled, rows, in_dim, out_dim, ep_c);
+        return e;
+    }
     const size_t blocks = static_cast<size_t>(rows) * (in_dim / kQ4kBlockValues);
     const uint8_t* ws = static_cast<const uint8_t*>(workspace);
     const int8_t* q = reinterpret_cast<const int8_t*>(ws);
     const float* d = reinterpret_cast<const float*>(ws + (static_cast<size_t>(rows) * in_dim + 255) / 256 * 256);
     const int* sums = reinterpret_cast<const int*>(d + blocks);
     const int kb = in_dim / kQ4kBlockValues;
-    if (tiled && kb <= 12) {
+    if (shares) {
+        const size_t lds = static_cast<size_t>(kb) * (1024 + 32) * 4;
+        static_assert(12 * (1024 + 32) * 4 <= 64 * 1024, "no raised LDS limit");
+        hipLaunchKernelGGL(linear_q4k_q8k_mfma_kernel, dim3((out_dim + 31) / 32, (rows + kQ8kMfmaRows - 1) / kQ8kMfmaRows, dst_c ? 3 : (dst_b ? 2 : 1)),
+                           dim3(64 * kb), lds, stream, dst, q, d, sums, weight, rows, in_dim, out_dim, ep, Q8kSecond{dst_b, weight_b, ep_b},
+                           Q8kSecond{dst_c, weight_c, ep_c});
+    } else if (tiled && kb <= 12) {
         // row groups: enough workgroups for the chip on narrow matrices, whole passes of eight rows each
         const int tiles = (out_dim + 31) / 32;
         int groups = (2 * gemv_compute_units() + tiles - 1) / tiles;

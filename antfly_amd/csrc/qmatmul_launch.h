@@ -162,7 +162,11 @@ int gemv_q4k_max_in_dim();
 size_t q4k_q8k_workspace_bytes(size_t rows, size_t in_dim);
 hipError_t launch_quantize_q8k(hipStream_t stream, const float* x, int rows, int in_dim, void* workspace);
 hipError_t launch_linear_q4k_q8k(hipStream_t stream, float* dst, const void* workspace, const uint8_t* weight, bool tiled, int rows,
-                                 int in_dim, int out_dim, const Epilogue& ep);
+                                 int in_dim, int out_dim, const Epilogue& ep = Epilogue{}, float* dst_b = nullptr,
+                                 const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{}, float* dst_c = nullptr,
+                                 const uint8_t* weight_c = nullptr, const Epilogue& ep_c = Epilogue{});
+// Whether that takes a second and third matrix of the same shape on the same X into one launch.
+bool linear_q4k_q8k_shares_launch(bool tiled, size_t rows, size_t in_dim);
 // One, two or four rows on the tile-major layout at K <= 3072: the quantizer runs inside the matmul launch
 // (same bits as the two launches; `workspace` is not touched).
 bool linear_q4k_q8k_fuses_quantizer(bool tiled, size_t rows, size_t in_dim);

@@ -358,6 +358,38 @@ def test_q8k_route_pair_and_bias():
     assert np.array_equal(yb2, ya + bias[None, :])
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(50, 512, 513), (64, 768, 2304), (77, 3072, 769), (154, 1536, 640), (514, 2048, 545)])
+def test_q8k_route_on_the_matrix_cores(rows, in_dim, out_dim):
+    """More than nine rows of the gated shapes: part tiles of rows (50 = 32 + 18, 77, 154, 514) and columns, two to twelve
+    super-blocks; a pair and Q/K/V through the backend are single calls, bit for bit."""
+    print(f"case: q4_k q8k mfma rows={rows} in={in_dim} out={out_dim}", flush=True)
+    assert O.uses_q4k_q8k_activation(rows, in_dim, out_dim)
+    ws = [synth.weights(Q4K, 91 + i, out_dim, in_dim) for i in range(3)]
+    bs = [synth.activations(94 + i, 1, out_dim)[0] for i in range(3)]
+    x = synth.activations(97, rows, in_dim)
+    x[1, :256] = 0.0  # a zero block: scale 1
+    wd = [device_weight(PREP, w, out_dim, in_dim) for w in ws]
+    y = [G.linear(Q4K, PREP, x, d, rows, in_dim, out_dim) for d in wd]
+    sample = np.r_[0:2, 17, 31:34, rows - 1]
+    for got, w in zip(y, ws):
+        assert G.max_rel_err(got[sample], O.linear_q4_k_q8k(x[sample], w, len(sample), in_dim, out_dim).astype(np.float64)) <= TIGHT
+    ya, yb = G.linear_pair(Q4K, PREP, x, wd[0], wd[1], rows, in_dim, out_dim)
+    assert np.array_equal(ya, y[0]) and np.array_equal(yb, y[1])
+    with HipCompute() as cb:
+        for i in range(3):
+            cb.insertWeightFromLoaded(f"{i}.weight", Q4K, ws[i], [out_dim, in_dim])
+        xt, bt = cb.fromFloat32(x, [rows, in_dim]), [cb.fromFloat32(b, [out_dim]) for b in bs]
+        wt = [cb.getWeight(f"{i}.weight") for i in range(3)]
+        triple = cb.linearTriple(xt, wt[0], bt[0], wt[1], bt[1], wt[2], bt[2], rows, in_dim, out_dim)
+        for got, want, b in zip(triple, y, bs):
+            assert np.array_equal(cb.toFloat32(got).reshape(rows, out_dim), want + b[None, :])
+        stats = cb.debugStats()
+        assert stats["launches_activation_quant"] == 1 and stats["launches_mm"] + stats["launches_small_batch"] == 3
+        bad = cb.fromFloat32(np.zeros(out_dim + 1, np.float32), [out_dim + 1])
+        with pytest.raises(_lib.InvalidShape):  # not a call for the shared launch: the single ops say what is wrong
+            cb.linearTriple(xt, wt[0], bt[0], wt[1], bt[1], wt[2], bad, rows, in_dim, out_dim)
+
+
 PREFILL_SHAPES = [(7, 4096, 64), (10, 1024, 300), (11, 512, 33), (40, 2048, 256), (41, 1024, 257), (100, 512, 1000),
                   (128, 4096, 512), (3, 14336, 40), (45, 14336, 96), (300, 256, 64), (8, 512, 40), (9, 512, 40), (12, 512, 40), (13, 4096, 300), (7, 4096, 300), (3, 14336, 64), (5, 14336, 200), (33, 1024, 64), (64, 1024, 96), (20, 2560, 700), (50, 14336, 64),
                   (81, 768, 500)]
