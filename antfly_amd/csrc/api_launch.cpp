@@ -525,13 +525,11 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
         const size_t partial_bytes = gemm_i8_partial_bytes(rows, in_dim, out_dim);
         float* partial = partial_bytes != 0 && workspace.len >= partial_at + partial_bytes
                              ? reinterpret_cast<float*>(workspace.ptr + partial_at) : nullptr;
+        // a pair goes down together: the second matrix reuses the quantized activations (and the partial sums' room)
         e = launch_gemm_i8(stream, tensor_type, want_dots ? nullptr : y, dot_out, ws.qx, ws.sx, w, static_cast<int>(rows),
-                           static_cast<int>(in_dim), static_cast<int>(out_dim), ep, partial);
-        if (e == hipSuccess && pair) {  // the second matrix reuses the quantized activations (and the partial sums' room)
-            if (counters) counters->mm++;
-            e = launch_gemm_i8(stream, tensor_type, y_b, nullptr, ws.qx, ws.sx, w_b, static_cast<int>(rows),
-                               static_cast<int>(in_dim), static_cast<int>(out_dim), ep_b, partial);
-        }
+                           static_cast<int>(in_dim), static_cast<int>(out_dim), ep, partial, pair ? y_b : nullptr,
+                           pair ? w_b : nullptr, ep_b);
+        if (counters && pair) counters->mm++;
         return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
     }
     // (Two rows up to K = 11008 stay on the decode kernel below: one launch, the K slices of a column group meet inside the

@@ -95,31 +95,19 @@ struct GemmShape {
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
 };
 
-// s_waitcnt for "at most n vector memory operations outstanding" (nothing else waited
-// for).  n is wave-uniform; the instruction needs an immediate.
-__device__ __forceinline__ void wait_vm_outstanding(int n) {
+// s_waitcnt for "at most kLeft vector memory operations outstanding" (nothing else waited for).
+template <int kLeft>
+__device__ __forceinline__ void wait_vm_outstanding() {
+    static_assert(kLeft >= 0 && kLeft < 64, "six bits");
     // simm16: vmcnt[3:0] | expcnt << 4 | lgkmcnt << 8 | vmcnt[5:4] << 14
-#define AFHIP_WAIT_VM(N) __builtin_amdgcn_s_waitcnt(((N) & 15) | (7 << 4) | (15 << 8) | (((N) >> 4) << 14))
-    switch (n) {
-        case 1: AFHIP_WAIT_VM(1); break;
-        case 2: AFHIP_WAIT_VM(2); break;
-        case 3: AFHIP_WAIT_VM(3); break;
-        case 4: AFHIP_WAIT_VM(4); break;
-        case 5: AFHIP_WAIT_VM(5); break;
-        case 6: AFHIP_WAIT_VM(6); break;
-        case 8: AFHIP_WAIT_VM(8); break;
-        case 10: AFHIP_WAIT_VM(10); break;
-        case 12: AFHIP_WAIT_VM(12); break;
-        default: AFHIP_WAIT_VM(0); break;  // 0, or a count not listed: waiting for everything is always safe
-    }
-#undef AFHIP_WAIT_VM
+    __builtin_amdgcn_s_waitcnt((kLeft & 15) | (7 << 4) | (15 << 8) | ((kLeft >> 4) << 14));
 }
 
 // One 64-lane load from global memory straight into LDS: lane l's `bytes` at
 // base + voff land at lds_addr + l * max(bytes, 4) (a 2-byte element is zero-extended
 // to 4).  Issued as inline assembly on purpose: the compiler would otherwise make
 // every later LDS read wait for all such loads in flight, which defeats the ring.
-// Completion is tracked with wait_vm_outstanding(); base and lds_addr are wave-uniform.
+// Completion is tracked with wait_vm_outstanding; base and lds_addr are wave-uniform.
 // M0 is declared as clobbered, so the compiler keeps nothing of its own in it across these statements.
 __device__ __forceinline__ void lds_load16(const void* base, uint32_t voff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
@@ -173,14 +161,20 @@ __device__ __forceinline__ void gemm_i8_body(
     const int wm = tile / kWavesN, wn = tile % kWavesN;
     const int lj = lane & 31, lh = lane >> 5;
 
-    // Workgroups that share a weight tile (same n tile, different m tiles) sit on
-    // the same XCD (consecutive workgroup ids go round-robin over the 8 XCDs), so
-    // each L2 reads every weight byte once.
-    const int id = blockIdx.x;
-    const int xcd = id & 7, slot_id = id >> 3;
-    const int m_tile = slot_id % m_tiles;
-    const int n_tile = (slot_id / m_tiles) * 8 + xcd;
-    if (n_tile >= n_tiles) return;
+    // Workgroups that share a weight tile (same n tile, different m tiles) sit on the same XCD (consecutive workgroup ids go
+    // round-robin over the eight), so each L2 reads every weight byte once.  The tiles of the columns that eight do not divide
+    // go to all XCDs in equal parts (whole columns to each: 5632 columns of 128 put six on four of them and five on the others).
+    const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3, whole = (n_tiles >> 3) * m_tiles;
+    int m_tile, n_tile;
+    if (slot_id < whole) {
+        m_tile = slot_id % m_tiles;
+        n_tile = (slot_id / m_tiles) * 8 + xcd;
+    } else {
+        const int rest = (n_tiles & 7) * m_tiles, part = (rest + 7) >> 3, index = xcd * part + slot_id - whole;
+        if (slot_id - whole >= part || index >= rest) return;
+        m_tile = index % m_tiles;
+        n_tile = (n_tiles & ~7) + index / m_tiles;
+    }
     const int m0 = m_tile * kTM, n0 = n_tile * kTN;
 
     const size_t blocks = static_cast<size_t>(out_dim) * kb_full;
@@ -197,15 +191,13 @@ __device__ __forceinline__ void gemm_i8_body(
     const int ub0 = (wave + kWaves - kStartB) % kWaves;
     const int usx0 = (wave + kWaves - kStartSx) % kWaves;
     const int usw0 = (wave + kWaves - kStartSw) % kWaves;
-    int loads_per_stage = 0;
-#pragma unroll
-    for (int i = 0; i < kPerA; ++i) loads_per_stage += ua0 + i * kWaves < kUnitsA;
-#pragma unroll
-    for (int i = 0; i < kPerB; ++i) loads_per_stage += ub0 + i * kWaves < kUnitsB;
-#pragma unroll
-    for (int i = 0; i < kPerSx; ++i) loads_per_stage += usx0 + i * kWaves < kUnitsSx;
-#pragma unroll
-    for (int i = 0; i < kPerSw; ++i) loads_per_stage += usw0 + i * kWaves < kUnitsSw;
+    // the round-robin leaves every wavefront kLoads loads a stage, or one more to some
+    constexpr int kUnits = kUnitsA + kUnitsB + kUnitsSx + kUnitsSw, kLoads = kUnits / kWaves, kOneMore = kUnits % kWaves;
+    const bool one_more = kOneMore != 0 && wave < kOneMore;
+    auto wait_for_stage = [&]() {  // all but the last stage issued
+        if (kOneMore != 0 && one_more) wait_vm_outstanding<kLoads + 1>();
+        else wait_vm_outstanding<kLoads>();
+    };
 
     // Per-lane byte offsets of the loads of a stage whose blocks from `blocks_here` on are clamped to the one before (the last
     // stage: nothing is read past a row's end; the scales of the clamped blocks are taken as zero).
@@ -417,7 +409,7 @@ __device__ __forceinline__ void gemm_i8_body(
     for (int d = 0; d < kRing - 1; ++d) issue_loads(d, d);
     // Loads complete in order: a stage has landed for this wavefront once at most the
     // loads of the stages issued after it are outstanding.
-    wait_vm_outstanding(loads_per_stage);
+    wait_for_stage();
     __syncthreads();
     {
         // The next stage's operands are read from LDS while this stage's arithmetic runs.
@@ -439,7 +431,7 @@ __device__ __forceinline__ void gemm_i8_body(
                 // the next stage reads its operands
                 uint64_t s0 = 0, s1 = 0;
                 if (kStamps) s0 = __builtin_readcyclecounter();
-                wait_vm_outstanding(loads_per_stage);
+                wait_for_stage();
                 if (kStamps) s1 = __builtin_readcyclecounter();
                 __syncthreads();
                 if (kStamps) {
@@ -456,7 +448,7 @@ __device__ __forceinline__ void gemm_i8_body(
 
     // Loads still in flight target ring slots nobody reads again; they must land before
     // the ring is reused for the reduction (and before the workgroup ends).
-    wait_vm_outstanding(0);
+    wait_vm_outstanding<0>();
     constexpr int kPerWave = kPerM * kPerN;
     if (kSplit > 1) {
         // ---- the kSplit partial sums of a tile meet in LDS
@@ -569,25 +561,42 @@ __device__ __forceinline__ void gemm_i8_body(
     }
 }
 
+// A second matrix of the same shape on the same activations (gate and up; blockIdx.z = 1).
+struct GemmSecond {
+    float* dst = nullptr;
+    const uint8_t* weight = nullptr;
+    Epilogue ep;
+};
+
 template <int kType, int kWavesM, int kWavesN, int kSplit, bool kWriteDots, bool kShareK = false, bool kStamps = false, int kPerM = 1,
           int kPerN = 1>
 __global__ __launch_bounds__(64 * kWavesM * kWavesN * kSplit) void gemm_i8_kernel(
     float* __restrict__ dst, int* __restrict__ dots, const int8_t* __restrict__ qx, const float* __restrict__ sx,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_tiles, int n_tiles,
-    int share_blocks, float* __restrict__ partial, Epilogue ep) {
+    int share_blocks, float* __restrict__ partial, Epilogue ep, GemmSecond second) {
+    if (!kWriteDots && !kShareK && !kStamps && blockIdx.z != 0) {
+        dst = second.dst;
+        weight = second.weight;
+        ep = second.ep;
+    }
     gemm_i8_body<kType, kWavesM, kWavesN, kSplit, kWriteDots, kShareK, kStamps, kPerM, kPerN>(
         dst, dots, qx, sx, weight, rows, in_dim, out_dim, m_tiles, n_tiles, share_blocks, partial, ep);
 }
 
 namespace {
 
+// Workgroups of a launch: an eighth of them for each XCD, whole columns of tiles and its part of the others.
+long long gemm_grid(int m_tiles, int n_tiles) {
+    return 8 * (static_cast<long long>(n_tiles >> 3) * m_tiles + ((n_tiles & 7) * static_cast<long long>(m_tiles) + 7) / 8);
+}
+
 // Grids that fill the compute units: f32 results of whole K only (no shares, no block dots).
 template <int kType, int kWavesM, int kWavesN, int kSplit, int kPerM, int kPerN>
 hipError_t launch_wide_tile(hipStream_t stream, float* dst, const int8_t* qx, const float* sx, const uint8_t* weight, int rows,
-                            int in_dim, int out_dim, const Epilogue& ep) {
+                            int in_dim, int out_dim, const Epilogue& ep, const GemmSecond& second) {
     using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2, kPerM, kPerN>;
     const int m_tiles = (rows + S::kTM - 1) / S::kTM, n_tiles = (out_dim + S::kTN - 1) / S::kTN;
-    const long long grid = static_cast<long long>((n_tiles + 7) / 8) * m_tiles * 8;
+    const long long grid = gemm_grid(m_tiles, n_tiles);
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     // per-lane load offsets are 32-bit, relative to the workgroup's first row
     if (static_cast<long long>(S::kTM > S::kTN ? S::kTM : S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -600,19 +609,18 @@ hipError_t launch_wide_tile(hipStream_t stream, float* dst, const int8_t* qx, co
             return e;
         attr_done.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(S::kThreads), S::kLdsBytes, stream, dst, nullptr, qx, sx, weight,
-                       rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, ep);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), 1, second.dst ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, stream, dst,
+                       nullptr, qx, sx, weight, rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, ep, second);
     return hipGetLastError();
 }
 
 template <int kType, int kWavesM, int kWavesN, int kSplit>
-hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
-                       const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial) {
+hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx, const uint8_t* weight, int rows,
+                       int in_dim, int out_dim, const Epilogue& ep, float* partial, const GemmSecond& second) {
     using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2>;
     const int m_tiles = (rows + S::kTM - 1) / S::kTM;
     const int n_tiles = (out_dim + S::kTN - 1) / S::kTN;
-    const int n_groups = (n_tiles + 7) / 8;
-    const long long grid = static_cast<long long>(n_groups) * m_tiles * 8;
+    const long long grid = gemm_grid(m_tiles, n_tiles);
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     // per-lane load offsets are 32-bit, relative to the workgroup's first row
     if (static_cast<long long>(S::kTM > S::kTN ? S::kTM : S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -622,7 +630,7 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
     const int share_blocks = (kb + splits - 1) / splits;
     const int shares = (kb + share_blocks - 1) / share_blocks;  // no empty share
     float* sums = shares > 1 ? partial : nullptr;
-    dim3 g(static_cast<unsigned>(grid), static_cast<unsigned>(shares)), b(S::kThreads);
+    dim3 g(static_cast<unsigned>(grid), static_cast<unsigned>(shares), second.dst && shares == 1 ? 2 : 1), b(S::kThreads);
     auto kernel_f32 = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false>;
     auto kernel_shares = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false, true>;
     auto kernel_dots = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, true>;
@@ -643,20 +651,26 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
     if (attr != hipSuccess) return attr;
     if (dots)
         hipLaunchKernelGGL(kernel_dots, g, b, S::kLdsBytes, stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim,
-                           m_tiles, n_tiles, share_blocks, sums, ep);
+                           m_tiles, n_tiles, share_blocks, sums, ep, second);
     else if (shares > 1)
         hipLaunchKernelGGL(kernel_shares, g, b, S::kLdsBytes, stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim,
-                           m_tiles, n_tiles, share_blocks, sums, ep);
+                           m_tiles, n_tiles, share_blocks, sums, ep, second);
     else
         hipLaunchKernelGGL(kernel_f32, g, b, S::kLdsBytes, stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim,
-                           m_tiles, n_tiles, share_blocks, sums, ep);
+                           m_tiles, n_tiles, share_blocks, sums, ep, second);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || shares == 1) return e;
-    return launch_splitk_reduce(stream, dst, sums, static_cast<size_t>(rows) * out_dim, out_dim, shares, ep);
+    if (hipError_t e = launch_splitk_reduce(stream, dst, sums, static_cast<size_t>(rows) * out_dim, out_dim, shares, ep);
+        e != hipSuccess || second.dst == nullptr)
+        return e;
+    // (the partial sums have room for one matrix: the second follows)
+    return launch_tile<kType, kWavesM, kWavesN, kSplit>(stream, second.dst, dots, qx, sx, second.weight, rows, in_dim, out_dim, second.ep,
+                                                        partial, GemmSecond{});
 }
 
 template <int kType>
 hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
-                       const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial) {
+                       const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial,
+                       const GemmSecond& second) {
     // us of the whole op, M x K x N; "before" is the 64 x 128 tile by sixteen wavefronts that served these grids.
     static const char* env_tile = std::getenv("AFHIP_GEMM_TILE");  // tuning: "S", "X", "Y", "V" or "L", see below
     const char force = dots == nullptr && env_tile ? env_tile[0] : '\0';
@@ -671,18 +685,17 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
         if (grid * 8 >= units * 11) tile = 'X';
     } else if (grid >= units) {
         // Q8_0, whose 64 x 128 stage does not fit twice: "Y" (64 x 64 outputs, two workgroups a unit) or "V" (128 x 128, two tiles
-        // a wavefront, one workgroup a unit), whichever the rounds make shorter.  An XCD (an eighth of the units) serves every
-        // eighth column of tiles, so it is the XCD with most columns whose rounds count.  K = 4096: a round of "V" takes about
-        // 50 us, one workgroup more on every unit about 15 of "Y".  Y / V (64 x 128 by sixteen wavefronts before):
-        // 333 x 4096 x 6144 49 / 52 (60), 512 x 4096 x 4096 36 / 53 (35), 512 x 4096 x 14336 106 / 101 (118), 777 x 4096 x 14336
-        // 170 / 192 (175), 1300 x 4096 x 5632 115 / 145 (121; six columns of tiles on four of the XCDs: three rounds of "V"),
-        // 2048 x 4096 x 14336 435 / 362 (425).  Over 349 sizes (96 .. 2048 rows, K 1024 .. 14336, N 2048 .. 14336) 0.2 % above the
-        // better of the two on the mean; counted over the whole chip instead 2.6 %, at worst 28 %.
+        // a wavefront, one workgroup a unit), whichever the rounds of an XCD's units make shorter (the two sum alike, so a pair, which
+        // is one launch of twice the tiles, may choose for itself).  K = 4096: a round of "V" takes about 50 us, one workgroup more on
+        // every unit about 15 of "Y".  Y / V: 333 x 4096 x 6144 47 / 52, 512 x 4096 x 4096 36 / 53, 512 x 4096 x 14336 103 / 103, 777 x
+        // 4096 x 14336 168 / 192, 1024 x 4096 x 14336 210 / 201 (twice 406 / 361), 2048 x 4096 x 14336 445 / 366; over 110 single
+        // calls and pairs (96 .. 2048 rows, K 1024 .. 14336, N 4096 .. 14336) at most 2 % above the better of the two but for
+        // 2048 x 5120 x 5120 (202 / 184).
         constexpr long long kXcds = 8;
         auto rounds = [&](long long tile_rows, long long tile_cols) {
-            const long long cols_of_xcd = ((out_dim + tile_cols - 1) / tile_cols + kXcds - 1) / kXcds;
+            const long long tiles = ((out_dim + tile_cols - 1) / tile_cols) * ((rows + tile_rows - 1) / tile_rows) * (second.dst ? 2 : 1);
             const long long units_of_xcd = units >= kXcds ? units / kXcds : 1;
-            return (cols_of_xcd * ((rows + tile_rows - 1) / tile_rows) + units_of_xcd - 1) / units_of_xcd;
+            return ((tiles + kXcds - 1) / kXcds + units_of_xcd - 1) / units_of_xcd;
         };
         // 33 .. 64 rows have one row of tiles and fetch every weight once, so nothing is gained by a second workgroup that shares
         // them: "L" (64 x 128, one tile for each of sixteen wavefronts), Y / L: 64 x 4096 x 65536 85.4 / 77.9, 64 x 8192 x 32768
@@ -695,14 +708,14 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
     if (force != '\0') tile = force;
     if (dots == nullptr) {
         if constexpr (kType == 2) {
-            if (tile == 'X') return launch_wide_tile<2, 1, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
+            if (tile == 'X') return launch_wide_tile<2, 1, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep, second);
         } else {
-            if (tile == 'L') return launch_wide_tile<8, 2, 4, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
-            if (tile == 'V') return launch_wide_tile<8, 2, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
-            if (tile == 'Y') return launch_wide_tile<8, 2, 2, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep);
+            if (tile == 'L') return launch_wide_tile<8, 2, 4, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep, second);
+            if (tile == 'V') return launch_wide_tile<8, 2, 4, 2, 2, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep, second);
+            if (tile == 'Y') return launch_wide_tile<8, 2, 2, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep, second);
         }
     }
-    return launch_tile<kType, 1, 2, 4>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial);
+    return launch_tile<kType, 1, 2, 4>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial, second);
 }
 
 }  // namespace
@@ -770,7 +783,7 @@ hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* q
                                  int rows, int in_dim, int out_dim) {
     using S = GemmShape<2, 2, 2, false>;
     const int m_tiles = (rows + S::kTM - 1) / S::kTM, n_tiles = (out_dim + S::kTN - 1) / S::kTN;
-    const long long grid = static_cast<long long>((n_tiles + 7) / 8) * m_tiles * 8;
+    const long long grid = gemm_grid(m_tiles, n_tiles);
     if (grid > 0x7fffffffLL || static_cast<long long>(S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
     if (static_cast<long long>(rows) * out_dim < grid * S::kWaves * 8) return hipErrorInvalidValue;
     auto kernel = gemm_i8_kernel<8, 2, 2, 2, false, false, true>;
@@ -779,14 +792,16 @@ hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* q
         e != hipSuccess)
         return e;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(S::kThreads), S::kLdsBytes, stream, dst, nullptr, qx, sx,
-                       weight, rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, Epilogue{});
+                       weight, rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, Epilogue{}, GemmSecond{});
     return hipGetLastError();
 }
 
 hipError_t launch_gemm_i8(hipStream_t stream, int tensor_type, float* dst, int* dots, const int8_t* qx, const float* sx,
-                          const uint8_t* weight_prepared, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial) {
-    if (tensor_type == 2) return launch_type<2>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial);
-    return launch_type<8>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial);
+                          const uint8_t* weight_prepared, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial,
+                          float* dst_b, const uint8_t* weight_b, const Epilogue& ep_b) {
+    const GemmSecond second{dst_b, weight_b, ep_b};
+    if (tensor_type == 2) return launch_type<2>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second);
+    return launch_type<8>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second);
 }
 
 }  // namespace afhip

@@ -118,7 +118,8 @@ hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* q
                                  int rows, int in_dim, int out_dim);
 hipError_t launch_gemm_i8(hipStream_t stream, int tensor_type, float* dst, int* dots, const int8_t* qx, const float* sx,
                           const uint8_t* weight_prepared, int rows, int in_dim, int out_dim,
-                          const Epilogue& ep = Epilogue{}, float* partial = nullptr);
+                          const Epilogue& ep = Epilogue{}, float* partial = nullptr,
+                          float* dst_b = nullptr, const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{});
 int gemm_i8_splits(int rows, int in_dim, int out_dim);
 size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim);
 // dst[i] = epilogue(sum over s < shares of partial[s * count + i]), i < count = rows * out_dim

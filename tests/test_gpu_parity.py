@@ -229,6 +229,24 @@ def test_prefill_grids_past_the_compute_units(fmt, rows, in_dim, out_dim):
 
 
 @pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(97, 1024, 520), (130, 2048, 5632), (333, 1024, 4164), (1300, 512, 5632)])
+def test_prefill_pair_in_one_launch(fmt, rows, in_dim, out_dim):
+    """Gate and up of a prefill: each half is the single call, bit for bit, on grids that share K out (two launches and their
+    sums), on one share and on each wide tile; tile counts that eight XCDs do not divide."""
+    print(f"case: prefill pair fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(911, rows, in_dim)
+    wa, wb = synth.weights(fmt, 912, out_dim, in_dim), synth.weights(fmt, 913, out_dim, in_dim)
+    da, db = G.prepare(fmt, wa, out_dim, in_dim), G.prepare(fmt, wb, out_dim, in_dim)
+    ya, yb = G.linear_pair(fmt, PREP, x, da, db, rows, in_dim, out_dim)
+    assert np.array_equal(ya, G.linear(fmt, PREP, x, da, rows, in_dim, out_dim))
+    assert np.array_equal(yb, G.linear(fmt, PREP, x, db, rows, in_dim, out_dim))
+    sample = np.r_[0:2, 31:33, rows - 1]
+    for got, w in ((ya, wa), (yb, wb)):
+        ref = O.linear_no_bias(fmt, x[sample], w, len(sample), in_dim, out_dim, workers=8)
+        assert G.max_rel_err(got[sample], ref.astype(np.float64)) <= TIGHT
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
 @pytest.mark.parametrize("rows,in_dim,out_dim", [
     (700, 160, 4097), (257, 672, 10921), (130, 544, 4100),  # the large tiles and 32 x 64
     (130, 1056, 520)])                                      # ... with K shared out over workgroups
