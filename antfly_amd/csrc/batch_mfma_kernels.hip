@@ -115,31 +115,33 @@ template <bool kByteOrder>
 __global__ __launch_bounds__(256) void quantize_fragments_kernel(const float* __restrict__ x, int rows, int in_dim, int row_tiles,
                                                                   uint32_t* __restrict__ qa, float* __restrict__ sa,
                                                                   float* __restrict__ zero_a, float* __restrict__ zero_b, size_t zero_count) {
+    // blockIdx.y is the (padded) row, a thread four values of it: nothing is divided (64-bit quotients of a flat index
+    // stood before the load), and the load leaves before the results are cleared.  What is left is the launch and one trip to
+    // memory: 32 x 4096 4.0 us as kernel time, a pass of 32 rows through four matrices' calls 566.7 -> 557.8 us.
     const int units_per_row = in_dim >> 2, kb = in_dim >> 5, padded = row_tiles * 32;
-    const size_t units = static_cast<size_t>(padded) * units_per_row;
+    const int r = blockIdx.y, c4 = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool mine = c4 < units_per_row;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (mine && r < rows) v = reinterpret_cast<const float4*>(x)[static_cast<size_t>(r) * units_per_row + c4];
     if (zero_a != nullptr) {
-        for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < zero_count; i += static_cast<size_t>(gridDim.x) * blockDim.x) {
+        const size_t first = (static_cast<size_t>(r) * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+        for (size_t i = first; i < zero_count; i += static_cast<size_t>(gridDim.x) * gridDim.y * blockDim.x) {
             zero_a[i] = 0.0f;
             if (zero_b != nullptr) zero_b[i] = 0.0f;
         }
     }
-    for (size_t u = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; u < units;
-         u += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const int r = static_cast<int>(u / units_per_row), c4 = static_cast<int>(u % units_per_row);
-        const int b = c4 >> 3, j = c4 & 7;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (r < rows) v = reinterpret_cast<const float4*>(x)[static_cast<size_t>(r) * units_per_row + c4];
-        float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-        m = max_over_8(m);
-        const float s = act_scale(m);
-        const float inv = m == 0.0f ? 0.0f : 1.0f / s;
-        const int q0 = act_quant(v.x, inv), q1 = act_quant(v.y, inv);
-        const int q2 = act_quant(v.z, inv), q3 = act_quant(v.w, inv);
-        const int half = kByteOrder ? (j >> 1) & 1 : j >> 2, dw = kByteOrder ? 2 * (j & 1) + (j >> 2) : j & 3;
-        const size_t lane_entry = (static_cast<size_t>(r >> 5) * kb + b) * 64 + half * 32 + (r & 31);
-        qa[lane_entry * 4 + dw] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
-        if (j == 0) sa[static_cast<size_t>(b) * padded + r] = r < rows ? s : 0.0f;
-    }
+    if (!mine) return;  // (whole groups of eight lanes: units_per_row is a multiple of eight)
+    const int b = c4 >> 3, j = c4 & 7;
+    float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    m = max_over_8(m);
+    const float s = act_scale(m);
+    const float inv = m == 0.0f ? 0.0f : 1.0f / s;
+    const int q0 = act_quant(v.x, inv), q1 = act_quant(v.y, inv);
+    const int q2 = act_quant(v.z, inv), q3 = act_quant(v.w, inv);
+    const int half = kByteOrder ? (j >> 1) & 1 : j >> 2, dw = kByteOrder ? 2 * (j & 1) + (j >> 2) : j & 3;
+    const size_t lane_entry = (static_cast<size_t>(r >> 5) * kb + b) * 64 + half * 32 + (r & 31);
+    qa[lane_entry * 4 + dw] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
+    if (j == 0) sa[static_cast<size_t>(b) * padded + r] = r < rows ? s : 0.0f;
 }
 
 template <int kType, int kRowTiles, int kLive>
@@ -423,38 +425,36 @@ __global__ __launch_bounds__(256) void quantize_fragments8_kernel(const float* _
                                                                    uint32_t* __restrict__ qa8, float* __restrict__ sa8,
                                                                    float* __restrict__ zero_a, float* __restrict__ zero_b, int zero_count) {
     const int kb = in_dim >> 5, slots = ((kb + 1) >> 1) * 2;  // block slots: whole pairs
-    const int units = 8 * slots * 8;                           // (row, block slot, eight lanes)
-    // blockIdx.y: the group of eight rows (rows 8 .. 15 of X make a second set of fragments and scales behind the first)
-    const int group = blockIdx.y;
-    x += static_cast<size_t>(group) * 8 * in_dim;
-    rows -= 8 * group;
-    qa8 += static_cast<size_t>(group) * (slots / 2) * 128;
-    sa8 += static_cast<size_t>(group) * (slots / 2) * 16;
-    if (zero_a != nullptr && group == 0) {
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < zero_count; i += gridDim.x * blockDim.x) {
+    // blockIdx.y: the row of a group of eight and the group (rows 8 .. 15 of X make a second set of fragments and scales behind the
+    // first); a thread takes four values of the row, so nothing is divided, and its load leaves before the results are cleared:
+    // 5 x 4096 2.8 us as kernel time, a pass of five rows through four matrices' calls 1537 -> 1515 us.
+    const int group = blockIdx.y >> 3, r = blockIdx.y & 7;
+    const int u = blockIdx.x * blockDim.x + threadIdx.x, j = u & 7, bs = u >> 3;
+    const bool real = 8 * group + r < rows && bs < kb;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (real) v = reinterpret_cast<const float4*>(x)[(static_cast<size_t>(blockIdx.y) * in_dim >> 2) + u];
+    if (zero_a != nullptr) {
+        for (int i = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x; i < zero_count; i += gridDim.x * gridDim.y * blockDim.x) {
             zero_a[i] = 0.0f;
             if (zero_b != nullptr) zero_b[i] = 0.0f;
         }
     }
-    for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < units; u += gridDim.x * blockDim.x) {
-        const int j = u & 7, bs = (u >> 3) % slots, r = (u >> 3) / slots;
-        const bool real = r < rows && bs < kb;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (real) v = reinterpret_cast<const float4*>(x)[(static_cast<size_t>(r) * in_dim >> 2) + bs * 8 + j];
-        float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-        m = max_over_8(m);
-        const float s = act_scale(m);
-        const float inv = m == 0.0f ? 0.0f : 1.0f / s;
-        const int q0 = act_quant(v.x, inv), q1 = act_quant(v.y, inv);
-        const int q2 = act_quant(v.z, inv), q3 = act_quant(v.w, inv);
-        const int pair = bs >> 1, hs = bs & 1, i = hs * 8 + r;
-        // values [4 j, 4 j + 4) of the block: which 16-byte half, which dword of it
-        const int h2 = kType == 2 ? (j >> 1) & 1 : j >> 2;
-        const int dw = kType == 2 ? 2 * (j & 1) + (j >> 2) : j & 3;
-        // entry 16 * s + 8 * h2 + r of the pair: sixteen bytes
-        qa8[static_cast<size_t>(pair) * 128 + (16 * hs + 8 * h2 + r) * 4 + dw] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
-        if (j == 0) sa8[pair * 16 + i] = real ? s : 0.0f;
-    }
+    if (bs >= slots) return;  // (whole groups of eight lanes)
+    qa8 += static_cast<size_t>(group) * (slots / 2) * 128;
+    sa8 += static_cast<size_t>(group) * (slots / 2) * 16;
+    float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    m = max_over_8(m);
+    const float s = act_scale(m);
+    const float inv = m == 0.0f ? 0.0f : 1.0f / s;
+    const int q0 = act_quant(v.x, inv), q1 = act_quant(v.y, inv);
+    const int q2 = act_quant(v.z, inv), q3 = act_quant(v.w, inv);
+    const int pair = bs >> 1, hs = bs & 1, i = hs * 8 + r;
+    // values [4 j, 4 j + 4) of the block: which 16-byte half, which dword of it
+    const int h2 = kType == 2 ? (j >> 1) & 1 : j >> 2;
+    const int dw = kType == 2 ? 2 * (j & 1) + (j >> 2) : j & 3;
+    // entry 16 * s + 8 * h2 + r of the pair: sixteen bytes
+    qa8[static_cast<size_t>(pair) * 128 + (16 * hs + 8 * h2 + r) * 4 + dw] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
+    if (j == 0) sa8[pair * 16 + i] = real ? s : 0.0f;
 }
 
 // kStamps (bench.py --probe timeline8): the same code, but instead of results every wavefront stores eight readings of the
@@ -1310,8 +1310,7 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     if (eight) {  // its own operand layout: 512 + 64 bytes per pair of blocks and group of eight rows, inside the same region
         const int pairs = (kb + 1) / 2;
         sa = reinterpret_cast<float*>(workspace + static_cast<size_t>(groups) * pairs * 512);
-        const int units = 8 * (2 * pairs) * 8;
-        const dim3 qgrid(static_cast<unsigned>((units + 255) / 256), static_cast<unsigned>(groups));
+        const dim3 qgrid(static_cast<unsigned>((2 * pairs * 8 + 255) / 256), static_cast<unsigned>(8 * groups));
         float* zero_a = accumulate ? dst : nullptr;
         float* zero_b = accumulate && weight_b_prepared ? dst_b : nullptr;
         const int zero_count = rows * out_dim;
@@ -1321,17 +1320,15 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
             hipLaunchKernelGGL(quantize_fragments8_kernel<8>, qgrid, dim3(256), 0, stream, input, rows, in_dim, qa, sa, zero_a, zero_b, zero_count);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     } else {
-        const size_t units = static_cast<size_t>(padded) * (in_dim / 4);
-        size_t grid = (units + 255) / 256;
-        if (grid > 4096) grid = 4096;
+        const dim3 qgrid(static_cast<unsigned>((in_dim / 4 + 255) / 256), static_cast<unsigned>(padded));
         float* zero_a = accumulate ? dst : nullptr;
         float* zero_b = accumulate && weight_b_prepared ? dst_b : nullptr;
         const size_t zero_count = static_cast<size_t>(rows) * out_dim;
         if (thirty_two && tensor_type == 2)
-            hipLaunchKernelGGL(quantize_fragments_kernel<true>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, input, rows, in_dim,
+            hipLaunchKernelGGL(quantize_fragments_kernel<true>, qgrid, dim3(256), 0, stream, input, rows, in_dim,
                                row_tiles, qa, sa, zero_a, zero_b, zero_count);
         else
-            hipLaunchKernelGGL(quantize_fragments_kernel<false>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, input, rows, in_dim,
+            hipLaunchKernelGGL(quantize_fragments_kernel<false>, qgrid, dim3(256), 0, stream, input, rows, in_dim,
                                row_tiles, qa, sa, zero_a, zero_b, zero_count);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }
@@ -1390,8 +1387,7 @@ hipError_t launch_batch8_timeline(hipStream_t stream, uint32_t* stamps, size_t s
     uint32_t* qa = reinterpret_cast<uint32_t*>(workspace);
     const int pairs = (kb + 1) / 2;
     float* sa = reinterpret_cast<float*>(workspace + static_cast<size_t>(pairs) * 512);
-    const int units = 8 * (2 * pairs) * 8;
-    hipLaunchKernelGGL(quantize_fragments8_kernel<2>, dim3(static_cast<unsigned>((units + 255) / 256)), dim3(256), 0, stream, input, rows, in_dim, qa, sa,
+    hipLaunchKernelGGL(quantize_fragments8_kernel<2>, dim3(static_cast<unsigned>((2 * pairs * 8 + 255) / 256), 8), dim3(256), 0, stream, input, rows, in_dim, qa, sa,
                        static_cast<float*>(nullptr), static_cast<float*>(nullptr), 0);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     int share_blocks = (kb + BmFormat<2>::kWaveBlocks - 1) / BmFormat<2>::kWaveBlocks * BmFormat<2>::kWaveBlocks;
