@@ -468,7 +468,10 @@ __global__ __launch_bounds__(256) void quantize_fragments8_kernel(const float* _
 // four of 112), and two shares need no reduce launch.
 // kGroups: groups of eight rows (one or two: nine to sixteen rows run every step's two MFMAs once per group on the same
 // weight operand; the second group's fragments and row scales lie behind the first's).
-template <int kType, int kCG, bool kStamps = false, bool kFullCols = false, int kHalves = 2, int kGroups = 1>
+// kQuantize: qa8 is X itself, f32 [rows][in_dim] (sa8 is not looked at), and every wavefront quantizes the values of its own
+// blocks before the first stage: no quantizer launch.  The wavefronts of a workgroup own different blocks, so within one
+// nothing is converted twice; every workgroup converts all of its K share, while its first weights travel.
+template <int kType, int kCG, bool kStamps = false, bool kFullCols = false, int kHalves = 2, int kGroups = 1, bool kQuantize = false>
 __global__ __launch_bounds__(kBmThreads, kGroups > 1 ? 2 : 4) void batch8_mfma_kernel(float* __restrict__ dst_a, float* __restrict__ partial_a,
                                                                      const uint32_t* __restrict__ qa8, const float* __restrict__ sa8,
                                                                      const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
@@ -547,7 +550,35 @@ __global__ __launch_bounds__(kBmThreads, kGroups > 1 ? 2 : 4) void batch8_mfma_k
     constexpr int kScaleLoads = (kPairs + 3) / 4;
     float sx_part[kGroups][kScaleLoads];
     bm_v4i packed[kGroups][kPairs / 2];
-    {
+    // (kQuantize: X instead.  A load is eight blocks of one row, eight lanes a block and four values a lane: whole lines)
+    typedef float bm_v4f __attribute__((ext_vector_type(4)));
+    constexpr int kRowLoads = kQuantize ? kWB / 8 : 1;
+    bm_v4f xv[kQuantize ? 8 : 1][kRowLoads];
+    const int live = nb > 0 ? rows : 0;
+    if constexpr (kQuantize) {
+        static_assert(kGroups == 1 && kWB % 8 == 0 && kWB <= 16, "the operand's place in the ring");
+        uint32_t x_off[kRowLoads];
+#pragma unroll
+        for (int c = 0; c < kRowLoads; ++c) {
+            x_off[c] = static_cast<uint32_t>(min(blk0 + 8 * c + (lane >> 3), kb_full - 1)) * 128u + (lane & 7) * 16u;
+            asm volatile("" : "+v"(x_off[c]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) {
+            if (r < live) {
+                const float* row0 = reinterpret_cast<const float*>(qa8) + static_cast<size_t>(r) * in_dim;
+                const float* row1 = r + 1 < live ? row0 + in_dim : row0;  // (an odd last row twice)
+#pragma unroll
+                for (int c = 0; c < kRowLoads; ++c) asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(xv[r][c]) : "v"(x_off[c]), "s"(row0) : "memory");
+#pragma unroll
+                for (int c = 0; c < kRowLoads; ++c) asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(xv[r + 1][c]) : "v"(x_off[c]), "s"(row1) : "memory");
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
         uint32_t frag_off[kPairs / 2], scale_off[kScaleLoads];
 #pragma unroll
         for (int q = 0; q < kPairs / 2; ++q) frag_off[q] = static_cast<uint32_t>(min(pair0 + 2 * q + (lane >> 5), pairs_total - 1) * 32 + (lane & 31)) * 16u;
@@ -606,13 +637,94 @@ __global__ __launch_bounds__(kBmThreads, kGroups > 1 ? 2 : 4) void batch8_mfma_k
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    // (kQuantize: Q8_0 requests its second stage in front of the conversions, K = 4096, eight rows: 14336 columns 14.4 -> 13.7 us,
+    // 11008 columns 12.3 -> 11.8; Q4_0 loses, a pair of 14336 columns 17.0 .. 17.3 -> 17.7 .. 18.6)
+    constexpr bool kStageOneEarly = kQuantize && kScalesInLds && kStages > 1 && kType == 8;
     issue_stage(0);
+    if (kStageOneEarly) issue_stage(1);
+    if constexpr (kQuantize) {
+        // X is there when at most the first stages' requests and the rounds of scale runs that every wavefront takes part in are
+        // in flight.  Quantized as quantize_fragments8_kernel does it, bit for bit.  kN vectors are converted together: of their
+        // kN maxima over eight lanes a lane ends with one (`pick`: lane % kN, mirrored in the upper four of the eight so that the
+        // last exchange, a mirror, stays within one maximum), divides for that one, and the quad hands the reciprocals round.
+        // The dwords go to the operand's order through LDS: the ring's slots 2 and 3, whose stages are requested once this has
+        // been read back.  Row r of block b is stored in row r ^ (b % 8) of the eight: the 64 lanes' dwords in 64 banks.
+        constexpr int kN = 2 * kRowLoads;
+        constexpr int kFullRounds = kScalesInLds ? 16 * kCG * kChunks / kBmThreads : 0;
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kStageOneEarly ? 4 : 2) + kFullRounds) : "memory");
+        unsigned char* own = bm_lds + wave * kBmWaveBytes + 4096;
+        const int bl = lane >> 3, j = lane & 7, pick = (j & 4 ? 7 - j : j) & (kN - 1);
+        const int h2 = kType == 2 ? (j >> 1) & 1 : j >> 2, dw = kType == 2 ? 2 * (j & 1) + (j >> 2) : j & 3;
+        const uint32_t q_base = (bl >> 1) * 512 + (16 * (bl & 1) + 8 * h2 + bl) * 16 + dw * 4;
+        float row_scale[4];  // of the lane's own pick
+        // (numbers or quiet NaNs on both sides: nothing to quieten first, which fmaxf would do.  The two wait states that a lane
+        // exchange of the result needs stand with it: the compiler does not look into the assembly)
+        auto max_with = [](float a, float other) { float m; asm("v_max_f32 %0, %1, %2\n\ts_nop 1" : "=v"(m) : "v"(a), "v"(other)); return m; };
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) {
+            row_scale[r / 2] = 0.0f;
+            if (r < live) {
+                float m[kN];
+#pragma unroll
+                for (int i = 0; i < kN; ++i) {
+                    bm_v4f& v = xv[r + i / kRowLoads][i % kRowLoads];
+                    asm volatile("" : "+v"(v));
+                    m[i] = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+                }
+                float mine = pick & 1 ? m[1] : m[0], other = pick & 1 ? m[0] : m[1];
+                mine = max_with(mine, dpp_move<kDppXor1>(other));
+                if constexpr (kN == 4) {
+                    float mine2 = pick & 1 ? m[3] : m[2], other2 = pick & 1 ? m[2] : m[3];
+                    mine2 = max_with(mine2, dpp_move<kDppXor1>(other2));
+                    other = pick & 2 ? mine : mine2;
+                    mine = pick & 2 ? mine2 : mine;
+                } else {
+                    other = mine;
+                }
+                mine = max_with(mine, dpp_move<kDppXor2>(other));
+                mine = max_with(mine, dpp_move<kDppHalfMirror>(mine));
+                const float s = act_scale(mine);
+                row_scale[r / 2] = s;
+                const float inv_mine = mine == 0.0f ? 0.0f : 1.0f / s;
+                // (the upper four lanes of eight back in order)
+                const float inv = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(inv_mine), __float_as_int(inv_mine), 0x1B, 0xF, 0xA, false));
+                auto convert = [&](int i, float inv_i) {
+                    const bm_v4f v = xv[r + i / kRowLoads][i % kRowLoads];
+                    const uint32_t q0 = act_quant(v[0], inv_i), q1 = act_quant(v[1], inv_i), q2 = act_quant(v[2], inv_i), q3 = act_quant(v[3], inv_i);
+                    const uint32_t low = __builtin_amdgcn_perm(q1, q0, 0x0C0C0400u), high = __builtin_amdgcn_perm(q3, q2, 0x0C0C0400u);
+                    *reinterpret_cast<uint32_t*>(own + (q_base ^ ((r + i / kRowLoads) << 4)) + (i % kRowLoads) * 2048) = low | high << 16;
+                };
+                convert(0, dpp_move<0x00>(inv));
+                convert(1, dpp_move<0x55>(inv));
+                if constexpr (kN == 4) {
+                    convert(2, dpp_move<0xAA>(inv));
+                    convert(3, dpp_move<0xFF>(inv));
+                }
+            }
+        }
+        // slot l16 of pair 4 q + g: row l16 % 8 of block 8 q + (2 g + l16 / 8), from the lane of that block that picked it
+#pragma unroll
+        for (int q = 0; q < kScaleLoads; ++q) {
+            const int from = 4 * ((2 * g + (l16 >> 3)) * 8 + (l16 & 1) * kRowLoads + q);
+            int got[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) got[p] = __builtin_amdgcn_ds_bpermute(from, __float_as_int(row_scale[p]));
+            sx_part[0][q] = __int_as_float(l16 & 4 ? (l16 & 2 ? got[3] : got[2]) : (l16 & 2 ? got[1] : got[0]));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+#pragma unroll
+        for (int q = 0; q < kPairs / 2; ++q) {
+            const int swz = (4 * q + 2 * (lane >> 5) + ((lane >> 4) & 1)) & 7;
+            packed[0][q] = *reinterpret_cast<const bm_v4i*>(own + (2 * q + (lane >> 5)) * 512 + ((lane & 24) + ((lane & 7) ^ swz)) * 16);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    }
     if (kScalesInLds) {
         // the scale runs are there when at most the first stage's two requests are in flight; the workgroup meets once they
         // are in LDS (the first stage is waited for behind that, with nothing else of the wavefront outstanding: behind
         // the second stage's requests the wait would also have to see those accepted by the memory pipeline, which for
         // the last wavefronts of a unit is well into the stream)
-        asm volatile("s_waitcnt vmcnt(2)" : : : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kStageOneEarly ? 4 : 2) : "memory");
 #pragma unroll
         for (int r = 0; r < kScaleRounds; ++r) {
             asm volatile("" : "+v"(scale_run[r]));
@@ -648,8 +760,8 @@ __global__ __launch_bounds__(kBmThreads, kGroups > 1 ? 2 : 4) void batch8_mfma_k
     }
     // Q4_0 asks for the second stage only when the first one and the register loads are there (below); Q8_0, whose
     // stages are half as many blocks, measured better with the second stage requested up front.
-    constexpr bool kStartupAlone = kType == 2;
-    if (!kStartupAlone) {
+    constexpr bool kStartupAlone = (kType == 2 || kQuantize) && !kStageOneEarly;
+    if (!kStartupAlone && !kStageOneEarly) {
 #pragma unroll
         for (int st = 1; st < kAheadStages; ++st) issue_stage(st);
     }
@@ -686,7 +798,6 @@ __global__ __launch_bounds__(kBmThreads, kGroups > 1 ? 2 : 4) void batch8_mfma_k
         typedef unsigned bm_v2u __attribute__((ext_vector_type(2)));
         typedef unsigned bm_v4u __attribute__((ext_vector_type(4)));
         typedef typename std::conditional<kType == 2, bm_v2u, bm_v4u>::type Raw;
-        typedef float bm_v4f __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) const Raw LdsRaw;
         Raw raw[2];
         bm_v4i afrag[kGroups][kHalfPairs];
@@ -1112,25 +1223,31 @@ static hipError_t bm_allow_large_lds(Kernel kernel, size_t lds, std::atomic<size
     return e;
 }
 
+constexpr bool bm8_can_quantize(int tensor_type, int halves, int groups) { return groups == 1 && halves <= (tensor_type == 2 ? 2 : 4); }
+
+// quantize: qa is X itself (at most sixteen blocks a wavefront: kHalves <= 2 for Q4_0, <= 4 for Q8_0)
 template <int kType, int kCG, int kHalves, int kGroups>
 hipError_t bm_launch8(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
-                      int in_dim, int out_dim, int shares, int share_blocks, int cols, bool accumulate, const Epilogue& ep, const BmSecond& second) {
+                      int in_dim, int out_dim, int shares, int share_blocks, int cols, bool accumulate, bool quantize, const Epilogue& ep,
+                      const BmSecond& second) {
     const dim3 grid(static_cast<unsigned>((out_dim + cols - 1) / cols), static_cast<unsigned>(shares), second.weight ? 2u : 1u), block(kBmThreads);
     if (accumulate || shares == 1) partial = nullptr;
     const size_t lds = bm8_lds_bytes(kType, kCG, kHalves);
-    static std::atomic<size_t> lds_limit[2] = {{64 * 1024}, {64 * 1024}};
-    if (cols == 16 * kCG) {
-        auto kernel = batch8_mfma_kernel<kType, kCG, false, true, kHalves, kGroups>;
-        if (hipError_t e = bm_allow_large_lds(kernel, lds, &lds_limit[0]); e != hipSuccess) return e;
+    static std::atomic<size_t> lds_limit[4] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
+    auto launch = [&](auto kernel, std::atomic<size_t>* limit) {
+        if (hipError_t e = bm_allow_large_lds(kernel, lds, limit); e != hipSuccess) return e;
         hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, share_blocks, cols,
                            accumulate ? 1 : 0, ep, second);
-    } else {
-        auto kernel = batch8_mfma_kernel<kType, kCG, false, false, kHalves, kGroups>;
-        if (hipError_t e = bm_allow_large_lds(kernel, lds, &lds_limit[1]); e != hipSuccess) return e;
-        hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, share_blocks, cols,
-                           accumulate ? 1 : 0, ep, second);
+        return hipGetLastError();
+    };
+    if constexpr (bm8_can_quantize(kType, kHalves, kGroups)) {
+        if (quantize) {
+            if (cols == 16 * kCG) return launch(batch8_mfma_kernel<kType, kCG, false, true, kHalves, kGroups, true>, &lds_limit[2]);
+            return launch(batch8_mfma_kernel<kType, kCG, false, false, kHalves, kGroups, true>, &lds_limit[3]);
+        }
     }
-    return hipGetLastError();
+    if (cols == 16 * kCG) return launch(batch8_mfma_kernel<kType, kCG, false, true, kHalves, kGroups>, &lds_limit[0]);
+    return launch(batch8_mfma_kernel<kType, kCG, false, false, kHalves, kGroups>, &lds_limit[1]);
 }
 
 
@@ -1307,7 +1424,27 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     // (cleared by the quantizer's launch), which saves the reduce launch -- two of them for a pair.
     const bool accumulate = real_shares == 2 && both_plain;
     const int groups = rows > 8 ? 2 : 1;  // (eight-row kernel) groups of eight rows
-    if (eight) {  // its own operand layout: 512 + 64 bytes per pair of blocks and group of eight rows, inside the same region
+    // One K share of at most sixteen blocks a wavefront on up to two workgroups per compute unit: the workgroups quantize X
+    // themselves, no quantizer launch.  What they convert they convert once per workgroup, so a grid of many rounds keeps the
+    // launch (us, fused against launched; weights from memory): Q4_0 5 x 4096 on 4096 columns 6.9 against 8.1 .. 8.9, 6144 8.4
+    // (9.0), 14336 10.2 (11.2), a pair of 14336 16.0 .. 16.7 (16.8 .. 17.9), 5 x 2048 x 8192 6.1 (8.0); 8 x 4096 on 32000 columns
+    // (500 workgroups) 18.4 (18.4), on 128256 (2004) 66 (54).  Q8_0 5 x 2048 x 8192 6.1 (8.8), 8 x 2048 x 32000 13.3 (15.3),
+    // 8 x 4096 x 14336 13.7 (14.0).  Two K shares keep it too: their result has to be cleared first.  So does a result that
+    // overlaps X, which here is read by workgroups that start while others store.
+    const size_t x_bytes = static_cast<size_t>(rows) * in_dim * 4, y_bytes = static_cast<size_t>(rows) * out_dim * 4;
+    auto apart = [&](const float* y) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(input), b = reinterpret_cast<uintptr_t>(y);
+        return b + y_bytes <= a || a + x_bytes <= b;
+    };
+    const long groups8 = !eight ? 0 : [&] {
+        const int cols = bm8_columns(real_shares, out_dim, weight_b_prepared != nullptr);
+        return static_cast<long>((out_dim + cols - 1) / cols) * (weight_b_prepared ? 2 : 1);
+    }();
+    const bool quantize = eight && real_shares == 1 && bm8_can_quantize(tensor_type, halves, groups) && groups8 <= 2 * gemv_compute_units() &&
+                          apart(dst) && (!weight_b_prepared || apart(dst_b));
+    if (quantize) {
+        qa = reinterpret_cast<uint32_t*>(const_cast<float*>(input));
+    } else if (eight) {  // its own operand layout: 512 + 64 bytes per pair of blocks and group of eight rows, inside the same region
         const int pairs = (kb + 1) / 2;
         sa = reinterpret_cast<float*>(workspace + static_cast<size_t>(groups) * pairs * 512);
         const dim3 qgrid(static_cast<unsigned>((2 * pairs * 8 + 255) / 256), static_cast<unsigned>(8 * groups));
@@ -1340,7 +1477,7 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     hipError_t e;
     if (eight) {
         const int cols = bm8_columns(real_shares, out_dim, weight_b_prepared != nullptr), cg = (cols + 15) / 16;
-#define AFHIP_BM8(T, CG, H, G) bm_launch8<T, CG, H, G>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, real_shares, share_blocks, cols, accumulate, ep, second)
+#define AFHIP_BM8(T, CG, H, G) bm_launch8<T, CG, H, G>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, real_shares, share_blocks, cols, accumulate, quantize, ep, second)
 #define AFHIP_BM8_CG(T, H, G) (cg == 4 ? AFHIP_BM8(T, 4, H, G) : (cg == 3 ? AFHIP_BM8(T, 3, H, G) : (cg == 2 ? AFHIP_BM8(T, 2, H, G) : AFHIP_BM8(T, 1, H, G))))
 #define AFHIP_BM8_G(T, H) (groups == 2 ? AFHIP_BM8_CG(T, H, 2) : AFHIP_BM8_CG(T, H, 1))
         // (Q4_0: two groups of rows only on a long K, which runs four stage rounds)

@@ -529,3 +529,49 @@ def test_thirty_two_row_kernel_with_k_shares_and_pairs(fmt, rows, in_dim, out_di
         finally:
             _lib.lib().afhip_tune_batch32_max_workgroups(-1)
 
+
+
+@pytest.mark.parametrize("fmt,rows,in_dim,out_dim,pair", [
+    (Q4, 5, 4096, 4096, False), (Q4, 8, 256, 4100, False), (Q4, 7, 1280, 6152, False), (Q4, 6, 3840, 12290, True),
+    (Q4, 4, 2048, 16400, False), (Q8, 8, 2048, 4096, False), (Q8, 5, 256, 8200, True), (Q8, 7, 1792, 14336, False),
+    (Q8, 6, 4096, 11008, False), (Q8, 8, 3328, 9000, False), (Q8, 3, 4096, 28672, False),
+])
+def test_eight_row_kernel_quantizes_like_its_quantizer_launch(fmt, rows, in_dim, out_dim, pair):
+    """One K share: the workgroups quantize X themselves, unless the result overlaps X -- then the quantizer's launch runs first.
+    The two must give the same bits: odd row counts, wavefronts with some or none of their blocks, every tile width, with zero
+    blocks, ties, huge and tiny values, infinities and NaNs in X."""
+    print(f"case: eight-row kernel's own quantizer fmt={fmt} rows={rows} in={in_dim} out={out_dim} pair={pair}", flush=True)
+    x = synth.activations(4200 + rows, rows, in_dim)
+    x[0, 32:64] = 0.0
+    x[1, :32] = np.arange(32) - 15.5
+    x[1, 31] = 127.0
+    x[rows - 1, 64:96] *= 1e30
+    x[rows - 1, 96:128] *= 1e-38
+    x[rows - 1, 128:160] = 1e-45
+    x[2, 160:164] = [np.nan, np.inf, -np.inf, 1.0]  # (row 2 alone: the other rows stay numbers)
+    x[2, 192:196] = np.nan
+    wd = [G.prepare(fmt, synth.weights(fmt, 4300 + i, out_dim, in_dim), out_dim, in_dim) for i in range(2 if pair else 1)]
+    ws = torch.empty(max(kernels.workspaceBytes(fmt, rows, in_dim, out_dim), 16), dtype=torch.uint8, device=G.DEV)
+
+    def run(overlap):
+        both = torch.full((rows * (in_dim + out_dim),), float("nan"), dtype=torch.float32, device=G.DEV)
+        at = 0 if overlap else rows * in_dim  # the (first) result: X's own place, or behind it
+        both[:rows * in_dim] = torch.from_numpy(x.ravel()).to(G.DEV)
+        xd, y = both[:rows * in_dim], both[at:at + rows * out_dim]
+        second = torch.full((rows * out_dim,), float("nan"), dtype=torch.float32, device=G.DEV)
+        if pair:
+            kernels.launchLinearPairF32(G.stream(), fmt, PREP, G.buf(y), G.buf(second), G.buf(xd), G.buf(wd[0]), G.buf(wd[1]), rows, in_dim,
+                                        out_dim, G.buf(ws))
+        else:
+            kernels.launchLinearF32(G.stream(), fmt, PREP, G.buf(y), G.buf(xd), G.buf(wd[0]), rows, in_dim, out_dim, G.buf(ws))
+        torch.cuda.synchronize()
+        return y.cpu().numpy().view(np.uint32), second.cpu().numpy().view(np.uint32)
+
+    apart, over = run(False), run(True)
+    assert np.array_equal(apart[0], over[0])
+    if pair:
+        assert np.array_equal(apart[1], over[1])
+    y = apart[0].view(np.float32).reshape(rows, out_dim)
+    keep = [r for r in range(rows) if r != 2]
+    ref = O.linear_no_bias(fmt, x[keep], synth.weights(fmt, 4300, out_dim, in_dim), len(keep), in_dim, out_dim, workers=8)
+    assert G.max_rel_err(y[keep], ref.astype(np.float64)) <= TIGHT
