@@ -482,14 +482,19 @@ __global__ __launch_bounds__(256) void q4k_zero_results_kernel(float* __restrict
 // K shares (grid.z = 2, `accumulate`): a matrix with so few column tiles that half the compute units would stay idle
 // gives each tile to two workgroups, each with half of K; both add their sums to the result array, cleared beforehand,
 // with a float atomic -- two addends on a zero give the same float in either order.  No epilogue then.
+// kHalfTile (one row): a workgroup takes sixteen of a tile's columns and all of K.  Lanes with c < 16 hold those columns of
+// one super-block, the others the same columns of the next one; the digits of the two super-blocks are MFMA rows 0 .. 3 and
+// 4 .. 7, so that columns 0 .. 15 find theirs in the lower lanes and columns 16 .. 31 theirs in the upper ones: as many live
+// results per MFMA as a whole tile gives one row.  Twice the workgroups of whole tiles, without K shares and the launch that
+// clears their result.
 struct Q4kSecond {
     float* dst;
     const uint8_t* weight;
     Epilogue ep;
 };
 
-template <int kGroups, int kFlight, int kMaxThreads, bool kPlanesGiven = false>
-__global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 8 : 4) void gemv_q4k_i8_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
+template <int kGroups, int kFlight, int kMaxThreads, bool kPlanesGiven = false, bool kHalfTile = false>
+__global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 && !kHalfTile ? 8 : 4) void gemv_q4k_i8_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
                                                                   const uint8_t* __restrict__ weight_a, int rows, int in_dim,
                                                                   int out_dim, int slices, int sb_per_slice, Epilogue ep_a,
                                                                   const uint8_t* __restrict__ frag, const float* __restrict__ frag_scale,
@@ -508,8 +513,11 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
     float* xsum = xscale + ((rows * kb + 3) & ~3);                                                          // [rows][kb * 8], 16-byte aligned
     float* partial = xsum + rows * kb * 8;                                                                  // [waves][kGroups][64]
 
+    static_assert(!kHalfTile || (kGroups == 1 && !kPlanesGiven), "one row, its digits made here");
+    constexpr int kStep = kHalfTile ? 2 : 1;  // super-blocks a lane set of requests covers
     const int n_tiles = (out_dim + kTileCols - 1) >> 5;
-    const int tile = blockIdx.x < static_cast<unsigned>(n_tiles) ? blockIdx.x : n_tiles - 1;
+    const int my_tile = kHalfTile ? blockIdx.x >> 1 : blockIdx.x, col0 = kHalfTile ? 16 * (blockIdx.x & 1) : 0;
+    const int tile = my_tile < n_tiles ? my_tile : n_tiles - 1;
     const int slice = static_cast<int>(blockIdx.z) * slices + wave;  // one tile per workgroup and K share: blockDim.x = 64 * slices
     const int sb_begin = slice * sb_per_slice;
     const int sb_end = min(kb, sb_begin + sb_per_slice);
@@ -524,8 +532,16 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
     auto request = [&](int sb_first) {
 #pragma unroll
         for (int f = 0; f < kFlight; ++f) {
-            const int sb = sb_first + f;
+            const int sb = sb_first + kStep * f;
             if (sb >= sb_end) continue;  // wave-uniform; the same test guards the use below
+            if constexpr (kHalfTile) {
+                const uint32_t at = static_cast<uint32_t>(min(sb + (c >> 4), sb_end - 1)) * kTileBytes + 16 * (col0 + (c & 15));
+                hdr[f] = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(tile_base + at));
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    qv[f][t] = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(tile_base + (at + 512 * g) + (512 + t * 1024)));
+                continue;
+            }
             const uint8_t* base = tile_base + static_cast<size_t>(sb) * kTileBytes;
             hdr[f] = __builtin_nontemporal_load(reinterpret_cast<const t_u32x4*>(base + 16 * (lane & 31)));
 #pragma unroll
@@ -566,7 +582,7 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
             if ((lane & 7) == 0) xsum[r * (kb * 8) + sb * 8 + (lane >> 3)] = dg.sub_sum;
             if (lane == 0) xscale[r * kb + sb] = dg.minus_s;
         };
-        constexpr int kAhead = 2;  // items requested before the weights (one row, or two rows, of a one-super-block slice)
+        constexpr int kAhead = kHalfTile ? 2 * kFlight : 2;  // items requested before the weights (one row, or two rows, of a one-super-block slice; a half tile's whole slice)
         float4 first[kAhead];
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) first[i] = i < n_items ? *item_ptr(i) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -586,7 +602,7 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
 
     // ---- 2. this lane's roles
     const bool a_live = (c >> 2) < rows;
-    const unsigned char* a_base = xdig + static_cast<size_t>(a_live ? c : 0) * plane_stride + 16 * g;
+    const unsigned char* a_base = xdig + static_cast<size_t>(kHalfTile ? c & 3 : (a_live ? c : 0)) * plane_stride + 16 * g;
     // results: D registers 4 G .. 4 G + 3 (digits) of lane half g belong to row 2 G + g, output column c of the tile
     const float* xsum_row[kGroups];
     const float* xscale_row[kGroups];
@@ -599,12 +615,14 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
         acc[G] = 0.0f;
     }
 
-    for (int sb_first = sb_begin; sb_first < sb_end; sb_first += kFlight) {
+    for (int sb_first = sb_begin; sb_first < sb_end; sb_first += kStep * kFlight) {
         if (sb_first != sb_begin) request(sb_first);
 #pragma unroll
         for (int f = 0; f < kFlight; ++f) {
-            const int sb = sb_first + f;
-            if (sb >= sb_end) continue;  // wave-uniform: nothing was requested for it
+            const int sb_step = sb_first + kStep * f;
+            if (sb_step >= sb_end) continue;  // wave-uniform: nothing was requested for it
+            const int sb = kHalfTile ? min(sb_step + (c >> 4), sb_end - 1) : sb_step;  // the lane's own
+            const int a_sb_at = kHalfTile ? min(sb_step + ((c >> 2) & 1), sb_end - 1) : sb_step;
             const t_u32x4 h = hdr[f];
             const float d = half_bits_to_f32(static_cast<uint16_t>(h.x & 0xFFFFu));
             const float dmin = half_bits_to_f32(static_cast<uint16_t>(h.x >> 16));
@@ -613,7 +631,7 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
             const uint32_t sc_lo = h.y & 0x3F3F3F3Fu, mn_lo = h.z & 0x3F3F3F3Fu;
             const uint32_t sc_hi = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
             const uint32_t mn_hi = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-            const unsigned char* a_sb = a_base + sb * kQ4kBlockValues;
+            const unsigned char* a_sb = a_base + a_sb_at * kQ4kBlockValues;
             // the sub-block sums of a row group: all eight at once for one or two groups, one by one for more (registers)
             constexpr bool kSumsAhead = kGroups <= 2;
             float xs[kSumsAhead ? kGroups : 1][8];
@@ -664,8 +682,8 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
                 // times 2^-s (xscale holds -s as a number, NaN for a super-block with an infinity or a NaN in it)
                 const float minus_s = xscale_row[G][sb];
                 S = __builtin_fmaf(minus_s, 0.0f, __builtin_ldexpf(S, static_cast<int>(minus_s)));
-                acc[G] = __builtin_fmaf(d, S, acc[G]);
-                acc[G] = __builtin_fmaf(-dmin, min_sum[G], acc[G]);
+                const float more = __builtin_fmaf(-dmin, min_sum[G], __builtin_fmaf(d, S, acc[G]));
+                if (!kHalfTile || sb_step + (c >> 4) < sb_end) acc[G] = more;
             }
         }
     }
@@ -674,6 +692,15 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 ? 
 #pragma unroll
     for (int G = 0; G < kGroups; ++G) partial[(wave * kGroups + G) * 64 + lane] = acc[G];
     __syncthreads();
+    if constexpr (kHalfTile) {
+        if (tid < 16) {
+            float total = 0.0f;
+            for (int sl = 0; sl < slices; ++sl) total += partial[sl * 64 + tid] + partial[sl * 64 + 48 + tid];
+            const int o = static_cast<int>(blockIdx.x) * 16 + tid;
+            if (o < out_dim) dst[o] = finish_output(ep, o, o, total);
+        }
+        return;
+    }
     for (int i = tid; i < kGroups * 64; i += threads) {
         const int G = i >> 6, ln = i & 63;
         float total = 0.0f;
@@ -1486,18 +1513,29 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
     // super-block per wavefront of two workgroups, no epilogue: two K shares (K = 14336 x 4096 columns: 128 tiles, one
     // row 12.7 us on half the chip).  A call with an epilogue keeps one share and sums in another order.
     auto plain = [](const Epilogue& e) { return e.bias == nullptr && e.residual == nullptr && e.activation == kActNone; };
+    // One row of such a matrix, from seventeen super-blocks on: half tiles, all of K (us, against one share of whole tiles up to
+    // 31 super-blocks and two shares with their clearing launch beyond; weights from memory): 4352 x 4096 columns 5.8 (6.1),
+    // 5120 5.5 (6.4), 7168 6.4 (7.2), 8192 6.5 (8.4), 11008 8.8 (9.9), 14336 10.3 (10.7), 16384 10.5 (11.1), 14336 x 1024 8.2
+    // (8.9), 8192 x 2048 5.6 (8.4).  4096 x 4096 columns is even (5.5) and stays.  A slice is whole pairs of super-blocks.  A
+    // pair keeps the other form where its half tiles would take two rounds (5120 x 4096 columns each 8.9 against 7.4, 14336
+    // 20 against 18.3): there its sums have another order than a single call's.
+    const bool half_tiles = kGroups == 1 && rows == 1 && use_i8 && env_slices == 0 && slices == 16 && kb > 16 &&
+                            (second != nullptr ? 4 : 2) * n_tiles <= gemv_compute_units();
     const bool two_shares = kGroups == 1 && use_i8 && env_slices == 0 && slices == 16 && kb >= 32 && plain(ep) &&
-                            (second == nullptr || plain(second->ep)) &&
+                            (second == nullptr || plain(second->ep)) && !half_tiles &&
                             2 * n_tiles <= gemv_compute_units();
-    const int sb_per_slice = (kb + (two_shares ? 2 : 1) * slices - 1) / ((two_shares ? 2 : 1) * slices);
+    if (half_tiles && kb < 32) slices = (kb + 1) / 2;
+    const int sb_per_slice = half_tiles ? ((kb + slices - 1) / slices + 1) / 2 * 2
+                                        : (kb + (two_shares ? 2 : 1) * slices - 1) / ((two_shares ? 2 : 1) * slices);
     int tiles_per_wg = use_i8 ? 1 : (slices > 8 ? 16 : 8) / slices;  // (the int8 kernel: its wavefronts partition K, nothing else)
     if (!use_i8 && env_tiles >= 1 && env_tiles * slices <= max_waves) tiles_per_wg = env_tiles;
     const int waves = slices * tiles_per_wg;
-    const int grid = (n_tiles + tiles_per_wg - 1) / tiles_per_wg;
+    const int grid = half_tiles ? (out_dim + 15) / 16 : (n_tiles + tiles_per_wg - 1) / tiles_per_wg;
     const size_t lds = q4k_mfma_lds_bytes(rows, in_dim, waves, kGroups);
     // super-blocks requested ahead: all of a short slice (fewer registers, more wavefronts
     // resident), four at a time of a long one
-    const int flight = sb_per_slice <= 1 ? 0 : (sb_per_slice <= 2 ? 1 : 2);
+    const int steps = half_tiles ? sb_per_slice / 2 : sb_per_slice;
+    const int flight = steps <= 1 ? 0 : (steps <= 2 ? 1 : 2);
     const int variant = (waves > 8 ? 3 : 0) + flight;
     const bool own_slice = kGroups == 1 && tiles_per_wg == 1 && env_shared == 0;
     if constexpr (kGroups <= 2) {
@@ -1516,13 +1554,17 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
             } else {
                 k8 = gemv_q4k_i8_kernel<2, 2, 512>;
             }
+            if constexpr (kGroups == 1) {
+                if (half_tiles) k8 = steps <= 1 ? gemv_q4k_i8_kernel<1, 1, 1024, false, true> : gemv_q4k_i8_kernel<1, 2, 1024, false, true>;
+            }
             const size_t lds8 = q4k_i8_lds_bytes(rows, in_dim, waves);
-            static std::atomic<bool> large_lds8[6] = {};
-            if (lds8 > 64 * 1024 && !large_lds8[variant]) {
+            static std::atomic<bool> large_lds8[12] = {};
+            const int limit8 = variant + (half_tiles ? 6 : 0);
+            if (lds8 > 64 * 1024 && !large_lds8[limit8]) {
                 if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k8), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
                     e != hipSuccess)
                     return e;
-                large_lds8[variant] = true;
+                large_lds8[limit8] = true;
             }
             if (two_shares) {
                 const int count = rows * out_dim;

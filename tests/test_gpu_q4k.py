@@ -278,6 +278,32 @@ def test_two_k_shares_pair_and_bias(rows, in_dim, out_dim):
     assert G.max_rel_err(yb_, (ya + bias[None, :]).astype(np.float64)) <= TIGHT
 
 
+@pytest.mark.parametrize("in_dim,out_dim", [(4352, 96), (7168, 70), (8192, 640), (8448, 4096), (11008, 17), (16384, 33)])
+def test_one_row_on_half_tiles(in_dim, out_dim):
+    """One row, few columns, more than sixteen super-blocks: sixteen columns a workgroup, two super-blocks at a time.  Odd counts
+    of super-blocks, idle wavefronts, a last half tile without columns; halves of a pair and a bias are the plain call's bits."""
+    print(f"case: q4_k half tiles in={in_dim} out={out_dim}", flush=True)
+    wa, wb = synth.weights(Q4K, 297, out_dim, in_dim), synth.weights(Q4K, 298, out_dim, in_dim)
+    x = synth.activations(299, 1, in_dim)
+    x[0, 256:512] *= 1e20
+    x[0, -256:] *= 1e-20
+    da, db = device_weight(PREP, wa, out_dim, in_dim), device_weight(PREP, wb, out_dim, in_dim)
+    y = G.linear(Q4K, PREP, x, da, 1, in_dim, out_dim)
+    assert G.max_rel_err(y, O.linear_q4_k(x, wa, 1, in_dim, out_dim, f64=True)) <= TIGHT
+    x[0, 256:512] *= 1e-40  # now the first super-blocks and the last ones count
+    y = G.linear(Q4K, PREP, x, da, 1, in_dim, out_dim)
+    assert G.max_rel_err(y, O.linear_q4_k(x, wa, 1, in_dim, out_dim, f64=True)) <= TIGHT
+    bias = synth.activations(300, 1, out_dim).reshape(-1)
+    assert np.array_equal(G.linear_bias(Q4K, PREP, x, da, bias, 1, in_dim, out_dim), y + bias[None, :])
+    ya, yb = G.linear_pair(Q4K, PREP, x, da, db, 1, in_dim, out_dim)
+    if out_dim <= 2048:
+        assert np.array_equal(ya, y) and np.array_equal(yb, G.linear(Q4K, PREP, x, db, 1, in_dim, out_dim))
+    for got, w in ((ya, wa), (yb, wb)):
+        assert G.max_rel_err(got, O.linear_q4_k(x, w, 1, in_dim, out_dim, f64=True)) <= TIGHT
+    x[0, in_dim - 1] = np.inf  # a super-block with an infinity reaches every column, a clamped one none twice
+    assert not np.isfinite(G.linear(Q4K, PREP, x, da, 1, in_dim, out_dim)).any()
+
+
 Q8K_SHAPES = [(1, 2048, 512), (1, 3072, 2048), (2, 3072, 600), (4, 512, 1000), (9, 768, 513), (64, 1536, 512), (77, 2048, 520)]
 
 
