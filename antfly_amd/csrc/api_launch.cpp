@@ -507,28 +507,39 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
     }
     if (layout == AFHIP_LAYOUT_PREPARED && kind == AFHIP_DISPATCH_MM) {
         // rows >= 9 (or a plan that asks for mul_mm): quantize X once, then the int8-MFMA GEMM
+        const int m32 = static_cast<int>(rows), k32 = static_cast<int>(in_dim), n32 = static_cast<int>(out_dim);
+        auto apart = [&](const float* out) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(out);
+            return b + out_count * 4 <= a || a + rows * in_dim * 4 <= b;
+        };
         const WorkspaceView ws = workspace_view(workspace.ptr, rows, in_dim);
         if (workspace.ptr == 0 || workspace.len < ws.bytes || workspace.ptr % 16 != 0) return AFHIP_ERR_INVALID_STATE;
         if (counters) {
             counters->mm++;
             counters->activation_quant++;
         }
-        hipError_t e = launch_quantize_activations(stream, x, static_cast<int>(rows), static_cast<int>(in_dim), ws.qx,
-                                                   ws.sx, ws.sums);
-        if (e == hipSuccess) {
-            mark_phase(counters, 1, stream);
-            *quantizer_marked = true;
-        }
-        if (e != hipSuccess) return static_cast<afhip_status>(e);
         // room behind the quantized activations for the partial sums of K shares (small grids): optional
         const size_t partial_at = (ws.bytes + 255) / 256 * 256;
         const size_t partial_bytes = gemm_i8_partial_bytes(rows, in_dim, out_dim);
         float* partial = partial_bytes != 0 && workspace.len >= partial_at + partial_bytes
                              ? reinterpret_cast<float*>(workspace.ptr + partial_at) : nullptr;
+        // Two shares (where their sums would have room) and nothing to do to the sums but add them: the quantizer's launch clears
+        // the result and the shares add to it: no reduce launch, and a pair stays one launch (us, weights from memory, with the
+        // reduce launch in brackets): Q4_0 77 x 2048 x 2048 9.1 (11.2), 77 x 5632 x 2048 14.4 (16.5), 120 x 14336 x 2048 26.5
+        // (28.3), a pair of 97 x 2048 x 2048 11.4 (20.0); Q8_0 the same, 97 x 14336 x 2048 twice 42 .. 45 (47 .. 49).  A result
+        // that overlaps X cannot be cleared while X is read.
+        const bool cleared = partial != nullptr && !want_dots && gemm_i8_adds_to_result(m32, k32, n32, ep) &&
+                             (!pair || gemm_i8_adds_to_result(m32, k32, n32, ep_b)) && apart(y) && (!pair || apart(y_b));
+        hipError_t e = launch_quantize_activations(stream, x, m32, k32, ws.qx, ws.sx, ws.sums, cleared ? y : nullptr,
+                                                   cleared && pair ? y_b : nullptr, out_count);
+        if (e == hipSuccess) {
+            mark_phase(counters, 1, stream);
+            *quantizer_marked = true;
+        }
+        if (e != hipSuccess) return static_cast<afhip_status>(e);
         // a pair goes down together: the second matrix reuses the quantized activations (and the partial sums' room)
-        e = launch_gemm_i8(stream, tensor_type, want_dots ? nullptr : y, dot_out, ws.qx, ws.sx, w, static_cast<int>(rows),
-                           static_cast<int>(in_dim), static_cast<int>(out_dim), ep, partial, pair ? y_b : nullptr,
-                           pair ? w_b : nullptr, ep_b);
+        e = launch_gemm_i8(stream, tensor_type, want_dots ? nullptr : y, dot_out, ws.qx, ws.sx, w, m32, k32, n32, ep, partial,
+                           pair ? y_b : nullptr, pair ? w_b : nullptr, ep_b, cleared);
         if (counters && pair) counters->mm++;
         return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
     }

@@ -149,7 +149,8 @@ __device__ __forceinline__ void gemm_i8_body(
     constexpr int kStartB = kUnitsA % kWaves, kStartSx = (kStartB + kUnitsB) % kWaves, kStartSw = (kStartSx + kUnitsSx) % kWaves;
 
     // K range of this workgroup: all of it, or (a small grid spread over more compute units)
-    // share blockIdx.y of share_blocks blocks, whose sums go to partial[share][rows][out_dim]
+    // share blockIdx.y of share_blocks blocks, whose sums go to partial[share][rows][out_dim], or, without room for them, are
+    // added to a cleared dst (two shares: 0 + a + b = 0 + b + a to the bit, whoever comes first)
     // for splitk_reduce_kernel.  kb_full is the row pitch, kb the blocks walked here.
     const int kb_full = in_dim >> 5;
     const int blk_begin = kShareK ? static_cast<int>(blockIdx.y) * share_blocks : 0;
@@ -529,7 +530,8 @@ __device__ __forceinline__ void gemm_i8_body(
                 asm volatile("" : : "v"(sum));  // the sum is formed, not stored
             } else if (m < rows && n < out_dim) {
                 const size_t at = static_cast<size_t>(m) * out_dim + n;
-                if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
+                if (kShareK && partial == nullptr) unsafeAtomicAdd(dst + at, sum);
+                else if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
                 else dst[at] = finish_output(ep, n, at, sum);
             }
         }
@@ -554,7 +556,8 @@ __device__ __forceinline__ void gemm_i8_body(
             if (m < rows && n < out_dim) {
                 const size_t at = static_cast<size_t>(m) * out_dim + n;
                 const float sum = acc[p / kPerN][p % kPerN][v];
-                if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
+                if (kShareK && partial == nullptr) unsafeAtomicAdd(dst + at, sum);
+                else if (kShareK) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
                 else dst[at] = finish_output(ep, n, at, sum);
             }
         }
@@ -574,7 +577,7 @@ __global__ __launch_bounds__(64 * kWavesM * kWavesN * kSplit) void gemm_i8_kerne
     float* __restrict__ dst, int* __restrict__ dots, const int8_t* __restrict__ qx, const float* __restrict__ sx,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_tiles, int n_tiles,
     int share_blocks, float* __restrict__ partial, Epilogue ep, GemmSecond second) {
-    if (!kWriteDots && !kShareK && !kStamps && blockIdx.z != 0) {
+    if (!kWriteDots && !kStamps && blockIdx.z != 0) {
         dst = second.dst;
         weight = second.weight;
         ep = second.ep;
@@ -616,7 +619,7 @@ hipError_t launch_wide_tile(hipStream_t stream, float* dst, const int8_t* qx, co
 
 template <int kType, int kWavesM, int kWavesN, int kSplit>
 hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx, const uint8_t* weight, int rows,
-                       int in_dim, int out_dim, const Epilogue& ep, float* partial, const GemmSecond& second) {
+                       int in_dim, int out_dim, const Epilogue& ep, float* partial, const GemmSecond& second, bool cleared) {
     using S = GemmShape<kWavesM, kWavesN, kSplit, kType == 2>;
     const int m_tiles = (rows + S::kTM - 1) / S::kTM;
     const int n_tiles = (out_dim + S::kTN - 1) / S::kTN;
@@ -629,8 +632,9 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
     const int splits = partial != nullptr && dots == nullptr ? gemm_i8_splits(rows, in_dim, out_dim) : 1;
     const int share_blocks = (kb + splits - 1) / splits;
     const int shares = (kb + share_blocks - 1) / share_blocks;  // no empty share
-    float* sums = shares > 1 ? partial : nullptr;
-    dim3 g(static_cast<unsigned>(grid), static_cast<unsigned>(shares), second.dst && shares == 1 ? 2 : 1), b(S::kThreads);
+    const bool add = cleared && shares == 2;
+    float* sums = shares > 1 && !add ? partial : nullptr;
+    dim3 g(static_cast<unsigned>(grid), static_cast<unsigned>(shares), second.dst && (shares == 1 || add) ? 2 : 1), b(S::kThreads);
     auto kernel_f32 = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false>;
     auto kernel_shares = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false, true>;
     auto kernel_dots = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, true>;
@@ -658,19 +662,19 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
     else
         hipLaunchKernelGGL(kernel_f32, g, b, S::kLdsBytes, stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim,
                            m_tiles, n_tiles, share_blocks, sums, ep, second);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess || shares == 1) return e;
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || shares == 1 || add) return e;
     if (hipError_t e = launch_splitk_reduce(stream, dst, sums, static_cast<size_t>(rows) * out_dim, out_dim, shares, ep);
         e != hipSuccess || second.dst == nullptr)
         return e;
     // (the partial sums have room for one matrix: the second follows)
     return launch_tile<kType, kWavesM, kWavesN, kSplit>(stream, second.dst, dots, qx, sx, second.weight, rows, in_dim, out_dim, second.ep,
-                                                        partial, GemmSecond{});
+                                                        partial, GemmSecond{}, false);
 }
 
 template <int kType>
 hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* qx, const float* sx,
                        const uint8_t* weight, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial,
-                       const GemmSecond& second) {
+                       const GemmSecond& second, bool cleared) {
     // us of the whole op, M x K x N; "before" is the 64 x 128 tile by sixteen wavefronts that served these grids.
     static const char* env_tile = std::getenv("AFHIP_GEMM_TILE");  // tuning: "S", "X", "Y", "V" or "L", see below
     const char force = dots == nullptr && env_tile ? env_tile[0] : '\0';
@@ -715,7 +719,7 @@ hipError_t launch_type(hipStream_t stream, float* dst, int* dots, const int8_t* 
             if (tile == 'Y') return launch_wide_tile<8, 2, 2, 2, 1, 1>(stream, dst, qx, sx, weight, rows, in_dim, out_dim, ep, second);
         }
     }
-    return launch_tile<kType, 1, 2, 4>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial, second);
+    return launch_tile<kType, 1, 2, 4>(stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim, ep, partial, second, cleared);
 }
 
 }  // namespace
@@ -729,6 +733,12 @@ int gemm_i8_splits(int rows, int in_dim, int out_dim) {
     int splits = 1;
     while (splits < 8 && workgroups * splits * 2 <= units && kb / (splits * 2) >= 16) splits *= 2;
     return splits;
+}
+
+bool gemm_i8_adds_to_result(int rows, int in_dim, int out_dim, const Epilogue& ep) {
+    if (ep.bias != nullptr || ep.residual != nullptr || ep.activation != kActNone) return false;
+    const int splits = gemm_i8_splits(rows, in_dim, out_dim), kb = in_dim / 32, share_blocks = (kb + splits - 1) / splits;
+    return (kb + share_blocks - 1) / share_blocks == 2;
 }
 
 size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim) {
@@ -798,10 +808,10 @@ hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* q
 
 hipError_t launch_gemm_i8(hipStream_t stream, int tensor_type, float* dst, int* dots, const int8_t* qx, const float* sx,
                           const uint8_t* weight_prepared, int rows, int in_dim, int out_dim, const Epilogue& ep, float* partial,
-                          float* dst_b, const uint8_t* weight_b, const Epilogue& ep_b) {
+                          float* dst_b, const uint8_t* weight_b, const Epilogue& ep_b, bool cleared) {
     const GemmSecond second{dst_b, weight_b, ep_b};
-    if (tensor_type == 2) return launch_type<2>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second);
-    return launch_type<8>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second);
+    if (tensor_type == 2) return launch_type<2>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second, cleared);
+    return launch_type<8>(stream, dst, dots, qx, sx, weight_prepared, rows, in_dim, out_dim, ep, partial, second, cleared);
 }
 
 }  // namespace afhip

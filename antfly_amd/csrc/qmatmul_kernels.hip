@@ -111,9 +111,18 @@ __device__ __forceinline__ void quantize_activations_body(const float* __restric
     }
 }
 
+// zero_a (and zero_b): result arrays of zero_count floats that the GEMM behind this launch adds its two K shares' sums to;
+// cleared here, by the launch that has to run first anyway.
 __global__ __launch_bounds__(256) void quantize_activations_kernel(const float* __restrict__ x, int rows, int in_dim,
                                                                     int8_t* __restrict__ q, float* __restrict__ scale,
-                                                                    int* __restrict__ sum) {
+                                                                    int* __restrict__ sum, float* __restrict__ zero_a,
+                                                                    float* __restrict__ zero_b, size_t zero_count) {
+    if (zero_a != nullptr) {
+        for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < zero_count; i += static_cast<size_t>(gridDim.x) * blockDim.x) {
+            zero_a[i] = 0.0f;
+            if (zero_b != nullptr) zero_b[i] = 0.0f;
+        }
+    }
     quantize_activations_body(x, rows, in_dim, q, scale, sum);
 }
 
@@ -474,13 +483,13 @@ hipError_t launch_status() { return hipGetLastError(); }
 }  // namespace
 
 hipError_t launch_quantize_activations(hipStream_t stream, const float* x, int rows, int in_dim, int8_t* q,
-                                       float* scale, int* sum) {
+                                       float* scale, int* sum, float* zero_a, float* zero_b, size_t zero_count) {
     const size_t units = static_cast<size_t>(rows) * (in_dim / 4);
     size_t grid = (units + 255) / 256;
     if (grid > 4096) grid = 4096;
     if (grid == 0) return hipSuccess;
     hipLaunchKernelGGL(quantize_activations_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, x, rows,
-                       in_dim, q, scale, sum);
+                       in_dim, q, scale, sum, zero_a, zero_b, zero_count);
     return launch_status();
 }
 

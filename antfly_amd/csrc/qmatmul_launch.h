@@ -113,21 +113,26 @@ hipError_t launch_gemv_argmax_keys(hipStream_t stream, int tensor_type, unsigned
 // weights; dots optional (int32 [rows][out][in/32]), dst may be null when dots is set.
 // `partial` (optional, gemm_i8_partial_bytes() bytes): lets a launch whose tiles would leave
 // compute units idle share K out over more workgroups (gemm_i8_splits() shares, partial sums
-// added in share order by a second kernel).
+// added in share order by a second kernel, or see `cleared`).
 hipError_t launch_gemm_i8_stamps(hipStream_t stream, float* dst, const int8_t* qx, const float* sx, const uint8_t* weight,
                                  int rows, int in_dim, int out_dim);
 hipError_t launch_gemm_i8(hipStream_t stream, int tensor_type, float* dst, int* dots, const int8_t* qx, const float* sx,
                           const uint8_t* weight_prepared, int rows, int in_dim, int out_dim,
                           const Epilogue& ep = Epilogue{}, float* partial = nullptr,
-                          float* dst_b = nullptr, const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{});
+                          float* dst_b = nullptr, const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{},
+                          bool cleared = false);
+// Two K shares and no epilogue: with dst (and dst_b) cleared ahead of the launch and `cleared` set, both shares add to it.
+bool gemm_i8_adds_to_result(int rows, int in_dim, int out_dim, const Epilogue& ep);
 int gemm_i8_splits(int rows, int in_dim, int out_dim);
 size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim);
 // dst[i] = epilogue(sum over s < shares of partial[s * count + i]), i < count = rows * out_dim
 hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* partial, size_t count, int out_dim, int shares,
                                 const Epilogue& ep);
 
+// zero_a, zero_b (optional): arrays of zero_count floats to clear in the same launch
 hipError_t launch_quantize_activations(hipStream_t stream, const float* x, int rows, int in_dim, int8_t* q,
-                                       float* scale, int* sum);
+                                       float* scale, int* sum, float* zero_a = nullptr, float* zero_b = nullptr,
+                                       size_t zero_count = 0);
 
 // Any layout / shape.  route_a: uses qx/sx (pre-quantized), else f32 `input`.  dst_b / weight_b (f32 `input` only): a second
 // matrix of the same shape in the same launch.

@@ -575,3 +575,33 @@ def test_eight_row_kernel_quantizes_like_its_quantizer_launch(fmt, rows, in_dim,
     keep = [r for r in range(rows) if r != 2]
     ref = O.linear_no_bias(fmt, x[keep], synth.weights(fmt, 4300, out_dim, in_dim), len(keep), in_dim, out_dim, workers=8)
     assert G.max_rel_err(y[keep], ref.astype(np.float64)) <= TIGHT
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim,pair", [(77, 2048, 2048, False), (97, 1024, 1000, True), (129, 1056, 1541, False),
+                                                      (161, 3040, 512, True), (400, 1088, 520, False)])
+def test_two_k_shares_of_the_prefill_gemm_add_to_the_result(fmt, rows, in_dim, out_dim, pair):
+    """A plain call of two K shares clears the result in the quantizer's launch and adds both shares to it.  Whatever the result
+    held before, it must be what the reduce launch gives (a call with a bias of zeros, and one whose result overlaps X)."""
+    print(f"case: two K shares added fmt={fmt} rows={rows} in={in_dim} out={out_dim} pair={pair}", flush=True)
+    x = synth.activations(611, rows, in_dim)
+    w = [synth.weights(fmt, 612 + i, out_dim, in_dim) for i in range(2 if pair else 1)]
+    wd = [G.prepare(fmt, each, out_dim, in_dim) for each in w]
+    want = [G.linear_bias(fmt, PREP, x, each, np.zeros(out_dim, np.float32), rows, in_dim, out_dim) for each in wd]
+    ws = torch.empty(max(kernels.workspaceBytes(fmt, rows, in_dim, out_dim), 16), dtype=torch.uint8, device=G.DEV)
+    room = torch.full((rows * (in_dim + out_dim),), float("nan"), dtype=torch.float32, device=G.DEV)
+    second = torch.full((rows * out_dim,), float("nan"), dtype=torch.float32, device=G.DEV)
+    for at in (rows * in_dim, rows * in_dim, 0):  # behind X, once more on the first results, in X's place
+        room[:rows * in_dim] = torch.from_numpy(x.ravel()).to(G.DEV)
+        xd, y = room[:rows * in_dim], room[at:at + rows * out_dim]
+        if pair:
+            kernels.launchLinearPairF32(G.stream(), fmt, PREP, G.buf(y), G.buf(second), G.buf(xd), G.buf(wd[0]), G.buf(wd[1]), rows, in_dim,
+                                        out_dim, G.buf(ws))
+        else:
+            kernels.launchLinearF32(G.stream(), fmt, PREP, G.buf(y), G.buf(xd), G.buf(wd[0]), rows, in_dim, out_dim, G.buf(ws))
+        torch.cuda.synchronize()
+        for got, ref in zip((y, second), want):
+            assert np.array_equal(got.cpu().numpy().reshape(rows, out_dim), ref)
+    sample = np.r_[0:2, rows - 1]
+    ref = O.linear_no_bias(fmt, x[sample], w[0], len(sample), in_dim, out_dim, workers=8)
+    assert G.max_rel_err(want[0][sample], ref.astype(np.float64)) <= TIGHT
