@@ -12,11 +12,16 @@
 // Three v_mfma_f32_16x16x32_bf16 per 16 rows x 16 columns x block then leave the block's dots, and one multiply-add per
 // element applies the scale, as before.
 //
-// A workgroup owns 16 rows x 16 * kTiles columns and all of K; its wavefronts take the blocks round robin (sixteen of them
-// where K allows) and their sums meet in LDS in wavefront order.  kTiles column tiles share one split of X: the split is
-// about 70 of 100 vector instructions at one tile, but a short prompt has too few tiles to give up workgroups for it.
-// Bound by the vector ALU (the split) on many rows, by latency on few.  A pair of 256 columns at K = 2048: 77 rows 39.0 us
-// (two launches of a wavefront per output: 46) -> 9.6, 2048 rows 961 -> 74.  Relative error against 64 bits 1.0e-7 (1.3e-7).
+// A workgroup owns 16 rows x 16 * kTiles columns and all of K; its wavefronts (sixteen where K allows) take a run of blocks each
+// and their sums meet in LDS in wavefront order.  kTiles column tiles share one split of X: the split is about 70 of 100 vector
+// instructions at one tile, but a short prompt has too few tiles to give up workgroups for it.
+// What bounded it on most shapes was neither the split nor latency but the address unit: with every lane loading the values it
+// multiplies, a load of X asks for sixteen lines, one a lane of a quad, and so does a load of weights -- about 800 cycles of
+// address work a wavefront and four blocks.  One column tile therefore loads whole lines and lets its lanes exchange them
+// through LDS (2 KB of X, up to 2 KB of weights a wavefront, where the sums go afterwards): about 180.
+// us before / now, Q4_0: a pair of 256 columns at K = 2048, 77 rows 9.5 / 6.1, 300 rows 24 / 13, 2048 rows 73 / 64; 333 x 4096 x
+// 100 16.7 / 10.9, 20 x 4096 x 500 16.1 / 9.6.  Now the vector ALU (the split) on many rows, launch and latency on few.
+// Relative error against 64 bits 1.0e-7.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -35,6 +40,13 @@ union Bf16x8 {
 
 constexpr int kRouteRows = 16;   // rows of a workgroup, and columns of a tile
 constexpr int kRouteDepth = 4;   // blocks a wavefront requests ahead of its arithmetic
+constexpr int kWaveFloats = 1024;  // of LDS: a block of X (2 KB), one tile's weights of four blocks (2 KB); at the end the sums
+
+// What a wavefront's own lanes hand each other through LDS: the operations of a wavefront complete in order, only the compiler
+// has to keep theirs.
+__device__ __forceinline__ void wave_order() {
+    asm volatile("" : : : "memory");
+}
 
 __device__ __forceinline__ uint32_t upper_halves(float a, float b) {  // bf16 bits of a, b (already exact in bf16): a low, b high
     return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
@@ -107,7 +119,7 @@ template <int kType, int kTiles>
 __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
                                                                const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
                                                                Epilogue ep_a, RouteSecond second) {
-    extern __shared__ __align__(16) float route_sums[];  // [wavefront][tile][4][64]
+    extern __shared__ __align__(16) float route_sums[];  // a wavefront's kWaveFloats; sums: [tile][4][64]
     const bool is_b = blockIdx.z != 0;
     float* dst = is_b ? second.dst : dst_a;
     const uint8_t* weight = is_b ? second.weight : weight_a;
@@ -119,7 +131,22 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
     const int c = lane & 15, g = lane >> 4;  // operand row / column, and the eight values 8 g .. 8 g + 7 of a block
     const int m0 = blockIdx.y * kRouteRows, n0 = blockIdx.x * (16 * kTiles);
     // rows and columns past the end repeat the last one; their results are not stored
-    const float* xrow = x + static_cast<size_t>(min(m0 + c, rows - 1)) * in_dim + 8 * g;
+    // One tile: X is loaded eight lanes a row and block (rows r8 and r8 + 8), whole lines, and goes to the operand's lanes through
+    // LDS, as the weights do.  A lane that loads what it multiplies asks for sixteen lines a load, four a quad of lanes, and the
+    // address unit was what bounded the kernel (with four tiles the registers do not allow it; loaded by its user there).
+    constexpr bool kStaged = kTiles == 1;
+    const int r8 = lane >> 3, ch = lane & 7;
+    const float* xrow[2];
+    if constexpr (kStaged) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) xrow[i] = x + static_cast<size_t>(min(m0 + r8 + 8 * i, rows - 1)) * in_dim + 4 * ch;
+    } else {
+        xrow[0] = x + static_cast<size_t>(min(m0 + c, rows - 1)) * in_dim + 8 * g;
+        xrow[1] = xrow[0] + 4;
+    }
+    float* own = route_sums + wave * kWaveFloats;
+    float4* own_x = reinterpret_cast<float4*>(own);                       // [row][chunk ^ row / 2], 16 bytes each: a read in 16 banks' groups
+    unsigned char* own_w = reinterpret_cast<unsigned char*>(own) + 2048;  // [block][16-byte half][column]
     const size_t blocks = static_cast<size_t>(out_dim) * kb;
     const uint16_t* scales = reinterpret_cast<const uint16_t*>(weight + blocks * kQuantBytes);
     size_t first[kTiles];  // first block of this lane's column in each tile
@@ -131,26 +158,59 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
     for (int t = 0; t < kTiles; ++t) acc[t] = r_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     uint64_t left_behind = 0;  // lanes that met a value below about 2^-110
-    for (int b0 = wave; b0 < kb; b0 += waves * kRouteDepth) {
+    // a wavefront's blocks follow each other: parts of the same lines of weights
+    const int per_wave = (kb + waves - 1) / waves, begin = wave * per_wave, end = min(begin + per_wave, kb);
+    for (int b0 = begin; b0 < end; b0 += kRouteDepth) {
         float4 xv[kRouteDepth][2];
         uint2 wq[kRouteDepth][kTiles];
         uint16_t ws[kRouteDepth][kTiles];
+        int sraw = 0;
 #pragma unroll
         for (int u = 0; u < kRouteDepth; ++u) {
-            const int b = min(b0 + u * waves, kb - 1);  // past the end: the last block again, not used
-            xv[u][0] = reinterpret_cast<const float4*>(xrow + b * 32)[0];
-            xv[u][1] = reinterpret_cast<const float4*>(xrow + b * 32)[1];
+            const int b = min(b0 + u, end - 1);  // past the end: the last block again, not used
+            xv[u][0] = *reinterpret_cast<const float4*>(xrow[0] + b * 32);
+            xv[u][1] = *reinterpret_cast<const float4*>(xrow[1] + b * 32);
 #pragma unroll
-            for (int t = 0; t < kTiles; ++t) {
+            for (int t = 0; t < (kStaged ? 0 : kTiles); ++t) {
                 wq[u][t] = *reinterpret_cast<const uint2*>(weight + (first[t] + b) * kQuantBytes + quant_offset<kType>(g));
                 ws[u][t] = scales[first[t] + b];
             }
         }
+        if constexpr (kStaged) {
+            // a column's four blocks are one load of 64 bytes (Q8_0: two loads of 64 lanes, 128 bytes a column), its four scales
+            // are four lanes'
+            constexpr int kWeightLoads = kType == 2 ? 1 : 2;
+            const int col = lane >> 2, b = min(b0 + (lane & 3), end - 1);
+            sraw = scales[static_cast<size_t>(min(n0 + col, out_dim - 1)) * kb + b];
+            uint4 wraw[kWeightLoads];
+#pragma unroll
+            for (int i = 0; i < kWeightLoads; ++i) {
+                const int wcol = kType == 2 ? col : 8 * i + r8, wb = kType == 2 ? b : min(b0 + (ch >> 1), end - 1), half = kType == 2 ? 0 : ch & 1;
+                wraw[i] = *reinterpret_cast<const uint4*>(weight + (static_cast<size_t>(min(n0 + wcol, out_dim - 1)) * kb + wb) * kQuantBytes + 16 * half);
+            }
+#pragma unroll
+            for (int i = 0; i < kWeightLoads; ++i) {
+                const int slot = kType == 2 ? (lane & 3) * 16 + col : ch * 16 + 8 * i + r8;
+                *reinterpret_cast<uint4*>(own_w + 16 * slot) = wraw[i];
+            }
+        }
 #pragma unroll
         for (int u = 0; u < kRouteDepth; ++u) {
-            if (b0 + u * waves >= kb) break;  // wavefront-uniform
+            if (b0 + u >= end) break;  // wavefront-uniform
             Bf16x8 part[3];
-            const float v[8] = {xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w, xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w};
+            float4 x0 = xv[u][0], x1 = xv[u][1];
+            if constexpr (kStaged) {
+                own_x[r8 * 8 + (ch ^ (r8 >> 1))] = x0;
+                own_x[(r8 + 8) * 8 + (ch ^ ((r8 + 8) >> 1))] = x1;
+                wave_order();
+                x0 = own_x[c * 8 + ((2 * g) ^ (c >> 1))];
+                x1 = own_x[c * 8 + ((2 * g + 1) ^ (c >> 1))];
+                const int slot = kType == 2 ? u * 16 + c : (u * 2 + (g >> 1)) * 16 + c;
+                wq[u][0] = *reinterpret_cast<const uint2*>(own_w + 16 * slot + 8 * (g & 1));
+                ws[u][0] = static_cast<uint16_t>(__builtin_amdgcn_ds_bpermute(4 * (4 * c + u), sraw));
+                wave_order();
+            }
+            const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) split_pair(v[2 * i], v[2 * i + 1], &part[0].u[i], &part[1].u[i], &part[2].u[i], &left_behind);
 #pragma unroll
@@ -168,7 +228,7 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
 #pragma unroll
     for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) route_sums[((wave * kTiles + t) * 4 + i) * 64 + lane] = acc[t][i];
+        for (int i = 0; i < 4; ++i) own[(t * 4 + i) * 64 + lane] = acc[t][i];
     // A second pass over the wavefront's blocks where a value left something behind, added to its own sums in LDS: no activation
     // of a model does, and nothing of this may take registers in the loop above: four tiles keep to the 64 that give a compute
     // unit two workgroups (as a branch in the loop 128; one workgroup: 4096 rows of K = 288 x 288 columns 11.0 -> 12.1 us).
@@ -178,7 +238,7 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
         const int c2 = again & 15, g2 = again >> 4;
         const float* row = x + static_cast<size_t>(min(m0 + c2, rows - 1)) * in_dim + 8 * g2;
 #pragma unroll 1
-        for (int b = wave; b < kb; b += waves) {
+        for (int b = begin; b < end; ++b) {
             const float4 x0 = reinterpret_cast<const float4*>(row + b * 32)[0], x1 = reinterpret_cast<const float4*>(row + b * 32)[1];
             Bf16x8 rest[2];
             left_pair(x0.x, x0.y, &rest[0].u[0], &rest[1].u[0]);
@@ -193,7 +253,7 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
 #pragma unroll
                 for (int q = 1; q >= 0; --q) dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rest[q].v, w, dot, 0, 0, 0);
                 const float d = half_bits_to_f32(scales[at]);
-                float* sums = route_sums + (wave * kTiles + t) * 256 + again;
+                float* sums = own + t * 256 + again;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (dot[i] != 0.0f) sums[64 * i] += d * dot[i] * 0x1p-100f;  // (d may be an infinity)
@@ -203,7 +263,7 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
     __syncthreads();
     for (int at = tid; at < kTiles * 256; at += blockDim.x) {
         float total = 0.0f;
-        for (int w = 0; w < waves; ++w) total += route_sums[w * (kTiles * 256) + at];
+        for (int w = 0; w < waves; ++w) total += route_sums[w * kWaveFloats + at];
         const int l = at & 63, i = (at >> 6) & 3, t = at >> 8;
         const int m = m0 + 4 * (l >> 4) + i, n = n0 + 16 * t + (l & 15);
         if (m < rows && n < out_dim) {
@@ -224,11 +284,14 @@ hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* ds
     for (int r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
         const int nr = rows - r0 < kRowsPerLaunch ? rows - r0 : kRowsPerLaunch;
         const unsigned groups = static_cast<unsigned>((nr + 15) / 16);
-        // one column tile while four of them a workgroup would leave compute units without one
+        // One column tile, whose loads go through LDS, or four, which share a split of X but not those loads (us, one / four; the
+        // two add alike): from K = 1056 on one everywhere -- a pair of 256 columns, 700 x 1536 19 / 29, 2048 x 1536 49 / 56,
+        // 1000 x 4096 61 / 75, 2048 x 5120 144 / 179 -- below, four on grids of two workgroups a compute unit: a pair of 2048 x
+        // 1024 x 256 38 .. 42 / 39, of 2048 x 768 31 / 25, 4096 x 288 x 288 15.5 / 10.5, but a pair of 700 x 1024 x 256 14.2 / 20.5.
         const long wide = static_cast<long>(groups) * ((out_dim + 63) / 64) * matrices;
-        const int tiles = wide >= gemv_compute_units() ? 4 : 1;
+        const int tiles = kb <= 32 && wide >= 2 * gemv_compute_units() ? 4 : 1;
         const dim3 grid(static_cast<unsigned>((out_dim + 16 * tiles - 1) / (16 * tiles)), groups, matrices), block(64 * waves);
-        const size_t lds = static_cast<size_t>(waves) * tiles * 1024;  // at most 64 KiB
+        const size_t lds = static_cast<size_t>(waves) * kWaveFloats * 4;  // at most 64 KiB
         Epilogue ep = ep0, ep_b = ep_b0;
         if (ep.residual) ep.residual += static_cast<size_t>(r0) * out_dim;
         if (ep_b.residual) ep_b.residual += static_cast<size_t>(r0) * out_dim;

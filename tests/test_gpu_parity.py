@@ -605,3 +605,23 @@ def test_two_k_shares_of_the_prefill_gemm_add_to_the_result(fmt, rows, in_dim, o
     sample = np.r_[0:2, rows - 1]
     ref = O.linear_no_bias(fmt, x[sample], w[0], len(sample), in_dim, out_dim, workers=8)
     assert G.max_rel_err(want[0][sample], ref.astype(np.float64)) <= TIGHT
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(77, 2048, 250), (33, 1056, 257), (70, 1088, 500), (530, 1312, 130), (2100, 64, 500),
+                                                 (1030, 1024, 510), (18, 5152, 490), (130, 96, 500)])
+def test_f32_route_tiles_and_runs_of_blocks(fmt, rows, in_dim, out_dim):
+    """One column tile (loads exchanged through LDS) and four: runs of one to eleven blocks a wavefront, the last ones short or
+    empty, ragged rows and columns.  Each half of a pair is the single call to the bit, whichever tile each of them takes."""
+    print(f"case: f32 route tiles fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(711, rows, in_dim)
+    x[rows // 2, in_dim // 2:] *= 1e-37  # values that three bf16 parts do not hold
+    wa, wb = synth.weights(fmt, 712, out_dim, in_dim), synth.weights(fmt, 713, out_dim, in_dim)
+    da, db = G.prepare(fmt, wa, out_dim, in_dim), G.prepare(fmt, wb, out_dim, in_dim)
+    ya, yb = G.linear_pair(fmt, PREP, x, da, db, rows, in_dim, out_dim)
+    assert np.array_equal(ya, G.linear(fmt, PREP, x, da, rows, in_dim, out_dim))
+    assert np.array_equal(yb, G.linear(fmt, PREP, x, db, rows, in_dim, out_dim))
+    sample = np.r_[0:2, rows // 2, rows - 2:rows]
+    for got, w in ((ya, wa), (yb, wb)):
+        ref = O.linear_no_bias(fmt, x[sample], w, len(sample), in_dim, out_dim, workers=8)
+        assert G.max_rel_err(got[sample], ref.astype(np.float64)) <= TIGHT
