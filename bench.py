@@ -28,6 +28,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_BPS = 8.0e12           # MI355X HBM3E
 INT8_MFMA_PEAK_OPS = 5.0e15     # MI355X dense int8 MFMA
 BF16_MFMA_PEAK_FLOPS = 2.5e15   # MI355X dense bf16 MFMA
+FP6_MFMA_PEAK_FLOPS = 10.0e15  # dense: 64 K values in the cycles of sixteen bf16 ones
 Q4, Q8, Q4K = 2, 8, 12
 BLOCK_BYTES = {Q4: 18, Q8: 34}
 
@@ -883,14 +884,15 @@ def main() -> int:
         for m in (32, 128, 512):
             w_s, e_s = time_config(Q4K, m, 4096, 14336, 40, 5, 2, 78)
             flops = 2.0 * m * 4096 * 14336
-            # the kernel issues three bf16 MFMA products per f32 product (X as hi + mid + lo parts), so the
-            # matrix-core work is 3 x 2MNK flop, priced against the dense bf16 peak
+            # up to 64 rows the kernel issues three bf16 MFMA products per f32 product (X as hi + mid + lo parts), past them
+            # eight 6-bit ones (X as eight 4-bit digits): priced against the dense peak of each
+            parts, name, peak = (3, "bf16", BF16_MFMA_PEAK_FLOPS) if m <= 64 else (8, "fp6", FP6_MFMA_PEAK_FLOPS)
             extra[f"q4k_gemm_m{m}_k4096_n14336"] = {
-                "what": "Q4_K prefill: X split once into three bf16 parts, bf16-MFMA GEMM, f32-accurate; per call incl. the split",
+                "what": f"Q4_K prefill: X split once into {parts} {name} parts, {name}-MFMA GEMM, f32-accurate; per call incl. the split",
                 "us_per_call": round(e_s / 40 * 1e6, 1),
                 "TFLOPs_f32_equivalent": round(flops * 40 / e_s / 1e12, 1),
-                "bf16_mfma_TFLOPs_issued": round(3 * flops * 40 / e_s / 1e12, 1),
-                "frac_bf16_mfma_peak": round(3 * flops * 40 / e_s / BF16_MFMA_PEAK_FLOPS, 4)}
+                f"{name}_mfma_TFLOPs_issued": round(parts * flops * 40 / e_s / 1e12, 1),
+                f"frac_{name}_mfma_peak": round(parts * flops * 40 / e_s / peak, 4)}
         for m in (128, 512, 2048):
             gsteps = 200
             w_s, e_s = time_config(Q8, m, 4096, 4096, gsteps, 20, 4, 7)
