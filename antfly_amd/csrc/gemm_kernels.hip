@@ -747,43 +747,34 @@ size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim) {
     return splits > 1 ? static_cast<size_t>(splits) * rows * out_dim * 4 : 0;
 }
 
-// dst = epilogue(sum over the K shares, in order): second kernel of a split-K launch.  kLanes values a thread (four where count
-// and both arrays allow 16-byte accesses; a lane's column is only worked out where an epilogue asks for it).
-template <int kLanes>
+// dst = epilogue(sum over the K shares, in order): second kernel of a split-K launch.  Four shares' values on their way at a
+// time; a column is only worked out where an epilogue asks for it.  (us a call, against a serial loop over the shares with a
+// remainder for every value: Q8_0 100 x 4096 x 1024 12.3 -> 11.7, Q4_0 32 x 14336 x 4096 19.4 -> 18.9.  Four values a thread did
+// no better there and lost where the shares are large: Q4_K 32 x 4096 x 14336 22.2 -> 24.4, 64 x 4096 x 4096 17.0 -> 19.8.)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(float* __restrict__ dst, const float* __restrict__ partial,
                                                             size_t count, int out_dim, int splits, Epilogue ep) {
-    typedef float Values __attribute__((ext_vector_type(kLanes)));
     const bool plain = ep.bias == nullptr && ep.residual == nullptr && ep.activation == kActNone;
-    const size_t groups = count / kLanes;
-    for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < groups;
+    for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < count;
          i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        Values total = 0.0f;
-        for (int z0 = 0; z0 < splits; z0 += 4) {  // four shares' values on their way at a time
-            Values part[4];
+        float total = 0.0f;
+        for (int z0 = 0; z0 < splits; z0 += 4) {
+            float part[4];
 #pragma unroll
-            for (int z = 0; z < 4; ++z)
-                part[z] = reinterpret_cast<const Values*>(partial + static_cast<size_t>(min(z0 + z, splits - 1)) * count)[i];
+            for (int z = 0; z < 4; ++z) part[z] = partial[static_cast<size_t>(min(z0 + z, splits - 1)) * count + i];
 #pragma unroll
             for (int z = 0; z < 4; ++z)
                 if (z0 + z < splits) total += part[z];
         }
-        if (!plain) {
-#pragma unroll
-            for (int k = 0; k < kLanes; ++k)
-                total[k] = finish_output(ep, static_cast<int>((i * kLanes + k) % out_dim), i * kLanes + k, total[k]);
-        }
-        reinterpret_cast<Values*>(dst)[i] = total;
+        dst[i] = plain ? total : finish_output(ep, static_cast<int>(i % out_dim), i, total);
     }
 }
 
 hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* partial, size_t count, int out_dim, int shares,
                                 const Epilogue& ep) {
-    const bool wide = count % 4 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0;
-    const size_t groups = wide ? count / 4 : count;
-    size_t grid = (groups + 255) / 256;
+    size_t grid = (count + 255) / 256;
     if (grid > 4096) grid = 4096;
-    auto kernel = wide ? splitk_reduce_kernel<4> : splitk_reduce_kernel<1>;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, dst, partial, count, out_dim, shares, ep);
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, dst, partial, count, out_dim,
+                       shares, ep);
     return hipGetLastError();
 }
 
