@@ -289,7 +289,8 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
     // more rows than one GEMV launch holds: X split once into the caller's scratch, then the
     // GEMM (without scratch the GEMV serves them a launch at a time)
     const size_t gemm_rows = static_cast<size_t>(gemm_q4k_min_rows(static_cast<int>(in_dim)));
-    const bool gemm = tiled && rows >= gemm_rows && workspace.ptr != 0 && workspace.ptr % 16 == 0 && workspace.len >= gemm_q4k_workspace_bytes(rows, in_dim, out_dim);
+    const bool gemm = tiled && rows >= gemm_rows && workspace.ptr != 0 && workspace.ptr % 16 == 0 &&
+                      gemm_q4k_fits(rows, in_dim, out_dim, workspace.len);
     for (int i = 0; i < (pair ? 2 : 1); ++i) {
         if (counters) {
             if (kind == AFHIP_DISPATCH_MMV) counters->mmv++;
@@ -299,7 +300,7 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
         if (gemm) {  // a pair goes down together: X is split once
             if (i == 1) continue;
             hipError_t e = launch_gemm_q4k_tiled(stream, reinterpret_cast<float*>(dst.ptr), reinterpret_cast<const float*>(input.ptr),
-                                                 reinterpret_cast<const uint8_t*>(weight.ptr), reinterpret_cast<void*>(workspace.ptr),
+                                                 reinterpret_cast<const uint8_t*>(weight.ptr), reinterpret_cast<void*>(workspace.ptr), workspace.len,
                                                  static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), ep,
                                                  pair ? reinterpret_cast<float*>(dst_b.ptr) : nullptr,
                                                  pair ? reinterpret_cast<const uint8_t*>(weight_b.ptr) : nullptr, ep_b);

@@ -38,9 +38,11 @@
 
 #include <stdint.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
+#include "antfly_hip_qmatmul.h"
 #include "device_common.h"
 #include "qmatmul_launch.h"
 
@@ -1708,32 +1710,63 @@ constexpr Q4kGemmCost kQ4kGemmCosts[4] = {
     {32, 128, 1, 4, {0.219, 0.329, 0.490, 0.627}, 0.0, 7.2, 2.5, 0.21, 3.1, 0.25},
 };
 
-// `pair`: for both matrices of a pair in one launch (one share); its tile may be another than the single call's, as a result's bits
-// depend on the shares alone (333 x 4096 x 14336 twice: 64 x 256 tiles 212 us, 64 x 128 231; once 124 / 119).
-// Up to 64 rows the bf16 kernel is the faster one (64 x 4096 x 4096 17.5 against 19.4 us, 32 x 4096 x 14336 21.4 / 22.4) and keeps its
-// own shares: one when its workgroups fill the compute units anyway, else as many as spread it over them.  Above, the tile and
-// share count that cost least -- one share where that costs at most 3 % more, since a pair is one launch then -- unless the bf16
-// kernel is expected within 3 % of it (small matrices: 200 x 2048 x 2048 17.3 against 20.4; 333 x 2048 x 5632 36.9 / 40.6, a grid that
-// just fills its rounds).
-Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, bool pair = false) {
-    const int kb = static_cast<int>(in_dim / kQ4kBlockValues);
-    const double m = static_cast<double>(rows), k = static_cast<double>(in_dim), n = static_cast<double>(out_dim);
-    auto allowed = [&](int s) { return s == 1 || (s <= 8 && kb / s >= 2); };
+// The parts or digits of X with the sub-block sums behind them (the fp6 kernel's rows are padded to even), and the partial sums of
+// K shares behind those.
+size_t gemm_q4k_digit_bytes(size_t rows, size_t in_dim) { return (rows + 1) / 2 * 2 * in_dim * 6; }
+size_t gemm_q4k_split_bytes(Q4kGemmKind kind, size_t rows, size_t in_dim) {
+    const size_t values = kind == kParts ? rows * in_dim * 6 : gemm_q4k_digit_bytes(rows, in_dim);
+    return (values + rows * (in_dim / 32) * 8 + 255) / 256 * 256;
+}
+size_t gemm_q4k_plan_bytes(const Q4kGemmPlan& plan, size_t rows, size_t in_dim, size_t out_dim) {
+    return gemm_q4k_split_bytes(plan.kind, rows, in_dim) + (plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * out_dim * 4 : 0);
+}
+
+bool gemm_q4k_shares_allowed(int splits, size_t in_dim) { return splits == 1 || (splits <= 8 && in_dim / kQ4kBlockValues / splits >= 2); }
+
+// The bf16 kernel's own shares: one when its workgroups fill the compute units anyway, else as many as spread it over them.
+Q4kGemmPlan gemm_q4k_parts_plan(size_t rows, size_t in_dim, size_t out_dim) {
     Q4kGemmPlan parts{kParts, 1};
     const long long workgroups = static_cast<long long>((out_dim + 255) / 256) * static_cast<long long>((rows + kG32Rows - 1) / kG32Rows);
-    while (workgroups * parts.splits * 2 <= device_units() && allowed(parts.splits * 2)) parts.splits *= 2;
-    if (rows <= 64) return parts;
-    Q4kGemmPlan best{kFp6Tile64x256, 1};
+    while (workgroups * parts.splits * 2 <= device_units() && gemm_q4k_shares_allowed(parts.splits * 2, in_dim)) parts.splits *= 2;
+    return parts;
+}
+
+// The scratch that a call may take: the cost of a plan says nothing of the memory it asks callers for (without a limit 129 x 5120 x 13824
+// took 31 MB where X is 4, 512 x 8192 x 28672 137 where X is 25).  A call whose bf16 plan fits the static entry's array keeps
+// fitting it; past that the partial sums may take twice what the bf16 plan takes.  us with this limit / without: 333 x 4096 x 6144
+// 72 / 70 (one share for four), 129 x 4096 x 4096 29.8 / 29.4, 512 x 8192 x 28672 482 / 466; by the cost model 2 % on the mean of 4000
+// shapes (65 .. 2048 rows), 3 % with the same room once, 11 % without any past the bf16 plan's.
+size_t gemm_q4k_most_bytes(size_t rows, size_t in_dim, size_t out_dim) {
+    const size_t parts = gemm_q4k_plan_bytes(gemm_q4k_parts_plan(rows, in_dim, out_dim), rows, in_dim, out_dim);
+    return parts <= AFHIP_STATIC_SCRATCH_BYTES ? static_cast<size_t>(AFHIP_STATIC_SCRATCH_BYTES) : 3 * parts;
+}
+
+// The plan of a call that lends `room` bytes (splits = 0: none fits).  Whoever lends gemm_q4k_workspace_bytes or more gets the
+// same one: the choice is over what fits, and the best of all that fits the most a call may take is the best of fewer.
+// `pair`: for both matrices of a pair in one launch (one share); its tile may be another than the single call's, as a result's bits
+// depend on the shares alone (333 x 4096 x 14336 twice: 64 x 256 tiles 212 us, 64 x 128 231; once 124 / 119).
+// Up to 64 rows the bf16 kernel is the faster one (64 x 4096 x 4096 17.5 against 19.4 us, 32 x 4096 x 14336 21.4 / 22.4).  Above, the
+// tile and share count that cost least -- one share where that costs at most 3 % more, since a pair is one launch then -- unless the
+// bf16 kernel is expected within 3 % of it (small matrices: 200 x 2048 x 2048 17.3 against 20.4; 333 x 2048 x 5632 36.9 / 40.6, a
+// grid that just fills its rounds).
+Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, size_t room, bool pair = false) {
+    const double m = static_cast<double>(rows), k = static_cast<double>(in_dim), n = static_cast<double>(out_dim);
+    room = std::min(room, gemm_q4k_most_bytes(rows, in_dim, out_dim));
+    auto fits = [&](const Q4kGemmPlan& p) { return gemm_q4k_plan_bytes(p, rows, in_dim, out_dim) <= room; };
+    const Q4kGemmPlan none{kParts, 0}, parts = gemm_q4k_parts_plan(rows, in_dim, out_dim);
+    if (rows <= 64) return fits(parts) ? parts : none;
+    Q4kGemmPlan best = none;
     double best_us = 1e30;
     for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
-        for (int s = 1; allowed(s); s *= 2) {
+        for (int s = 1; gemm_q4k_shares_allowed(s, in_dim); s *= 2) {
+            const Q4kGemmPlan plan{static_cast<Q4kGemmKind>(kind), s};
             const double us = kQ4kGemmCosts[kind].us(m, k, n, s) * (s == 1 ? 1.0 : 1.03);
-            if (us < best_us) {
+            if (us < best_us && fits(plan)) {
                 best_us = us;
-                best = {static_cast<Q4kGemmKind>(kind), s};
+                best = plan;
             }
         }
-    if (kQ4kGemmCosts[kParts].us(m, k, n, parts.splits) * 0.97 < best_us) return parts;
+    if (fits(parts) && kQ4kGemmCosts[kParts].us(m, k, n, parts.splits) * 0.97 < best_us) return parts;
     if (pair && best.splits == 1) {
         best_us = 1e30;
         for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
@@ -1743,13 +1776,6 @@ Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, bool pair 
             }
     }
     return best;
-}
-
-// The parts or digits of X; the fp6 kernel's rows are padded to even.
-size_t gemm_q4k_digit_bytes(size_t rows, size_t in_dim) { return (rows + 1) / 2 * 2 * in_dim * 6; }
-size_t gemm_q4k_split_bytes(const Q4kGemmPlan& plan, size_t rows, size_t in_dim) {
-    const size_t values = plan.kind == kParts ? rows * in_dim * 6 : gemm_q4k_digit_bytes(rows, in_dim);
-    return (values + rows * (in_dim / 32) * 8 + 255) / 256 * 256;
 }
 
 struct Q4kGemmCall {
@@ -1784,21 +1810,25 @@ hipError_t launch_fp6_tile(const Q4kGemmCall& q) {
 }  // namespace
 
 size_t gemm_q4k_workspace_bytes(size_t rows, size_t in_dim, size_t out_dim) {
-    const Q4kGemmPlan plan = gemm_q4k_plan(rows, in_dim, out_dim);
-    return gemm_q4k_split_bytes(plan, rows, in_dim) + (plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * out_dim * 4 : 0);
+    return gemm_q4k_plan_bytes(gemm_q4k_plan(rows, in_dim, out_dim, SIZE_MAX), rows, in_dim, out_dim);
+}
+
+bool gemm_q4k_fits(size_t rows, size_t in_dim, size_t out_dim, size_t workspace_bytes) {
+    return gemm_q4k_plan(rows, in_dim, out_dim, workspace_bytes).splits != 0;
 }
 
 hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, void* workspace,
-                                 int rows, int in_dim, int out_dim, const Epilogue& ep, float* dst_b, const uint8_t* weight_b,
-                                 const Epilogue& ep_b) {
+                                 size_t workspace_bytes, int rows, int in_dim, int out_dim, const Epilogue& ep, float* dst_b,
+                                 const uint8_t* weight_b, const Epilogue& ep_b) {
     if (in_dim % kQ4kBlockValues != 0 || rows < 1 || workspace == nullptr) return hipErrorInvalidValue;
     const Q4kGemmPlan plan = gemm_q4k_plan(static_cast<size_t>(rows), static_cast<size_t>(in_dim), static_cast<size_t>(out_dim),
-                                           dst_b != nullptr);
+                                           workspace_bytes, dst_b != nullptr);
+    if (plan.splits == 0) return hipErrorInvalidValue;
     const int kb = in_dim / kQ4kBlockValues;
     const int sb_per_split = (kb + plan.splits - 1) / plan.splits;
     const int shares = (kb + sb_per_split - 1) / sb_per_split;  // no empty share
     uint8_t* const space = static_cast<uint8_t*>(workspace);
-    float* partial = shares > 1 ? reinterpret_cast<float*>(space + gemm_q4k_split_bytes(plan, rows, in_dim)) : nullptr;
+    float* partial = shares > 1 ? reinterpret_cast<float*>(space + gemm_q4k_split_bytes(plan.kind, rows, in_dim)) : nullptr;
     const int m_tiles = (rows + kG32Rows - 1) / kG32Rows;
     if (m_tiles > 65535) return hipErrorInvalidValue;
     uint32_t* parts = static_cast<uint32_t*>(workspace);

@@ -211,14 +211,16 @@ hipError_t launch_gemv_q4k_i8_rows(hipStream_t stream, float* dst, const void* w
                                    int out_dim, const Epilogue& ep, float* dst_b = nullptr, const uint8_t* weight_b = nullptr,
                                    const Epilogue& ep_b = Epilogue{}, bool results_cleared = false);
 // More rows than one launch of the kernel above holds (gemv_q4k_tiled_rows_per_launch): X is split
-// once into `workspace` (gemm_q4k_workspace_bytes, 16-byte aligned; it also holds the partial sums when a
-// small problem splits K over several workgroups) and a GEMM multiplies.  Any in_dim that is a multiple of 256.  dst_b and
-// weight_b: a second matrix on the same X.
+// once into `workspace` (16-byte aligned; it also holds the partial sums when a small problem splits K over several
+// workgroups) and a GEMM multiplies.  Any in_dim that is a multiple of 256.  dst_b and weight_b: a second matrix on the same X.
+// gemm_q4k_workspace_bytes: what the best plan takes.  With less (past 64 rows) K is split over fewer workgroups, or not at all;
+// gemm_q4k_fits: whether any plan finds room.
 int gemv_q4k_tiled_rows_per_launch(int in_dim);
 int gemm_q4k_min_rows(int in_dim);  // fewer rows fit one GEMV launch (or are two rows)
 size_t gemm_q4k_workspace_bytes(size_t rows, size_t in_dim, size_t out_dim);
+bool gemm_q4k_fits(size_t rows, size_t in_dim, size_t out_dim, size_t workspace_bytes);
 hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, void* workspace,
-                                 int rows, int in_dim, int out_dim, const Epilogue& ep = Epilogue{}, float* dst_b = nullptr,
+                                 size_t workspace_bytes, int rows, int in_dim, int out_dim, const Epilogue& ep = Epilogue{}, float* dst_b = nullptr,
                                  const uint8_t* weight_b = nullptr, const Epilogue& ep_b = Epilogue{});
 hipError_t launch_dequantize_q4k_tiled_rows(hipStream_t stream, float* dst, const uint8_t* weight, const long long* ids,
                                             size_t rows, int dim, size_t weight_rows);

@@ -158,7 +158,9 @@ int afhip_uses_q8k_activation_quant(int tensor_type, size_t rows, size_t in_dim,
  * ---------------------------------------------------------------------- */
 
 /* Bytes of device scratch a launch needs (quantized activations for the
- * int8-MFMA GEMM and for unfused GEMV); 0 when the call needs none. */
+ * int8-MFMA GEMM and for unfused GEMV); 0 when the call needs none.  From nine rows on (Q4_K: past 64)
+ * the figure may hold room for the partial sums of K shares, which is optional: a launch that finds
+ * less runs on fewer shares or one, its sums in another order. */
 size_t afhip_linear_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, size_t out_dim);
 
 /* Y = X * W^T.  `layout` says how `weight` is stored; `dispatch` is -1 to let

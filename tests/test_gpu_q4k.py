@@ -515,6 +515,32 @@ def test_prefill_past_64_rows_on_extreme_activations():
     assert np.array_equal(got[~hit], y[~hit])
 
 
+def test_prefill_past_64_rows_in_a_workspace_without_room_for_partial_sums():
+    """A workspace that holds the split of X but not the sums of the K shares: the GEMM on one share -- the bits of the same columns
+    in a matrix so wide that K is not shared out -- and in one that holds three parts a value but not an even number of rows of digits
+    still a result within tolerance."""
+    rows, in_dim, out_dim, wide = 129, 4096, 4096, 11008
+    print("case: q4_k prefill in a short workspace", flush=True)
+    w = synth.weights(Q4K, 95, wide, in_dim)
+    x = synth.activations(96, rows, in_dim)
+    narrow = w[:out_dim * (in_dim // 256) * 144]
+    digits = 130 * in_dim * 6 + 129 * (in_dim // 256) * 64
+    assert kernels.workspaceBytes(Q4K, rows, in_dim, out_dim) > digits + rows * out_dim * 8
+    assert kernels.workspaceBytes(Q4K, rows, in_dim, wide) == (digits + 255) // 256 * 256
+    want = G.linear(Q4K, PREP, x, device_weight(PREP, w, wide, in_dim), rows, in_dim, wide)[:, :out_dim]
+    xd, wd = G.to_dev(x), device_weight(PREP, narrow, out_dim, in_dim)
+    sample = np.r_[0:2, 31:34, rows - 1]
+    ref = O.linear_q4_k(x[sample], narrow, len(sample), in_dim, out_dim, f64=True)
+    for spare in (0, 256, -in_dim * 6):
+        lent = torch.empty((digits + 255) // 256 * 256 + spare, dtype=torch.uint8, device=G.DEV)
+        y = torch.full((rows, out_dim), float("nan"), dtype=torch.float32, device=G.DEV)
+        kernels.launchLinearF32(G.stream(), Q4K, PREP, G.buf(y), G.buf(xd), G.buf(wd), rows, in_dim, out_dim, G.buf(lent))
+        torch.cuda.synchronize()
+        if spare >= 0:
+            assert np.array_equal(y.cpu().numpy(), want)
+        assert G.max_rel_err(y.cpu().numpy()[sample], ref) <= TIGHT
+
+
 def test_linear_argument_checks():
     w = G.to_dev(synth.weights(Q4K, 1, 4, 256))
     x = G.to_dev(synth.activations(2, 1, 256))

@@ -5,6 +5,7 @@ import ctypes as C
 import os
 import re
 
+import numpy as np
 import pytest
 
 from antfly_amd import _lib, kernels, quant_matmul as qm
@@ -131,6 +132,33 @@ def test_q4_k_prefill_workspace_sizes():
     assert kernels.workspaceBytes(Q4K, 2048, 4096, 14336) == 2048 * 4096 * 6 + 2048 * 16 * 64
     # the smallest prefill on a small matrix spreads K over workgroups
     assert kernels.workspaceBytes(Q4K, 13, 4096, 4096) > 13 * 4096 * 6 + 13 * 16 * 64
+
+
+def test_q4_k_prefill_workspace_is_bounded():
+    """Past 64 rows: what the bf16 kernel takes (the split of X and the sums of the K shares that spread a small grid over 256
+    compute units) decides.  Calls that fit the static entry's scratch with it keep fitting; beyond, at most three times that.  A
+    one-share call needs no more than the split of X, its rows rounded up to even."""
+    Q4K, limit = _lib.TYPE_Q4_K, kernels.STATIC_SCRATCH_BYTES
+
+    def bf16_kernel(rows, k, n):
+        workgroups, shares = (n + 255) // 256 * ((rows + 31) // 32), 1
+        while workgroups * shares * 2 <= 256 and shares < 8 and k // 256 // (2 * shares) >= 2:
+            shares *= 2
+        return (rows * k * 6 + rows * (k // 256) * 64 + 255) // 256 * 256 + (shares * rows * n * 4 if shares > 1 else 0)
+
+    rng = np.random.default_rng(17)
+    shapes = [(333, 4096, 6144), (256, 4096, 4096), (129, 5120, 13824), (512, 8192, 28672), (1397, 24576, 24528), (333, 14336, 4096)]
+    shapes += [(int(m), 256 * int(k), int(n)) for m, k, n in zip(rng.integers(65, 1500, 4000), rng.integers(1, 57, 4000),
+                                                               np.exp(rng.uniform(np.log(32), np.log(28672), 4000)))]
+    for rows, k, n in shapes:
+        if _lib.lib().afhip_uses_q8k_activation_quant(Q4K, rows, k, n):
+            continue
+        got, least = kernels.workspaceBytes(Q4K, rows, k, n), bf16_kernel(rows, k, n)
+        digits = ((rows + 1) // 2 * 2 * k * 6 + rows * (k // 256) * 64 + 255) // 256 * 256
+        assert min(least, digits) <= got <= max(digits, limit if least <= limit else 3 * least), (rows, k, n, got, least)
+    # odd rows whose X fits by less than a row of digits: the bf16 kernel
+    assert bf16_kernel(655, 4096, 14336) <= limit < 656 * 4096 * 6 + 655 * 16 * 64
+    assert kernels.workspaceBytes(Q4K, 655, 4096, 14336) == bf16_kernel(655, 4096, 14336)
 
 
 def test_linear_workspace_covers_every_kernel_family():

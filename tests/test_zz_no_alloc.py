@@ -55,6 +55,21 @@ def test_static_scratch_entry_matches_workspace_entry(fmt):
         assert G.max_rel_err(got, ref.astype(np.float64)) <= 2e-5
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(333, 4096, 6144), (256, 4096, 4096), (129, 5120, 3072)])
+def test_static_scratch_entry_serves_q4_k_prefills(rows, in_dim, out_dim):
+    """Q4_K past 64 rows whose split of X fits the array: the K shares' sums must not push it out (and the lent workspace of
+    the same size gives the same bits)."""
+    print(f"case: static scratch q4_k prefill rows={rows} in={in_dim} out={out_dim}", flush=True)
+    kernels.staticScratchInit()
+    fmt = _lib.TYPE_Q4_K
+    x, w = synth.activations(7100, rows, in_dim), synth.weights(fmt, 7101, out_dim, in_dim)
+    wd = G.prepare(fmt, w, out_dim, in_dim)
+    got = static_linear(fmt, x, wd, rows, in_dim, out_dim)
+    assert np.array_equal(got, G.linear(fmt, PREP, x, wd, rows, in_dim, out_dim))
+    sample = np.r_[0:2, 31:33, rows - 1]
+    assert G.max_rel_err(got[sample], O.linear_q4_k(x[sample], w, len(sample), in_dim, out_dim, f64=True)) <= 2e-5
+
+
 def test_static_scratch_entry_refuses_what_does_not_fit():
     rows, in_dim, out_dim = 4096, 14336, 512  # 56 MiB of quantized activations
     assert kernels.workspaceBytes(Q4, rows, in_dim, out_dim) > kernels.STATIC_SCRATCH_BYTES
