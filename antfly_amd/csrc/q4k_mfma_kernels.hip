@@ -489,13 +489,14 @@ __global__ __launch_bounds__(256) void q4k_zero_results_kernel(float* __restrict
 // 4 .. 7, so that columns 0 .. 15 find theirs in the lower lanes and columns 16 .. 31 theirs in the upper ones: as many live
 // results per MFMA as a whole tile gives one row.  Twice the workgroups of whole tiles, without K shares and the launch that
 // clears their result.
+// kByParity: whole tiles with the sums of half tiles, bit for bit: the even and the odd super-blocks of a slice apart.
 struct Q4kSecond {
     float* dst;
     const uint8_t* weight;
     Epilogue ep;
 };
 
-template <int kGroups, int kFlight, int kMaxThreads, bool kPlanesGiven = false, bool kHalfTile = false>
+template <int kGroups, int kFlight, int kMaxThreads, bool kPlanesGiven = false, bool kHalfTile = false, bool kByParity = false>
 __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 && !kHalfTile ? 8 : 4) void gemv_q4k_i8_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
                                                                   const uint8_t* __restrict__ weight_a, int rows, int in_dim,
                                                                   int out_dim, int slices, int sb_per_slice, Epilogue ep_a,
@@ -515,7 +516,8 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 &&
     float* xsum = xscale + ((rows * kb + 3) & ~3);                                                          // [rows][kb * 8], 16-byte aligned
     float* partial = xsum + rows * kb * 8;                                                                  // [waves][kGroups][64]
 
-    static_assert(!kHalfTile || (kGroups == 1 && !kPlanesGiven), "one row, its digits made here");
+    static_assert(!(kHalfTile || kByParity) || (kGroups == 1 && !kPlanesGiven), "one row, its digits made here");
+    static_assert(!kByParity || (!kHalfTile && kFlight == 2), "a slice begins with an even super-block");
     constexpr int kStep = kHalfTile ? 2 : 1;  // super-blocks a lane set of requests covers
     const int n_tiles = (out_dim + kTileCols - 1) >> 5;
     const int my_tile = kHalfTile ? blockIdx.x >> 1 : blockIdx.x, col0 = kHalfTile ? 16 * (blockIdx.x & 1) : 0;
@@ -608,7 +610,7 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 &&
     // results: D registers 4 G .. 4 G + 3 (digits) of lane half g belong to row 2 G + g, output column c of the tile
     const float* xsum_row[kGroups];
     const float* xscale_row[kGroups];
-    float acc[kGroups];
+    float acc[kGroups], odd = 0.0f;  // (odd: kByParity)
 #pragma unroll
     for (int G = 0; G < kGroups; ++G) {
         const int my_row = min(2 * G + g, rows - 1);
@@ -684,13 +686,15 @@ __global__ __launch_bounds__(kMaxThreads, kMaxThreads == 1024 && kFlight == 1 &&
                 // times 2^-s (xscale holds -s as a number, NaN for a super-block with an infinity or a NaN in it)
                 const float minus_s = xscale_row[G][sb];
                 S = __builtin_fmaf(minus_s, 0.0f, __builtin_ldexpf(S, static_cast<int>(minus_s)));
-                const float more = __builtin_fmaf(-dmin, min_sum[G], __builtin_fmaf(d, S, acc[G]));
-                if (!kHalfTile || sb_step + (c >> 4) < sb_end) acc[G] = more;
+                float& sum = kByParity && (f & 1) ? odd : acc[G];
+                const float more = __builtin_fmaf(-dmin, min_sum[G], __builtin_fmaf(d, S, sum));
+                if (!kHalfTile || sb_step + (c >> 4) < sb_end) sum = more;
             }
         }
     }
 
     // ---- 3. K-slices meet in LDS, in slice order
+    if (kByParity) acc[0] += odd;
 #pragma unroll
     for (int G = 0; G < kGroups; ++G) partial[(wave * kGroups + G) * 64 + lane] = acc[G];
     __syncthreads();
@@ -1510,25 +1514,27 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
     while (slices > kb) slices /= 2;
     static const int env_slices = tuning_int("AFHIP_Q4K_SLICES"), env_tiles = tuning_int("AFHIP_Q4K_TILES_PER_WG");
     if (env_slices >= 1 && env_slices <= max_waves && (env_slices & (env_slices - 1)) == 0 && env_slices <= kb) slices = env_slices;
-    // The int8 kernel at one or two rows on a matrix whose column tiles occupy at most half the compute units (one
-    // matrix counted, so that each half of a pair takes the single op's path and has its bits), K long enough for a
-    // super-block per wavefront of two workgroups, no epilogue: two K shares (K = 14336 x 4096 columns: 128 tiles, one
-    // row 12.7 us on half the chip).  A call with an epilogue keeps one share and sums in another order.
+    // The int8 kernel at two rows on a matrix whose column tiles occupy at most half the compute units (one matrix
+    // counted, so that each half of a pair takes the single op's path and has its bits), K long enough for a
+    // super-block per wavefront of two workgroups, no epilogue: two K shares.  A call with an epilogue keeps one share and sums in
+    // another order.  One row takes half tiles there, or their order of sums.
     auto plain = [](const Epilogue& e) { return e.bias == nullptr && e.residual == nullptr && e.activation == kActNone; };
     // One row of such a matrix, from seventeen super-blocks on: half tiles, all of K (us, against one share of whole tiles up to
     // 31 super-blocks and two shares with their clearing launch beyond; weights from memory): 4352 x 4096 columns 5.8 (6.1),
     // 5120 5.5 (6.4), 7168 6.4 (7.2), 8192 6.5 (8.4), 11008 8.8 (9.9), 14336 10.3 (10.7), 16384 10.5 (11.1), 14336 x 1024 8.2
     // (8.9), 8192 x 2048 5.6 (8.4).  4096 x 4096 columns is even (5.5) and stays.  A slice is whole pairs of super-blocks.  A
-    // pair keeps the other form where its half tiles would take two rounds (5120 x 4096 columns each 8.9 against 7.4, 14336
-    // 20 against 18.3): there its sums have another order than a single call's.
-    const bool half_tiles = kGroups == 1 && rows == 1 && use_i8 && env_slices == 0 && slices == 16 && kb > 16 &&
-                            (second != nullptr ? 4 : 2) * n_tiles <= gemv_compute_units();
+    // pair whose half tiles would take two rounds (5120 x 4096 columns each 8.9, 14336 20) takes whole tiles that add in the
+    // half tiles' order (against one share, or two with their clearing launch): 5120 x 4096 7.2 (7.2), 8192 9.1 (10.0), 14336
+    // 15.6 (17.1).
+    const bool half_sums = kGroups == 1 && rows == 1 && use_i8 && env_slices == 0 && slices == 16 && kb > 16 &&
+                           2 * n_tiles <= gemv_compute_units();
+    const bool half_tiles = half_sums && (second == nullptr || 4 * n_tiles <= gemv_compute_units());
     const bool two_shares = kGroups == 1 && use_i8 && env_slices == 0 && slices == 16 && kb >= 32 && plain(ep) &&
-                            (second == nullptr || plain(second->ep)) && !half_tiles &&
+                            (second == nullptr || plain(second->ep)) && !half_sums &&
                             2 * n_tiles <= gemv_compute_units();
-    if (half_tiles && kb < 32) slices = (kb + 1) / 2;
-    const int sb_per_slice = half_tiles ? ((kb + slices - 1) / slices + 1) / 2 * 2
-                                        : (kb + (two_shares ? 2 : 1) * slices - 1) / ((two_shares ? 2 : 1) * slices);
+    if (half_sums && kb < 32) slices = (kb + 1) / 2;
+    const int sb_per_slice = half_sums ? ((kb + slices - 1) / slices + 1) / 2 * 2
+                                       : (kb + (two_shares ? 2 : 1) * slices - 1) / ((two_shares ? 2 : 1) * slices);
     int tiles_per_wg = use_i8 ? 1 : (slices > 8 ? 16 : 8) / slices;  // (the int8 kernel: its wavefronts partition K, nothing else)
     if (!use_i8 && env_tiles >= 1 && env_tiles * slices <= max_waves) tiles_per_wg = env_tiles;
     const int waves = slices * tiles_per_wg;
@@ -1557,11 +1563,12 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
                 k8 = gemv_q4k_i8_kernel<2, 2, 512>;
             }
             if constexpr (kGroups == 1) {
+                if (half_sums) k8 = gemv_q4k_i8_kernel<1, 2, 1024, false, false, true>;
                 if (half_tiles) k8 = steps <= 1 ? gemv_q4k_i8_kernel<1, 1, 1024, false, true> : gemv_q4k_i8_kernel<1, 2, 1024, false, true>;
             }
             const size_t lds8 = q4k_i8_lds_bytes(rows, in_dim, waves);
-            static std::atomic<bool> large_lds8[12] = {};
-            const int limit8 = variant + (half_tiles ? 6 : 0);
+            static std::atomic<bool> large_lds8[13] = {};
+            const int limit8 = half_tiles ? variant + 6 : (half_sums ? 12 : variant);
             if (lds8 > 64 * 1024 && !large_lds8[limit8]) {
                 if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k8), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
                     e != hipSuccess)

@@ -296,12 +296,28 @@ def test_one_row_on_half_tiles(in_dim, out_dim):
     bias = synth.activations(300, 1, out_dim).reshape(-1)
     assert np.array_equal(G.linear_bias(Q4K, PREP, x, da, bias, 1, in_dim, out_dim), y + bias[None, :])
     ya, yb = G.linear_pair(Q4K, PREP, x, da, db, 1, in_dim, out_dim)
-    if out_dim <= 2048:
-        assert np.array_equal(ya, y) and np.array_equal(yb, G.linear(Q4K, PREP, x, db, 1, in_dim, out_dim))
+    assert np.array_equal(ya, y) and np.array_equal(yb, G.linear(Q4K, PREP, x, db, 1, in_dim, out_dim))
     for got, w in ((ya, wa), (yb, wb)):
         assert G.max_rel_err(got, O.linear_q4_k(x, w, 1, in_dim, out_dim, f64=True)) <= TIGHT
     x[0, in_dim - 1] = np.inf  # a super-block with an infinity reaches every column, a clamped one none twice
     assert not np.isfinite(G.linear(Q4K, PREP, x, da, 1, in_dim, out_dim)).any()
+
+
+@pytest.mark.parametrize("in_dim,out_dim", [(5120, 2049), (4608, 4096), (7168, 3000), (8448, 4096), (14336, 2080), (4352, 4128)])
+def test_one_row_pairs_in_the_order_of_half_tiles(in_dim, out_dim):
+    """One row on 2049 .. 4096 columns: a single call takes half tiles, a pair whole ones; each half of the pair is the single call,
+    bit for bit, with one pair of super-blocks a slice and two, odd counts of super-blocks, and biases.  (4128 columns: neither.)"""
+    print(f"case: q4_k one-row pair in={in_dim} out={out_dim}", flush=True)
+    wa, wb = synth.weights(Q4K, 197, out_dim, in_dim), synth.weights(Q4K, 198, out_dim, in_dim)
+    x = synth.activations(199, 1, in_dim)
+    da, db = device_weight(PREP, wa, out_dim, in_dim), device_weight(PREP, wb, out_dim, in_dim)
+    ya, yb = G.linear_pair(Q4K, PREP, x, da, db, 1, in_dim, out_dim)
+    assert np.array_equal(ya, G.linear(Q4K, PREP, x, da, 1, in_dim, out_dim))
+    assert np.array_equal(yb, G.linear(Q4K, PREP, x, db, 1, in_dim, out_dim))
+    assert G.max_rel_err(ya, O.linear_q4_k(x, wa, 1, in_dim, out_dim, f64=True)) <= TIGHT
+    ba, bb = synth.activations(200, 2, out_dim)
+    ya_, yb_ = G.linear_pair_bias(Q4K, PREP, x, da, ba, db, bb, 1, in_dim, out_dim)
+    assert np.array_equal(ya_, ya + ba[None, :]) and np.array_equal(yb_, yb + bb[None, :])
 
 
 Q8K_SHAPES = [(1, 2048, 512), (1, 3072, 2048), (2, 3072, 600), (4, 512, 1000), (9, 768, 513), (64, 1536, 512), (77, 2048, 520)]
