@@ -967,13 +967,12 @@ __global__ __launch_bounds__(512, 4) void gemm_q4k_rows32_kernel(float* __restri
 // More than 64 rows: X is split once by its own kernel, then a GEMM on the 6-bit matrix
 // instructions.  v_mfma_scale_f32_32x32x64_f8f6f4 multiplies 64 fp6 (e2m3) numbers a column in the 33 cycles that
 // v_mfma_f32_32x32x16_bf16 needs for 16 bf16 ones, and to it
-//   * the fp6 codes 0 .. 15 are the numbers n / 8, so a weight nibble is its own code (with two zero bits on top);
-//   * an activation is eight 4-bit digits with its sign: |x| = sum over d of digit_d * 2^(e - 4 (d + 1)), with
-//     2^(e - 1) <= max |x| < 2^e over the sub-block.  Rounded to 2^-33 of that maximum (24-bit numbers down to 2^-8 of it are
-//     exact); products with the scales 2^(e - 4 d) that the instruction applies to 32 values at a time are exact.
+//   * the fp6 codes 0 .. 16 are the numbers n / 8 (a sign in front), so a weight nibble is its own code;
+//   * an activation is eight digits from -16 to 16: x = sum over d of digit_d * 2^(e - 4 - 5 d), with 2^(e - 1) <= max |x| < 2^e over the
+//     sub-block.  Rounded to 2^(e - 39): 24-bit numbers down to 2^(e - 16) are exact, for smaller ones see add_lost; products with the
+//     scales that the instruction applies to 32 values at a time are exact.
 // A sub-block of 32 values is four such instructions -- lane half g of number p multiplies digit 2 p + g -- against six bf16
-// ones, and its result needs no conversion: (d sc) * D is added to the sum.  Against 64 bits the four leave 4.4e-8 of a
-// sub-block's sum, the three bf16 parts of the kernel above 6.9e-8 (32 normal values; 3.9e-8 / 6.7e-8 with outliers).
+// ones, and its result needs no conversion: (d sc) * D is added to the sum.
 //
 // The order of the 16 values of a lane half inside its three 32-bit words of codes: the one in which nine instructions spread
 // the nibbles of the tile-major layout (expand_nibbles).
@@ -981,10 +980,35 @@ constexpr int kFp6Order[16] = {0, 12, 5, 10, 3, 15, 4, 9, 2, 14, 7, 8, 1, 13, 6,
 
 // Workspace: the digits, for every 32 rows (the last tile: its rows, rounded up to even) and sub-block the operands of the four
 // instructions, each [half g][row] 16 bytes and then [half g][row] 8 bytes (a lane's six words); behind them, for every row and
-// super-block 64 bytes: the eight sub-block sums as three bf16 parts, [part][sub-block], and the sub-blocks' scale bytes.
+// super-block 64 bytes: the eight sub-block sums as three bf16 parts, [part][sub-block], the sub-blocks' scale bytes, and in the first
+// row of 32 a byte per sub-block that says whether the digits left something of these 32 rows' values behind.
 constexpr int kDigitBytes = 192;  // of a row and sub-block
 
 __device__ __forceinline__ int rows_of_tile(int rows, int tile) { return (min(kG32Rows, rows - tile * kG32Rows) + 1) & ~1; }
+
+// Four digits each: x = (high * 2^20 + low) * 2^(e - 39) + what is left, `exponent` = e + 126 being the biased exponent of the sub-block's
+// largest value.  Returns what is left (at most 2^(e - 40), exact); NaN for an infinity or a NaN.
+__device__ __forceinline__ float digits_of(float x, int exponent, int* high, int* low) {
+    const float h = __builtin_rintf(__builtin_ldexpf(x, 145 - exponent));
+    const float rest = x - __builtin_ldexpf(h, exponent - 145);
+    const float l = __builtin_rintf(__builtin_ldexpf(rest, 165 - exponent));
+    *high = static_cast<int>(h);
+    *low = static_cast<int>(l);
+    return rest - __builtin_ldexpf(l, exponent - 165);
+}
+
+// Sixteen 6-bit fields, digit + 16 (0 .. 32) each, as fp6 codes: bit 5 the sign, below it the magnitude.  A carry leaves no field.
+typedef unsigned __int128 Fp6Fields;
+constexpr Fp6Fields each_field(uint32_t v) {
+    Fp6Fields all = 0;
+    for (int f = 0; f < 16; ++f) all |= static_cast<Fp6Fields>(v) << (6 * f);
+    return all;
+}
+__device__ __forceinline__ Fp6Fields fp6_codes(Fp6Fields shifted) {
+    const Fp6Fields u = shifted + each_field(16);        // bit 5: not negative, and the magnitude below it
+    const Fp6Fields one = (~u & each_field(32)) >> 5;    // of the negative ones: 32 - magnitude in the low bits
+    return (u ^ each_field(32) ^ ((one << 5) - one)) + one;
+}
 
 // One wavefront per 32 rows and sub-block, a lane for 16 values; the image is put together in LDS and written as it lies.
 __global__ __launch_bounds__(64) void q4k_split_digits_kernel(const float* __restrict__ x, uint8_t* __restrict__ digits,
@@ -1009,29 +1033,31 @@ __global__ __launch_bounds__(64) void q4k_split_digits_kernel(const float* __res
 #pragma unroll
     for (int i = 0; i < 16; ++i) peak = max(peak, __float_as_uint(v[i]) & 0x7FFFFFFFu);
     peak = max(peak, static_cast<uint32_t>(dpp_move<kDppXor1>(static_cast<int>(peak))));
-    // the biased exponent is the scale byte of digit 0; below 4 (2^-122) the digits reach 2^-154, under every f32, and the scales
+    // the biased exponent is the scale byte of digit 0; below 5 (2^-121) the digits reach 2^-160, under every f32, and the scales
     // of the lower ones would leave their range.  255: an infinity or a NaN, which the instruction takes as NaN
-    const int exponent = max(static_cast<int>(peak >> 23), 4);
-    uint32_t u[16], sign[3] = {0u, 0u, 0u};
+    const int exponent = max(static_cast<int>(peak >> 23), 5);
+    constexpr int kBias = 16 * (1 + 32 + 32 * 32 + 32 * 32 * 32);  // a 16 on every digit
+    int u[2][16];
+    bool left = false;
 #pragma unroll
     for (int f = 0; f < 16; ++f) {
-        const float value = v[kFp6Order[f]];
-        u[f] = static_cast<uint32_t>(__builtin_rintf(__builtin_ldexpf(__builtin_fabsf(value), 158 - exponent)));
-        const int at = 6 * f + 5;
-        sign[at >> 5] |= (__float_as_uint(value) >> 31) << (at & 31);
+        left |= digits_of(v[kFp6Order[f]], exponent, &u[0][f], &u[1][f]) != 0.0f;
+        u[0][f] += kBias;
+        u[1][f] += kBias;
     }
+    const bool any_left = __builtin_amdgcn_ballot_w64(left) != 0;
     uint8_t* img = reinterpret_cast<uint8_t*>(image);
     if (r < tile_rows) {
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
-            uint32_t w[3] = {sign[0], sign[1], sign[2]};
+            Fp6Fields shifted = 0;
 #pragma unroll
             for (int f = 0; f < 16; ++f) {
-                const uint32_t digit = (u[f] >> (28 - 4 * d)) & 15u;
-                const int at = 6 * f;
-                w[at >> 5] |= digit << (at & 31);
-                if ((at & 31) > 28) w[(at >> 5) + 1] |= digit >> (32 - (at & 31));
+                const uint32_t at = static_cast<uint32_t>(u[d >> 2][f]) >> (15 - 5 * (d & 3));
+                shifted |= static_cast<Fp6Fields>((d & 3) == 0 ? at & 63u : at & 31u) << (6 * f);
             }
+            const Fp6Fields codes = fp6_codes(shifted);
+            const uint32_t w[3] = {static_cast<uint32_t>(codes), static_cast<uint32_t>(codes >> 32), static_cast<uint32_t>(codes >> 64)};
             const int p = d >> 1, g = d & 1;
             uint32_t* wide = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + (g * tile_rows + r) * 16);
             uint32_t* rest = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + tile_rows * 32 + (g * tile_rows + r) * 8);
@@ -1054,6 +1080,7 @@ __global__ __launch_bounds__(64) void q4k_split_digits_kernel(const float* __res
         part[8] = static_cast<uint16_t>(mid);
         part[16] = static_cast<uint16_t>(lo);
         cell[48 + (sub & 7)] = static_cast<uint8_t>(exponent);
+        if (r == 0) cell[56 + (sub & 7)] = any_left;
     }
     __syncthreads();
     uint4* out = reinterpret_cast<uint4*>(digits + static_cast<size_t>(tile) * kG32Rows * in_dim * 6 +
@@ -1118,7 +1145,7 @@ template <int kWaves, int kR, int kC, int kOcc>
 __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
     float* __restrict__ dst, const uint8_t* __restrict__ digits, const uint8_t* __restrict__ sums,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_groups, int n_groups, int band, int sb_per_split,
-    float* __restrict__ partial, Epilogue ep, Q4kSecond second) {
+    float* __restrict__ partial, Epilogue ep, Q4kSecond second, const float* __restrict__ x) {
     using S = G6Shape<kWaves, kR, kC>;
     if (blockIdx.z != 0) {  // a second matrix on the same X
         dst = second.dst;
@@ -1281,7 +1308,7 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
         }
     };
 
-    const int b_scale = 130 | 122 << 8 | 114 << 16 | 106 << 24;  // 2^(3 - 8 p): codes are eighths, digit pair p weighs 2^(-8 p)
+    const int b_scale = 130 | 120 << 8 | 110 << 16 | 100 << 24;  // 2^(3 - 10 p): codes are eighths, digit pair p weighs 2^(-10 p)
     issue(0, sb_begin & 1);
     issue(1, 0);
     issue(2, 0);
@@ -1321,6 +1348,15 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
         asm volatile("" : "+v"(acc[i][j]));
     };
     read_scales(sb_begin, 0);
+    // whether the min terms outweigh what the digits leave behind (see add_lost): bit 7 of every byte while no 6-bit min is zero, and
+    // the least of 16 |dmin| - |d|
+    uint32_t mins_live[kC];
+    float slack[kC];
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+        mins_live[j] = 0xFFFFFFFFu;
+        slack[j] = 0.0f;
+    }
     for (int sb = sb_begin; sb < sb_end; ++sb) {
         const unsigned char* cell = q4k_mfma_lds + S::kSumsAt + (sb & 1) * S::kSums;
         t_u32x4 hdr[kC];
@@ -1339,7 +1375,7 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
             const int to_issue = loads_of((s + 3) & 7);
             if ((s & 3) == 0) {
 #pragma unroll
-                for (int i = 0; i < kR; ++i) a_scale[i] = a_scale_next[i] - 0x04040404 * g;
+                for (int i = 0; i < kR; ++i) a_scale[i] = a_scale_next[i] - 0x05050505 * g;
             }
 #pragma unroll
             for (int i = 0; i < kR; ++i) {
@@ -1385,6 +1421,7 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
                                                  bf16_pair(ubyte_to_f32(mn_hi, 0), ubyte_to_f32(mn_hi, 1)),
                                                  bf16_pair(ubyte_to_f32(mn_hi, 2), ubyte_to_f32(mn_hi, 3)));
                             asm volatile("" : "+v"(mins[j].x), "+v"(mins[j].y), "+v"(mins[j].z), "+v"(mins[j].w));
+                            mins_live[j] &= (mn_lo + 0x7F7F7F7Fu) & (mn_hi + 0x7F7F7F7Fu);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
@@ -1412,7 +1449,10 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
                             __builtin_amdgcn_sched_barrier(0);
                             if (m == 1 && j == kC - 1 && i + 1 < kR) read_sums(i + 1);
                             accumulate(before, i_before, j, 8 * m, 8 * (m + 1));
-                            if (m == 1) factor[now][j] = -half_bits_to_f32(static_cast<uint16_t>(hdr[j].x >> 16));
+                            if (m == 1) {
+                                factor[now][j] = -half_bits_to_f32(static_cast<uint16_t>(hdr[j].x >> 16));
+                                if (i == 0) slack[j] = fminf(slack[j], __builtin_fmaf(16.0f, __builtin_fabsf(factor[now][j]), -__builtin_fabsf(d[j])));
+                            }
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
@@ -1435,6 +1475,110 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
 #pragma unroll
     for (int j = 0; j < kC; ++j) accumulate(1, kR - 1, j, 0, 16);
     q4k_wait_vm<0>();  // what is still on its way to LDS lands before the workgroup ends
+
+    // add_lost: what the digits left behind of an activation, at most 2^(e - 40), where it can count.  A sub-block's dot holds the
+    // values near 2^e with their nibbles and loses more than that when it is rounded -- unless those nibbles are zero; then the
+    // products are (-dmin m) x, and where dmin m is at least d sc / 1024 their own rounding in 24 bits is the larger.  Columns
+    // of which no super-block is below that line (16 |dmin| >= |d|, no m of zero) end the call here: all of ordinary weights,
+    // whose min is about 8 steps of d sc.  The others look for sub-blocks with something left, take it from X itself, in three bf16
+    // parts as gemm_q4k_rows32_kernel multiplies them, and decide by 32 rows x 32 columns x sub-block, so that
+    // a result does not depend on the workgroup's tile.  Without this a channel 2^16 times the others, on weights that are zero,
+    // would cost 1.8e-7 of a row's largest result, at 2^20 3.3e-6, at 2^30 3e-3.  us before / with this: 512 x 4096 x 14336 141.6 / 141.3, 333 x 14336
+    // x 4096 120.4 / 119.7; weights of random bytes, where a 64th of the mins is zero, 148 / 174 and 125 / 146.
+    bool below = false;
+#pragma unroll
+    for (int j = 0; j < kC; ++j) below |= (mins_live[j] & 0x80808080u) != 0x80808080u || slack[j] < 0.0f;
+    if (__builtin_amdgcn_ballot_w64(below) != 0) {
+#pragma unroll
+        for (int i = 0; i < kR; ++i) {
+            const int mt = min(m_group * kR + i, m_tiles - 1), row = min(mt * kG32Rows + c, rows - 1);
+            const uint8_t* const left_at = sums + static_cast<size_t>(mt) * kG32Rows * kb * 64 + 56;
+            const uint8_t* const exponent_at = sums + static_cast<size_t>(row) * kb * 64 + 48;
+            const float* const xrow = x + static_cast<size_t>(row) * in_dim + 16 * g;
+#pragma unroll 1
+            for (int sb0 = sb_begin; sb0 < sb_end; sb0 += 64) {
+                uint64_t some = 0;  // a lane's super-block: the eight flags
+                if (sb0 + lane < sb_end) some = *reinterpret_cast<const uint64_t*>(left_at + static_cast<size_t>(sb0 + lane) * 64);
+                uint64_t todo = __builtin_amdgcn_ballot_w64(some != 0);
+#pragma unroll 1
+                while (todo != 0) {
+                    const int from = __builtin_ctzll(todo), sb = sb0 + from;
+                    todo &= todo - 1;
+                    const uint64_t flags = static_cast<uint64_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(some >> 32), from)) << 32 |
+                                           static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(some), from));
+                    const uint8_t* base[kC];
+                    t_u32x4 h[kC];
+#pragma unroll
+                    for (int j = 0; j < kC; ++j) {
+                        base[j] = tile_at(wave * kC + j) + static_cast<size_t>(sb) * kTileBytes;
+                        h[j] = *reinterpret_cast<const t_u32x4*>(base[j] + 16 * c);
+                    }
+#pragma unroll 1
+                    for (int sub = 0; sub < 8; ++sub) {
+                        if ((flags >> (8 * sub) & 0xFFu) == 0) continue;
+                        // everything is requested ahead of the look at the headers: this pass is a chain of trips to memory
+                        const int exponent = exponent_at[static_cast<size_t>(sb) * 64 + sub];
+                        float4 v[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) v[k] = reinterpret_cast<const float4*>(xrow + sb * kQ4kBlockValues + sub * 32)[k];
+                        t_u32x4 q[kC];
+#pragma unroll
+                        for (int j = 0; j < kC; ++j) q[j] = *reinterpret_cast<const t_u32x4*>(base[j] + 512 + (sub >> 1) * 1024 + 16 * lane);
+                        const int shift = 8 * (sub & 3);
+                        float dsc[kC];
+                        bool counts[kC], any = false;
+#pragma unroll
+                        for (int j = 0; j < kC; ++j) {
+                            const uint32_t sc = sub < 4 ? h[j].y & 0x3F3F3F3Fu : (h[j].w & 0x0F0F0F0Fu) | ((h[j].y >> 2) & 0x30303030u);
+                            const uint32_t mn = sub < 4 ? h[j].z & 0x3F3F3F3Fu : ((h[j].w >> 4) & 0x0F0F0F0Fu) | ((h[j].z >> 2) & 0x30303030u);
+                            dsc[j] = half_bits_to_f32(static_cast<uint16_t>(h[j].x & 0xFFFFu)) * static_cast<float>(sc >> shift & 0xFFu);
+                            const float min_term = half_bits_to_f32(static_cast<uint16_t>(h[j].x >> 16)) * static_cast<float>(mn >> shift & 0xFFu);
+                            counts[j] = __builtin_amdgcn_ballot_w64(1024.0f * __builtin_fabsf(min_term) < __builtin_fabsf(dsc[j])) != 0;
+                            any |= counts[j];
+                        }
+                        if (!any) continue;
+                        union {
+                            t_bf16x8 v;
+                            uint32_t u[4];
+                        } part[3][2];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            int high, low;
+                            const float r[4] = {digits_of(v[k].x, exponent, &high, &low), digits_of(v[k].y, exponent, &high, &low),
+                                                digits_of(v[k].z, exponent, &high, &low), digits_of(v[k].w, exponent, &high, &low)};
+#pragma unroll
+                            for (int e = 0; e < 2; ++e)
+                                split3_pair(r[2 * e], r[2 * e + 1], &part[0][k >> 1].u[2 * (k & 1) + e], &part[1][k >> 1].u[2 * (k & 1) + e],
+                                            &part[2][k >> 1].u[2 * (k & 1) + e]);
+                        }
+#pragma unroll
+                        for (int j = 0; j < kC; ++j) {
+                            if (!counts[j]) continue;
+                            t_f32x16 dot = t_f32x16{};
+#pragma unroll
+                            for (int m = 0; m < 2; ++m) {
+                                union {
+                                    t_bf16x8 v;
+                                    t_bf16x2 pair[4];
+                                } w;
+#pragma unroll
+                                for (int k = 0; k < 2; ++k) {
+                                    const int nibbles = static_cast<int>(q[j][2 * m + k] >> (4 * (sub & 1)) & 0x0F0F0F0Fu);
+                                    w.pair[2 * k] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(nibbles, 512.0f, false);
+                                    w.pair[2 * k + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(nibbles, 512.0f, true);
+                                }
+#pragma unroll
+                                for (int t = 2; t >= 0; --t) dot = __builtin_amdgcn_mfma_f32_32x32x16_bf16(part[t][m].v, w.v, dot, 0, 0, 0);
+                            }
+#pragma unroll
+                            for (int e = 0; e < 16; ++e)  // (dsc may be an infinity)
+                                if (dot[e] != 0.0f) acc[i][j][e] = __builtin_fmaf(dsc[j], dot[e], acc[i][j][e]);
+                        }
+                    }
+                }
+            }
+        }
+    }
 
     // Results.  Plain ones go straight out of the registers; an epilogue is a loop over a copy in LDS, not 64 copies of its code
     // in a row (45 KB of them: 333 x 4096 x 4096 79 -> 76 us without).
@@ -1787,6 +1931,7 @@ Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, size_t roo
 
 struct Q4kGemmCall {
     hipStream_t stream;
+    const float* x;
     float* dst;
     const uint8_t *digits, *sums, *weight;
     int rows, in_dim, out_dim, sb_per_split, shares;
@@ -1811,7 +1956,7 @@ hipError_t launch_fp6_tile(const Q4kGemmCall& q) {
     }
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), q.shares, q.second ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, q.stream, q.dst,
                        q.digits, q.sums, q.weight, q.rows, q.in_dim, q.out_dim, m_groups, n_groups, 8, q.sb_per_split, q.partial, q.ep,
-                       q.second ? *q.second : Q4kSecond{nullptr, nullptr, Epilogue{}});
+                       q.second ? *q.second : Q4kSecond{nullptr, nullptr, Epilogue{}}, q.x);
     return hipGetLastError();
 }
 }  // namespace
@@ -1828,9 +1973,18 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
                                  size_t workspace_bytes, int rows, int in_dim, int out_dim, const Epilogue& ep, float* dst_b,
                                  const uint8_t* weight_b, const Epilogue& ep_b) {
     if (in_dim % kQ4kBlockValues != 0 || rows < 1 || workspace == nullptr) return hipErrorInvalidValue;
-    const Q4kGemmPlan plan = gemm_q4k_plan(static_cast<size_t>(rows), static_cast<size_t>(in_dim), static_cast<size_t>(out_dim),
-                                           workspace_bytes, dst_b != nullptr);
+    const size_t m = rows, k = in_dim, n = out_dim;
+    Q4kGemmPlan plan = gemm_q4k_plan(m, k, n, workspace_bytes, dst_b != nullptr);
     if (plan.splits == 0) return hipErrorInvalidValue;
+    // the fp6 kernel may look at X again when other workgroups have stored results
+    auto over_x = [&](const float* y) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+        return y != nullptr && b < a + m * k * 4 && a < b + m * n * 4;
+    };
+    if (plan.kind != kParts && (over_x(dst) || over_x(dst_b))) {
+        plan = gemm_q4k_parts_plan(m, k, n);
+        if (gemm_q4k_plan_bytes(plan, m, k, n) > workspace_bytes) plan.splits = 1;
+    }
     const int kb = in_dim / kQ4kBlockValues;
     const int sb_per_split = (kb + plan.splits - 1) / plan.splits;
     const int shares = (kb + sb_per_split - 1) / sb_per_split;  // no empty share
@@ -1853,7 +2007,7 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     const Q4kSecond second{dst_b, weight_b, ep_b};
     auto multiply = [&](float* y, const uint8_t* w, const Epilogue& epilogue, const Q4kSecond* with) {
-        const Q4kGemmCall q{stream, y, space, digit_sums, w, rows, in_dim, out_dim, sb_per_split, shares, partial, epilogue, with};
+        const Q4kGemmCall q{stream, x, y, space, digit_sums, w, rows, in_dim, out_dim, sb_per_split, shares, partial, epilogue, with};
         hipError_t e;
         if (plan.kind == kFp6Tile64x256) e = launch_fp6_tile<4, 2, 2, 2>(q);
         else if (plan.kind == kFp6Tile64x128) e = launch_fp6_tile<4, 2, 1, 2>(q);

@@ -885,7 +885,7 @@ def main() -> int:
             w_s, e_s = time_config(Q4K, m, 4096, 14336, 40, 5, 2, 78)
             flops = 2.0 * m * 4096 * 14336
             # up to 64 rows the kernel issues three bf16 MFMA products per f32 product (X as hi + mid + lo parts), past them
-            # eight 6-bit ones (X as eight 4-bit digits): priced against the dense peak of each
+            # eight 6-bit ones (X as eight base-32 digits): priced against the dense peak of each
             parts, name, peak = (3, "bf16", BF16_MFMA_PEAK_FLOPS) if m <= 64 else (8, "fp6", FP6_MFMA_PEAK_FLOPS)
             extra[f"q4k_gemm_m{m}_k4096_n14336"] = {
                 "what": f"Q4_K prefill: X split once into {parts} {name} parts, {name}-MFMA GEMM, f32-accurate; per call incl. the split",

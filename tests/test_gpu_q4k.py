@@ -531,6 +531,56 @@ def test_prefill_past_64_rows_on_extreme_activations():
     assert np.array_equal(got[~hit], y[~hit])
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(66, 512, 1000), (140, 6144, 5000), (200, 1536, 8192)])
+def test_prefill_past_64_rows_keeps_small_values_beside_large_ones(rows, in_dim, out_dim):
+    """One channel in 32 is 2^8 .. 2^100 times as large as the others, and its weights are exact zeros (nibble 0, no min, by the
+    super-block's dmin in even columns, by the sub-blocks' 6-bit mins in odd ones): the result is what the small values make, and every
+    one of their 24 bits counts.  Against the float64 oracle, as without the large channel; pairs and biases keep the call's bits."""
+    print(f"case: q4_k fp6 prefill, large activations on zero weights rows={rows} in={in_dim} out={out_dim}", flush=True)
+    assert not O.uses_q4k_q8k_activation(rows, in_dim, out_dim)
+    ws = []
+    for seed in (87, 88):
+        w = synth.weights(Q4K, seed, out_dim, in_dim).reshape(out_dim, in_dim // 256, 144)
+        w[0::2, :, 2:4] = 0        # dmin
+        w[1::2, :, 8:12] = 0       # mins 0 .. 3
+        w[1::2, :, 12:16] &= 0x0F  # mins 4 .. 7, low bits (their upper two are in the bytes above)
+        w[:, :, 16 + 5::32] = 0    # nibble 5 of every sub-block
+        ws.append(w.reshape(-1))
+    wa, wb = ws
+    da, db = device_weight(PREP, wa, out_dim, in_dim), device_weight(PREP, wb, out_dim, in_dim)
+    small = synth.activations(89, rows, in_dim)
+    sample = np.unique(np.r_[0, 1, 31:34, rows - 1])
+    ref = None
+    for ratio in (8, 12, 16, 18, 20, 24, 30, 45, 60, 100):
+        x = small.copy()
+        x[:, 5::32] = np.float32(2.0) ** ratio * (1 + np.arange(rows, dtype=np.float32)[:, None] / 256)
+        if ref is None:
+            ref = O.linear_q4_k(x[sample], wa, len(sample), in_dim, out_dim, f64=True)
+        y = G.linear(Q4K, PREP, x, da, rows, in_dim, out_dim)
+        err = G.max_rel_err(y[sample], ref)
+        assert err <= 2e-6, (ratio, err)  # 32-bit sums of in_dim products: measured 3e-7 without the large channel
+    ya, yb = G.linear_pair(Q4K, PREP, x, da, db, rows, in_dim, out_dim)
+    assert np.array_equal(ya, y) and np.array_equal(yb, G.linear(Q4K, PREP, x, db, rows, in_dim, out_dim))
+    b = synth.activations(90, 1, out_dim)[0]
+    assert np.array_equal(G.linear_bias(Q4K, PREP, x, da, b, rows, in_dim, out_dim), y + b[None, :])
+
+
+def test_prefill_past_64_rows_over_its_own_input():
+    """A result in X's place is outside the header's contract; it has always come out right because X is split before anything is
+    stored, and the kernel that may look at X again must not serve it."""
+    rows, in_dim, out_dim = 66, 1024, 1000
+    print("case: q4_k prefill, result over X", flush=True)
+    w, x = synth.weights(Q4K, 101, out_dim, in_dim), synth.activations(102, rows, in_dim)
+    x[:, 5::32] *= np.float32(2.0) ** 20  # (values with bits that the digits do not hold)
+    xd, wd = G.to_dev(x), device_weight(PREP, w, out_dim, in_dim)
+    y = xd.reshape(-1)[:rows * out_dim]
+    ws = torch.empty(kernels.workspaceBytes(Q4K, rows, in_dim, out_dim), dtype=torch.uint8, device=G.DEV)
+    kernels.launchLinearF32(G.stream(), Q4K, PREP, G.buf(y), G.buf(xd), G.buf(wd), rows, in_dim, out_dim, G.buf(ws))
+    torch.cuda.synchronize()
+    ref = O.linear_q4_k(x, w, rows, in_dim, out_dim, f64=True)
+    assert G.max_rel_err(y.cpu().numpy().reshape(rows, out_dim), ref) <= TIGHT
+
+
 def test_prefill_past_64_rows_in_a_workspace_without_room_for_partial_sums():
     """A workspace that holds the split of X but not the sums of the K shares: the GEMM on one share -- the bits of the same columns
     in a matrix so wide that K is not shared out -- and in one that holds three parts a value but not an even number of rows of digits
