@@ -983,109 +983,113 @@ constexpr int kFp6Order[16] = {0, 12, 5, 10, 3, 15, 4, 9, 2, 14, 7, 8, 1, 13, 6,
 // super-block 64 bytes: the eight sub-block sums as three bf16 parts, [part][sub-block], the sub-blocks' scale bytes, and in the first
 // row of 32 a byte per sub-block that says whether the digits left something of these 32 rows' values behind.
 constexpr int kDigitBytes = 192;  // of a row and sub-block
+typedef int t_i32x6 __attribute__((ext_vector_type(6)));
 
 __device__ __forceinline__ int rows_of_tile(int rows, int tile) { return (min(kG32Rows, rows - tile * kG32Rows) + 1) & ~1; }
 
-// Four digits each: x = (high * 2^20 + low) * 2^(e - 39) + what is left, `exponent` = e + 126 being the biased exponent of the sub-block's
-// largest value.  Returns what is left (at most 2^(e - 40), exact); NaN for an infinity or a NaN.
-__device__ __forceinline__ float digits_of(float x, int exponent, int* high, int* low) {
-    const float h = __builtin_rintf(__builtin_ldexpf(x, 145 - exponent));
-    const float rest = x - __builtin_ldexpf(h, exponent - 145);
-    const float l = __builtin_rintf(__builtin_ldexpf(rest, 165 - exponent));
-    *high = static_cast<int>(h);
-    *low = static_cast<int>(l);
-    return rest - __builtin_ldexpf(l, exponent - 165);
+// What the digits leave of a value, exact (at most 2^(e - 40)); `exponent` = e + 126, the biased exponent of the sub-block's largest value.
+// In two steps, as the digits are made: together they are the value rounded to 2^(e - 39), to the even neighbour from halfway.
+__device__ __forceinline__ float left_behind(float x, int exponent) {
+    const float rest = x - __builtin_ldexpf(__builtin_rintf(__builtin_ldexpf(x, 145 - exponent)), exponent - 145);
+    return rest - __builtin_ldexpf(__builtin_rintf(__builtin_ldexpf(rest, 165 - exponent)), exponent - 165);
 }
 
-// Sixteen 6-bit fields, digit + 16 (0 .. 32) each, as fp6 codes: bit 5 the sign, below it the magnitude.  A carry leaves no field.
-typedef unsigned __int128 Fp6Fields;
-constexpr Fp6Fields each_field(uint32_t v) {
-    Fp6Fields all = 0;
-    for (int f = 0; f < 16; ++f) all |= static_cast<Fp6Fields>(v) << (6 * f);
-    return all;
-}
-__device__ __forceinline__ Fp6Fields fp6_codes(Fp6Fields shifted) {
-    const Fp6Fields u = shifted + each_field(16);        // bit 5: not negative, and the magnitude below it
-    const Fp6Fields one = (~u & each_field(32)) >> 5;    // of the negative ones: 32 - magnitude in the low bits
-    return (u ^ each_field(32) ^ ((one << 5) - one)) + one;
+// 32 values as 6-bit codes: code f is even[f / 2] (odd[f / 2]) / scale rounded to eighths, the even one from halfway.  (As assembly: with
+// the builtin the compiler may give the result the scale's register, which the instruction still reads after its first words.)
+__device__ __forceinline__ t_i32x6 fp6_codes(t_f32x16 even, t_f32x16 odd, float scale) {
+    t_i32x6 codes;
+    asm("v_cvt_scalef32_2xpk16_fp6_f32 %0, %1, %2, %3" : "=&v"(codes) : "v"(even), "v"(odd), "v"(scale));
+    return codes;
 }
 
-// One wavefront per 32 rows and sub-block, a lane for 16 values; the image is put together in LDS and written as it lies.
-__global__ __launch_bounds__(64) void q4k_split_digits_kernel(const float* __restrict__ x, uint8_t* __restrict__ digits,
-                                                            uint8_t* __restrict__ sums, int rows, int in_dim) {
-    __shared__ __align__(16) uint32_t image[kG32Rows * kDigitBytes / 4];
-    const int lane = threadIdx.x, tile = blockIdx.y, sub = blockIdx.x;
-    const int tile_rows = rows_of_tile(rows, tile);
-    const int r = lane >> 1, half = lane & 1, row = tile * kG32Rows + r;
-    float v[16];
-    if (row < rows) {
-        const float4* src = reinterpret_cast<const float4*>(x + static_cast<size_t>(row) * in_dim + sub * 32 + half * 16);
+// A workgroup per 32 rows and sub-block, a lane for a row and one of the eight digits: X less what the digits above take of it -- adding
+// and subtracting 1.5 * 2^23 units rounds to a unit; from the fifth digit on in two steps, as 24 bits reach no further -- and the
+// conversion rounds to the digit itself.  X comes in by whole lines and is handed round in LDS.
+// Bound by the launch and a trip to memory on short calls, the vector ALU on long ones.  us of kernel time by rocprofv3, against a lane
+// for 16 values and all digits, packed by shifts: 75 x 256 4.1 -> 1.8, 333 x 4096 7.3 -> 6.1, 2048 x 4096 17.7 (four-bit digits 19.0).
+__global__ __launch_bounds__(256) void q4k_split_digits_kernel(const float* __restrict__ x, uint8_t* __restrict__ digits,
+                                                             uint8_t* __restrict__ sums, int rows, int in_dim) {
+    __shared__ float4 staged[kG32Rows * 8];  // [row][chunk ^ row % 8]
+    const int tid = threadIdx.x, tile = blockIdx.y, sub = blockIdx.x;
+    {
+        const int r = tid >> 3, chunk = tid & 7, row = tile * kG32Rows + r;
+        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (row < rows) q = *reinterpret_cast<const float4*>(x + static_cast<size_t>(row) * in_dim + sub * 32 + chunk * 4);
+        staged[r * 8 + (chunk ^ (r & 7))] = q;
+    }
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), digit = tid >> 5;
+    const int r = tid & 31, row = tile * kG32Rows + r, tile_rows = rows_of_tile(rows, tile);
+    float v[32];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 q = src[i];
-            v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = 0.0f;
+    for (int c = 0; c < 8; ++c) {
+        const float4 q = staged[r * 8 + (c ^ (r & 7))];
+        v[4 * c] = q.x; v[4 * c + 1] = q.y; v[4 * c + 2] = q.z; v[4 * c + 3] = q.w;
     }
     uint32_t peak = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) peak = max(peak, __float_as_uint(v[i]) & 0x7FFFFFFFu);
-    peak = max(peak, static_cast<uint32_t>(dpp_move<kDppXor1>(static_cast<int>(peak))));
+    for (int i = 0; i < 32; ++i) peak = max(peak, __float_as_uint(v[i]) & 0x7FFFFFFFu);
     // the biased exponent is the scale byte of digit 0; below 5 (2^-121) the digits reach 2^-160, under every f32, and the scales
     // of the lower ones would leave their range.  255: an infinity or a NaN, which the instruction takes as NaN
     const int exponent = max(static_cast<int>(peak >> 23), 5);
-    constexpr int kBias = 16 * (1 + 32 + 32 * 32 + 32 * 32 * 32);  // a 16 on every digit
-    int u[2][16];
-    bool left = false;
+    uint8_t* const cell = sums + (static_cast<size_t>(row) * (in_dim >> 8) + (sub >> 3)) * 64;
+    if (wave == 0) {
+        float s = 0.0f;
+        {
+            float part[16];
 #pragma unroll
-    for (int f = 0; f < 16; ++f) {
-        left |= digits_of(v[kFp6Order[f]], exponent, &u[0][f], &u[1][f]) != 0.0f;
-        u[0][f] += kBias;
-        u[1][f] += kBias;
-    }
-    const bool any_left = __builtin_amdgcn_ballot_w64(left) != 0;
-    uint8_t* img = reinterpret_cast<uint8_t*>(image);
-    if (r < tile_rows) {
+            for (int i = 0; i < 16; ++i) part[i] = v[2 * i] + v[2 * i + 1];
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            Fp6Fields shifted = 0;
+            for (int n = 8; n >= 1; n /= 2)
 #pragma unroll
-            for (int f = 0; f < 16; ++f) {
-                const uint32_t at = static_cast<uint32_t>(u[d >> 2][f]) >> (15 - 5 * (d & 3));
-                shifted |= static_cast<Fp6Fields>((d & 3) == 0 ? at & 63u : at & 31u) << (6 * f);
-            }
-            const Fp6Fields codes = fp6_codes(shifted);
-            const uint32_t w[3] = {static_cast<uint32_t>(codes), static_cast<uint32_t>(codes >> 32), static_cast<uint32_t>(codes >> 64)};
-            const int p = d >> 1, g = d & 1;
-            uint32_t* wide = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + (g * tile_rows + r) * 16);
-            uint32_t* rest = reinterpret_cast<uint32_t*>(img + p * tile_rows * 48 + tile_rows * 32 + (g * tile_rows + r) * 8);
-            if (half == 0) {
-                wide[0] = w[0]; wide[1] = w[1]; wide[2] = w[2];
-            } else {
-                wide[3] = w[0]; rest[0] = w[1]; rest[1] = w[2];
-            }
+                for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
+            s = part[0];
         }
+        if (digit == 0 && row < rows) {
+            uint32_t hi, mid, lo;
+            split3_pair(s, 0.0f, &hi, &mid, &lo);
+            uint16_t* part = reinterpret_cast<uint16_t*>(cell) + (sub & 7);
+            part[0] = static_cast<uint16_t>(hi);
+            part[8] = static_cast<uint16_t>(mid);
+            part[16] = static_cast<uint16_t>(lo);
+            cell[48 + (sub & 7)] = static_cast<uint8_t>(exponent);
+        }
+    } else if (wave == 1) {
+        // the digits may leave something of a value whose last bit is below 2^(e - 39) (zeros wrap round to the largest number)
+        uint32_t least = 0xFFFFFFFFu;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) least = min(least, (__float_as_uint(v[i]) << 1) - 1u);
+        const bool left = least != 0xFFFFFFFFu && static_cast<int>((least + 1) >> 24) < exponent - 15;
+        const bool any_left = __builtin_amdgcn_ballot_w64(left) != 0;
+        if (tid == 64) cell[56 + (sub & 7)] = any_left;  // (row 0)
     }
-    float s = (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]))) +
-              (((v[8] + v[9]) + (v[10] + v[11])) + ((v[12] + v[13]) + (v[14] + v[15])));
-    s += dpp_move<kDppXor1>(s);
-    if (half == 0 && row < rows) {
-        uint32_t hi, mid, lo;
-        split3_pair(s, 0.0f, &hi, &mid, &lo);
-        uint8_t* cell = sums + (static_cast<size_t>(row) * (in_dim >> 8) + (sub >> 3)) * 64;
-        uint16_t* part = reinterpret_cast<uint16_t*>(cell) + (sub & 7);
-        part[0] = static_cast<uint16_t>(hi);
-        part[8] = static_cast<uint16_t>(mid);
-        part[16] = static_cast<uint16_t>(lo);
-        cell[48 + (sub & 7)] = static_cast<uint8_t>(exponent);
-        if (r == 0) cell[56 + (sub & 7)] = any_left;
+    // The units and the scale as floats, for which sub-blocks near the ends of f32 are brought to 2^0.
+    const bool far = exponent < 70 || exponent > 220;
+    const int base = far ? 127 : exponent;
+    if (__builtin_amdgcn_ballot_w64(far && peak != 0) != 0) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] = __builtin_ldexpf(v[i], base - exponent);
     }
-    __syncthreads();
-    uint4* out = reinterpret_cast<uint4*>(digits + static_cast<size_t>(tile) * kG32Rows * in_dim * 6 +
-                                          static_cast<size_t>(sub) * tile_rows * kDigitBytes);
-    for (int i = lane; i < tile_rows * (kDigitBytes / 16); i += 64) out[i] = reinterpret_cast<const uint4*>(img)[i];
+    auto take_off = [&](int biased) {  // multiples of 2^(biased - 150)
+        const float c = __uint_as_float(static_cast<uint32_t>(biased) << 23 | 0x400000u);
+#pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] -= (v[i] + c) - c;
+    };
+    if (wave >= 2) take_off(base + 5);
+    take_off(base + 25 - 5 * digit);
+    t_f32x16 even, odd;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        even[i] = v[(i & 8) * 2 + kFp6Order[2 * i & 15]];
+        odd[i] = v[(i & 8) * 2 + kFp6Order[(2 * i & 15) + 1]];
+    }
+    const t_i32x6 codes = fp6_codes(even, odd, __uint_as_float(static_cast<uint32_t>(base - 5 * digit) << 23));
+    if (r < tile_rows) {
+        uint8_t* image = digits + static_cast<size_t>(tile) * kG32Rows * in_dim * 6 + (static_cast<size_t>(sub) * 4 + (digit >> 1)) * tile_rows * 48;
+        const int at = (digit & 1) * tile_rows + r;
+        reinterpret_cast<int4*>(image)[at] = make_int4(codes[0], codes[1], codes[2], codes[3]);
+        reinterpret_cast<int2*>(image + tile_rows * 32)[at] = make_int2(codes[4], codes[5]);
+    }
 }
 
 // (x & mask) | (y & ~mask) and (x & mask) | y in one instruction at the fast rate (v_bitop3_b32 2.4 cycles; v_and_or_b32 and the
@@ -1111,7 +1115,6 @@ __device__ __forceinline__ void q4k_lds_load16(const void* base, uint32_t& off, 
 
 typedef int t_i32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t t_u32x2 __attribute__((ext_vector_type(2)));
-typedef int t_i32x6 __attribute__((ext_vector_type(6)));
 
 // s_waitcnt for "at most kLeft vector memory operations outstanding".
 template <int kLeft>
@@ -1545,9 +1548,8 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
                         } part[3][2];
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
-                            int high, low;
-                            const float r[4] = {digits_of(v[k].x, exponent, &high, &low), digits_of(v[k].y, exponent, &high, &low),
-                                                digits_of(v[k].z, exponent, &high, &low), digits_of(v[k].w, exponent, &high, &low)};
+                            const float r[4] = {left_behind(v[k].x, exponent), left_behind(v[k].y, exponent), left_behind(v[k].z, exponent),
+                                                left_behind(v[k].w, exponent)};
 #pragma unroll
                             for (int e = 0; e < 2; ++e)
                                 split3_pair(r[2 * e], r[2 * e + 1], &part[0][k >> 1].u[2 * (k & 1) + e], &part[1][k >> 1].u[2 * (k & 1) + e],
@@ -2004,7 +2006,7 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
         hipLaunchKernelGGL(q4k_split_parts_kernel, dim3(static_cast<unsigned>(split_grid)), dim3(256), 0, stream, x, parts, part_sums,
                            groups, in_dim >> 3);
     } else {
-        hipLaunchKernelGGL(q4k_split_digits_kernel, dim3(in_dim / 32, m_tiles), dim3(64), 0, stream, x, space, digit_sums, rows, in_dim);
+        hipLaunchKernelGGL(q4k_split_digits_kernel, dim3(in_dim / 32, m_tiles), dim3(256), 0, stream, x, space, digit_sums, rows, in_dim);
     }
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     const Q4kSecond second{dst_b, weight_b, ep_b};

@@ -565,6 +565,32 @@ def test_prefill_past_64_rows_keeps_small_values_beside_large_ones(rows, in_dim,
     assert np.array_equal(G.linear_bias(Q4K, PREP, x, da, b, rows, in_dim, out_dim), y + b[None, :])
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(65, 256, 100), (97, 1024, 520)])
+def test_prefill_past_64_rows_on_activations_of_every_size(rows, in_dim, out_dim):
+    """The splitter works on X as it is except near the ends of f32: sub-blocks on both sides of either line, in one row and in
+    different rows.  A power of two on X is one on Y, to the bit; zero sub-blocks and a zero row stay zeros."""
+    print(f"case: q4_k fp6 prefill, powers of two rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(103, rows, in_dim)
+    x[3, 32:64] = 0.0
+    x[rows - 2] = 0.0
+    w = synth.weights(Q4K, 104, out_dim, in_dim)
+    wd = device_weight(PREP, w, out_dim, in_dim)
+    y = G.linear(Q4K, PREP, x, wd, rows, in_dim, out_dim)
+    ref = O.linear_q4_k(x[:8], w, 8, in_dim, out_dim, f64=True)
+    assert G.max_rel_err(y[:8], ref) <= TIGHT and not y[rows - 2].any()
+    powers = np.array([-62, -59, -58, -57, -20, 40, 91, 92, 93, 94, 100], np.float32)
+    for p in powers:
+        got = G.linear(Q4K, PREP, x * np.float32(2) ** p, wd, rows, in_dim, out_dim)
+        assert np.array_equal(got, y * np.float32(2) ** p), p
+    each = np.float32(2) ** powers[np.arange(rows) % len(powers)][:, None]  # every row its own
+    assert np.array_equal(G.linear(Q4K, PREP, x * each, wd, rows, in_dim, out_dim), y * each)
+    tiny = x.copy()
+    tiny[:, :32] *= np.float32(2) ** -90  # a sub-block of its own size, the whole of row 5
+    tiny[5, 32:] = 0.0
+    ref = O.linear_q4_k(tiny[:8], w, 8, in_dim, out_dim, f64=True)
+    assert G.max_rel_err(G.linear(Q4K, PREP, tiny, wd, rows, in_dim, out_dim)[:8], ref) <= TIGHT
+
+
 def test_prefill_past_64_rows_over_its_own_input():
     """A result in X's place is outside the header's contract; it has always come out right because X is split before anything is
     stored, and the kernel that may look at X again must not serve it."""
