@@ -295,15 +295,20 @@ struct PreparedWeights<8> {
 };
 
 // The value stored for output column o (element idx of Y) whose total is v.
-__device__ __forceinline__ float finish_output(const Epilogue& ep, int o, size_t idx, float v) {
-    if (ep.bias != nullptr) v += ep.bias[o];
-    if (ep.activation == kActRelu) {
+__device__ __forceinline__ float activate(int activation, float v) {
+    if (activation == kActRelu) {
         v = v < 0.0f ? 0.0f : v;
-    } else if (ep.activation == kActQuickGelu) {
+    } else if (activation == kActQuickGelu) {
         v = v / (1.0f + expf(-1.702f * v));
-    } else if (ep.activation == kActGelu) {
+    } else if (activation == kActGelu) {
         v = 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
     }
+    return v;
+}
+
+__device__ __forceinline__ float finish_output(const Epilogue& ep, int o, size_t idx, float v) {
+    if (ep.bias != nullptr) v += ep.bias[o];
+    v = activate(ep.activation, v);
     if (ep.residual != nullptr) v += ep.residual[idx];
     return v;
 }

@@ -161,6 +161,37 @@ def test_fused_epilogues(fmt, rows, in_dim, out_dim):
         assert G.max_rel_err(relu, ref.astype(np.float64)) <= TIGHT
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(69, 256, 1000), (333, 4096, 4090), (669, 1024, 5603), (130, 6144, 1030)])
+def test_fused_epilogues_of_q4_k_prefills(rows, in_dim, out_dim):
+    """Past 64 rows: each tile of the 6-bit kernel on odd rows and columns, and K shares (the reduce kernel's epilogue): the stored
+    value is act(product + bias) + residual, also where the residual lies in the result's place."""
+    print(f"case: q4_k prefill epilogues rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x, w = synth.activations(670, rows, in_dim) * 4.0, synth.weights(Q4K, 671, out_dim, in_dim)
+    b, res = bias_vector(672, out_dim), synth.activations(673, rows, out_dim)
+    wd = G.prepare(Q4K, w, out_dim, in_dim)
+    plain = G.linear(Q4K, PREP, x, wd, rows, in_dim, out_dim)
+
+    def run(**more):
+        return linear_epilogue(Q4K, PREP, x, wd, rows, in_dim, out_dim, **more)
+
+    biased = run(bias=b)
+    assert np.array_equal(biased, plain + b[None, :]) and (biased < 0).any() and (biased > 0).any()
+    assert np.array_equal(run(residual=res), plain + res)
+    assert np.array_equal(run(bias=b, residual=res), biased + res)
+    assert np.array_equal(run(activation=_lib.ACTIVATION_RELU), np.maximum(plain, 0))
+    assert np.array_equal(run(bias=b, residual=res, activation=_lib.ACTIVATION_RELU), np.maximum(biased, 0) + res)
+    for act, kind in ((_lib.ACTIVATION_QUICK_GELU, O.QUICK_GELU), (_lib.ACTIVATION_GELU, O.GELU)):
+        got, want = run(bias=b, activation=act), O.apply_activation(kind, biased)
+        assert np.allclose(got, want, rtol=3e-6, atol=1e-6 * np.abs(biased).max()), (act, np.abs(got - want).max())
+        assert np.array_equal(run(bias=b, residual=res, activation=act), got + res)
+    xd, bd, y = G.to_dev(x.astype(np.float32)), G.to_dev(b), G.to_dev(res.astype(np.float32))
+    ws = torch.empty(max(kernels.workspaceBytes(Q4K, rows, in_dim, out_dim), 16), dtype=torch.uint8, device=G.DEV)
+    kernels.launchLinearEpilogueF32(G.stream(), Q4K, PREP, G.buf(y), G.buf(xd), G.buf(wd), rows, in_dim, out_dim, G.buf(bd), G.buf(y),
+                                    _lib.ACTIVATION_RELU, G.buf(ws))
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), np.maximum(biased, 0) + res)
+
+
 def test_bias_argument_errors():
     rows, in_dim, out_dim = 2, 512, 512
     x = G.to_dev(synth.activations(1, rows, in_dim))
