@@ -19,8 +19,8 @@
 // multiplies, a load of X asks for sixteen lines, one a lane of a quad, and so does a load of weights -- about 800 cycles of
 // address work a wavefront and four blocks.  One column tile therefore loads whole lines and lets its lanes exchange them
 // through LDS (2 KB of X, up to 2 KB of weights a wavefront, where the sums go afterwards): about 180.
-// us before / now, Q4_0: a pair of 256 columns at K = 2048, 77 rows 9.5 / 6.1, 300 rows 24 / 13, 2048 rows 73 / 64; 333 x 4096 x
-// 100 16.7 / 10.9, 20 x 4096 x 500 16.1 / 9.6.  Now the vector ALU (the split) on many rows, launch and latency on few.
+// us, loaded by its user / by lines, Q4_0: a pair of 256 columns at K = 2048, 77 rows 9.8 / 6.6, 300 rows 24 / 13.5, 2048 rows 73 / 62;
+// 333 x 4096 x 100 17.3 / 11.5, 20 x 4096 x 500 16.5 / 9.6.  Now the vector ALU (the split) on many rows, launch and latency on few.
 // Relative error against 64 bits 1.0e-7.
 #include <hip/hip_runtime.h>
 
@@ -39,7 +39,6 @@ union Bf16x8 {
 };
 
 constexpr int kRouteRows = 16;   // rows of a workgroup, and columns of a tile
-constexpr int kRouteDepth = 4;   // blocks a wavefront requests ahead of its arithmetic
 constexpr int kWaveFloats = 1024;  // of LDS: a block of X (2 KB), one tile's weights of four blocks (2 KB); at the end the sums
 
 // What a wavefront's own lanes hand each other through LDS: the operations of a wavefront complete in order, only the compiler
@@ -115,7 +114,8 @@ struct RouteSecond {
     Epilogue ep;
 };
 
-template <int kType, int kTiles>
+// kDepth: blocks a wavefront requests ahead of its arithmetic.
+template <int kType, int kTiles, int kDepth>
 __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restrict__ dst_a, const float* __restrict__ x,
                                                                const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
                                                                Epilogue ep_a, RouteSecond second) {
@@ -146,27 +146,48 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
     }
     float* own = route_sums + wave * kWaveFloats;
     float4* own_x = reinterpret_cast<float4*>(own);                       // [row][chunk ^ row / 2], 16 bytes each: a read in 16 banks' groups
-    unsigned char* own_w = reinterpret_cast<unsigned char*>(own) + 2048;  // [block][16-byte half][column]
+    // [block][16-byte half][column ^ 2 * place of block and half]: written by lanes of one column and all places, read by all columns
+    // of one place, in different banks both times
+    unsigned char* own_w = reinterpret_cast<unsigned char*>(own) + 2048;
+    auto weight_slot = [](int place, int column) { return place * 16 + (column ^ (2 * place & 15)); };
     const size_t blocks = static_cast<size_t>(out_dim) * kb;
     const uint16_t* scales = reinterpret_cast<const uint16_t*>(weight + blocks * kQuantBytes);
     size_t first[kTiles];  // first block of this lane's column in each tile
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) first[t] = static_cast<size_t>(min(n0 + 16 * t + c, out_dim - 1)) * kb;
 
+    // (one tile) a column's four blocks are one load of 64 bytes (Q8_0: two loads of 64 lanes, 128 bytes a column), its four scales are
+    // four lanes'
+    constexpr int kWeightLoads = kType == 2 ? 1 : 2;
+    const uint8_t* wcol[kWeightLoads];
+    const uint16_t* scol = scales + static_cast<size_t>(min(n0 + (lane >> 2), out_dim - 1)) * kb;
+#pragma unroll
+    for (int i = 0; i < kWeightLoads; ++i) {
+        const int col = kType == 2 ? lane >> 2 : 8 * i + r8, half = kType == 2 ? 0 : ch & 1;
+        wcol[i] = weight + static_cast<size_t>(min(n0 + col, out_dim - 1)) * kb * kQuantBytes + 16 * half;
+    }
+
     r_f32x4 acc[kTiles];
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) acc[t] = r_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     uint64_t left_behind = 0;  // lanes that met a value below about 2^-110
-    // a wavefront's blocks follow each other: parts of the same lines of weights
-    const int per_wave = (kb + waves - 1) / waves, begin = wave * per_wave, end = min(begin + per_wave, kb);
-    for (int b0 = begin; b0 < end; b0 += kRouteDepth) {
-        float4 xv[kRouteDepth][2];
-        uint2 wq[kRouteDepth][kTiles];
-        uint16_t ws[kRouteDepth][kTiles];
+    // a wavefront's blocks follow each other, parts of the same lines of weights; the first kb % waves wavefronts have one more
+    const int per_wave = kb / waves, more = kb - per_wave * waves, begin = wave * per_wave + min(wave, more), end = begin + per_wave + (wave < more);
+    for (int b0 = begin; b0 < end; b0 += kDepth) {
+        float4 xv[kDepth][2];
+        uint2 wq[kDepth][kTiles];
+        uint16_t ws[kDepth][kTiles];
         int sraw = 0;
+        uint4 wraw[kWeightLoads];
+        if constexpr (kStaged) {
 #pragma unroll
-        for (int u = 0; u < kRouteDepth; ++u) {
+            for (int i = 0; i < kWeightLoads; ++i)
+                wraw[i] = *reinterpret_cast<const uint4*>(wcol[i] + min(b0 + (kType == 2 ? lane & 3 : ch >> 1), end - 1) * kQuantBytes);
+            sraw = scol[min(b0 + (lane & 3), end - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < kDepth; ++u) {
             const int b = min(b0 + u, end - 1);  // past the end: the last block again, not used
             xv[u][0] = *reinterpret_cast<const float4*>(xrow[0] + b * 32);
             xv[u][1] = *reinterpret_cast<const float4*>(xrow[1] + b * 32);
@@ -177,25 +198,12 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
             }
         }
         if constexpr (kStaged) {
-            // a column's four blocks are one load of 64 bytes (Q8_0: two loads of 64 lanes, 128 bytes a column), its four scales
-            // are four lanes'
-            constexpr int kWeightLoads = kType == 2 ? 1 : 2;
-            const int col = lane >> 2, b = min(b0 + (lane & 3), end - 1);
-            sraw = scales[static_cast<size_t>(min(n0 + col, out_dim - 1)) * kb + b];
-            uint4 wraw[kWeightLoads];
 #pragma unroll
-            for (int i = 0; i < kWeightLoads; ++i) {
-                const int wcol = kType == 2 ? col : 8 * i + r8, wb = kType == 2 ? b : min(b0 + (ch >> 1), end - 1), half = kType == 2 ? 0 : ch & 1;
-                wraw[i] = *reinterpret_cast<const uint4*>(weight + (static_cast<size_t>(min(n0 + wcol, out_dim - 1)) * kb + wb) * kQuantBytes + 16 * half);
-            }
-#pragma unroll
-            for (int i = 0; i < kWeightLoads; ++i) {
-                const int slot = kType == 2 ? (lane & 3) * 16 + col : ch * 16 + 8 * i + r8;
-                *reinterpret_cast<uint4*>(own_w + 16 * slot) = wraw[i];
-            }
+            for (int i = 0; i < kWeightLoads; ++i)
+                *reinterpret_cast<uint4*>(own_w + 16 * (kType == 2 ? weight_slot(lane & 3, lane >> 2) : weight_slot(ch, 8 * i + r8))) = wraw[i];
         }
 #pragma unroll
-        for (int u = 0; u < kRouteDepth; ++u) {
+        for (int u = 0; u < kDepth; ++u) {
             if (b0 + u >= end) break;  // wavefront-uniform
             Bf16x8 part[3];
             float4 x0 = xv[u][0], x1 = xv[u][1];
@@ -205,7 +213,7 @@ __global__ __launch_bounds__(1024, 8) void linear_f32_rows_kernel(float* __restr
                 wave_order();
                 x0 = own_x[c * 8 + ((2 * g) ^ (c >> 1))];
                 x1 = own_x[c * 8 + ((2 * g + 1) ^ (c >> 1))];
-                const int slot = kType == 2 ? u * 16 + c : (u * 2 + (g >> 1)) * 16 + c;
+                const int slot = weight_slot(kType == 2 ? u : u * 2 + (g >> 1), c);
                 wq[u][0] = *reinterpret_cast<const uint2*>(own_w + 16 * slot + 8 * (g & 1));
                 ws[u][0] = static_cast<uint16_t>(__builtin_amdgcn_ds_bpermute(4 * (4 * c + u), sraw));
                 wave_order();
@@ -284,12 +292,15 @@ hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* ds
     for (int r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
         const int nr = rows - r0 < kRowsPerLaunch ? rows - r0 : kRowsPerLaunch;
         const unsigned groups = static_cast<unsigned>((nr + 15) / 16);
-        // One column tile, whose loads go through LDS, or four, which share a split of X but not those loads (us, one / four; the
-        // two add alike): from K = 1056 on one everywhere -- a pair of 256 columns, 700 x 1536 19 / 29, 2048 x 1536 49 / 56,
-        // 1000 x 4096 61 / 75, 2048 x 5120 144 / 179 -- below, four on grids of two workgroups a compute unit: a pair of 2048 x
-        // 1024 x 256 38 .. 42 / 39, of 2048 x 768 31 / 25, 4096 x 288 x 288 15.5 / 10.5, but a pair of 700 x 1024 x 256 14.2 / 20.5.
-        const long wide = static_cast<long>(groups) * ((out_dim + 63) / 64) * matrices;
-        const int tiles = kb <= 32 && wide >= 2 * gemv_compute_units() ? 4 : 1;
+        // One column tile, whose loads go through LDS, or four, which share a split of X but not those loads (the two add alike).  Four
+        // where their workgroups leave the compute units' last round at least 65 % full, K is no multiple of 512 (there the rows that
+        // a load of X touches meet in the caches: us, one / four, a pair of 927 x 1536 x 223 25 / 31, 817 x 1024 x 321 22 / 30) and, with
+        // Q4_0, up to K = 4096: Q8_0, pairs, 1917 x 1376 x 411 72 / 53, 671 x 672 x 292 14.3 / 10.4, Q4_0 1090 x 1120 x 305 28 / 21,
+        // 1764 x 352 x 384 19.9 / 13.0, but 478 x 992 x 256 (47 % full) 10 / 13.  Over 1200 shapes (16 .. 2048 rows, K 256 .. 8192, 64 .. 511
+        // columns) 0.6 % above the better of the two on the mean.
+        const long units = gemv_compute_units(), wide = static_cast<long>(groups) * ((out_dim + 63) / 64) * matrices;
+        const bool full = wide * 100 >= 65 * units * ((wide + units - 1) / units);
+        const int tiles = full && in_dim % 512 != 0 && (tensor_type == 8 || in_dim <= 4096) ? 4 : 1;
         const dim3 grid(static_cast<unsigned>((out_dim + 16 * tiles - 1) / (16 * tiles)), groups, matrices), block(64 * waves);
         const size_t lds = static_cast<size_t>(waves) * kWaveFloats * 4;  // at most 64 KiB
         Epilogue ep = ep0, ep_b = ep_b0;
@@ -298,12 +309,20 @@ hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* ds
         float* d = dst + static_cast<size_t>(r0) * out_dim;
         const float* in = x + static_cast<size_t>(r0) * in_dim;
         const RouteSecond second{dst_b ? dst_b + static_cast<size_t>(r0) * out_dim : nullptr, weight_b, ep_b};
+        const int per_wave = (kb + waves - 1) / waves;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+        };
         if (tensor_type == 2) {
-            if (tiles == 4) hipLaunchKernelGGL((linear_f32_rows_kernel<2, 4>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
-            else hipLaunchKernelGGL((linear_f32_rows_kernel<2, 1>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+            if (tiles == 4) launch(linear_f32_rows_kernel<2, 4, 4>);
+            else if (per_wave == 1) launch(linear_f32_rows_kernel<2, 1, 1>);
+            else if (per_wave == 2) launch(linear_f32_rows_kernel<2, 1, 2>);
+            else launch(linear_f32_rows_kernel<2, 1, 4>);
         } else {
-            if (tiles == 4) hipLaunchKernelGGL((linear_f32_rows_kernel<8, 4>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
-            else hipLaunchKernelGGL((linear_f32_rows_kernel<8, 1>), grid, block, lds, stream, d, in, weight_prepared, nr, in_dim, out_dim, ep, second);
+            if (tiles == 4) launch(linear_f32_rows_kernel<8, 4, 4>);
+            else if (per_wave == 1) launch(linear_f32_rows_kernel<8, 1, 1>);
+            else if (per_wave == 2) launch(linear_f32_rows_kernel<8, 1, 2>);
+            else launch(linear_f32_rows_kernel<8, 1, 4>);
         }
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }

@@ -625,3 +625,11 @@ def test_f32_route_tiles_and_runs_of_blocks(fmt, rows, in_dim, out_dim):
     for got, w in ((ya, wa), (yb, wb)):
         ref = O.linear_no_bias(fmt, x[sample], w, len(sample), in_dim, out_dim, workers=8)
         assert G.max_rel_err(got[sample], ref.astype(np.float64)) <= TIGHT
+
+
+@pytest.mark.parametrize("fmt", [Q8, Q4])
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(168, 352, 187), (40, 512, 200), (671, 672, 292), (1090, 1120, 305), (530, 3616, 250),
+                                                 (520, 4640, 257), (460, 544, 490)])
+def test_f32_route_runs_of_unequal_length(fmt, rows, in_dim, out_dim):
+    """Runs of one, two and more blocks a wavefront, some one block longer than the others, on one column tile and on four."""
+    test_f32_route_tiles_and_runs_of_blocks(fmt, rows, in_dim, out_dim)
