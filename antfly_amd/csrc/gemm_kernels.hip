@@ -149,9 +149,9 @@ __device__ __forceinline__ void gemm_i8_body(
     constexpr int kStartB = kUnitsA % kWaves, kStartSx = (kStartB + kUnitsB) % kWaves, kStartSw = (kStartSx + kUnitsSx) % kWaves;
 
     // K range of this workgroup: all of it, or (a small grid spread over more compute units)
-    // share blockIdx.y of share_blocks blocks, whose sums go to partial[share][rows][out_dim], or, without room for them, are
-    // added to a cleared dst (two shares: 0 + a + b = 0 + b + a to the bit, whoever comes first)
-    // for splitk_reduce_kernel.  kb_full is the row pitch, kb the blocks walked here.
+    // share blockIdx.y of share_blocks blocks, whose sums go to partial[share][rows][out_dim] for splitk_reduce_kernel, or, of two
+    // shares without an epilogue, are added to a dst that the quantizer's launch has cleared (partial is null then;
+    // 0 + a + b = 0 + b + a to the bit, whoever comes first).  kb_full is the row pitch, kb the blocks walked here.
     const int kb_full = in_dim >> 5;
     const int blk_begin = kShareK ? static_cast<int>(blockIdx.y) * share_blocks : 0;
     const int kb = kShareK ? min(share_blocks, kb_full - blk_begin) : kb_full;
@@ -747,16 +747,17 @@ size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim) {
     return splits > 1 ? static_cast<size_t>(splits) * rows * out_dim * 4 : 0;
 }
 
-// dst = epilogue(sum over the K shares, in order): second kernel of a split-K launch.  Four shares' values on their way at a
+// dst = epilogue(sum over the K shares, in order): second kernel of a split-K launch.  first_in_dst: the first share's sums are in dst.  Four shares' values on their way at a
 // time; a column is only worked out where an epilogue asks for it.  (us a call, against a serial loop over the shares with a
 // remainder for every value: Q8_0 100 x 4096 x 1024 12.3 -> 11.7, Q4_0 32 x 14336 x 4096 19.4 -> 18.9.  Four values a thread did
 // no better there and lost where the shares are large: Q4_K 32 x 4096 x 14336 22.2 -> 24.4, 64 x 4096 x 4096 17.0 -> 19.8.)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(float* __restrict__ dst, const float* __restrict__ partial,
-                                                            size_t count, int out_dim, int splits, Epilogue ep) {
+                                                            size_t count, int out_dim, int splits, Epilogue ep, int first_in_dst) {
     const bool plain = ep.bias == nullptr && ep.residual == nullptr && ep.activation == kActNone;
     for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < count;
          i += static_cast<size_t>(gridDim.x) * blockDim.x) {
         float total = 0.0f;
+        if (first_in_dst) total += dst[i];
         for (int z0 = 0; z0 < splits; z0 += 4) {
             float part[4];
 #pragma unroll
@@ -770,11 +771,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(float* __restrict__ 
 }
 
 hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* partial, size_t count, int out_dim, int shares,
-                                const Epilogue& ep) {
+                                const Epilogue& ep, bool first_in_dst) {
     size_t grid = (count + 255) / 256;
     if (grid > 4096) grid = 4096;
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, dst, partial, count, out_dim,
-                       shares, ep);
+                       first_in_dst ? shares - 1 : shares, ep, first_in_dst ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -1148,7 +1148,7 @@ template <int kWaves, int kR, int kC, int kOcc>
 __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
     float* __restrict__ dst, const uint8_t* __restrict__ digits, const uint8_t* __restrict__ sums,
     const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim, int m_groups, int n_groups, int band, int sb_per_split,
-    float* __restrict__ partial, Epilogue ep, Q4kSecond second, const float* __restrict__ x) {
+    float* __restrict__ partial, int first_to_dst, Epilogue ep, Q4kSecond second, const float* __restrict__ x) {
     using S = G6Shape<kWaves, kR, kC>;
     if (blockIdx.z != 0) {  // a second matrix on the same X
         dst = second.dst;
@@ -1156,7 +1156,8 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
         ep = second.ep;
     }
     const int kb = in_dim >> 8;
-    // K range of this workgroup: all of it, or share blockIdx.y, whose sums go to partial[share][rows][out_dim]
+    // K range of this workgroup: all of it, or share blockIdx.y, whose sums go to partial[share][rows][out_dim] (first_to_dst = 1: the
+    // first share's to dst, the others' to partial[share - 1])
     const int sb_begin = blockIdx.y * sb_per_split;
     const int sb_end = min(kb, sb_begin + sb_per_split);
     const int lane = threadIdx.x & 63;
@@ -1642,7 +1643,8 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
                     for (int v = 0; v < 16; ++v) acc[i][j][v] += residual[i][j][v];
         }
     }
-    float* out = partial != nullptr ? partial + static_cast<size_t>(blockIdx.y) * rows * out_dim : dst;
+    float* out = partial == nullptr || (blockIdx.y == 0 && first_to_dst != 0) ? dst
+                                                                              : partial + static_cast<size_t>(blockIdx.y - first_to_dst) * rows * out_dim;
 #pragma unroll
     for (int j = 0; j < kC; ++j) {
         if (col0 + j * kTileCols >= out_dim) continue;
@@ -1866,7 +1868,7 @@ int device_units() {
 }
 
 // What serves a GEMM call: the bf16 kernel (kParts), or the fp6 kernel with one of its tiles; and over how many workgroups K is
-// shared out (a power of two, at most eight, at least two super-blocks each).
+// shared out (at most eight, at least two super-blocks each, no empty one; kParts: a power of two).
 enum Q4kGemmKind { kParts, kFp6Tile64x256, kFp6Tile64x128, kFp6Tile32x128 };
 struct Q4kGemmPlan {
     Q4kGemmKind kind;
@@ -1874,29 +1876,29 @@ struct Q4kGemmPlan {
 };
 
 // Time of a call in us, from the rounds of the busiest XCD's compute units.  `steps[n]`: a sub-block of a wavefront's tiles with n + 1
-// workgroups on the unit; `round`: start and drain of a workgroup; `shares`, `share_mb`: the reduce launch and its MB; `split`: per
-// million values of X; `out`: per MB of Y.  Fitted to 1600 timed calls (65 .. 2048 rows, K 1024 .. 14336, N 1536 .. 14336; 5 % rms);
-// over these the choice is 3 % from the best tile and share count on the mean.
+// workgroups on the unit; `base`: launches, start and drain; `shares`, `share_mb`: the reduce launch and its MB; `split`: per million
+// values of X; `out`: per MB of Y.  Fitted to 5400 timed plans of 420 calls (65 .. 2048 rows, K 256 .. 14336, N 64 .. 14336; 7 % rms);
+// over these the choice is 1 % from the best tile and share count on the mean, 17 % at worst.
 struct Q4kGemmCost {
     int rows, cols, tiles, resident;
-    double steps[4], round, base, shares, share_mb, split, out;
+    double steps[4], base, shares, share_mb, split, out;
     double us(double m, double k, double n, int s) const {
         const long long groups = static_cast<long long>((m + rows - 1) / rows) * static_cast<long long>((n + cols - 1) / cols);
         const long long units = device_units() >= 8 ? device_units() / 8 : 1;
         const long long per_unit = ((groups + 7) / 8 * s + units - 1) / units, kb = static_cast<long long>(k / kQ4kBlockValues);
         const double work = static_cast<double>(tiles * 8 * ((kb + s - 1) / s)), mb = m * n * 4e-6;
         const long long full = per_unit / resident, rest = per_unit % resident;
-        double t = static_cast<double>(full) * work * steps[resident - 1] + static_cast<double>(full + (rest > 0)) * round + base;
+        double t = static_cast<double>(full) * work * steps[resident - 1] + base;
         if (rest > 0) t += work * steps[rest - 1];
         if (s > 1) t += shares + share_mb * (s + 1) * mb;
         return t + split * m * k * 1e-6 + out * mb;
     }
 };
 constexpr Q4kGemmCost kQ4kGemmCosts[4] = {
-    {32, 256, 1, 2, {0.351, 0.609, 0, 0}, 3.2, 3.2, 0.0, 0.40, 3.3, 0.32},
-    {64, 256, 4, 2, {0.108, 0.213, 0, 0}, 3.2, 5.7, 3.2, 0.16, 3.7, 0.31},
-    {64, 128, 2, 2, {0.138, 0.258, 0, 0}, 1.2, 6.3, 2.8, 0.20, 3.5, 0.26},
-    {32, 128, 1, 4, {0.219, 0.329, 0.490, 0.627}, 0.0, 7.2, 2.5, 0.21, 3.1, 0.25},
+    {32, 256, 1, 2, {0.377, 0.664, 0, 0}, 6.1, 1.3, 0.63, 1.8, 0.41},
+    {64, 256, 4, 2, {0.110, 0.214, 0, 0}, 8.3, 4.0, 0.26, 2.0, 0.30},
+    {64, 128, 2, 2, {0.141, 0.255, 0, 0}, 7.0, 3.9, 0.27, 2.2, 0.295},
+    {32, 128, 1, 4, {0.225, 0.319, 0.480, 0.620}, 6.6, 3.7, 0.24, 2.0, 0.27},
 };
 
 // The parts or digits of X with the sub-block sums behind them (the fp6 kernel's rows are padded to even), and the partial sums of
@@ -1906,25 +1908,33 @@ size_t gemm_q4k_split_bytes(Q4kGemmKind kind, size_t rows, size_t in_dim) {
     const size_t values = kind == kParts ? rows * in_dim * 6 : gemm_q4k_digit_bytes(rows, in_dim);
     return (values + rows * (in_dim / 32) * 8 + 255) / 256 * 256;
 }
+// (the fp6 kernel's first share stores where the result goes: one array of sums fewer)
+size_t gemm_q4k_sum_arrays(const Q4kGemmPlan& plan) {
+    return plan.splits <= 1 ? 0 : static_cast<size_t>(plan.kind == kParts ? plan.splits : plan.splits - 1);
+}
 size_t gemm_q4k_plan_bytes(const Q4kGemmPlan& plan, size_t rows, size_t in_dim, size_t out_dim) {
-    return gemm_q4k_split_bytes(plan.kind, rows, in_dim) + (plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * out_dim * 4 : 0);
+    return gemm_q4k_split_bytes(plan.kind, rows, in_dim) + gemm_q4k_sum_arrays(plan) * rows * out_dim * 4;
 }
 
-bool gemm_q4k_shares_allowed(int splits, size_t in_dim) { return splits == 1 || (splits <= 8 && in_dim / kQ4kBlockValues / splits >= 2); }
+bool gemm_q4k_shares_allowed(int splits, size_t in_dim) {
+    const size_t kb = in_dim / kQ4kBlockValues, s = static_cast<size_t>(splits), each = (kb + s - 1) / s;
+    return splits == 1 || (splits <= 8 && kb / s >= 2 && (kb + each - 1) / each == s);
+}
 
 // The bf16 kernel's own shares: one when its workgroups fill the compute units anyway, else as many as spread it over them.
 Q4kGemmPlan gemm_q4k_parts_plan(size_t rows, size_t in_dim, size_t out_dim) {
     Q4kGemmPlan parts{kParts, 1};
     const long long workgroups = static_cast<long long>((out_dim + 255) / 256) * static_cast<long long>((rows + kG32Rows - 1) / kG32Rows);
-    while (workgroups * parts.splits * 2 <= device_units() && gemm_q4k_shares_allowed(parts.splits * 2, in_dim)) parts.splits *= 2;
+    while (workgroups * parts.splits * 2 <= device_units() && parts.splits < 8 && in_dim / kQ4kBlockValues / (2 * parts.splits) >= 2) parts.splits *= 2;
     return parts;
 }
 
 // The scratch that a call may take: the cost of a plan says nothing of the memory it asks callers for (without a limit 129 x 5120 x 13824
 // took 31 MB where X is 4, 512 x 8192 x 28672 137 where X is 25).  A call whose bf16 plan fits the static entry's array keeps
-// fitting it; past that the partial sums may take twice what the bf16 plan takes.  us with this limit / without: 333 x 4096 x 6144
-// 72 / 70 (one share for four), 129 x 4096 x 4096 29.8 / 29.4, 512 x 8192 x 28672 482 / 466; by the cost model 2 % on the mean of 4000
-// shapes (65 .. 2048 rows), 3 % with the same room once, 11 % without any past the bf16 plan's.
+// fitting it; past that the partial sums may take twice what the bf16 plan takes.  By the cost model the limit is 0.5 % on the mean of
+// 4000 shapes (65 .. 2048 rows), 128 of them more than 5 % -- 815, and 2.7 %, with powers of two alone and an array for every share.
+// us with the limit / eight shares allowed without one: 113 x 11008 x 6144 62 / 60, 333 x 4096 x 6144 71 / 69, but 167 x 12288 x 2580
+// 54 / 47, 176 x 7680 x 11008 119 / 103 (one share), 243 x 8448 x 5375 109 / 81.
 size_t gemm_q4k_most_bytes(size_t rows, size_t in_dim, size_t out_dim) {
     const size_t parts = gemm_q4k_plan_bytes(gemm_q4k_parts_plan(rows, in_dim, out_dim), rows, in_dim, out_dim);
     return parts <= AFHIP_STATIC_SCRATCH_BYTES ? static_cast<size_t>(AFHIP_STATIC_SCRATCH_BYTES) : 3 * parts;
@@ -1947,7 +1957,8 @@ Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, size_t roo
     Q4kGemmPlan best = none;
     double best_us = 1e30;
     for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
-        for (int s = 1; gemm_q4k_shares_allowed(s, in_dim); s *= 2) {
+        for (int s = 1; s <= 8; ++s) {
+            if (!gemm_q4k_shares_allowed(s, in_dim)) continue;
             const Q4kGemmPlan plan{static_cast<Q4kGemmKind>(kind), s};
             const double us = kQ4kGemmCosts[kind].us(m, k, n, s) * (s == 1 ? 1.0 : 1.03);
             if (us < best_us && fits(plan)) {
@@ -1974,6 +1985,7 @@ struct Q4kGemmCall {
     const uint8_t *digits, *sums, *weight;
     int rows, in_dim, out_dim, sb_per_split, shares;
     float* partial;
+    bool first_to_dst;
     const Epilogue& ep;
     const Q4kSecond* second;
 };
@@ -1993,7 +2005,7 @@ hipError_t launch_fp6_tile(const Q4kGemmCall& q) {
         attr_done.store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), q.shares, q.second ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, q.stream, q.dst,
-                       q.digits, q.sums, q.weight, q.rows, q.in_dim, q.out_dim, m_groups, n_groups, 8, q.sb_per_split, q.partial, q.ep,
+                       q.digits, q.sums, q.weight, q.rows, q.in_dim, q.out_dim, m_groups, n_groups, 8, q.sb_per_split, q.partial, q.first_to_dst ? 1 : 0, q.ep,
                        q.second ? *q.second : Q4kSecond{nullptr, nullptr, Epilogue{}}, q.x);
     return hipGetLastError();
 }
@@ -2023,6 +2035,13 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
         plan = gemm_q4k_parts_plan(m, k, n);
         if (gemm_q4k_plan_bytes(plan, m, k, n) > workspace_bytes) plan.splits = 1;
     }
+    // (a residual in the result's place has to outlast the first share: the sums take an array each then, and fewer shares where
+    // those have no room)
+    const bool over_residual = ep.residual != nullptr && reinterpret_cast<uintptr_t>(ep.residual) < reinterpret_cast<uintptr_t>(dst) + m * n * 4 &&
+                               reinterpret_cast<uintptr_t>(dst) < reinterpret_cast<uintptr_t>(ep.residual) + m * n * 4;
+    const bool first_to_dst = plan.kind != kParts && plan.splits > 1 && !over_residual;
+    if (plan.kind != kParts && over_residual)
+        while (plan.splits > 1 && gemm_q4k_split_bytes(plan.kind, m, k) + plan.splits * m * n * 4 > workspace_bytes) --plan.splits;
     const int kb = in_dim / kQ4kBlockValues;
     const int sb_per_split = (kb + plan.splits - 1) / plan.splits;
     const int shares = (kb + sb_per_split - 1) / sb_per_split;  // no empty share
@@ -2045,7 +2064,7 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     const Q4kSecond second{dst_b, weight_b, ep_b};
     auto multiply = [&](float* y, const uint8_t* w, const Epilogue& epilogue, const Q4kSecond* with) {
-        const Q4kGemmCall q{stream, x, y, space, digit_sums, w, rows, in_dim, out_dim, sb_per_split, shares, partial, epilogue, with};
+        const Q4kGemmCall q{stream, x, y, space, digit_sums, w, rows, in_dim, out_dim, sb_per_split, shares, partial, first_to_dst, epilogue, with};
         hipError_t e;
         if (plan.kind == kFp6Tile64x256) e = launch_fp6_tile<4, 2, 2, 2>(q);
         else if (plan.kind == kFp6Tile64x128) e = launch_fp6_tile<4, 2, 1, 2>(q);
@@ -2058,7 +2077,7 @@ hipError_t launch_gemm_q4k_tiled(hipStream_t stream, float* dst, const float* x,
             e = hipGetLastError();
         }
         if (e != hipSuccess || shares == 1) return e;
-        return launch_splitk_reduce(stream, y, partial, static_cast<size_t>(rows) * out_dim, out_dim, shares, epilogue);
+        return launch_splitk_reduce(stream, y, partial, static_cast<size_t>(rows) * out_dim, out_dim, shares, epilogue, first_to_dst);
     };
     if (dst_b == nullptr) return multiply(dst, weight, ep, nullptr);
     if (shares == 1 && plan.kind != kParts) return multiply(dst, weight, ep, &second);

@@ -125,9 +125,10 @@ hipError_t launch_gemm_i8(hipStream_t stream, int tensor_type, float* dst, int* 
 bool gemm_i8_adds_to_result(int rows, int in_dim, int out_dim, const Epilogue& ep);
 int gemm_i8_splits(int rows, int in_dim, int out_dim);
 size_t gemm_i8_partial_bytes(size_t rows, size_t in_dim, size_t out_dim);
-// dst[i] = epilogue(sum over s < shares of partial[s * count + i]), i < count = rows * out_dim
+// dst[i] = epilogue(sum over s < shares of partial[s * count + i]), i < count = rows * out_dim.  first_in_dst: share 0's sums are
+// in dst itself, partial begins with share 1's.
 hipError_t launch_splitk_reduce(hipStream_t stream, float* dst, const float* partial, size_t count, int out_dim, int shares,
-                                const Epilogue& ep);
+                                const Epilogue& ep, bool first_in_dst = false);
 
 // zero_a, zero_b (optional): arrays of zero_count floats to clear in the same launch
 hipError_t launch_quantize_activations(hipStream_t stream, const float* x, int rows, int in_dim, int8_t* q,

@@ -617,7 +617,7 @@ def test_prefill_past_64_rows_in_a_workspace_without_room_for_partial_sums():
     x = synth.activations(96, rows, in_dim)
     narrow = w[:out_dim * (in_dim // 256) * 144]
     digits = 130 * in_dim * 6 + 129 * (in_dim // 256) * 64
-    assert kernels.workspaceBytes(Q4K, rows, in_dim, out_dim) > digits + rows * out_dim * 8
+    assert kernels.workspaceBytes(Q4K, rows, in_dim, out_dim) >= digits + rows * out_dim * 4  # (one array of sums at the least)
     assert kernels.workspaceBytes(Q4K, rows, in_dim, wide) == (digits + 255) // 256 * 256
     want = G.linear(Q4K, PREP, x, device_weight(PREP, w, wide, in_dim), rows, in_dim, wide)[:, :out_dim]
     xd, wd = G.to_dev(x), device_weight(PREP, narrow, out_dim, in_dim)
