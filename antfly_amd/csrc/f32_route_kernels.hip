@@ -293,14 +293,16 @@ hipError_t launch_linear_f32_rows(hipStream_t stream, int tensor_type, float* ds
         const int nr = rows - r0 < kRowsPerLaunch ? rows - r0 : kRowsPerLaunch;
         const unsigned groups = static_cast<unsigned>((nr + 15) / 16);
         // One column tile, whose loads go through LDS, or four, which share a split of X but not those loads (the two add alike).  Four
-        // where their workgroups leave the compute units' last round at least 65 % full, K is no multiple of 512 (there the rows that
-        // a load of X touches meet in the caches: us, one / four, a pair of 927 x 1536 x 223 25 / 31, 817 x 1024 x 321 22 / 30) and, with
-        // Q4_0, up to K = 4096: Q8_0, pairs, 1917 x 1376 x 411 72 / 53, 671 x 672 x 292 14.3 / 10.4, Q4_0 1090 x 1120 x 305 28 / 21,
-        // 1764 x 352 x 384 19.9 / 13.0, but 478 x 992 x 256 (47 % full) 10 / 13.  Over 1200 shapes (16 .. 2048 rows, K 256 .. 8192, 64 .. 511
-        // columns) 0.6 % above the better of the two on the mean.
+        // where their workgroups fill the compute units' rounds: to 65 % up to K = 1024, 75 % up to 4096, 90 % beyond (Q8_0; Q4_0 not at
+        // all), and not where K is a multiple of 256 past 1024, or of 512 (the rows that a load of X touches meet in the caches).  us, one /
+        // four: Q8_0, pairs, 1917 x 1376 x 411 72 / 53, 671 x 672 x 292 14.3 / 10.4, Q4_0 1090 x 1120 x 305 28 / 21, 1764 x 352 x 384
+        // 19.9 / 13.0, but 478 x 992 x 256 (47 % full) 10 / 13, 863 x 2816 x 256 40 / 42, 927 x 1536 x 223 25 / 31.  Over 1200 shapes (16 ..
+        // 2048 rows, K 256 .. 8192, 64 .. 511 columns) 0.3 % above the better of the two on the mean.
         const long units = gemv_compute_units(), wide = static_cast<long>(groups) * ((out_dim + 63) / 64) * matrices;
-        const bool full = wide * 100 >= 65 * units * ((wide + units - 1) / units);
-        const int tiles = full && in_dim % 512 != 0 && (tensor_type == 8 || in_dim <= 4096) ? 4 : 1;
+        const long fill = 100 * wide / (units * ((wide + units - 1) / units));
+        const bool apart = in_dim % 256 != 0 || (in_dim <= 1024 && in_dim % 512 != 0);
+        const long least = in_dim <= 1024 && in_dim % 256 != 0 ? 65 : (in_dim <= 4096 ? 75 : (tensor_type == 8 ? 90 : 101));
+        const int tiles = apart && fill >= least ? 4 : 1;
         const dim3 grid(static_cast<unsigned>((out_dim + 16 * tiles - 1) / (16 * tiles)), groups, matrices), block(64 * waves);
         const size_t lds = static_cast<size_t>(waves) * kWaveFloats * 4;  // at most 64 KiB
         Epilogue ep = ep0, ep_b = ep_b0;

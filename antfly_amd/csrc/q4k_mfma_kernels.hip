@@ -1590,18 +1590,12 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
     // took everything a value at a time, one trip to memory each (in brackets the bias alone): 75 x 256 x 2048 14.7 -> 11.4
     // (11.1 -> 8.1), 670 x 1024 x 5632 65 -> 44 (42 -> 34), 512 x 4096 x 14336 185 -> 163 (159 -> 150).
     const int row0 = m_group * S::kRows + 4 * g, col0 = (tile0 + wave * kC) * kTileCols + c;
-    if (partial == nullptr && ep.bias != nullptr) {
+    if (partial == nullptr && (ep.bias != nullptr || ep.residual != nullptr || ep.activation != kActNone)) {
+        float bias[kC], residual[kR][kC][16];
+        if (ep.bias != nullptr) {
 #pragma unroll
-        for (int j = 0; j < kC; ++j) {
-            const float bias = ep.bias[min(col0 + j * kTileCols, out_dim - 1)];
-#pragma unroll
-            for (int i = 0; i < kR; ++i)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] += bias;
+            for (int j = 0; j < kC; ++j) bias[j] = ep.bias[min(col0 + j * kTileCols, out_dim - 1)];
         }
-    }
-    if (partial == nullptr && (ep.residual != nullptr || ep.activation != kActNone)) {
-        float residual[kR][kC][16];
         if (ep.residual != nullptr) {  // (past the end: the last row's, the last column's; not stored)
 #pragma unroll
             for (int i = 0; i < kR; ++i)
@@ -1613,6 +1607,14 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
                 }
         }
         asm volatile("" : : : "memory");  // (requested here, not where they are used)
+        if (ep.bias != nullptr) {
+#pragma unroll
+            for (int j = 0; j < kC; ++j)
+#pragma unroll
+                for (int i = 0; i < kR; ++i)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] += bias[j];
+        }
         if (ep.activation != kActNone) {
             __syncthreads();  // every wavefront's loads have landed: the ring is free
             static_assert(kR * kC * kWaves * 4096 <= S::kLdsBytes, "a tile of results is 4 KB");
@@ -1942,39 +1944,50 @@ size_t gemm_q4k_most_bytes(size_t rows, size_t in_dim, size_t out_dim) {
 
 // The plan of a call that lends `room` bytes (splits = 0: none fits).  Whoever lends gemm_q4k_workspace_bytes or more gets the
 // same one: the choice is over what fits, and the best of all that fits the most a call may take is the best of fewer.
-// `pair`: for both matrices of a pair in one launch (one share); its tile may be another than the single call's, as a result's bits
-// depend on the shares alone (333 x 4096 x 14336 twice: 64 x 256 tiles 212 us, 64 x 128 231; once 124 / 119).
-// Up to 64 rows the bf16 kernel is the faster one (64 x 4096 x 4096 17.5 against 19.4 us, 32 x 4096 x 14336 21.4 / 22.4).  Above, the
-// tile and share count that cost least -- one share where that costs at most 3 % more, since a pair is one launch then -- unless the
-// bf16 kernel is expected within 3 % of it (small matrices: 200 x 2048 x 2048 17.3 against 20.4; 333 x 2048 x 5632 36.9 / 40.6, a
-// grid that just fills its rounds).
+// A result's bits depend on the shares alone, and a pair's halves have the single call's, while a pair is one launch on one share only.
+// Columns of at least twice K, which mostly come in pairs (gate and up): a quarter of the pair's time counts beside the call's own
+// (99 x 2816 x 9728 twice: one share 51 us, two 59, a call 29.7 and 28.8; 99 x 2048 x 4096 a call 17.4 on the bf16 kernel's shares and 21
+// on one of the 6-bit kernel's).  Other shapes: the call's own, one share where that costs at most 3 % more.
+// `pair`: the tile may be another than the single call's (333 x 4096 x 14336 twice: 64 x 256 tiles 212 us, 64 x 128 231; once 124 / 119).
+// An activation is sixteen values and more a lane of the matrix kernels, about 3 us, and one a thread of the reduce launch: a third of
+// that is counted (65 x 1024 x 4096 plain 13.7 us on the bf16 kernel's shares and 13.3 on one of the 6-bit kernel's, with gelu 14.5 and 16.7).
+// Up to 64 rows the bf16 kernel is the faster one (64 x 4096 x 4096 17.5 against 19.4 us, 32 x 4096 x 14336 21.4 / 22.4), above where it is
+// expected within 3 %.
+constexpr double kEpilogueUs = 1.0;
 Q4kGemmPlan gemm_q4k_plan(size_t rows, size_t in_dim, size_t out_dim, size_t room, bool pair = false) {
     const double m = static_cast<double>(rows), k = static_cast<double>(in_dim), n = static_cast<double>(out_dim);
     room = std::min(room, gemm_q4k_most_bytes(rows, in_dim, out_dim));
     auto fits = [&](const Q4kGemmPlan& p) { return gemm_q4k_plan_bytes(p, rows, in_dim, out_dim) <= room; };
     const Q4kGemmPlan none{kParts, 0}, parts = gemm_q4k_parts_plan(rows, in_dim, out_dim);
     if (rows <= 64) return fits(parts) ? parts : none;
-    Q4kGemmPlan best = none;
-    double best_us = 1e30;
+    Q4kGemmKind pair_kind = kFp6Tile64x256;  // of one share
+    double pair_us = 1e30;
     for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
-        for (int s = 1; s <= 8; ++s) {
-            if (!gemm_q4k_shares_allowed(s, in_dim)) continue;
+        if (const double us = kQ4kGemmCosts[kind].us(m, k, 2 * n, 1); us < pair_us) {
+            pair_us = us;
+            pair_kind = static_cast<Q4kGemmKind>(kind);
+        }
+    auto cost = [&](const Q4kGemmPlan& plan) {
+        const double epilogue = plan.splits == 1 ? kEpilogueUs : 0.0;
+        const double us = kQ4kGemmCosts[plan.kind].us(m, k, n, plan.splits) * (plan.kind == kParts ? 0.97 : 1.0) + epilogue;
+        if (out_dim < 2 * in_dim) return us * (plan.kind != kParts && plan.splits > 1 ? 1.03 : 1.0);
+        const bool together = plan.kind != kParts && plan.splits == 1;
+        return us + 0.25 * (together ? pair_us + epilogue : 2 * us - kQ4kGemmCosts[plan.kind].split * m * k * 1e-6);
+    };
+    Q4kGemmPlan best = none;
+    double best_cost = 1e60;
+    for (int s = 1; s <= 8; ++s) {
+        if (!gemm_q4k_shares_allowed(s, in_dim)) continue;
+        for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind) {
             const Q4kGemmPlan plan{static_cast<Q4kGemmKind>(kind), s};
-            const double us = kQ4kGemmCosts[kind].us(m, k, n, s) * (s == 1 ? 1.0 : 1.03);
-            if (us < best_us && fits(plan)) {
-                best_us = us;
+            if (const double c = cost(plan); c < best_cost && fits(plan)) {
+                best_cost = c;
                 best = plan;
             }
         }
-    if (fits(parts) && kQ4kGemmCosts[kParts].us(m, k, n, parts.splits) * 0.97 < best_us) return parts;
-    if (pair && best.splits == 1) {
-        best_us = 1e30;
-        for (int kind = kFp6Tile64x256; kind <= kFp6Tile32x128; ++kind)
-            if (const double us = kQ4kGemmCosts[kind].us(m, k, 2 * n, 1); us < best_us) {
-                best_us = us;
-                best.kind = static_cast<Q4kGemmKind>(kind);
-            }
     }
+    if (fits(parts) && cost(parts) < best_cost) return parts;
+    if (pair && best.splits == 1) best.kind = pair_kind;
     return best;
 }
 

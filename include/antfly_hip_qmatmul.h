@@ -154,7 +154,9 @@ int afhip_uses_q8k_activation_quant(int tensor_type, size_t rows, size_t in_dim,
  * is a successful no-op.  The result buffers must not overlap the activations, the
  * weights, the workspace or each other (every workgroup reads all of X while others
  * already write Y, and some launches clear Y before they read X), as in the
- * reference, whose launchers write a freshly allocated output.
+ * reference, whose launchers write a freshly allocated output.  An overlap is not
+ * refused, and some launches that notice a result over X take kernels which have read X
+ * by then, but nothing is promised for such calls.
  * ---------------------------------------------------------------------- */
 
 /* Bytes of device scratch a launch needs (quantized activations for the
