@@ -1489,7 +1489,8 @@ __global__ __launch_bounds__(64 * kWaves, kOcc) void gemm_q4k_fp6_kernel(
     // a result does not depend on the workgroup's tile.  Without this a channel 2^16 times the others, on weights that are zero,
     // would cost 1.8e-7 of a row's largest result, at 2^20 3.3e-6, at 2^30 3e-3.  us before / with this: 512 x 4096 x 14336 141.6 / 141.3, 333 x 14336
     // x 4096 120.4 / 119.7; weights of random bytes, where a 64th of the mins is zero, 148 / 174 and 125 / 146.
-    // (a tile's columns past the matrix are zeros, which are below every line: they do not count.  us, counted / not: a pair of 130 x 14336 x 1877 115 / 100, 917 x 1024 x 1512 32.3 / 29.5)
+    // (a tile's columns past the matrix are zeros, which are below every line: they do not count.  us, counted / not: a pair of
+    // 130 x 14336 x 1877 115 / 100, 917 x 1024 x 1512 32.3 / 29.5)
     bool below = false;
 #pragma unroll
     for (int j = 0; j < kC; ++j)
