@@ -238,8 +238,11 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
         // (which reads no workspace; the stand-alone quantizer writes the Q8_K rows there)
         if (!fused && (workspace.ptr == 0 || workspace.ptr % 16 != 0 || workspace.len < q4k_q8k_workspace_bytes(rows, in_dim)))
             return AFHIP_ERR_INVALID_STATE;
+        // small calls of the matrix-core form likewise, where no result lies over X, which its workgroups read while others store
+        auto apart = [&](const afhip_buffer& y) { return y.ptr == 0 || y.ptr + out_count * 4 <= input.ptr || input.ptr + in_count * 4 <= y.ptr; };
+        const bool fused_rows = tiled && !fused && linear_q4k_q8k_rows_fuses_quantizer(rows, in_dim, out_dim, pair ? 2 : 1) && apart(dst) && apart(dst_b);
         if (counters) counters->activation_quant++;
-        hipError_t e = fused ? hipSuccess
+        hipError_t e = fused || fused_rows ? hipSuccess
                              : launch_quantize_q8k(stream, reinterpret_cast<const float*>(input.ptr), static_cast<int>(rows),
                                                    static_cast<int>(in_dim), reinterpret_cast<void*>(workspace.ptr));
         for (int i = 0; e == hipSuccess && i < (pair ? 2 : 1); ++i) {
@@ -256,6 +259,9 @@ static afhip_status linear_q4k_impl(hipStream_t stream, int layout, afhip_buffer
             if (fused)
                 e = launch_linear_q4k_q8k_fused(stream, y, reinterpret_cast<const float*>(input.ptr), w, static_cast<int>(rows),
                                                 static_cast<int>(in_dim), static_cast<int>(out_dim), ep, y_b, w_b, ep_b);
+            else if (fused_rows)
+                e = launch_linear_q4k_q8k_fused_rows(stream, y, reinterpret_cast<const float*>(input.ptr), w, static_cast<int>(rows),
+                                                     static_cast<int>(in_dim), static_cast<int>(out_dim), ep, y_b, w_b, ep_b);
             else
                 e = launch_linear_q4k_q8k(stream, y, reinterpret_cast<const void*>(workspace.ptr), w, tiled, static_cast<int>(rows),
                                           static_cast<int>(in_dim), static_cast<int>(out_dim), ep, y_b, w_b, ep_b);
@@ -349,11 +355,23 @@ afhip_status linear_triple_impl(void* stream_v, const afhip_buffer (&dst)[3], af
         const int kind = afhip_quant_matmul_select(rows, in_dim, out_dim, AFHIP_FORMAT_Q4_K);
         (kind == AFHIP_DISPATCH_MMV ? counters->mmv : kind == AFHIP_DISPATCH_SMALL_BATCH ? counters->small_batch : counters->mm) += 3;
     }
+    Epilogue ep[3];
+    bool fused = linear_q4k_q8k_rows_fuses_quantizer(rows, in_dim, out_dim, 3);
+    for (int i = 0; i < 3; ++i) {
+        ep[i].bias = reinterpret_cast<const float*>(bias[i].ptr);
+        fused = fused && (dst[i].ptr + y_bytes <= input.ptr || input.ptr + rows * in_dim * 4 <= dst[i].ptr);
+    }
+    if (fused) {
+        const hipError_t e = launch_linear_q4k_q8k_fused_rows(
+            stream, reinterpret_cast<float*>(dst[0].ptr), reinterpret_cast<const float*>(input.ptr), reinterpret_cast<const uint8_t*>(weight[0].ptr),
+            static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), ep[0], reinterpret_cast<float*>(dst[1].ptr),
+            reinterpret_cast<const uint8_t*>(weight[1].ptr), ep[1], reinterpret_cast<float*>(dst[2].ptr),
+            reinterpret_cast<const uint8_t*>(weight[2].ptr), ep[2]);
+        return e == hipSuccess ? AFHIP_OK : static_cast<afhip_status>(e);
+    }
     hipError_t e = launch_quantize_q8k(stream, reinterpret_cast<const float*>(input.ptr), static_cast<int>(rows), static_cast<int>(in_dim),
                                        reinterpret_cast<void*>(workspace.ptr));
     if (e != hipSuccess) return static_cast<afhip_status>(e);
-    Epilogue ep[3];
-    for (int i = 0; i < 3; ++i) ep[i].bias = reinterpret_cast<const float*>(bias[i].ptr);
     e = launch_linear_q4k_q8k(stream, reinterpret_cast<float*>(dst[0].ptr), reinterpret_cast<const void*>(workspace.ptr),
                               reinterpret_cast<const uint8_t*>(weight[0].ptr), true, static_cast<int>(rows), static_cast<int>(in_dim),
                               static_cast<int>(out_dim), ep[0], reinterpret_cast<float*>(dst[1].ptr),

@@ -827,6 +827,145 @@ __global__ __launch_bounds__(768) void linear_q4k_q8k_mfma_kernel(float* __restr
     }
 }
 
+// The same with the quantizer inside, for calls that are one round of small workgroups: sixteen rows x 32 columns, wavefront w
+// quantizes super-block w of the workgroup's rows (a row a load, four values a lane, the maxima of sixteen rows reduced together), hands
+// the bytes round in LDS and multiplies them as above -- the same values in the same order, so the bits of the two launches.  What a
+// workgroup quantizes every column tile quantizes again; against that stand the launch and the trip to memory of the quantizer's.
+// Sixteen rows and not 32: the quantizer's vector work (560 instructions a wavefront) is what the launch waits for, and small calls have
+// compute units to spare for it.  us a call as a graph node, against the two launches: 77 x 768 x 768 8.1 -> 5.3, 77 x 768 x 3072 8.6 ->
+// 7.4, 77 x 3072 x 768 10.3 -> 8.5, 50 x 512 x 2048 8.0 -> 5.5, 64 x 2048 x 2048 8.5 -> 6.7; an encoder's layers (77 rows, launched one by
+// one, where a launch costs the host 3.6 us) 168 -> 126 a pass.
+constexpr int kQ8kFusedRows = 16;
+constexpr int kQ8kStageRow = kQ4kBlockValues + 16;                       // bytes: sixteen rows' fragments in different banks
+constexpr int kQ8kStageBytes = kQ8kFusedRows * kQ8kStageRow;             // of a wavefront, its sums in the same place afterwards
+static_assert(kQ8kStageBytes >= 8 * 64 * 4, "room for the sums");
+
+__global__ __launch_bounds__(768) void linear_q4k_q8k_fused_rows_kernel(float* __restrict__ dst, const float* __restrict__ x,
+                                                                       const uint8_t* __restrict__ weight, int rows, int in_dim, int out_dim,
+                                                                       Epilogue ep, Q8kSecond second, Q8kSecond third) {
+    if (blockIdx.z != 0) {
+        dst = blockIdx.z == 1 ? second.dst : third.dst;
+        weight = blockIdx.z == 1 ? second.weight : third.weight;
+        ep = blockIdx.z == 1 ? second.ep : third.ep;
+    }
+    extern __shared__ __align__(16) unsigned char q8k_lds[];
+    const int kb = in_dim / kQ4kBlockValues;
+    const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int tile = blockIdx.x, row0 = blockIdx.y * kQ8kFusedRows;
+    unsigned char* const own = q8k_lds + wave * kQ8kStageBytes;
+    float* const xd_s = reinterpret_cast<float*>(q8k_lds + kb * kQ8kStageBytes) + wave * kQ8kFusedRows;
+
+    float4 v[kQ8kFusedRows];
+#pragma unroll
+    for (int r = 0; r < kQ8kFusedRows; ++r)  // (rows past the end repeat the last one and are not stored)
+        v[r] = reinterpret_cast<const float4*>(x + static_cast<size_t>(min(row0 + r, rows - 1)) * in_dim + wave * kQ4kBlockValues)[lane];
+    const uint8_t* tbase = weight + (static_cast<size_t>(tile) * kb + wave) * (32 * kQ4kBlockBytes);
+    const q4k_u32x4 header = *reinterpret_cast<const q4k_u32x4*>(tbase + c * 16);
+    q4k_u32x4 nib[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) nib[t] = *reinterpret_cast<const q4k_u32x4*>(tbase + 512 + t * 1024 + lane * 16);
+
+    // The maximum of every row: over sixteen lanes for each, then two and four rows a register.
+    float m[kQ8kFusedRows];
+#pragma unroll
+    for (int r = 0; r < kQ8kFusedRows; ++r) {
+        m[r] = fmaxf(fmaxf(fabsf(v[r].x), fabsf(v[r].y)), fmaxf(fabsf(v[r].z), fabsf(v[r].w)));
+        m[r] = max_over_8(m[r]);
+        m[r] = fmaxf(m[r], dpp_move<kDppRowMirror>(m[r]));
+    }
+    float four[kQ8kFusedRows / 4];  // sixteen lanes k: row 4 q + k
+#pragma unroll
+    for (int q = 0; q < kQ8kFusedRows / 4; ++q) {
+        float two[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const auto swapped = __builtin_amdgcn_permlane16_swap(__float_as_uint(m[4 * q + 2 * h]), __float_as_uint(m[4 * q + 2 * h + 1]), false, false);
+            two[h] = fmaxf(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
+        }
+        const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(two[0]), __float_as_uint(two[1]), false, false);
+        four[q] = fmaxf(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
+    }
+    const float peak = lane & 2 ? (lane & 1 ? four[3] : four[2]) : (lane & 1 ? four[1] : four[0]);  // of row 4 (lane % 4) + lane / 16
+    const float scale = act_scale(peak);
+    const float inverse = peak == 0.0f ? 0.0f : 1.0f / scale;
+    if ((lane & 15) < 4) xd_s[4 * (lane & 3) + (lane >> 4)] = scale;
+#pragma unroll
+    for (int r = 0; r < kQ8kFusedRows; ++r) {
+        const float inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inverse), 16 * (r & 3) + (r >> 2)));
+        const uint32_t q0 = act_quant(v[r].x, inv), q1 = act_quant(v[r].y, inv), q2 = act_quant(v[r].z, inv), q3 = act_quant(v[r].w, inv);
+        const uint32_t low = __builtin_amdgcn_perm(q1, q0, 0x0C0C0400u), high = __builtin_amdgcn_perm(q3, q2, 0x0C0C0400u);
+        *reinterpret_cast<uint32_t*>(own + r * kQ8kStageRow + lane * 4) = low | high << 16;
+    }
+    // (a wavefront reads back what its own lanes wrote: LDS operations of a wavefront complete in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    q8k_v4i a[8];
+#pragma unroll
+    for (int sub = 0; sub < 8; ++sub)
+        a[sub] = *reinterpret_cast<const q8k_v4i*>(own + (c & (kQ8kFusedRows - 1)) * kQ8kStageRow + sub * 32 + g * 16);
+    float xd[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xd[i] = xd_s[8 * (i >> 2) + 4 * g + (i & 3)];
+
+    float dsc[8], dmn[8];
+    {
+        const float d = half_bits_to_f32(static_cast<uint16_t>(header.x & 0xFFFFu));
+        const float dmin = half_bits_to_f32(static_cast<uint16_t>(header.x >> 16));
+#pragma unroll
+        for (int sub = 0; sub < 8; ++sub) {
+            float sc, mn;
+            q4k_scale_min(header, sub, &sc, &mn);
+            dsc[sub] = d * sc;
+            dmn[sub] = dmin * mn;
+        }
+    }
+    q8k_v16f part = {};
+#pragma unroll
+    for (int sub = 0; sub < 8; ++sub) {
+        if ((sub & 1) == 0) {
+            // the sums of sub-blocks sub and sub + 1: a lane's half of each, then lane half g has the whole of sub + g
+            uint32_t half_sum[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                int t = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) t = dot4(a[sub + h][i], 0x01010101, t);
+                half_sum[h] = static_cast<uint32_t>(t);
+            }
+            const auto swapped = __builtin_amdgcn_permlane32_swap(half_sum[0], half_sum[1], false, false);
+            const int total = static_cast<int>(swapped[0] + swapped[1]);
+            part = __builtin_amdgcn_mfma_f32_32x32x2f32(static_cast<float>(total), g ? -dmn[sub + 1] : -dmn[sub], part, 0, 0, 0);
+        }
+        const q4k_u32x4 p = nib[sub >> 1];
+        const int sh = (sub & 1) * 4;  // low nibbles = sub-block 2t, high nibbles = 2t + 1
+        const q8k_v4i b = {static_cast<int>((p.x >> sh) & 0x0F0F0F0Fu), static_cast<int>((p.y >> sh) & 0x0F0F0F0Fu),
+                           static_cast<int>((p.z >> sh) & 0x0F0F0F0Fu), static_cast<int>((p.w >> sh) & 0x0F0F0F0Fu)};
+        const q8k_v16i zero = {};
+        const q8k_v16i dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[sub], b, zero, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) part[i] = __builtin_fmaf(dsc[sub], static_cast<float>(dot[i]), part[i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float* const sums = reinterpret_cast<float*>(own);  // [8][64]: the fragments have been read
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sums[i * 64 + lane] = xd[i] * part[i];
+    __syncthreads();
+    for (int i = tid; i < 512; i += threads) {
+        float total = 0.0f;
+        for (int w = 0; w < kb; ++w) total += reinterpret_cast<const float*>(q8k_lds + w * kQ8kStageBytes)[i];
+        const int reg = i >> 6, l = i & 63;
+        const int r = row0 + 8 * (reg >> 2) + 4 * (l >> 5) + (reg & 3), n = tile * 32 + (l & 31);
+        if (r < rows && n < out_dim) {
+            const size_t at = static_cast<size_t>(r) * out_dim + n;
+            dst[at] = finish_output(ep, n, at, total);
+        }
+    }
+}
+
 // int8 [rows][in_dim] (padded to 256 bytes), f32 d [rows][in_dim / 256], int32 sums [rows][in_dim / 32]
 size_t q4k_q8k_workspace_bytes(size_t rows, size_t in_dim) {
     return (rows * in_dim + 255) / 256 * 256 + rows * (in_dim / 256) * 4 + rows * (in_dim / 32) * 4;
@@ -914,6 +1053,29 @@ hipError_t launch_linear_q4k_q8k_fused(hipStream_t stream, float* dst, const flo
     else if (rows == 2) AFHIP_Q8K_FUSED(2);
     else AFHIP_Q8K_FUSED(4);
 #undef AFHIP_Q8K_FUSED
+    return hipGetLastError();
+}
+
+// Whether the matrix-core form quantizes in the matmul launch: up to eight wavefronts a compute unit, two on a SIMD.  Past that the
+// repeated quantizing costs more than its launch (us, fused / two launches; wavefronts a unit): 64 x 2048 x 2048 (8) 6.7 / 8.5, 514 x 512 x
+// 512 (4.1) 7.3 / 8.6, but 197 x 768 x 3072 (14.6) 11.8 / 10.7, 154 x 1536 x 1536 (11) 10.8 / 8.8, 514 x 768 x 3072 (37) 24.4 / 15.2.
+constexpr size_t kQ8kFusedWaves = 8;
+bool linear_q4k_q8k_rows_fuses_quantizer(size_t rows, size_t in_dim, size_t out_dim, int matrices) {
+    const size_t groups = (rows + kQ8kFusedRows - 1) / kQ8kFusedRows, tiles = (out_dim + 31) / 32;
+    return linear_q4k_q8k_shares_launch(true, rows, in_dim) && groups <= 65535 &&
+           groups * tiles * static_cast<size_t>(matrices) * (in_dim / kQ4kBlockValues) <= kQ8kFusedWaves * static_cast<size_t>(gemv_compute_units());
+}
+
+hipError_t launch_linear_q4k_q8k_fused_rows(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
+                                            int out_dim, const Epilogue& ep, float* dst_b, const uint8_t* weight_b, const Epilogue& ep_b,
+                                            float* dst_c, const uint8_t* weight_c, const Epilogue& ep_c) {
+    if (rows == 0 || out_dim == 0) return hipSuccess;
+    const int kb = in_dim / kQ4kBlockValues;
+    const size_t lds = static_cast<size_t>(kb) * (kQ8kStageBytes + kQ8kFusedRows * 4);
+    static_assert(12 * (kQ8kStageBytes + kQ8kFusedRows * 4) <= 64 * 1024, "no raised LDS limit");
+    hipLaunchKernelGGL(linear_q4k_q8k_fused_rows_kernel,
+                       dim3((out_dim + 31) / 32, (rows + kQ8kFusedRows - 1) / kQ8kFusedRows, dst_c ? 3 : (dst_b ? 2 : 1)), dim3(64 * kb), lds, stream, dst,
+                       x, weight, rows, in_dim, out_dim, ep, Q8kSecond{dst_b, weight_b, ep_b}, Q8kSecond{dst_c, weight_c, ep_c});
     return hipGetLastError();
 }
 

@@ -400,6 +400,45 @@ def test_q8k_route_pair_and_bias():
     assert np.array_equal(yb2, ya + bias[None, :])
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim,pair", [
+    (50, 512, 512, True), (77, 768, 777, False), (64, 2048, 2048, False), (50, 3072, 513, False),  # column remainders, twelve wavefronts
+    (514, 512, 512, False), (231, 512, 550, True), (50, 2048, 2049, False)])  # a last group of two rows; the last: past the line, two launches
+def test_q8k_rows_quantized_by_the_matmul_launch(rows, in_dim, out_dim, pair):
+    """Small calls quantize X inside the matmul launch; a call whose result lies over X keeps the quantizer's own launch.  Both give
+    the same bits: zero super-blocks, large and small ones, infinities and NaNs among them."""
+    print(f"case: q4_k q8k rows, quantizer inside rows={rows} in={in_dim} out={out_dim} pair={pair}", flush=True)
+    x = synth.activations(811 + rows, rows, in_dim)
+    x[1, :256] = 0.0
+    x[2, 256:] *= np.float32(1e-30)
+    x[3, 7] = 1e30
+    x[rows - 1, 5], x[rows - 2, 3] = np.inf, np.nan
+    w = [synth.weights(Q4K, 812 + i, out_dim, in_dim) for i in range(2 if pair else 1)]
+    wd = [G.prepare(Q4K, each, out_dim, in_dim) for each in w]
+    ws = torch.empty(kernels.workspaceBytes(Q4K, rows, in_dim, out_dim), dtype=torch.uint8, device=G.DEV)
+    room = torch.empty(rows * (in_dim + out_dim), dtype=torch.float32, device=G.DEV)
+    second = torch.empty(rows * out_dim, dtype=torch.float32, device=G.DEV)
+    results = []
+    for at in (rows * in_dim, 0):  # behind X, in X's place
+        room.fill_(float("nan"))
+        second.fill_(float("nan"))
+        room[:rows * in_dim] = torch.from_numpy(x.ravel()).to(G.DEV)
+        xd, y = room[:rows * in_dim], room[at:at + rows * out_dim]
+        if pair:
+            kernels.launchLinearPairF32(G.stream(), Q4K, PREP, G.buf(y), G.buf(second), G.buf(xd), G.buf(wd[0]), G.buf(wd[1]), rows, in_dim,
+                                        out_dim, G.buf(ws))
+        else:
+            kernels.launchLinearF32(G.stream(), Q4K, PREP, G.buf(y), G.buf(xd), G.buf(wd[0]), rows, in_dim, out_dim, G.buf(ws))
+        torch.cuda.synchronize()
+        results.append([t.cpu().numpy().view(np.uint32).reshape(rows, out_dim) for t in ((y, second) if pair else (y,))])
+    finite = np.r_[0:rows - 2]
+    for inside, apart in zip(*results):
+        assert np.array_equal(inside[finite], apart[finite])
+        assert np.array_equal(np.isfinite(inside.view(np.float32)), np.isfinite(apart.view(np.float32)))
+    sample = np.r_[0:4, rows - 3]
+    ref = O.linear_q4_k_q8k(x[sample], w[0], len(sample), in_dim, out_dim)
+    assert G.max_rel_err(results[0][0].view(np.float32)[sample], ref.astype(np.float64)) <= 2e-5
+
+
 @pytest.mark.parametrize("rows,in_dim,out_dim", [(50, 512, 513), (64, 768, 2304), (77, 3072, 769), (154, 1536, 640), (514, 2048, 545)])
 def test_q8k_route_on_the_matrix_cores(rows, in_dim, out_dim):
     """More than nine rows of the gated shapes: part tiles of rows (50 = 32 + 18, 77, 154, 514) and columns, two to twelve
