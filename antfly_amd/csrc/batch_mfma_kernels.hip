@@ -32,9 +32,12 @@
 //     batch8_mfma_kernel (further down): the 16x16x64 MFMA on two blocks at once, tiles of 8 .. 64
 //     columns, weights requested two stages ahead instead of all at once, a long K in at most two
 //     shares where that is possible.
-//   * Nine to 64 rows whose 64-column tiles times K shares make a grid of five eighths to all of
-//     the compute units take batch32_mfma_kernel (further down): this kernel's arithmetic, staged
-//     weight requests, one workgroup per compute unit.
+//   * Nine to 64 rows take batch_groups_mfma_kernel (further down) on most shapes: this kernel's
+//     arithmetic, 32 rows a workgroup whose operands stay in registers while it walks over groups
+//     of columns, one workgroup per compute unit.
+//   * Those that do not, and whose 64-column tiles times K shares make a grid of five eighths to
+//     all of the compute units, take batch32_mfma_kernel (further down): this kernel's arithmetic,
+//     staged weight requests, one workgroup per compute unit.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -66,6 +69,21 @@ struct BmFormat {
     static constexpr int kShareBlocks = kBmWaves * kWaveBlocks;            // 128 / 64
 };
 
+// Column-group kernel.  A stage is the weights and scales of 32 columns and kStageBlocks blocks, 5 KB; kHalves stages are a wavefront's part of
+// the workgroup's share of K, which kParts wavefronts share out (the others take other columns).  LDS: a ring of stages for each
+// wavefront, the room where the sums meet, and two counters.
+template <int kType, int kLive, int kHalves, int kParts>
+struct BatchGroups {
+    static constexpr int kStageBlocks = kType == 2 ? 8 : 4;
+    static constexpr int kRun = kParts * kStageBlocks;  // consecutive blocks that the wavefronts' stages share out
+    static constexpr int kSlots = 3, kSlotBytes = 5120;
+    static constexpr int kGroupCols = 32 * (kBmWaves / kParts);  // columns the workgroup works on at a time
+    static constexpr int kSumsAt = kBmWaves * kSlots * kSlotBytes, kCountersAt = kSumsAt + kBmWaves * kLive * 256;
+    static constexpr int kLdsBytes = kCountersAt + 16;
+    static constexpr int kSets = kHalves == 4 ? 1 : 2;  // register sets of MFMA results
+    static_assert(kLdsBytes <= 160 * 1024, "LDS");
+};
+
 // One 64-lane load from global memory straight into LDS: lane l's 16 bytes at base + voff land
 // at lds_addr + 16 * l.  Inline assembly: the compiler does not track these loads, which is why
 // the kernel waits for them by hand before anything reads the LDS region.
@@ -73,7 +91,12 @@ __device__ __forceinline__ void bm_lds_load16(const void* base, uint32_t voff, u
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
 }
 
-extern __shared__ __align__(16) unsigned char bm_lds[];
+// the same where other workgroups are about to read the bytes too (no streaming hint)
+__device__ __forceinline__ void bm_lds_load16_kept(const void* base, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
+}
+
+extern __shared__ __align__(1024) unsigned char bm_lds[];  // (operand addresses inside rows of 128 bytes are formed by XOR)
 
 // the second matrix of a pair launch (grid.z == 2)
 struct BmSecond {
@@ -1172,15 +1195,385 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch32_mfma_kernel(float* __re
             const int m = rt * 32 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3);
             const int n = n0 + 32 * cg + (l & 31);
             if (m < rows && n < out_dim) {
-                float sum = red[i];
+                float half[2];
 #pragma unroll
-                for (int w = 1; w < kBmWaves; ++w) sum += red[w * kItems + i];
+                for (int h = 0; h < 2; ++h) {  // (batch_mfma_kernel's order, for the same bits)
+                    half[h] = red[(kBmWaves / 2) * h * kItems + i];
+#pragma unroll
+                    for (int w = 1; w < kBmWaves / 2; ++w) half[h] += red[((kBmWaves / 2) * h + w) * kItems + i];
+                }
+                const float sum = half[0] + half[1];
                 const size_t at = static_cast<size_t>(m) * out_dim + n;
                 if (partial != nullptr) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = sum;
                 else if (accumulate) unsafeAtomicAdd(dst + at, sum);  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
                 else dst[at] = finish_output(ep, n, at, sum);
             }
         }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Nine to 64 rows, one round of workgroups, a compute unit each: a workgroup takes 32 rows and walks over as many groups of 32 (64)
+// columns as that round needs, its operand fragments staying in registers.  The arithmetic is the kernels' above; what is
+// different is what stands around it, which is what such calls spend their time on:
+//   * K is shared out over the wavefronts in runs: every wavefront fetches its fragments once, whatever the number of columns, the first
+//     run's ahead of everybody's other requests;
+//   * weights and scales (from the tile-order copy: one request brings 32 columns') go through a ring of three stages in LDS that nothing
+//     but hand-counted waits stands before;
+//   * the matrix instructions of a pair of blocks leave between the conversions and multiply-adds of the pair before (two sets of result
+//     registers; runs of four stages, whose fragments fill the registers, keep one set);
+//   * the wavefronts' sums meet in LDS behind counters, half a column group later: no barrier in the loop.
+// Bound by the vector unit beside the matrix unit, about 200 SIMD cycles per 32 x 32 outputs and block (176 by the instructions alone), and
+// by the first bytes' way from memory, 5000 cycles until a wavefront can start.  Q4_0, weights from memory, against the two kernels above
+// (us): 32 rows, K = 4096, 4096 columns 10.5 -> 9.8, 6144 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8; 48 rows, 2048 x 2048 11.9 -> 7.4;
+// 64 rows, a pair of 14336 columns 51.0 -> 35.6.
+template <int kType, int kLive, int kHalves, int kParts, bool kApart, bool kShared, bool kOne>
+__global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float* __restrict__ dst_a, float* __restrict__ partial_a,
+                                                                      const uint32_t* __restrict__ qa, const float* __restrict__ sa,
+                                                                      const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
+                                                                      int share_blocks, int row_groups, int col_groups, Epilogue ep_a,
+                                                                      BmSecond second, int accumulate) {
+    using B = BatchGroups<kType, kLive, kHalves, kParts>;
+    const bool is_b = blockIdx.z != 0;
+    float* dst = is_b ? second.dst : dst_a;
+    const uint8_t* weight = is_b ? second.weight : weight_a;
+    const Epilogue ep = is_b ? second.ep : ep_a;
+    float* partial = partial_a == nullptr ? nullptr : partial_a + (is_b ? static_cast<size_t>(gridDim.y) * rows * out_dim : 0);
+    constexpr int kQB = kType == 2 ? 16 : 32, kHB = B::kStageBlocks, kPairs = kHB / 2, kRun = B::kRun;
+    constexpr int kSlots = B::kSlots, kSets = B::kSets, kSteps = kHalves * kPairs;
+    static_assert(kSteps % 2 == 0, "the two register sets alternate over a column group");
+    const int kb_full = in_dim >> 5;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lj = lane & 31, lh = lane >> 5;
+    // row groups of the same columns on one XCD (workgroup ids go round-robin over the eight), so that an L2 reads a weight once
+    int col_tile = blockIdx.x, group = 0;
+    if (kShared) {
+        const int slot = blockIdx.x >> 3;
+        group = slot % row_groups;
+        col_tile = slot / row_groups * 8 + (blockIdx.x & 7);
+    }
+    const int n_first = col_tile * B::kGroupCols * (kOne ? 1 : col_groups);
+    if (n_first >= out_dim) return;
+    const int groups_here = kOne ? 1 : min(col_groups, (out_dim - n_first + B::kGroupCols - 1) / B::kGroupCols);
+    const int padded = row_groups * 32, row0 = group * 32;
+    const int share_begin = static_cast<int>(blockIdx.y) * share_blocks;
+    const int share_end = min(share_begin + share_blocks, kb_full);
+    const int part = wave % kParts, side = wave / kParts;  // of K; of the group's columns
+    // Run hb of this wavefront is the kHB blocks first_of(hb) + [0, kHB).  Two runs follow on each other, a slice of blocks as
+    // batch_mfma_kernel's; four, and those whose sums are kept apart, are a row of all wavefronts' each.  Indices past the end are
+    // clamped to a valid block for every load; their activation scales are zero.
+    auto first_of = [&](int hb) { return share_begin + (kHalves == 2 && !kApart ? (part * 2 + hb) * kHB : hb * kRun + part * kHB); };
+    auto clamp_blk = [&](int hb, int j) { return min(first_of(hb) + j, share_end - 1); };
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(bm_lds)));
+    const uint32_t lds_slots = lds0 + wave * (kSlots * B::kSlotBytes);
+
+    auto load16 = [&](const uint8_t* base, uint32_t off, uint32_t at) {
+        if (kShared) bm_lds_load16_kept(base, off, at);
+        else bm_lds_load16(base, off, at);
+    };
+    // Requests of a stage: the columns' whole 128-byte lines (eight lanes each), chunk slots XOR-swizzled by the column; the scales in
+    // the tile order (tile_scale_index) -- of a tile of four (Q8_0: two) columns and 128 blocks the stage's blocks are 128 (64) bytes on
+    // end, so one request brings those of 32 columns -- in 16-byte units XOR-swizzled by the tile.
+    const size_t blocks_total = static_cast<size_t>(out_dim) * kb_full;
+    const uint8_t* scale_tiles = weight + ((blocks_total * (kQB + 2) + 15) & ~static_cast<size_t>(15));
+    constexpr int kTileCols = kType == 2 ? 4 : 2, kTileBytes = kType == 2 ? 1024 : 512, kUnits = kType == 2 ? 8 : 4;
+    const int slices = (kb_full + 127) >> 7, last_tile = (out_dim - 1) / kTileCols;
+    // (a unit of eight columns is eight times the row pitch on, its chunks an XOR by four in the odd ones: two offsets a lane serve every
+    // stage but those at the matrix's last columns)
+    const int c8 = lane >> 3, s8 = lane & 7;
+    const uint32_t pitch = static_cast<uint32_t>(kb_full) * kQB;
+    const int unit_tile = lane / kUnits, unit_at = (lane % kUnits) ^ (kType == 2 ? unit_tile >> 1 : unit_tile >> 2);
+    const uint32_t weights_at = c8 * pitch + (s8 ^ (c8 >> 1)) * 16;  // (the pitch is a multiple of 128)
+    const uint32_t scales_lane = static_cast<uint32_t>(unit_tile * slices) * kTileBytes + unit_at * 16;
+    auto issue = [&](int cg, int hb, int slot) {
+        const int n0 = min(n_first + cg * B::kGroupCols + side * 32, out_dim - 1) & ~31;  // (a side past the matrix repeats its last columns)
+        const uint32_t at = lds_slots + slot * B::kSlotBytes;
+        const int first = min(first_of(hb), share_end - kHB);  // (shares and K are whole stages; what is read for one past the end counts for nothing)
+        const uint8_t* sbase = scale_tiles + (static_cast<size_t>(n0 / kTileCols) * slices + (first >> 7)) * kTileBytes + (first & (kType == 2 ? 63 : 31)) * 16;
+        const uint8_t* wbase = weight + static_cast<size_t>(n0) * pitch + static_cast<size_t>(first) * kQB;
+        if (n0 + 32 <= out_dim) {
+            load16(sbase, scales_lane, at + 4096);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) load16(wbase + static_cast<size_t>(8 * u) * pitch, weights_at ^ (u & 1 ? 64u : 0u), at + u * 1024);
+        } else {  // rows clamped to the matrix
+            int l = lane;
+            asm volatile("" : "+v"(l));  // (nothing of this takes registers in the loop)
+            const int t = l / kUnits, tile = min(t, last_tile - n0 / kTileCols);
+            load16(sbase, static_cast<uint32_t>(tile * slices) * kTileBytes + ((l % kUnits) ^ (kType == 2 ? t >> 1 : t >> 2)) * 16, at + 4096);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int c = 8 * u + (l >> 3);
+                load16(wbase, static_cast<uint32_t>(min(c, out_dim - 1 - n0)) * pitch + ((l & 7) ^ ((c >> 1) & 7)) * 16, at + u * 1024);
+            }
+        }
+    };
+    // stage st is run st % kHalves of column group st / kHalves
+    const int stages = groups_here * kHalves;
+    auto issue_stage = [&](int st, int slot) { issue(st / kHalves, st % kHalves, slot); };
+
+    typedef __attribute__((address_space(3))) volatile uint32_t LdsCount;
+    const uint32_t counters = lds0 + B::kCountersAt;
+    if (tid < 2) *reinterpret_cast<LdsCount*>(counters + 4 * tid) = 0;
+    issue_stage(0, 0);
+    // A fragments and row scales: all of the wavefront's share, for every column group.  Rows that exist live in the first
+    // 2 * kLive lanes of each half of a fragment; the other lanes repeat a live lane's address.
+    const int lr = lj % (2 * kLive);
+    typedef const __attribute__((address_space(1))) bm_v4i* Fragments;
+    typedef const __attribute__((address_space(1))) float* Scales;
+    Fragments fragments_at = reinterpret_cast<Fragments>(reinterpret_cast<uintptr_t>(qa));
+    Scales scales_at = reinterpret_cast<Scales>(reinterpret_cast<uintptr_t>(sa));
+    bm_v4i afrag[kHalves][kHB];
+    float ta[kHalves][kPairs];
+    auto load_run = [&](int hb) {
+#pragma unroll
+        for (int j = 0; j < kHB; ++j) afrag[hb][j] = fragments_at[(static_cast<size_t>(group) * kb_full + clamp_blk(hb, j)) * 64 + lh * 32 + lr];
+#pragma unroll
+        for (int p = 0; p < kPairs; ++p) ta[hb][p] = scales_at[static_cast<size_t>(clamp_blk(hb, 2 * p + lh)) * padded + row0 + lr];
+    };
+    // The compiler counts only its own loads: a wait of its for one of them would be a wait for every request that left in
+    // between.  So they are taken here, before the requests of the later stages leave.
+    auto take_run = [&](int hb) {
+#pragma unroll
+        for (int j = 0; j < kHB; ++j) asm volatile("" : "+v"(afrag[hb][j]) : : "memory");
+#pragma unroll
+        for (int p = 0; p < kPairs; ++p) {
+            asm volatile("" : "+v"(ta[hb][p]) : : "memory");
+            if (first_of(hb) + 2 * p + lh >= share_end) ta[hb][p] = 0.0f;
+        }
+    };
+    // The first run's of all wavefronts go first: a barrier, reached within a few instructions, keeps the others behind them.  (Their
+    // addresses pass through it, so that the compiler cannot lift them.)
+    load_run(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : "+s"(fragments_at), "+s"(scales_at) : : "memory");
+#pragma unroll
+    for (int hb = 1; hb < kHalves; ++hb) load_run(hb);
+#pragma unroll
+    for (int hb = 0; hb < 1; ++hb) take_run(hb);  // (the others where they are needed)
+#pragma unroll
+    for (int st = 1; st < kSlots; ++st)
+        if (st < stages) issue_stage(st, st);
+
+    typedef unsigned bm_v2u __attribute__((ext_vector_type(2)));
+    typedef unsigned bm_v4u __attribute__((ext_vector_type(4)));
+    typedef typename std::conditional<kType == 2, bm_v2u, bm_v4u>::type Raw;
+    typedef __attribute__((address_space(3))) const Raw LdsRaw;
+    typedef __attribute__((address_space(3))) const uint16_t LdsHalf;
+    // this lane's B operand inside a slot: column lj, block j of the run (chunk j, or 2j + lh), k half lh -- an XOR away from block 0's
+    const uint32_t frag0 = lj * 128 + (((lj >> 1) & 7) ^ (kType == 2 ? 0 : lh)) * 16 + (kType == 2 ? 8 * lh : 0);
+    // ... and its scale: unit 2q + lh of its tile, the half of column lj and of the run's place in the slice
+    const int lt = lj / kTileCols;
+    const uint32_t scale0 = 4096 + lt * (kUnits * 16) + ((lh ^ (kType == 2 ? lt >> 1 : lt >> 2)) << 4) + (lj % kTileCols) * 2;
+    auto place_of_run = [&](int hb) {  // Q4_0: blocks 64 apart share a unit; Q8_0: blocks 32 apart
+        return kType == 2 ? ((first_of(hb) >> 6) & 1) * 8 : ((first_of(hb) >> 5) & 3) * 4;
+    };
+    auto unpack = [&](const Raw& w) {
+        bm_v4i b;
+        if constexpr (kType == 2) {
+            auto byte = [](uint32_t x) { return static_cast<int>((x & 0xF0F0F0F0u) ^ 0x80808080u); };  // 16 (n - 8) of each high nibble n
+            b = bm_v4i{byte(w[0] << 4), byte(w[0]), byte(w[1] << 4), byte(w[1])};
+        } else {
+            b = bm_v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[kType == 2 ? 0 : 2]), static_cast<int>(w[kType == 2 ? 1 : 3])};
+        }
+        return b;
+    };
+    // stage `st` has landed when at most the requests of the stages behind it are in flight
+    auto wait_stage = [&](int st) {
+        if (st + 2 < stages) asm volatile("s_waitcnt vmcnt(10)" : : : "memory");
+        else if (st + 1 < stages) asm volatile("s_waitcnt vmcnt(5)" : : : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    };
+
+    const bm_v16i zi = {};
+    const bm_v32f zf = {};
+    Raw raw0, raw1;
+    uint16_t half;
+    int st_read = 0, slot_read = 0;  // the stage that operands are read from, and its slot
+    auto read_step = [&](int p) {
+        const int hb = p / kPairs, q = p % kPairs;
+        const uint32_t slot_at = lds_slots + slot_read * B::kSlotBytes;
+        raw0 = *reinterpret_cast<LdsRaw*>(slot_at + (frag0 ^ ((kType == 2 ? 2 * q : 4 * q) * 16)));
+        raw1 = *reinterpret_cast<LdsRaw*>(slot_at + (frag0 ^ ((kType == 2 ? 2 * q + 1 : 4 * q + 2) * 16)));
+        half = *reinterpret_cast<LdsHalf*>(slot_at + place_of_run(hb) + (scale0 ^ (32 * q)));
+    };
+    bm_v32f t[kSets];
+    bm_v16i c0[kSets], c1[kSets];
+    bm_v4i b0, b1;
+    float tb;
+    auto take_operands = [&](int hb) {
+        b0 = unpack(raw0);
+        b1 = unpack(raw1);
+        tb = half_bits_to_f32(half) * (kType == 2 ? 0.0625f : 1.0f);
+        if (first_of(hb) >= share_end) tb = 0.0f;  // a run past the share (inside one, scales past the matrix are zeros)
+    };
+    // A chain of additions is at most sixteen blocks long.  Runs of four stages put the first half's sums down in the
+    // wavefront's own part of the room below.
+    constexpr bool kPutDown = kHalves == 4;
+    static_assert(!kPutDown || kOne, "the room is free for the one column group only");
+    constexpr int kSums = kApart ? kHalves : 1;
+    float acc[kSums][16];
+
+    // ---- the wavefronts' sums meet in LDS: [side][part of K][v][lane]; a thread adds up neighbouring columns of a row.  kApart: the sums
+    // of a share's runs are added each for itself, in order.  counters[0]: wavefronts that have stored theirs, counters[1]: that have
+    // added up; looked at half a column group later, so that nobody waits who is not a half ahead.
+    float* red = reinterpret_cast<float*>(bm_lds + B::kSumsAt);
+    constexpr int kSideThreads = 64 * kParts, kPer = kLive * 64 / kSideThreads;
+    typedef float Terms __attribute__((ext_vector_type(kPer)));
+    Terms total;
+    const bool plain = ep.bias == nullptr && ep.residual == nullptr && ep.activation == kActNone && partial == nullptr && !accumulate;
+    auto wait_count = [&](int which, uint32_t count) {
+        while (static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(*reinterpret_cast<LdsCount*>(counters + 4 * which)))) < count)
+            __builtin_amdgcn_s_sleep(1);
+        asm volatile("" : : : "memory");
+    };
+    auto count_up = [&](int which) {
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        if (lane == 0) asm volatile("ds_add_u32 %0, %1" : : "v"(counters + 4 * which), "v"(1u) : "memory");
+    };
+    auto store_sums = [&](int s) {
+#pragma unroll
+        for (int v = 0; v < kLive; ++v) red[(wave * kLive + v) * 64 + lane] = acc[s][v];
+    };
+    auto add_up = [&](int cg, int s) {
+        int side_tid = tid % kSideThreads;
+        asm volatile("" : "+v"(side_tid));  // (its addresses are formed here and take no registers elsewhere)
+        Terms term[kParts];
+#pragma unroll
+        for (int w = 0; w < kParts; ++w) term[w] = reinterpret_cast<const Terms*>(red)[(side * kParts + w) * kSideThreads + side_tid];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            // (batch_mfma_kernel's order, for the same bits)
+            float sum = ((term[0][k] + term[1][k]) + term[2][k]) + term[3][k];
+            if constexpr (kParts == 8) sum += ((term[4][k] + term[5][k]) + term[6][k]) + term[7][k];
+            total[k] = s == 0 ? sum : total[k] + sum;
+        }
+        if (s + 1 < kSums) return;
+        const int l = side_tid * kPer & 63, v = side_tid * kPer >> 6;
+        const int m = row0 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3);
+        const int n = n_first + cg * B::kGroupCols + side * 32 + (l & 31);
+        if (plain && n + kPer <= out_dim) {
+            if (m < rows) {
+                float* const to = dst + static_cast<size_t>(m) * out_dim + n;
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) to[k] = total[k];
+            }
+            return;
+        }
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            if (m < rows && n + k < out_dim) {
+                const size_t at = static_cast<size_t>(m) * out_dim + n + k;
+                if (partial != nullptr) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = total[k];
+                else if (accumulate) unsafeAtomicAdd(dst + at, total[k]);  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
+                else dst[at] = finish_output(ep, n + k, at, total[k]);
+            }
+        }
+    };
+
+    wait_stage(0);
+    read_step(0);
+    if (kSets == 2) {
+        take_operands(0);
+        c0[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[0][0], b0, zi, 0, 0, 0);
+        t[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(ta[0][0], tb, zf, 0, 0, 0);
+        c1[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[0][1], b1, zi, 0, 0, 0);
+        read_step(1);
+    }
+    // A column group.  The first one stands by itself: the fragments of the later runs are taken there, when they are needed.
+    auto column_group = [&](int cg, auto first_one) {
+        constexpr bool kFirst = decltype(first_one)::value;
+#pragma unroll
+        for (int s = 0; s < kSums; ++s)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[s][v] = 0.0f;
+#pragma unroll
+        for (int p = 0; p < kSteps; ++p) {
+            // The step whose matrix instructions go out here (two sets: the next one, possibly of the next column group), and the one
+            // whose operands are read here.
+            constexpr int kAhead = kSets - 1;
+            const int pm = (p + kAhead) % kSteps, pr = (p + kAhead + 1) % kSteps;
+            const int hm = pm / kPairs, qm = pm % kPairs;
+            const bool beyond = kOne && p + kAhead >= kSteps;  // nothing follows
+            take_operands(hm);
+            if (qm == kPairs - 1) {
+                // the last operands of a stage are in registers: the stage three on takes its slot
+                if (kFirst && hm + 1 < kHalves && p + kAhead < kSteps) take_run(hm + 1);
+                const int st = st_read, slot = slot_read;
+                slot_read = slot_read + 1 == kSlots ? 0 : slot_read + 1;
+                ++st_read;
+                if (st + kSlots < stages) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+                    issue_stage(st + kSlots, slot);
+                }
+                if (st_read < stages) wait_stage(st_read);
+            }
+            if (!beyond) read_step(pr);
+            const int set = kSets == 2 ? (p + 1) & 1 : 0, cur = kSets == 2 ? p & 1 : 0;
+            float(&sum)[16] = acc[kApart ? p / kPairs : 0];
+            auto multiply = [&](const bm_v16i& c, int h, int first, int last) {
+#pragma unroll
+                for (int v = 0; v < kLive; ++v)
+                    if (v >= first && v < last) sum[v] = __builtin_fmaf(t[cur][16 * h + v], static_cast<float>(c[v]), sum[v]);
+            };
+            if constexpr (kSets == 2) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (!beyond) c0[set] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm], b0, zi, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c0[cur], 0, 0, kLive / 2);
+                __builtin_amdgcn_sched_barrier(0);
+                if (!beyond) t[set] = __builtin_amdgcn_mfma_f32_32x32x1f32(ta[hm][qm], tb, zf, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c0[cur], 0, kLive / 2, kLive);
+                multiply(c1[cur], 1, 0, kLive / 2);
+                __builtin_amdgcn_sched_barrier(0);
+                if (!beyond) c1[set] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm + 1], b1, zi, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c1[cur], 1, kLive / 2, kLive);
+            } else {
+                __builtin_amdgcn_sched_barrier(0);
+                t[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(ta[hm][qm], tb, zf, 0, 0, 0);
+                c0[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm], b0, zi, 0, 0, 0);
+                c1[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm + 1], b1, zi, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c0[0], 0, 0, kLive);
+                multiply(c1[0], 1, 0, kLive);
+            }
+            fence_registers(sum);
+            if (kPutDown && p == kSteps / 2 - 1) {
+                store_sums(0);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+            }
+            if (!kApart && !kOne && !kFirst && p == kSteps / 2 - 1) {
+                wait_count(0, cg * kBmWaves);
+                add_up(cg - 1, 0);
+                count_up(1);
+            }
+        }
+        if (kPutDown) {
+#pragma unroll
+            for (int v = 0; v < kLive; ++v) acc[0][v] = red[(wave * kLive + v) * 64 + lane] + acc[0][v];
+        }
+        if (kApart || kOne) {
+#pragma unroll
+            for (int s = 0; s < kSums; ++s) {
+                if (s > 0 || !kFirst) __syncthreads();
+                store_sums(s);
+                __syncthreads();
+                add_up(cg, s);
+            }
+        } else {
+            if (!kFirst) wait_count(1, cg * kBmWaves);
+            store_sums(0);
+            count_up(0);
+        }
+    };
+    column_group(0, std::true_type{});
+    if (!kOne)
+        for (int cg = 1; cg < groups_here; ++cg) column_group(cg, std::false_type{});
+    if (!kApart && !kOne) {
+        __syncthreads();
+        add_up(groups_here - 1, 0);
     }
 }
 
@@ -1331,6 +1724,105 @@ hipError_t bm_launch32(hipStream_t stream, float* dst, float* partial, const uin
     return hipGetLastError();
 }
 
+// How a launch of the column-group kernel cuts its work up: workgroups over the rows, column groups a workgroup, wavefronts that share K out,
+// stages a wavefront and column group, K shares.
+struct BatchGroupsPlan {
+    int row_groups, column_groups, parts, halves, shares, share_blocks;
+    bool apart;
+    bool own_sums;  // the sums are not formed in the older kernels' order
+    long grid;  // workgroups
+};
+
+template <int kType, int kHalves, int kParts, bool kApart>
+hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
+                       int in_dim, int out_dim, const BatchGroupsPlan& plan, const Epilogue& ep, const BmSecond& second, bool accumulate) {
+    const int cols = 32 * (kBmWaves / kParts) * plan.column_groups, col_tiles = (out_dim + cols - 1) / cols;
+    const dim3 grid(static_cast<unsigned>(plan.row_groups == 1 ? col_tiles : (col_tiles + 7) / 8 * 8 * plan.row_groups), static_cast<unsigned>(plan.shares),
+                    second.weight ? 2u : 1u),
+        block(kBmThreads);
+    static std::atomic<size_t> lds_limit[6] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
+    auto launch = [&](auto kernel, int lds, std::atomic<size_t>* limit) {
+        if (hipError_t e = bm_allow_large_lds(kernel, lds, limit); e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, plan.shares > 1 && !accumulate ? partial : nullptr, qa, sa, weight, rows, in_dim,
+                           out_dim, plan.share_blocks, plan.row_groups, plan.column_groups, ep, second, accumulate ? 1 : 0);
+        return hipGetLastError();
+    };
+    auto launch_for = [&](auto live, auto shared, int at) {
+        constexpr int kLive = decltype(live)::value;
+        constexpr bool kShared = decltype(shared)::value;
+        constexpr int lds = BatchGroups<kType, kLive, kHalves, kParts>::kLdsBytes;
+        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kShared, true>, lds, &lds_limit[at]);
+        if constexpr (kHalves == 4 || kApart) return hipErrorInvalidValue;  // (not among the plans)
+        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kShared, false>, lds, &lds_limit[at + 1]);
+    };
+    if (plan.row_groups > 1) return launch_for(std::integral_constant<int, 16>{}, std::true_type{}, 0);
+    if (rows <= 16) return launch_for(std::integral_constant<int, 8>{}, std::false_type{}, 2);
+    return launch_for(std::integral_constant<int, 16>{}, std::false_type{}, 4);
+}
+
+template <int kType>
+hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
+                            int in_dim, int out_dim, const BatchGroupsPlan& plan, const Epilogue& ep, const BmSecond& second, bool accumulate) {
+#define AFHIP_BMG(H, P, APART) bm_launch_groups_of<kType, H, P, APART>(stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, plan, ep, second, accumulate)
+    if (plan.apart) return plan.halves == 2 && plan.parts == 8 ? AFHIP_BMG(2, 8, true) : hipErrorInvalidValue;
+    switch (plan.parts * 10 + plan.halves) {
+        case 81: return AFHIP_BMG(1, 8, false);
+        case 82: return AFHIP_BMG(2, 8, false);
+        case 84: return AFHIP_BMG(4, 8, false);
+        case 42: return AFHIP_BMG(2, 4, false);
+        default: return hipErrorInvalidValue;
+    }
+#undef AFHIP_BMG
+}
+
+// The column-group kernel's cut of a call.  Runs and shares depend on one matrix alone, and the sums of an op with an epilogue are formed in
+// the plain op's order, so that the halves of a pair and a biased op keep the plain single op's bits; column groups do not enter a sum.
+//   * Few columns (a matrix's 32 x 32 tiles fill at most half of the units): K goes to twice the workgroups, two shares that add to the
+//     result; an op with an epilogue keeps the two runs' sums apart instead (no reduce launch).  32 rows, 2048 x 2048 9.3 -> 7.7 us.
+//   * Four runs a share on few columns only, where a launch is mostly its way to the first bytes (K = 14336 x 4096 columns 19.1 -> 18.1,
+//     11008 18.1 -> 17.6); on more columns the older kernels' K shares are better (8192 x 8192 18.4 against 16.4).
+//   * Q8_0, twice the bytes for the same arithmetic, is bound by the bytes sooner: few columns on 32 rows from K = 1024 up only at an
+//     eighth of the units (1024 columns, K = 2048 7.6 -> 6.7, a pair of 4096 x 4096 columns 13.2 against 14.6 here); one run on many
+//     columns only at 33 rows and more (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
+bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool pair, bool adds, BatchGroupsPlan* plan) {
+    const int kb = in_dim / 32, stage_blocks = tensor_type == 2 ? 8 : 4;
+    if (kb % 8 != 0) return false;
+    const long units = gemv_compute_units();
+    BatchGroupsPlan p;
+    p.row_groups = (rows + 31) / 32;
+    const long columns = (out_dim + 31) / 32;
+    const bool few = 2 * columns * p.row_groups <= units;
+    p.parts = kb <= 8 * stage_blocks && columns * p.row_groups > units ? 4 : 8;
+    const int run = p.parts * stage_blocks, runs = (kb + run - 1) / run;
+    p.shares = (runs + 3) / 4;
+    p.apart = false;
+    if (few && runs > 1 && p.shares == 1) {
+        if (adds || runs > 2) p.shares = 2;
+        else p.apart = true;
+    }
+    p.halves = (runs + p.shares - 1) / p.shares;
+    p.share_blocks = p.halves * run;
+    if (p.halves == 3) p.halves = 4;
+    if (p.parts == 4) p.halves = 2;
+    p.shares = (kb + p.share_blocks - 1) / p.share_blocks;
+    // one workgroup a compute unit: each takes as many column groups as that needs
+    const long per = (pair ? 2 : 1) * p.row_groups * static_cast<long>(p.shares), wide = 8 / p.parts;
+    auto grid = [&](long groups) {
+        const long tiles = (columns + groups * wide - 1) / (groups * wide);
+        return (p.row_groups == 1 ? tiles : (tiles + 7) / 8 * 8) * per;
+    };
+    long groups = 1;
+    if (p.halves == 4 && (!few || tensor_type == 8)) return false;
+    if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 ? 8 : 4 * p.row_groups) * columns > units) return false;
+    if (tensor_type == 8 && !few && p.halves == 1 && p.row_groups == 1) return false;
+    while (!p.apart && p.halves != 4 && grid(groups) > units && groups < columns) ++groups;
+    p.own_sums = few || p.halves != 2;
+    p.column_groups = static_cast<int>(groups);
+    p.grid = grid(groups);
+    *plan = p;
+    return true;
+}
+
 }  // namespace
 
 bool batch_mfma_supports(int tensor_type, size_t rows, size_t in_dim, size_t out_dim) {
@@ -1371,7 +1863,7 @@ size_t batch_mfma_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, s
     return (front + 255) / 256 * 256 + (shares > 1 ? 2 * shares * rows * out_dim * 4 : 0);  // (twice: a pair of matrices)
 }
 
-// Largest grid the 32-row kernel is chosen for; negative: one workgroup per compute unit.
+// Largest grid batch32_mfma_kernel is chosen for; negative: one workgroup per compute unit; 0: neither it nor the column-group kernel.
 static std::atomic<long> batch32_bound{-1};
 void set_batch32_max_workgroups(long bound) { batch32_bound.store(bound, std::memory_order_relaxed); }
 
@@ -1404,10 +1896,33 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     // columns) 13.8 -> 12.7 and 13.9 -> 12.8, Q8_0 160 (5120 columns) 11.0 -> 9.9; 128 workgroups lose (8192 columns
     // 10.6 -> 12.5).  set_batch32_max_workgroups overrides the bound (tests
     // reach the kernel's K shares and pair launches that way; 0 switches the kernel off).
+    const size_t x_bytes = static_cast<size_t>(rows) * in_dim * 4, y_bytes = static_cast<size_t>(rows) * out_dim * 4;
+    auto apart = [&](const float* y) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(input), b = reinterpret_cast<uintptr_t>(y);
+        return b + y_bytes <= a || a + x_bytes <= b;
+    };
     const long bound_set = batch32_bound.load(std::memory_order_relaxed);
     const long bound = bound_set >= 0 ? bound_set : gemv_compute_units();
     const long groups32 = static_cast<long>((out_dim + 63) / 64) * real_shares * (weight_b_prepared ? 2 : 1);
-    const bool thirty_two = !eight && rows <= 64 && kb % 8 == 0 && groups32 >= gemv_compute_units() * 5 / 8 && groups32 <= bound;
+    const bool old_thirty_two = !eight && rows <= 64 && kb % 8 == 0 && groups32 >= gemv_compute_units() * 5 / 8 && groups32 <= bound;
+    // Column groups: where the plan's sums are its own, for every form of the call (the bits of a pair's halves); elsewhere they are the
+    // older kernels' and the faster one takes the call (us, Q4_0, K = 4096): one column group and three and more win (6144 columns
+    // 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8, 32000 29.8 -> 26.6), two on up to 32 rows lose to batch32_mfma_kernel where that can
+    // run (14336 columns 16.4 against 17.1, a pair of 6144 15.2 against 15.9).  A slice that K fills to less than three quarters is a
+    // loss of its own, which only more than 48 rows make up for (K = 2304 x 12290 columns, 40 rows 21.2 against 22.2; 64 rows x 32000
+    // columns 49.1 -> 39.2).  Q8_0 wins with one column group (K = 2048 x 8192 columns 9.8 -> 9.2; pairs of 5632 11.7 against 12.6).
+    const bool adds = both_plain && apart(dst) && (!weight_b_prepared || apart(dst_b));
+    BatchGroupsPlan plan;
+    const bool column_groups = !eight && rows <= 64 && bound_set != 0 &&
+                               batch_groups_plan(tensor_type, rows, in_dim, out_dim, weight_b_prepared != nullptr, adds, &plan) &&
+                               (plan.own_sums || plan.column_groups == 1 ||
+                                (tensor_type == 2 && (plan.parts == 4 || 4 * kb >= 3 * plan.share_blocks || rows > 48) &&
+                                 (plan.column_groups > 2 || rows > 32 || !old_thirty_two)));
+    const bool thirty_two = old_thirty_two && !column_groups;
+    if (column_groups) {
+        real_shares = plan.shares;
+        share_blocks = plan.share_blocks;
+    }
     // batch_mfma_kernel on a K of one share that more than four of its wavefronts work on, few column tiles (at most
     // half the compute units' worth, one matrix counted) and no epilogue: two shares of four wavefronts each.  The
     // kernel adds its wavefronts' sums as (first four) + (last four), so the two shares' sums are exactly those halves
@@ -1415,14 +1930,14 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     // for it).  Four wavefronts a workgroup on twice the workgroups, sixteen rows: 4096 x 4096 columns 9.8 -> 8.8 us,
     // 2048 columns 9.3 -> 8.2, 48 rows 14.5 -> 12.8.  (Beyond one workgroup per compute unit it loses: 6144 columns
     // 10.1 -> 11.8, 8192 columns at 64 rows 15.7 -> 22.4.)
-    if (!eight && !thirty_two && real_shares == 1 && both_plain && kb > (kBmWaves / 2) * wave_blocks &&
+    if (!eight && !thirty_two && !column_groups && real_shares == 1 && adds && kb > (kBmWaves / 2) * wave_blocks &&
         2 * static_cast<long>((out_dim + 31) / 32) <= gemv_compute_units()) {
         share_blocks = (kBmWaves / 2) * wave_blocks;
         real_shares = 2;
     }
     // Two K shares and nothing to do to the sums but add them: the kernel's shares add to the result themselves
-    // (cleared by the quantizer's launch), which saves the reduce launch -- two of them for a pair.
-    const bool accumulate = real_shares == 2 && both_plain;
+    // (cleared by the quantizer's launch, so the result must be apart from X), which saves the reduce launch -- two of them for a pair.
+    const bool accumulate = real_shares == 2 && adds;
     const int groups = rows > 8 ? 2 : 1;  // (eight-row kernel) groups of eight rows
     // One K share of at most sixteen blocks a wavefront on up to two workgroups per compute unit: the workgroups quantize X
     // themselves, no quantizer launch.  What they convert they convert once per workgroup, so a grid of many rounds keeps the
@@ -1431,11 +1946,6 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     // (500 workgroups) 18.4 (18.4), on 128256 (2004) 66 (54).  Q8_0 5 x 2048 x 8192 6.1 (8.8), 8 x 2048 x 32000 13.3 (15.3),
     // 8 x 4096 x 14336 13.7 (14.0).  Two K shares keep it too: their result has to be cleared first.  So does a result that
     // overlaps X, which here is read by workgroups that start while others store.
-    const size_t x_bytes = static_cast<size_t>(rows) * in_dim * 4, y_bytes = static_cast<size_t>(rows) * out_dim * 4;
-    auto apart = [&](const float* y) {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(input), b = reinterpret_cast<uintptr_t>(y);
-        return b + y_bytes <= a || a + x_bytes <= b;
-    };
     const long groups8 = !eight ? 0 : [&] {
         const int cols = bm8_columns(real_shares, out_dim, weight_b_prepared != nullptr);
         return static_cast<long>((out_dim + cols - 1) / cols) * (weight_b_prepared ? 2 : 1);
@@ -1461,7 +1971,7 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
         float* zero_a = accumulate ? dst : nullptr;
         float* zero_b = accumulate && weight_b_prepared ? dst_b : nullptr;
         const size_t zero_count = static_cast<size_t>(rows) * out_dim;
-        if (thirty_two && tensor_type == 2)
+        if ((thirty_two || column_groups) && tensor_type == 2)
             hipLaunchKernelGGL(quantize_fragments_kernel<true>, qgrid, dim3(256), 0, stream, input, rows, in_dim,
                                row_tiles, qa, sa, zero_a, zero_b, zero_count);
         else
@@ -1487,6 +1997,9 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
 #undef AFHIP_BM8_CG
 #undef AFHIP_BM8
     }
+    else if (column_groups)
+        e = tensor_type == 2 ? bm_launch_groups<2>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, plan, ep, second, accumulate)
+                             : bm_launch_groups<8>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, plan, ep, second, accumulate);
     else if (thirty_two)
         e = tensor_type == 2 ? bm_launch32<2>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, real_shares, share_blocks, ep, second, accumulate)
                              : bm_launch32<8>(stream, dst, partial, qa, sa, weight_prepared, rows, in_dim, out_dim, real_shares, share_blocks, ep, second, accumulate);

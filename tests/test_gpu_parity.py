@@ -531,6 +531,46 @@ def test_thirty_two_row_kernel_with_k_shares_and_pairs(fmt, rows, in_dim, out_di
 
 
 
+@pytest.mark.parametrize("fmt,rows,in_dim,out_dim,pair,same", [
+    (Q4, 9, 256, 32, False, False), (Q4, 16, 512, 1, True, False), (Q4, 17, 2304, 4095, False, False),  # few columns: one run, two
+    (Q4, 32, 4096, 4096, True, False), (Q4, 25, 5632, 2050, True, False), (Q4, 12, 11008, 4096, False, False),  # ... and long K
+    (Q4, 64, 14336, 2047, True, False), (Q4, 31, 2048, 8191, True, False), (Q4, 33, 256, 8223, True, True),
+    (Q4, 32, 4096, 6145, False, True), (Q4, 16, 3328, 33000, False, True), (Q4, 33, 4096, 4097, True, True),  # column groups
+    (Q4, 63, 4096, 14337, True, True), (Q4, 64, 1280, 33001, True, True), (Q4, 9, 2048, 65600, False, True),
+    (Q8, 9, 256, 33, False, False), (Q8, 17, 1024, 4096, True, False), (Q8, 33, 4096, 1023, True, False),
+    (Q8, 48, 1024, 4095, True, False), (Q8, 32, 2048, 8191, False, True), (Q8, 20, 1024, 14000, False, True),
+])
+def test_column_groups_of_the_thirty_two_row_kernel(fmt, rows, in_dim, out_dim, pair, same):
+    """32 rows a workgroup on one and more groups of columns, at the edges of row tiles, column tiles, runs and shares of K: the
+    oracle's result, the bits of the kernel it stands in for where the sums have its order (`same`), a pair's halves those of single
+    calls, and a call with a bias (two runs in one share) or one whose result lies over X those of the plain call."""
+    print(f"case: column groups fmt={fmt} rows={rows} in={in_dim} out={out_dim} pair={pair}", flush=True)
+    x = synth.activations(5300 + rows, rows, in_dim)
+    w = [synth.weights(fmt, 5301 + i, out_dim, in_dim) for i in range(2 if pair else 1)]
+    wd = [G.prepare(fmt, each, out_dim, in_dim) for each in w]
+    single = [G.linear(fmt, PREP, x, each, rows, in_dim, out_dim) for each in wd]
+    got = G.linear_pair(fmt, PREP, x, wd[0], wd[1], rows, in_dim, out_dim) if pair else single
+    _lib.lib().afhip_tune_batch32_max_workgroups(0)
+    try:
+        older = [G.linear(fmt, PREP, x, each, rows, in_dim, out_dim) for each in wd]
+    finally:
+        _lib.lib().afhip_tune_batch32_max_workgroups(-1)
+    for one, half, old in zip(single, got, older):
+        assert np.array_equal(one, half)
+        assert np.array_equal(one, old) if same else G.max_rel_err(one, old.astype(np.float64)) <= TIGHT
+    zeros = np.zeros(out_dim, np.float32)
+    assert np.array_equal(G.linear_bias(fmt, PREP, x, wd[0], zeros, rows, in_dim, out_dim), single[0])
+    ws = torch.empty(max(kernels.workspaceBytes(fmt, rows, in_dim, out_dim), 16), dtype=torch.uint8, device=G.DEV)
+    room = torch.full((rows * (in_dim + out_dim),), float("nan"), dtype=torch.float32, device=G.DEV)
+    room[:rows * in_dim] = torch.from_numpy(x.ravel()).to(G.DEV)
+    kernels.launchLinearF32(G.stream(), fmt, PREP, G.buf(room[:rows * out_dim]), G.buf(room[:rows * in_dim]), G.buf(wd[0]), rows, in_dim,
+                            out_dim, G.buf(ws))
+    torch.cuda.synchronize()
+    assert np.array_equal(room[:rows * out_dim].cpu().numpy(), single[0].ravel())
+    ref = O.linear_no_bias(fmt, x, w[-1], rows, in_dim, out_dim, workers=8)
+    assert G.max_rel_err(got[-1], ref.astype(np.float64)) <= TIGHT
+
+
 @pytest.mark.parametrize("fmt,rows,in_dim,out_dim,pair", [
     (Q4, 5, 4096, 4096, False), (Q4, 8, 256, 4100, False), (Q4, 7, 1280, 6152, False), (Q4, 6, 3840, 12290, True),
     (Q4, 4, 2048, 16400, False), (Q8, 8, 2048, 4096, False), (Q8, 5, 256, 8200, True), (Q8, 7, 1792, 14336, False),
