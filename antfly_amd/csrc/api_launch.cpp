@@ -113,6 +113,12 @@ static int env_int(const char* name) {
     return v && *v ? std::atoi(v) : 0;
 }
 
+static long batch_mfma_min_rows() {
+    static const char* v = std::getenv("AFHIP_BATCH_MFMA_MIN_ROWS");
+    static const long forced = v && *v ? std::atol(v) : -1;
+    return forced;
+}
+
 // Whether the single-shot MFMA kernel serves this shape (measured against the kernels it replaces;
 // AFHIP_BATCH_MFMA_MIN_ROWS overrides the lower row bound for tuning runs, 0 switches the kernel off):
 // from five rows on (six on a K longer than 4096, where the split-K GEMV still wins at five) up to 64
@@ -121,9 +127,8 @@ static int env_int(const char* name) {
 // the eight-row kernel requests weights as it goes and needs neither condition.  Two to four rows where measured
 // faster than the decode kernels (the rules below).
 static bool batch_mfma_preferred(int tensor_type, size_t rows, size_t in_dim, size_t out_dim, bool pair) {
-    static const char* v = std::getenv("AFHIP_BATCH_MFMA_MIN_ROWS");
-    static const long forced = v && *v ? std::atol(v) : -1;
-    // Up to 64 rows everywhere; 65 .. 96 of Q4_0 where the GEMM's grid of 32 x 64 tiles passes one workgroup a compute unit (on
+    const long forced = batch_mfma_min_rows();
+    // Up to 64 rows everywhere; 65 .. 96 of Q4_0 (beside batch_mfma_column_groups, whose kernel is the better one on its shapes) where the GEMM's grid of 32 x 64 tiles passes one workgroup a compute unit (on
     // one it takes 15.5 us at K = 4096 x 4608 columns) and this kernel's 32-column tiles need few rounds.  It takes 17 us for every
     // unit's worth of workgroups whatever K up to a share of 128 blocks, so K has to be near that (this kernel / the GEMM, 65 rows):
     //  * one share and one round, K over 3072: 3104 x 6144 columns 19.2 / 20.2, 4096 x 8192 19.5 / 20.7; 3072 x 6144 18.1 / 17.0
@@ -500,11 +505,13 @@ static afhip_status linear_impl_body(void* stream_v, int tensor_type, int layout
                           in_dim <= static_cast<size_t>(gemv_fused_max_in_dim());
     // Five to 64 (96) rows: the weights are read once, so the single-shot MFMA kernel (X quantized into
     // MFMA operand order first) beats both the row-by-row GEMV and the tiled GEMM.
+    const bool workspace_holds_batch = workspace.ptr != 0 && workspace.ptr % 16 == 0 &&
+                                       workspace.len >= batch_mfma_workspace_bytes(tensor_type, rows, in_dim, out_dim);
     if (layout == AFHIP_LAYOUT_PREPARED && !want_dots && kind != AFHIP_DISPATCH_SCALAR &&
-        batch_mfma_preferred(tensor_type, rows, in_dim, out_dim, pair) &&
-        // (below five rows the decode kernel, which needs no workspace, remains for a caller that lends none)
-        (rows >= kBatchMfmaMinRows || (workspace.ptr != 0 && workspace.ptr % 16 == 0 &&
-                                       workspace.len >= batch_mfma_workspace_bytes(tensor_type, rows, in_dim, out_dim)))) {
+        // (below five rows the decode kernel, which needs no workspace, remains for a caller that lends none; on the column-group
+        // kernel's own shapes beyond 64 rows the GEMM, for one that lends less than the shape's workspace size)
+        ((batch_mfma_preferred(tensor_type, rows, in_dim, out_dim, pair) && (rows >= kBatchMfmaMinRows || workspace_holds_batch)) ||
+         (workspace_holds_batch && batch_mfma_min_rows() < 0 && batch_mfma_column_groups(tensor_type, rows, in_dim, out_dim)))) {
         const size_t need = batch_mfma_workspace_bytes(tensor_type, rows, in_dim, out_dim);
         if (workspace.ptr == 0 || workspace.len < need || workspace.ptr % 16 != 0) return AFHIP_ERR_INVALID_STATE;
         if (counters) {

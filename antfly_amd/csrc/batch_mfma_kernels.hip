@@ -1411,7 +1411,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
     constexpr bool kPutDown = kHalves == 4;
     static_assert(!kPutDown || kOne, "the room is free for the one column group only");
     constexpr int kSums = kApart ? kHalves : 1;
-    float acc[kSums][16];
+    // ... and where a run's sums are added up by themselves, four: even and odd blocks apart.
+    constexpr bool kOdd = kHalves == 1 || kApart;
+    float acc[kSums][16], odd[16];
 
     // ---- the wavefronts' sums meet in LDS: [side][part of K][v][lane]; a thread adds up neighbouring columns of a row.  kApart: the sums
     // of a share's runs are added each for itself, in order.  counters[0]: wavefronts that have stored theirs, counters[1]: that have
@@ -1486,6 +1488,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
         for (int s = 0; s < kSums; ++s)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[s][v] = 0.0f;
+        if (kOdd) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) odd[v] = 0.0f;
+        }
 #pragma unroll
         for (int p = 0; p < kSteps; ++p) {
             // The step whose matrix instructions go out here (two sets: the next one, possibly of the next column group), and the one
@@ -1509,8 +1515,8 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             }
             if (!beyond) read_step(pr);
             const int set = kSets == 2 ? (p + 1) & 1 : 0, cur = kSets == 2 ? p & 1 : 0;
-            float(&sum)[16] = acc[kApart ? p / kPairs : 0];
             auto multiply = [&](const bm_v16i& c, int h, int first, int last) {
+                float(&sum)[16] = kOdd && h == 1 ? odd : acc[kApart ? p / kPairs : 0];
 #pragma unroll
                 for (int v = 0; v < kLive; ++v)
                     if (v >= first && v < last) sum[v] = __builtin_fmaf(t[cur][16 * h + v], static_cast<float>(c[v]), sum[v]);
@@ -1538,11 +1544,21 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
                 multiply(c0[0], 0, 0, kLive);
                 multiply(c1[0], 1, 0, kLive);
             }
-            fence_registers(sum);
+            fence_registers(acc[kApart ? p / kPairs : 0]);
+            if (kOdd) {
+                fence_registers(odd);
+                if (p % kPairs == kPairs - 1) {
+#pragma unroll
+                    for (int v = 0; v < kLive; ++v) {
+                        acc[kApart ? p / kPairs : 0][v] += odd[v];
+                        odd[v] = 0.0f;
+                    }
+                }
+            }
             if (kPutDown && p == kSteps / 2 - 1) {
                 store_sums(0);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+                for (int v = 0; v < 16; ++v) acc[0][v] = 0.0f;
             }
             if (!kApart && !kOne && !kFirst && p == kSteps / 2 - 1) {
                 wait_count(0, cg * kBmWaves);
@@ -1769,6 +1785,7 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
         case 81: return AFHIP_BMG(1, 8, false);
         case 82: return AFHIP_BMG(2, 8, false);
         case 84: return AFHIP_BMG(4, 8, false);
+        case 41: return AFHIP_BMG(1, 4, false);
         case 42: return AFHIP_BMG(2, 4, false);
         default: return hipErrorInvalidValue;
     }
@@ -1777,13 +1794,16 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
 
 // The column-group kernel's cut of a call.  Runs and shares depend on one matrix alone, and the sums of an op with an epilogue are formed in
 // the plain op's order, so that the halves of a pair and a biased op keep the plain single op's bits; column groups do not enter a sum.
+//   * A run that fits four wavefronts is given to four, the others take the next 32 columns (K = 1024, 32 rows, 14336 columns 10.2 -> 8.6,
+//     48 rows, a pair of 4096 10.3 -> 8.2); one of up to eight wavefronts on many columns likewise, two stages each, unless eight
+//     wavefronts and 32 columns leave fewer rounds (K = 2048: 128256 columns 46 against 51, but 77 rows, 5632 columns 13.8 -> 12.4).
 //   * Few columns (a matrix's 32 x 32 tiles fill at most half of the units): K goes to twice the workgroups, two shares that add to the
 //     result; an op with an epilogue keeps the two runs' sums apart instead (no reduce launch).  32 rows, 2048 x 2048 9.3 -> 7.7 us.
 //   * Four runs a share on few columns only, where a launch is mostly its way to the first bytes (K = 14336 x 4096 columns 19.1 -> 18.1,
 //     11008 18.1 -> 17.6); on more columns the older kernels' K shares are better (8192 x 8192 18.4 against 16.4).
 //   * Q8_0, twice the bytes for the same arithmetic, is bound by the bytes sooner: few columns on 32 rows from K = 1024 up only at an
-//     eighth of the units (1024 columns, K = 2048 7.6 -> 6.7, a pair of 4096 x 4096 columns 13.2 against 14.6 here); one run on many
-//     columns only at 33 rows and more (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
+//     eighth of the units (1024 columns, K = 2048 7.6 -> 6.7, a pair of 4096 x 4096 columns 13.2 against 14.6 here); one run of eight
+//     wavefronts on many columns only at 33 rows and more (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
 bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool pair, bool adds, BatchGroupsPlan* plan) {
     const int kb = in_dim / 32, stage_blocks = tensor_type == 2 ? 8 : 4;
     if (kb % 8 != 0) return false;
@@ -1792,7 +1812,24 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     p.row_groups = (rows + 31) / 32;
     const long columns = (out_dim + 31) / 32;
     const bool few = 2 * columns * p.row_groups <= units;
-    p.parts = kb <= 8 * stage_blocks && columns * p.row_groups > units ? 4 : 8;
+    // one workgroup a compute unit: each takes as many column groups as that needs
+    auto grid = [&](long groups, int matrices) {
+        const long wide = 8 / p.parts, tiles = (columns + groups * wide - 1) / (groups * wide);
+        return (p.row_groups == 1 ? tiles : (tiles + 7) / 8 * 8) * matrices * p.row_groups * static_cast<long>(p.shares);
+    };
+    auto groups_for = [&](int matrices) {
+        long groups = 1;
+        while (grid(groups, matrices) > units && groups < columns) ++groups;
+        return groups;
+    };
+    p.parts = 8;
+    p.shares = 1;
+    if (kb <= 4 * stage_blocks) p.parts = 4;
+    else if (columns * p.row_groups > units && kb <= 8 * stage_blocks) {
+        const long groups8 = groups_for(1);
+        p.parts = 4;
+        if (2 * groups_for(1) > groups8) p.parts = 8;
+    }
     const int run = p.parts * stage_blocks, runs = (kb + run - 1) / run;
     p.shares = (runs + 3) / 4;
     p.apart = false;
@@ -1803,22 +1840,13 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     p.halves = (runs + p.shares - 1) / p.shares;
     p.share_blocks = p.halves * run;
     if (p.halves == 3) p.halves = 4;
-    if (p.parts == 4) p.halves = 2;
     p.shares = (kb + p.share_blocks - 1) / p.share_blocks;
-    // one workgroup a compute unit: each takes as many column groups as that needs
-    const long per = (pair ? 2 : 1) * p.row_groups * static_cast<long>(p.shares), wide = 8 / p.parts;
-    auto grid = [&](long groups) {
-        const long tiles = (columns + groups * wide - 1) / (groups * wide);
-        return (p.row_groups == 1 ? tiles : (tiles + 7) / 8 * 8) * per;
-    };
-    long groups = 1;
+    p.own_sums = few || p.halves != 2;
     if (p.halves == 4 && (!few || tensor_type == 8)) return false;
     if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 ? 8 : 4 * p.row_groups) * columns > units) return false;
-    if (tensor_type == 8 && !few && p.halves == 1 && p.row_groups == 1) return false;
-    while (!p.apart && p.halves != 4 && grid(groups) > units && groups < columns) ++groups;
-    p.own_sums = few || p.halves != 2;
-    p.column_groups = static_cast<int>(groups);
-    p.grid = grid(groups);
+    if (tensor_type == 8 && !few && p.halves == 1 && p.parts == 8 && p.row_groups == 1) return false;
+    p.column_groups = p.apart || p.halves == 4 ? 1 : static_cast<int>(groups_for(pair ? 2 : 1));
+    p.grid = grid(p.column_groups, pair ? 2 : 1);
     *plan = p;
     return true;
 }
@@ -1861,6 +1889,27 @@ size_t batch_mfma_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, s
     const size_t shares = static_cast<size_t>(bm_shares(tensor_type, static_cast<int>(in_dim)));
     const size_t front = padded * in_dim + (in_dim / 32) * padded * 4;
     return (front + 255) / 256 * 256 + (shares > 1 ? 2 * shares * rows * out_dim * 4 : 0);  // (twice: a pair of matrices)
+}
+
+// 65 to 96 rows: the column-group kernel or the tiled GEMM (Q4_0; us, GEMM first).  One matrix's columns decide, also for a pair.  One
+// column group: always (77 rows, 2048 x 2048 9.7 -> 7.7, 1024 x 1024 8.7 -> 7.0, K = 4096 x 2048 columns 12.0 -> 10.2).  Several, each with
+// what its share of K leaves idle, against the GEMM's rounds: while two of its 32 x 64 tiles a compute unit take the matrix, its one round
+// is as long as three column groups and a little more (K = 4096, 96 rows: 4096 columns, two groups, 16.0 -> 14.2; 6144, three, 21.3 -> 18.2;
+// 8192, four, 21.7 against 22.2), with one run of K four (K = 2048: 5632 columns 14.4 -> 12.4, a pair 21.0 -> 17.8, 8192 15.0 -> 14.1);
+// beyond, it starts another round (K = 4096: 11008 columns 31.8 -> 26.2, 14336 32.4 -> 29.5, a pair 56 -> 49.5; K = 2048 x 16384 22.3 / 22.6,
+// 24576 34.4 -> 27.0).  K that fills less than seven eighths of the wavefronts' stages stays with the GEMM (3072 x 8192 18.8 against 21.6).
+// The error against 64 bits is that of the calls of fewer rows, 6.2e-8 .. 1.0e-7 (the GEMM's 6.4e-8 .. 1.5e-7).
+bool batch_mfma_column_groups(int tensor_type, size_t rows, size_t in_dim, size_t out_dim) {
+    BatchGroupsPlan plan;
+    if (rows <= 64 || !batch_mfma_supports(tensor_type, rows, in_dim, out_dim) ||
+        !batch_groups_plan(tensor_type, static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), false, true, &plan))
+        return false;
+    const long room = static_cast<long>(plan.halves) * plan.parts * (tensor_type == 2 ? 8 : 4), kb = static_cast<long>(in_dim / 32);
+    const long gemm_grid = static_cast<long>((rows + 31) / 32 * ((out_dim + 63) / 64));
+    if (plan.column_groups == 1) return true;
+    if (plan.shares == 1 && 8 * kb < 7 * room) return false;
+    if (gemm_grid <= 2 * gemv_compute_units()) return plan.column_groups <= (plan.halves == 2 && plan.parts == 8 ? 3 : 4);
+    return true;
 }
 
 // Largest grid batch32_mfma_kernel is chosen for; negative: one workgroup per compute unit; 0: neither it nor the column-group kernel.
@@ -1913,11 +1962,12 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     // columns 49.1 -> 39.2).  Q8_0 wins with one column group (K = 2048 x 8192 columns 9.8 -> 9.2; pairs of 5632 11.7 against 12.6).
     const bool adds = both_plain && apart(dst) && (!weight_b_prepared || apart(dst_b));
     BatchGroupsPlan plan;
-    const bool column_groups = !eight && rows <= 64 && bound_set != 0 &&
+    const bool column_groups = !eight && bound_set != 0 &&
                                batch_groups_plan(tensor_type, rows, in_dim, out_dim, weight_b_prepared != nullptr, adds, &plan) &&
-                               (plan.own_sums || plan.column_groups == 1 ||
-                                (tensor_type == 2 && (plan.parts == 4 || 4 * kb >= 3 * plan.share_blocks || rows > 48) &&
-                                 (plan.column_groups > 2 || rows > 32 || !old_thirty_two)));
+                               (rows > 64 ? batch_mfma_column_groups(tensor_type, rows, in_dim, out_dim)
+                                          : plan.own_sums || plan.column_groups == 1 ||
+                                                (tensor_type == 2 && (plan.parts == 4 || 4 * kb >= 3 * plan.share_blocks || rows > 48) &&
+                                                 (plan.column_groups > 2 || rows > 32 || !old_thirty_two)));
     const bool thirty_two = old_thirty_two && !column_groups;
     if (column_groups) {
         real_shares = plan.shares;

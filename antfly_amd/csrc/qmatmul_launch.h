@@ -90,6 +90,8 @@ int gemv_compute_units();
 bool batch_mfma_supports(int tensor_type, size_t rows, size_t in_dim, size_t out_dim);
 // whether launch_batch_mfma takes its eight-row kernel for this shape (the faster one where it applies)
 bool batch_mfma_eight_rows(int tensor_type, size_t rows, size_t in_dim, size_t out_dim);
+// whether launch_batch_mfma is the better route for 65 rows and more (its column-group kernel)
+bool batch_mfma_column_groups(int tensor_type, size_t rows, size_t in_dim, size_t out_dim);
 size_t batch_mfma_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, size_t out_dim);
 void set_batch32_max_workgroups(long bound);
 // Timing diagnostics: the eight-row kernel (Q4_0, a matrix it takes in tiles of more than 48 columns, K of one share) storing

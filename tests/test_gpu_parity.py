@@ -532,12 +532,15 @@ def test_thirty_two_row_kernel_with_k_shares_and_pairs(fmt, rows, in_dim, out_di
 
 
 @pytest.mark.parametrize("fmt,rows,in_dim,out_dim,pair,same", [
-    (Q4, 9, 256, 32, False, False), (Q4, 16, 512, 1, True, False), (Q4, 17, 2304, 4095, False, False),  # few columns: one run, two
+    (Q4, 9, 256, 512, False, False), (Q4, 16, 512, 513, True, False), (Q4, 17, 2304, 4095, False, False),  # few columns: one run, two
     (Q4, 32, 4096, 4096, True, False), (Q4, 25, 5632, 2050, True, False), (Q4, 12, 11008, 4096, False, False),  # ... and long K
-    (Q4, 64, 14336, 2047, True, False), (Q4, 31, 2048, 8191, True, False), (Q4, 33, 256, 8223, True, True),
+    (Q4, 64, 14336, 2047, True, False), (Q4, 31, 2048, 8191, True, False), (Q4, 33, 256, 8223, True, False),
     (Q4, 32, 4096, 6145, False, True), (Q4, 16, 3328, 33000, False, True), (Q4, 33, 4096, 4097, True, True),  # column groups
-    (Q4, 63, 4096, 14337, True, True), (Q4, 64, 1280, 33001, True, True), (Q4, 9, 2048, 65600, False, True),
-    (Q8, 9, 256, 33, False, False), (Q8, 17, 1024, 4096, True, False), (Q8, 33, 4096, 1023, True, False),
+    (Q4, 63, 4096, 14337, True, True), (Q4, 64, 1280, 32001, True, True), (Q4, 9, 2048, 65505, False, True),
+    (Q4, 64, 1280, 33001, True, False), (Q4, 65, 2048, 2047, False, False), (Q4, 96, 2048, 5633, True, False),  # ... beyond 64 rows
+    (Q4, 77, 4096, 6143, True, True), (Q4, 95, 3584, 10999, True, True), (Q4, 70, 14336, 1000, True, False),
+    (Q4, 96, 1024, 33001, True, False), (Q4, 65, 768, 513, True, False),
+    (Q8, 17, 256, 545, False, False), (Q8, 17, 1024, 4096, True, False), (Q8, 33, 4096, 1023, True, False),
     (Q8, 48, 1024, 4095, True, False), (Q8, 32, 2048, 8191, False, True), (Q8, 20, 1024, 14000, False, True),
 ])
 def test_column_groups_of_the_thirty_two_row_kernel(fmt, rows, in_dim, out_dim, pair, same):
