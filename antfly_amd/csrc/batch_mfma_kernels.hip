@@ -1784,7 +1784,9 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
     switch (plan.parts * 10 + plan.halves) {
         case 81: return AFHIP_BMG(1, 8, false);
         case 82: return AFHIP_BMG(2, 8, false);
-        case 84: return AFHIP_BMG(4, 8, false);
+        case 84:  // (Q4_0 alone)
+            if constexpr (kType == 2) return AFHIP_BMG(4, 8, false);
+            else return hipErrorInvalidValue;
         case 41: return AFHIP_BMG(1, 4, false);
         case 42: return AFHIP_BMG(2, 4, false);
         default: return hipErrorInvalidValue;
