@@ -1227,13 +1227,16 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch32_mfma_kernel(float* __re
 // by the first bytes' way from memory, 5000 cycles until a wavefront can start.  Q4_0, weights from memory, against the two kernels above
 // (us): 32 rows, K = 4096, 4096 columns 10.5 -> 9.8, 6144 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8; 48 rows, 2048 x 2048 11.9 -> 7.4;
 // 64 rows, a pair of 14336 columns 51.0 -> 35.6.
-template <int kType, int kLive, int kHalves, int kParts, bool kApart, bool kShared, bool kOne>
+//
+// kRows: the most rows a call has, 32 (one group of rows), 64 or (Q4_0) 96.
+template <int kType, int kLive, int kHalves, int kParts, bool kApart, int kRows, bool kOne>
 __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float* __restrict__ dst_a, float* __restrict__ partial_a,
                                                                       const uint32_t* __restrict__ qa, const float* __restrict__ sa,
                                                                       const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
                                                                       int share_blocks, int row_groups, int col_groups, Epilogue ep_a,
                                                                       BmSecond second, int accumulate) {
     using B = BatchGroups<kType, kLive, kHalves, kParts>;
+    constexpr bool kShared = kRows > 32;
     const bool is_b = blockIdx.z != 0;
     float* dst = is_b ? second.dst : dst_a;
     const uint8_t* weight = is_b ? second.weight : weight_a;
@@ -1331,6 +1334,13 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
 #pragma unroll
         for (int p = 0; p < kPairs; ++p) ta[hb][p] = scales_at[static_cast<size_t>(clamp_blk(hb, 2 * p + lh)) * padded + row0 + lr];
     };
+    // A packed nibble in its byte is sixteen times its value, which the weight scale takes back.  A sixteenth of a product of scales
+    // below 2^-122 is subnormal where the product may not be, though, and loses up to four of its bits.  Beyond 64 rows, where the other
+    // route is the GEMM, which keeps them, a wavefront that holds an activation scale below 2^-98 (the smallest fp16 scale is 2^-24; a
+    // block of activations below 4e-28, not all zeros) forms its sums again (form_again).  Up to 64 rows the kernels above, whose bits
+    // these are, lose them too.
+    constexpr bool kAgain = kType == 2 && kRows > 64;
+    bool small_scales = false;  // of the wavefront
     // The compiler counts only its own loads: a wait of its for one of them would be a wait for every request that left in
     // between.  So they are taken here, before the requests of the later stages leave.
     auto take_run = [&](int hb) {
@@ -1340,6 +1350,12 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
         for (int p = 0; p < kPairs; ++p) {
             asm volatile("" : "+v"(ta[hb][p]) : : "memory");
             if (first_of(hb) + 2 * p + lh >= share_end) ta[hb][p] = 0.0f;
+        }
+        if (kAgain) {
+            uint32_t least = ~0u;  // (a zero is no small scale: it wraps round to the largest)
+#pragma unroll
+            for (int p = 0; p < kPairs; ++p) least = min(least, __float_as_uint(ta[hb][p]) - 1u);
+            small_scales = small_scales || __ballot(least < 0x0E800000u - 1u) != 0;  // 2^-98
         }
     };
     // The first run's of all wavefronts go first: a barrier, reached within a few instructions, keeps the others behind them.  (Their
@@ -1435,6 +1451,52 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
     auto store_sums = [&](int s) {
 #pragma unroll
         for (int v = 0; v < kLive; ++v) red[(wave * kLive + v) * 64 + lane] = acc[s][v];
+    };
+    // The sums of runs [first, last) of a column group once more from plain products, operands straight from memory, where one of them is
+    // small enough to feel what was lost (as in gemm_i8_body: 2^-122 in all, which no sum from 2^-96 on does).
+    // Activations of 2^-111, products of scales just above 2^-126: the bits of ordinary ones scaled, as on the GEMM; a call without such
+    // scales pays for the test alone (77 rows, 2048 x 2048 7.74 -> 7.78 us, 96 rows, 4096 x 6144 18.4 / 18.3).
+    auto form_again = [&](int cg, int first, int last, float (&sum)[16]) {
+        int l = lane;
+        asm volatile("" : "+v"(l));  // (nothing of this takes registers in the loop)
+        const int column = l & 31, half_k = l >> 5;
+        float least = __builtin_huge_valf();
+#pragma unroll
+        for (int v = 0; v < kLive; ++v)
+            if (row0 + 8 * (v >> 2) + 4 * half_k + (v & 3) < rows) least = fminf(least, fabsf(sum[v]));
+        if (__ballot(least < 0x1p-96f) == 0) return;
+        float second[16];  // the odd blocks' sums where they are kept apart
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = second[v] = 0.0f;
+        const size_t n = min(n_first + cg * B::kGroupCols + side * 32 + column, out_dim - 1);
+        const uint16_t* block_scales = reinterpret_cast<const uint16_t*>(weight + blocks_total * kQB) + n * kb_full;
+#pragma unroll 1
+        for (int run = first; run < last && first_of(run) < share_end; ++run) {
+#pragma unroll 1
+            for (int blk = first_of(run); blk < first_of(run) + kHB; blk += 2) {
+                const bm_v4i* a = reinterpret_cast<const bm_v4i*>(qa) + (static_cast<size_t>(group) * kb_full + blk) * 64 + l;
+                const uint2* w = reinterpret_cast<const uint2*>(weight + (n * kb_full + blk) * kQB) + half_k;
+                const bm_v32f products = __builtin_amdgcn_mfma_f32_32x32x1f32(sa[static_cast<size_t>(blk + half_k) * padded + row0 + column],
+                                                                             half_bits_to_f32(block_scales[blk + half_k]), bm_v32f{}, 0, 0, 0);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint2 nibbles = w[h * (kQB / 8)];
+                    auto byte = [](uint32_t x) { return static_cast<int>((x & 0xF0F0F0F0u) ^ 0x80808080u); };
+                    const bm_v4i b = {byte(nibbles.x << 4), byte(nibbles.x), byte(nibbles.y << 4), byte(nibbles.y)};
+                    const bm_v16i dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[h * 64], b, bm_v16i{}, 0, 0, 0);
+                    float(&to)[16] = kOdd && h == 1 ? second : sum;
+#pragma unroll
+                    for (int v = 0; v < kLive; ++v) to[v] = __builtin_fmaf(products[16 * h + v], static_cast<float>(dot[v] >> 4), to[v]);
+                }
+            }
+            if (kOdd) {
+#pragma unroll
+                for (int v = 0; v < kLive; ++v) {
+                    sum[v] += second[v];
+                    second[v] = 0.0f;
+                }
+            }
+        }
     };
     auto add_up = [&](int cg, int s) {
         int side_tid = tid % kSideThreads;
@@ -1555,7 +1617,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
                     }
                 }
             }
+            if (kAgain && kApart && p % kPairs == kPairs - 1 && small_scales) form_again(cg, p / kPairs, p / kPairs + 1, acc[p / kPairs]);
             if (kPutDown && p == kSteps / 2 - 1) {
+                if (kAgain && small_scales) form_again(cg, 0, kHalves / 2, acc[0]);
                 store_sums(0);
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[0][v] = 0.0f;
@@ -1566,6 +1630,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
                 count_up(1);
             }
         }
+        if (kAgain && !kApart && small_scales) form_again(cg, kPutDown ? kHalves / 2 : 0, kHalves, acc[0]);
         if (kPutDown) {
 #pragma unroll
             for (int v = 0; v < kLive; ++v) acc[0][v] = red[(wave * kLive + v) * 64 + lane] + acc[0][v];
@@ -1756,24 +1821,25 @@ hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, c
     const dim3 grid(static_cast<unsigned>(plan.row_groups == 1 ? col_tiles : (col_tiles + 7) / 8 * 8 * plan.row_groups), static_cast<unsigned>(plan.shares),
                     second.weight ? 2u : 1u),
         block(kBmThreads);
-    static std::atomic<size_t> lds_limit[6] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
+    static std::atomic<size_t> lds_limit[8] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
     auto launch = [&](auto kernel, int lds, std::atomic<size_t>* limit) {
         if (hipError_t e = bm_allow_large_lds(kernel, lds, limit); e != hipSuccess) return e;
         hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, plan.shares > 1 && !accumulate ? partial : nullptr, qa, sa, weight, rows, in_dim,
                            out_dim, plan.share_blocks, plan.row_groups, plan.column_groups, ep, second, accumulate ? 1 : 0);
         return hipGetLastError();
     };
-    auto launch_for = [&](auto live, auto shared, int at) {
-        constexpr int kLive = decltype(live)::value;
-        constexpr bool kShared = decltype(shared)::value;
+    auto launch_for = [&](auto live, auto rows_to, int at) {
+        constexpr int kLive = decltype(live)::value, kRows = decltype(rows_to)::value;
         constexpr int lds = BatchGroups<kType, kLive, kHalves, kParts>::kLdsBytes;
-        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kShared, true>, lds, &lds_limit[at]);
+        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kRows, true>, lds, &lds_limit[at]);
         if constexpr (kHalves == 4 || kApart) return hipErrorInvalidValue;  // (not among the plans)
-        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kShared, false>, lds, &lds_limit[at + 1]);
+        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kRows, false>, lds, &lds_limit[at + 1]);
     };
-    if (plan.row_groups > 1) return launch_for(std::integral_constant<int, 16>{}, std::true_type{}, 0);
-    if (rows <= 16) return launch_for(std::integral_constant<int, 8>{}, std::false_type{}, 2);
-    return launch_for(std::integral_constant<int, 16>{}, std::false_type{}, 4);
+    if constexpr (kType == 2)
+        if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
+    if (rows > 32) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 64>{}, 0);
+    if (rows <= 16) return launch_for(std::integral_constant<int, 8>{}, std::integral_constant<int, 32>{}, 2);
+    return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 32>{}, 4);
 }
 
 template <int kType>

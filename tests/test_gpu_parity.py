@@ -273,6 +273,36 @@ def test_prefill_keeps_small_activations(fmt, rows, in_dim, out_dim):
     assert np.array_equal(G.linear(fmt, PREP, x_small, wd, rows, in_dim, out_dim), want)
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim,bias", [
+    (77, 2048, 2048, False), (96, 2048, 5632, False), (65, 3584, 2001, False),  # a run a wavefront on one group of columns, on several; two
+    (96, 4096, 6145, False), (66, 4096, 1000, True), (80, 4096, 1000, False),   # ... on several, two apart, two K shares
+    (70, 14336, 1000, False), (90, 14336, 1000, True),                          # four a wavefront
+    (65, 768, 513, False), (96, 1024, 33001, False)])                           # four wavefronts on K
+def test_short_prompts_keep_small_activations(rows, in_dim, out_dim, bias):
+    """65 to 96 rows of Q4_0: rows scaled by powers of two give the same bits scaled, from scale products just above 2^-126 (as
+    test_prefill_keeps_small_activations) to activations of 2^100, and rows of one call do not feel each other.  Rows around 2^87
+    whose parts of K differ by a factor of two cross the line above which a row's scales are divided by 16, in either order."""
+    print(f"case: small activations, short prompts rows={rows} in={in_dim} out={out_dim} bias={bias}", flush=True)
+    rng = np.random.default_rng(19 * rows + in_dim)
+    x = rng.uniform(-1.0, 1.0, (rows, in_dim)).astype(np.float32)
+    x[:, ::32] = rng.uniform(1.0, 1.5, x[:, ::32].shape)  # every block's peak: all scales within a factor of three
+    w = synth.weights(Q4, out_dim + 3, out_dim, in_dim)
+    blocks = w.reshape(out_dim * in_dim // 32, -1)
+    blocks[:, :2] = rng.uniform(2.0 ** -8, 2.0 ** -7, len(blocks)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    block = np.arange(in_dim) // 32
+    doubled = [block // 8 % 2 == 1, 2 * block >= in_dim // 32, 2 * block < in_dim // 32]
+    for i, part in enumerate(doubled):
+        x[2 + i::6, part] *= 2.0
+    factor = np.array([2.0 ** (-126 + 15), 2.0 ** 100, 2.0 ** 86, 2.0 ** 86, 2.0 ** 86, 1.0])[np.arange(rows) % 6]
+    scaled = (x.astype(np.float64) * factor[:, None]).astype(np.float32)
+    wd = G.prepare(Q4, w, out_dim, in_dim)
+    if bias:
+        y, got = (G.linear_bias(Q4, PREP, each, wd, np.zeros(out_dim, np.float32), rows, in_dim, out_dim) for each in (x, scaled))
+    else:
+        y, got = (G.linear(Q4, PREP, each, wd, rows, in_dim, out_dim) for each in (x, scaled))
+    assert np.array_equal(got, (y.astype(np.float64) * factor[:, None]).astype(np.float32))
+
+
 SHAPES_B = [(1, 32, 3), (2, 64, 600), (3, 96, 11), (4, 4096, 100), (1, 64, 4096), (12, 128, 40)]
 
 
