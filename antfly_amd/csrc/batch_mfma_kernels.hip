@@ -55,6 +55,7 @@ namespace {
 
 typedef int bm_v4i __attribute__((ext_vector_type(4)));
 typedef int bm_v16i __attribute__((ext_vector_type(16)));
+typedef float bm_v16f __attribute__((ext_vector_type(16)));
 typedef float bm_v32f __attribute__((ext_vector_type(32)));
 
 constexpr int kBmWaves = 8;
@@ -1228,15 +1229,16 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch32_mfma_kernel(float* __re
 // (us): 32 rows, K = 4096, 4096 columns 10.5 -> 9.8, 6144 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8; 48 rows, 2048 x 2048 11.9 -> 7.4;
 // 64 rows, a pair of 14336 columns 51.0 -> 35.6.
 //
-// kRows: the most rows a call has, 32 (one group of rows), 64 or (Q4_0) 96.
-template <int kType, int kLive, int kHalves, int kParts, bool kApart, int kRows, bool kOne>
+// kRows: the most rows a call has, 32 (one group of rows), 64 or (Q4_0) 96.  kChains: 0, a wavefront's blocks are added up one after
+// the other (a single run's even and odd ones apart); 1, even and odd ones apart; 2, and the sums of its runs too.
+template <int kType, int kLive, int kHalves, int kParts, int kChains, int kRows, bool kOne>
 __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float* __restrict__ dst_a, float* __restrict__ partial_a,
                                                                       const uint32_t* __restrict__ qa, const float* __restrict__ sa,
                                                                       const uint8_t* __restrict__ weight_a, int rows, int in_dim, int out_dim,
                                                                       int share_blocks, int row_groups, int col_groups, Epilogue ep_a,
                                                                       BmSecond second, int accumulate) {
     using B = BatchGroups<kType, kLive, kHalves, kParts>;
-    constexpr bool kShared = kRows > 32;
+    constexpr bool kShared = kRows > 32, kApart = kChains == 2;
     const bool is_b = blockIdx.z != 0;
     float* dst = is_b ? second.dst : dst_a;
     const uint8_t* weight = is_b ? second.weight : weight_a;
@@ -1264,9 +1266,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
     const int share_end = min(share_begin + share_blocks, kb_full);
     const int part = wave % kParts, side = wave / kParts;  // of K; of the group's columns
     // Run hb of this wavefront is the kHB blocks first_of(hb) + [0, kHB).  Two runs follow on each other, a slice of blocks as
-    // batch_mfma_kernel's; four, and those whose sums are kept apart, are a row of all wavefronts' each.  Indices past the end are
+    // batch_mfma_kernel's; four, and two in chains of their own, are a row of all wavefronts' each.  Indices past the end are
     // clamped to a valid block for every load; their activation scales are zero.
-    auto first_of = [&](int hb) { return share_begin + (kHalves == 2 && !kApart ? (part * 2 + hb) * kHB : hb * kRun + part * kHB); };
+    auto first_of = [&](int hb) { return share_begin + (kHalves == 2 && kChains == 0 ? (part * 2 + hb) * kHB : hb * kRun + part * kHB); };
     auto clamp_blk = [&](int hb, int j) { return min(first_of(hb) + j, share_end - 1); };
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(bm_lds)));
     const uint32_t lds_slots = lds0 + wave * (kSlots * B::kSlotBytes);
@@ -1428,7 +1430,11 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
     static_assert(!kPutDown || kOne, "the room is free for the one column group only");
     constexpr int kSums = kApart ? kHalves : 1;
     // ... and where a run's sums are added up by themselves, four: even and odd blocks apart.
-    constexpr bool kOdd = kHalves == 1 || kApart;
+    constexpr bool kOdd = kHalves == 1 || kChains > 0;
+    // Two runs' fragments, even and odd sums and two sets of results are more than the registers hold (12 spilled, reloaded in the loop):
+    // there the next pair's dots take the registers of this pair's as these are read, half a step before they are needed.
+    constexpr bool kOneResult = kHalves == 2 && kChains == 1 && !kOne;
+    auto last_of_chain = [](int run) { return kApart || run + 1 == kHalves; };  // where even and odd blocks meet
     float acc[kSums][16], odd[16];
 
     // ---- the wavefronts' sums meet in LDS: [side][part of K][v][lane]; a thread adds up neighbouring columns of a row.  kApart: the sums
@@ -1476,26 +1482,23 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             for (int blk = first_of(run); blk < first_of(run) + kHB; blk += 2) {
                 const bm_v4i* a = reinterpret_cast<const bm_v4i*>(qa) + (static_cast<size_t>(group) * kb_full + blk) * 64 + l;
                 const uint2* w = reinterpret_cast<const uint2*>(weight + (n * kb_full + blk) * kQB) + half_k;
-                const bm_v32f products = __builtin_amdgcn_mfma_f32_32x32x1f32(sa[static_cast<size_t>(blk + half_k) * padded + row0 + column],
-                                                                             half_bits_to_f32(block_scales[blk + half_k]), bm_v32f{}, 0, 0, 0);
+                const float x_scale = sa[static_cast<size_t>(blk + half_k) * padded + row0 + column], w_scale = half_bits_to_f32(block_scales[blk + half_k]);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
+                    const bm_v16f products = __builtin_amdgcn_mfma_f32_32x32x2f32(half_k == h ? x_scale : 0.0f, half_k == h ? w_scale : 0.0f, bm_v16f{}, 0, 0, 0);
                     const uint2 nibbles = w[h * (kQB / 8)];
                     auto byte = [](uint32_t x) { return static_cast<int>((x & 0xF0F0F0F0u) ^ 0x80808080u); };
                     const bm_v4i b = {byte(nibbles.x << 4), byte(nibbles.x), byte(nibbles.y << 4), byte(nibbles.y)};
                     const bm_v16i dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[h * 64], b, bm_v16i{}, 0, 0, 0);
                     float(&to)[16] = kOdd && h == 1 ? second : sum;
 #pragma unroll
-                    for (int v = 0; v < kLive; ++v) to[v] = __builtin_fmaf(products[16 * h + v], static_cast<float>(dot[v] >> 4), to[v]);
+                    for (int v = 0; v < kLive; ++v) to[v] = __builtin_fmaf(products[v], static_cast<float>(dot[v] >> 4), to[v]);
                 }
             }
-            if (kOdd) {
+        }
+        if (kOdd) {
 #pragma unroll
-                for (int v = 0; v < kLive; ++v) {
-                    sum[v] += second[v];
-                    second[v] = 0.0f;
-                }
-            }
+            for (int v = 0; v < kLive; ++v) sum[v] += second[v];
         }
     };
     auto add_up = [&](int cg, int s) {
@@ -1583,7 +1586,20 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
                 for (int v = 0; v < kLive; ++v)
                     if (v >= first && v < last) sum[v] = __builtin_fmaf(t[cur][16 * h + v], static_cast<float>(c[v]), sum[v]);
             };
-            if constexpr (kSets == 2) {
+            if constexpr (kOneResult) {
+                multiply(c0[0], 0, 0, kLive / 2);
+                __builtin_amdgcn_sched_barrier(0);
+                t[set] = __builtin_amdgcn_mfma_f32_32x32x1f32(ta[hm][qm], tb, zf, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c0[0], 0, kLive / 2, kLive);
+                __builtin_amdgcn_sched_barrier(0);
+                c0[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm], b0, zi, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(c1[0], 1, 0, kLive);
+                __builtin_amdgcn_sched_barrier(0);
+                c1[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm + 1], b1, zi, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            } else if constexpr (kSets == 2) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (!beyond) c0[set] = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag[hm][2 * qm], b0, zi, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1609,7 +1625,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             fence_registers(acc[kApart ? p / kPairs : 0]);
             if (kOdd) {
                 fence_registers(odd);
-                if (p % kPairs == kPairs - 1) {
+                if (p % kPairs == kPairs - 1 && last_of_chain(p / kPairs)) {
 #pragma unroll
                     for (int v = 0; v < kLive; ++v) {
                         acc[kApart ? p / kPairs : 0][v] += odd[v];
@@ -1809,12 +1825,12 @@ hipError_t bm_launch32(hipStream_t stream, float* dst, float* partial, const uin
 // stages a wavefront and column group, K shares.
 struct BatchGroupsPlan {
     int row_groups, column_groups, parts, halves, shares, share_blocks;
-    bool apart;
+    int chains;  // kChains
     bool own_sums;  // the sums are not formed in the older kernels' order
     long grid;  // workgroups
 };
 
-template <int kType, int kHalves, int kParts, bool kApart>
+template <int kType, int kHalves, int kParts, int kChains>
 hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
                        int in_dim, int out_dim, const BatchGroupsPlan& plan, const Epilogue& ep, const BmSecond& second, bool accumulate) {
     const int cols = 32 * (kBmWaves / kParts) * plan.column_groups, col_tiles = (out_dim + cols - 1) / cols;
@@ -1831,10 +1847,14 @@ hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, c
     auto launch_for = [&](auto live, auto rows_to, int at) {
         constexpr int kLive = decltype(live)::value, kRows = decltype(rows_to)::value;
         constexpr int lds = BatchGroups<kType, kLive, kHalves, kParts>::kLdsBytes;
-        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kRows, true>, lds, &lds_limit[at]);
-        if constexpr (kHalves == 4 || kApart) return hipErrorInvalidValue;  // (not among the plans)
-        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kApart, kRows, false>, lds, &lds_limit[at + 1]);
+        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, true>, lds, &lds_limit[at]);
+        if constexpr (kHalves == 4 || kChains == 2) return hipErrorInvalidValue;  // (not among the plans)
+        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, false>, lds, &lds_limit[at + 1]);
     };
+    if constexpr (kChains == 1) {
+        if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
+        return hipErrorInvalidValue;  // (not among the plans)
+    }
     if constexpr (kType == 2)
         if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
     if (rows > 32) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 64>{}, 0);
@@ -1845,16 +1865,21 @@ hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, c
 template <int kType>
 hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
                             int in_dim, int out_dim, const BatchGroupsPlan& plan, const Epilogue& ep, const BmSecond& second, bool accumulate) {
-#define AFHIP_BMG(H, P, APART) bm_launch_groups_of<kType, H, P, APART>(stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, plan, ep, second, accumulate)
-    if (plan.apart) return plan.halves == 2 && plan.parts == 8 ? AFHIP_BMG(2, 8, true) : hipErrorInvalidValue;
+#define AFHIP_BMG(H, P, CHAINS) bm_launch_groups_of<kType, H, P, CHAINS>(stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, plan, ep, second, accumulate)
+    if (plan.chains == 2) return plan.halves == 2 && plan.parts == 8 ? AFHIP_BMG(2, 8, 2) : hipErrorInvalidValue;
+    if (plan.chains == 1) {
+        if constexpr (kType == 2)
+            if (plan.halves == 2) return plan.parts == 8 ? AFHIP_BMG(2, 8, 1) : AFHIP_BMG(2, 4, 1);
+        return hipErrorInvalidValue;
+    }
     switch (plan.parts * 10 + plan.halves) {
-        case 81: return AFHIP_BMG(1, 8, false);
-        case 82: return AFHIP_BMG(2, 8, false);
+        case 81: return AFHIP_BMG(1, 8, 0);
+        case 82: return AFHIP_BMG(2, 8, 0);
         case 84:  // (Q4_0 alone)
-            if constexpr (kType == 2) return AFHIP_BMG(4, 8, false);
+            if constexpr (kType == 2) return AFHIP_BMG(4, 8, 0);
             else return hipErrorInvalidValue;
-        case 41: return AFHIP_BMG(1, 4, false);
-        case 42: return AFHIP_BMG(2, 4, false);
+        case 41: return AFHIP_BMG(1, 4, 0);
+        case 42: return AFHIP_BMG(2, 4, 0);
         default: return hipErrorInvalidValue;
     }
 #undef AFHIP_BMG
@@ -1869,6 +1894,11 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
 //     result; an op with an epilogue keeps the two runs' sums apart instead (no reduce launch).  32 rows, 2048 x 2048 9.3 -> 7.7 us.
 //   * Four runs a share on few columns only, where a launch is mostly its way to the first bytes (K = 14336 x 4096 columns 19.1 -> 18.1,
 //     11008 18.1 -> 17.6); on more columns the older kernels' K shares are better (8192 x 8192 18.4 against 16.4).
+//   * Beyond 64 rows, where the other route is the GEMM, which shares K out on one group of columns: a wavefront's two runs go into chains
+//     of even and odd blocks, and K shares are equal.  Error against the GEMM's, a chain of sixteen in brackets: 77 x 4096 x 2048 0.89
+//     (1.01), 96 x 2304 x 1500 0.95 (1.14), 66 x 4352 x 1024 0.95 (1.13), 77 x 2048 x 8192 0.87 (1.00); 10.28 -> 10.33, 9.78 -> 9.91, 10.7 ->
+//     10.9, 14.1 -> 14.3 us.  On several groups of columns the GEMM takes K whole, a chain of sixteen has 0.81 .. 1.0 of its error, and
+//     the bits are batch_mfma_kernel's.
 //   * Q8_0, twice the bytes for the same arithmetic, is bound by the bytes sooner: few columns on 32 rows from K = 1024 up only at an
 //     eighth of the units (1024 columns, K = 2048 7.6 -> 6.7, a pair of 4096 x 4096 columns 13.2 against 14.6 here); one run of eight
 //     wavefronts on many columns only at 33 rows and more (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
@@ -1900,20 +1930,24 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     }
     const int run = p.parts * stage_blocks, runs = (kb + run - 1) / run;
     p.shares = (runs + 3) / 4;
-    p.apart = false;
+    p.chains = 0;
     if (few && runs > 1 && p.shares == 1) {
         if (adds || runs > 2) p.shares = 2;
-        else p.apart = true;
+        else p.chains = 2;
     }
     p.halves = (runs + p.shares - 1) / p.shares;
     p.share_blocks = p.halves * run;
     if (p.halves == 3) p.halves = 4;
     p.shares = (kb + p.share_blocks - 1) / p.share_blocks;
-    p.own_sums = few || p.halves != 2;
+    p.own_sums = few || p.halves != 2;  // (up to 64 rows)
     if (p.halves == 4 && (!few || tensor_type == 8)) return false;
     if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 ? 8 : 4 * p.row_groups) * columns > units) return false;
     if (tensor_type == 8 && !few && p.halves == 1 && p.parts == 8 && p.row_groups == 1) return false;
-    p.column_groups = p.apart || p.halves == 4 ? 1 : static_cast<int>(groups_for(pair ? 2 : 1));
+    if (rows > 64 && p.halves == 2 && p.chains == 0 && (few || p.parts == 4 || groups_for(1) == 1)) {
+        p.chains = 1;
+        if (p.shares > 1) p.share_blocks = ((kb + p.shares - 1) / p.shares + stage_blocks - 1) / stage_blocks * stage_blocks;
+    }
+    p.column_groups = p.chains == 2 || p.halves == 4 ? 1 : static_cast<int>(groups_for(pair ? 2 : 1));
     p.grid = grid(p.column_groups, pair ? 2 : 1);
     *plan = p;
     return true;
@@ -1966,7 +2000,7 @@ size_t batch_mfma_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, s
 // 8192, four, 21.7 against 22.2), with one run of K four (K = 2048: 5632 columns 14.4 -> 12.4, a pair 21.0 -> 17.8, 8192 15.0 -> 14.1);
 // beyond, it starts another round (K = 4096: 11008 columns 31.8 -> 26.2, 14336 32.4 -> 29.5, a pair 56 -> 49.5; K = 2048 x 16384 22.3 / 22.6,
 // 24576 34.4 -> 27.0).  K that fills less than seven eighths of the wavefronts' stages stays with the GEMM (3072 x 8192 18.8 against 21.6).
-// The error against 64 bits is that of the calls of fewer rows, 6.2e-8 .. 1.0e-7 (the GEMM's 6.4e-8 .. 1.5e-7).
+// The error against 64 bits is 0.81 to 1.0 of the GEMM's (5.6e-8 .. 9.8e-8 on 48 shapes, the GEMM's 5.7e-8 .. 1.16e-7).
 bool batch_mfma_column_groups(int tensor_type, size_t rows, size_t in_dim, size_t out_dim) {
     BatchGroupsPlan plan;
     if (rows <= 64 || !batch_mfma_supports(tensor_type, rows, in_dim, out_dim) ||

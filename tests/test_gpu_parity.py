@@ -303,6 +303,56 @@ def test_short_prompts_keep_small_activations(rows, in_dim, out_dim, bias):
     assert np.array_equal(got, (y.astype(np.float64) * factor[:, None]).astype(np.float32))
 
 
+def short_chain_sums(dots: np.ndarray, products: np.ndarray, shares: int, wavefronts: int) -> np.ndarray:
+    """f32 sums over blocks (the last axis) of products * dots as K shares, runs of eight blocks a wavefront, even and odd blocks of a
+    wavefront, then its four (and four) wavefronts make them.  (Fused multiply-adds in float64 rounded to f32: the product of 24 and 20
+    bits is exact, a double rounding takes a tie of one in 2^29.)"""
+    blocks = dots.shape[-1]
+    share_blocks = (blocks + 8 * shares - 1) // (8 * shares) * 8
+    total = None
+    for begin in range(0, blocks, share_blocks):
+        end = min(begin + share_blocks, blocks)
+        waves = []
+        for part in range(wavefronts):
+            mine = [b for first in range(begin + 8 * part, end, 8 * wavefronts) for b in range(first, min(first + 8, end))]
+            chains = []
+            for odd in (0, 1):
+                acc = np.zeros(dots.shape[:-1], np.float32)
+                for b in mine[odd::2]:
+                    acc = (products[..., b].astype(np.float64) * dots[..., b] + acc).astype(np.float32)
+                chains.append(acc)
+            waves.append(chains[0] + chains[1])
+        halves = [((waves[i] + waves[i + 1]) + waves[i + 2]) + waves[i + 3] for i in range(0, wavefronts, 4)]
+        share = halves[0] if wavefronts == 4 else halves[0] + halves[1]
+        total = share if total is None else total + share
+    return total
+
+
+@pytest.mark.parametrize("rows,in_dim,out_dim,shares,wavefronts", [
+    (77, 4096, 2048, 1, 8), (65, 3584, 2559, 1, 8), (96, 2304, 1500, 1, 8),  # two runs, one group of columns (a pair: two)
+    (70, 6144, 700, 2, 8), (66, 4352, 1000, 2, 8), (80, 8192, 1344, 2, 8),   # ... on two K shares
+    (77, 2048, 2730, 1, 4), (96, 1792, 8201, 1, 4),                          # ... of four wavefronts, several groups
+    (77, 2048, 2048, 1, 8), (65, 768, 513, 1, 4)])                           # one run
+def test_short_prompts_add_up_in_short_chains(rows, in_dim, out_dim, shares, wavefronts):
+    """65 to 96 rows of Q4_0 where the GEMM shares K out: no chain of additions longer than eight blocks, bit for bit the sums in that
+    order, from the plain call, a pair and a call with a bias."""
+    print(f"case: short chains rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x = synth.activations(6100 + rows, rows, in_dim)
+    w = [synth.weights(Q4, 6101 + i, out_dim, in_dim) for i in range(2)]
+    wd = [G.prepare(Q4, each, out_dim, in_dim) for each in w]
+    got = [G.linear(Q4, PREP, x, wd[0], rows, in_dim, out_dim)]
+    got += [G.linear_pair(Q4, PREP, x, wd[1], wd[0], rows, in_dim, out_dim)[1]]
+    got += [G.linear_bias(Q4, PREP, x, wd[0], np.zeros(out_dim, np.float32), rows, in_dim, out_dim)]
+    sample, columns = np.r_[0, 31:34, rows - 1], np.r_[0:32, out_dim - 65:out_dim]
+    _, row_scales, _ = O.quantize_activation_rows(x[sample], len(sample), in_dim)
+    blocks = w[0].reshape(out_dim, -1, 18)[columns]
+    scales = blocks[..., :2].copy().view(np.float16)[..., 0].astype(np.float32)
+    want = short_chain_sums(O.block_dots(Q4, x[sample], blocks.reshape(-1), len(sample), in_dim, len(columns)),
+                            row_scales[:, None, :] * scales[None], shares, wavefronts)
+    for y in got:
+        assert np.array_equal(y[np.ix_(sample, columns)], want)
+
+
 SHAPES_B = [(1, 32, 3), (2, 64, 600), (3, 96, 11), (4, 4096, 100), (1, 64, 4096), (12, 128, 40)]
 
 
