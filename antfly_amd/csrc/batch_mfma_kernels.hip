@@ -1526,14 +1526,35 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             }
             return;
         }
+        // finish_output for neighbouring columns together, the activations out of the way: one column after the other it took 0.7 us of a small
+        // call (Q8_0 17 x 256 x 512 with a bias 6.86 -> 6.16, without 5.7; Q4_0 48 x 4096 x 8192 with a bias 17.2 -> 16.65)
+        if (partial == nullptr && !accumulate) {
+            if (ep.bias != nullptr) {
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) total[k] += ep.bias[min(n + k, out_dim - 1)];
+            }
+            if (__builtin_expect(ep.activation != kActNone, 0)) {
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) total[k] = activate(ep.activation, total[k]);
+            }
+            if (ep.residual != nullptr) {
+#pragma unroll
+                for (int k = 0; k < kPer; ++k)
+                    total[k] += ep.residual[static_cast<size_t>(min(m, rows - 1)) * out_dim + min(n + k, out_dim - 1)];
+            }
+        }
+        if (m >= rows) return;
+        float* const to = (partial != nullptr ? partial + static_cast<size_t>(blockIdx.y) * rows * out_dim : dst) + static_cast<size_t>(m) * out_dim + n;
+        if (!accumulate && n + kPer <= out_dim) {
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) to[k] = total[k];
+            return;
+        }
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            if (m < rows && n + k < out_dim) {
-                const size_t at = static_cast<size_t>(m) * out_dim + n + k;
-                if (partial != nullptr) partial[static_cast<size_t>(blockIdx.y) * rows * out_dim + at] = total[k];
-                else if (accumulate) unsafeAtomicAdd(dst + at, total[k]);  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
-                else dst[at] = finish_output(ep, n + k, at, total[k]);
-            }
+            if (n + k >= out_dim) break;
+            if (accumulate) unsafeAtomicAdd(to + k, total[k]);  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
+            else to[k] = total[k];
         }
     };
 

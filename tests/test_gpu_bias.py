@@ -161,6 +161,31 @@ def test_fused_epilogues(fmt, rows, in_dim, out_dim):
         assert G.max_rel_err(relu, ref.astype(np.float64)) <= TIGHT
 
 
+@pytest.mark.parametrize("fmt,rows,in_dim,out_dim", [
+    (Q8, 17, 256, 2047), (Q8, 40, 2048, 1023), (Q4, 32, 4096, 6145), (Q4, 13, 1024, 9001),  # one group of columns; two runs apart
+    (Q4, 63, 4096, 6145), (Q4, 16, 3328, 33001), (Q4, 77, 4096, 6143), (Q4, 66, 4096, 1001)])  # several; beyond 64 rows
+def test_fused_epilogues_of_column_groups(fmt, rows, in_dim, out_dim):
+    """The column-group kernel, which finishes neighbouring columns together, with odd rows and columns: the stored value is
+    act(product + bias) + residual, also where the residual lies in the result's place."""
+    print(f"case: column-group epilogues fmt={fmt} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    x, w = synth.activations(680 + rows, rows, in_dim) * 4.0, synth.weights(fmt, 681, out_dim, in_dim)
+    b, res = bias_vector(682, out_dim), synth.activations(683, rows, out_dim)
+    wd = G.prepare(fmt, w, out_dim, in_dim)
+    plain = G.linear(fmt, PREP, x, wd, rows, in_dim, out_dim)
+    biased = linear_epilogue(fmt, PREP, x, wd, rows, in_dim, out_dim, bias=b)
+    assert np.array_equal(biased, plain + b)
+    assert np.array_equal(linear_epilogue(fmt, PREP, x, wd, rows, in_dim, out_dim, residual=res), plain + res)
+    both = linear_epilogue(fmt, PREP, x, wd, rows, in_dim, out_dim, bias=b, residual=res, activation=_lib.ACTIVATION_RELU)
+    assert np.array_equal(both, np.maximum(biased, 0) + res)
+    gelu = linear_epilogue(fmt, PREP, x, wd, rows, in_dim, out_dim, bias=b, activation=_lib.ACTIVATION_GELU)
+    assert np.allclose(gelu, O.apply_activation(O.GELU, biased), rtol=3e-6, atol=1e-6 * np.abs(biased).max())
+    y, xd, bd = G.to_dev(res), G.to_dev(x), G.to_dev(b)
+    ws = torch.empty(max(kernels.workspaceBytes(fmt, rows, in_dim, out_dim), 16), dtype=torch.uint8, device=G.DEV)
+    kernels.launchLinearEpilogueF32(G.stream(), fmt, PREP, G.buf(y), G.buf(xd), G.buf(wd), rows, in_dim, out_dim, G.buf(bd), G.buf(y), 0, G.buf(ws))
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), biased + res)
+
+
 @pytest.mark.parametrize("rows,in_dim,out_dim", [(69, 256, 1000), (333, 4096, 4090), (669, 1024, 5603), (130, 6144, 1030)])
 def test_fused_epilogues_of_q4_k_prefills(rows, in_dim, out_dim):
     """Past 64 rows: each tile of the 6-bit kernel on odd rows and columns, and K shares (the reduce kernel's epilogue): the stored
