@@ -1913,16 +1913,21 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
 //     wavefronts and 32 columns leave fewer rounds (K = 2048: 128256 columns 46 against 51, but 77 rows, 5632 columns 13.8 -> 12.4).
 //   * Few columns (a matrix's 32 x 32 tiles fill at most half of the units): K goes to twice the workgroups, two shares that add to the
 //     result; an op with an epilogue keeps the two runs' sums apart instead (no reduce launch).  32 rows, 2048 x 2048 9.3 -> 7.7 us.
-//   * Four runs a share on few columns only, where a launch is mostly its way to the first bytes (K = 14336 x 4096 columns 19.1 -> 18.1,
-//     11008 18.1 -> 17.6); on more columns the older kernels' K shares are better (8192 x 8192 18.4 against 16.4).
+//   * Two shares of two runs add a reduce launch to an op with an epilogue and take twice the workgroups: on 32 rows only where a pair is one
+//     round too (K = 5632: 2048 columns 10.9 -> 10.5, but a pair of 4096 14.6 against 16.8), beyond 64 where one matrix is (1344 columns with
+//     a bias 14.7 against 17.1).
+//   * Four runs a share on 33 to 64 rows and few columns only (a pair in one round: 48 rows, K = 14336 x 1024 columns 18.6 -> 16.3, with a bias
+//     18.9 -> 18.5, 2048 columns 19.4 -> 17.9, but a pair 29.6 against 31.1).  On 32 rows the older kernels' K shares are better, most of all
+//     for an op with an epilogue (14336 x 1024 14.1 against 16.1, with a bias 14.3 against 18.5; 14336 x 4096 19.1 -> 18.3, but with a bias
+//     19.3 against 21.3), beyond 64 the GEMM's (11008 x 512 15.1 against 16.2, with a bias 15.5 against 18.8).
 //   * Beyond 64 rows, where the other route is the GEMM, which shares K out on one group of columns: a wavefront's two runs go into chains
 //     of even and odd blocks, and K shares are equal.  Error against the GEMM's, a chain of sixteen in brackets: 77 x 4096 x 2048 0.89
 //     (1.01), 96 x 2304 x 1500 0.95 (1.14), 66 x 4352 x 1024 0.95 (1.13), 77 x 2048 x 8192 0.87 (1.00); 10.28 -> 10.33, 9.78 -> 9.91, 10.7 ->
 //     10.9, 14.1 -> 14.3 us.  On several groups of columns the GEMM takes K whole, a chain of sixteen has 0.81 .. 1.0 of its error, and
 //     the bits are batch_mfma_kernel's.
-//   * Q8_0, twice the bytes for the same arithmetic, is bound by the bytes sooner: few columns on 32 rows from K = 1024 up only at an
-//     eighth of the units (1024 columns, K = 2048 7.6 -> 6.7, a pair of 4096 x 4096 columns 13.2 against 14.6 here); one run of eight
-//     wavefronts on many columns only at 33 rows and more (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
+//   * Q8_0, twice the bytes for the same arithmetic, is bound by the bytes sooner: two runs on few columns only at 33 rows and more (32 rows,
+//     1280 x 1024 7.1 -> 6.55, but with a bias 8.0 against 8.4; a pair of 4096 x 4096 columns 13.2 against 14.6); one run of eight wavefronts
+//     on many columns likewise (a pair of 8192 columns, K = 1024, 32 rows 10.5 against 10.8).
 bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool pair, bool adds, BatchGroupsPlan* plan) {
     const int kb = in_dim / 32, stage_blocks = tensor_type == 2 ? 8 : 4;
     if (kb % 8 != 0) return false;
@@ -1961,10 +1966,11 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     if (p.halves == 3) p.halves = 4;
     p.shares = (kb + p.share_blocks - 1) / p.share_blocks;
     p.own_sums = few || p.halves != 2;  // (up to 64 rows)
-    if (p.halves == 4 && (!few || tensor_type == 8)) return false;
-    if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 ? 8 : 4 * p.row_groups) * columns > units) return false;
+    if (p.shares == 2 && p.halves == 2 && (p.row_groups == 1 ? grid(1, 2) : (p.row_groups == 3 ? grid(1, 1) : 0)) > units) return false;
+    if (p.halves == 4 && (!few || tensor_type == 8 || p.row_groups != 2 || grid(1, 2) > units)) return false;
+    if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 || 4 * p.row_groups * columns > units)) return false;
     if (tensor_type == 8 && !few && p.halves == 1 && p.parts == 8 && p.row_groups == 1) return false;
-    if (rows > 64 && p.halves == 2 && p.chains == 0 && (few || p.parts == 4 || groups_for(1) == 1)) {
+    if (rows > 64 && p.halves == 2 && p.chains == 0 && (p.parts == 4 || groups_for(1) == 1)) {
         p.chains = 1;
         if (p.shares > 1) p.share_blocks = ((kb + p.shares - 1) / p.shares + stage_blocks - 1) / stage_blocks * stage_blocks;
     }
@@ -2021,6 +2027,10 @@ size_t batch_mfma_workspace_bytes(int tensor_type, size_t rows, size_t in_dim, s
 // 8192, four, 21.7 against 22.2), with one run of K four (K = 2048: 5632 columns 14.4 -> 12.4, a pair 21.0 -> 17.8, 8192 15.0 -> 14.1);
 // beyond, it starts another round (K = 4096: 11008 columns 31.8 -> 26.2, 14336 32.4 -> 29.5, a pair 56 -> 49.5; K = 2048 x 16384 22.3 / 22.6,
 // 24576 34.4 -> 27.0).  K that fills less than seven eighths of the wavefronts' stages stays with the GEMM (3072 x 8192 18.8 against 21.6).
+// From three rounds of the GEMM on (a unit's tiles, of which one is a column group of four wavefronts' K or two of eight's) no more column
+// groups than rounds: 80 rows, K = 2048: 14336 columns, three and three, 21.3 -> 19.7, 16384, four and three, 21.4 against 22.5 (with a bias
+// 21.9 against 24.2), 18432, four and four, 25.4 -> 22.7; K = 3584 x 16384, seven and three, 32.5 against 32.9 (bias 33.1 against 35.3).  A
+// pair in its own rounds where eight XCDs share the tile columns evenly (8192 columns, K = 2048 21.4 against 22.3; 8064 22.8 -> 22.4).
 // The error against 64 bits is 0.81 to 1.0 of the GEMM's (5.6e-8 .. 9.8e-8 on 48 shapes, the GEMM's 5.7e-8 .. 1.16e-7).
 bool batch_mfma_column_groups(int tensor_type, size_t rows, size_t in_dim, size_t out_dim) {
     BatchGroupsPlan plan;
@@ -2028,10 +2038,17 @@ bool batch_mfma_column_groups(int tensor_type, size_t rows, size_t in_dim, size_
         !batch_groups_plan(tensor_type, static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), false, true, &plan))
         return false;
     const long room = static_cast<long>(plan.halves) * plan.parts * (tensor_type == 2 ? 8 : 4), kb = static_cast<long>(in_dim / 32);
-    const long gemm_grid = static_cast<long>((rows + 31) / 32 * ((out_dim + 63) / 64));
+    const long units = gemv_compute_units(), gemm_cols = static_cast<long>((out_dim + 63) / 64), gemm_grid = static_cast<long>((rows + 31) / 32) * gemm_cols;
     if (plan.column_groups == 1) return true;
     if (plan.shares == 1 && 8 * kb < 7 * room) return false;
-    if (gemm_grid <= 2 * gemv_compute_units()) return plan.column_groups <= (plan.halves == 2 && plan.parts == 8 ? 3 : 4);
+    const long per_tile = plan.parts == 8 ? 2 : 1;
+    auto fits = [&](long tiles, long groups) { return tiles <= 2 * units || groups <= per_tile * ((tiles + units - 1) / units); };
+    if (!fits(gemm_grid, plan.column_groups)) return false;
+    BatchGroupsPlan pair;
+    if (gemm_cols % 8 == 0 && batch_groups_plan(tensor_type, static_cast<int>(rows), static_cast<int>(in_dim), static_cast<int>(out_dim), true, true, &pair) &&
+        !fits(2 * gemm_grid, pair.column_groups))
+        return false;
+    if (gemm_grid <= 2 * units) return plan.column_groups <= (plan.halves == 2 && plan.parts == 8 ? 3 : 4);
     return true;
 }
 
@@ -2079,18 +2096,19 @@ hipError_t launch_batch_mfma(hipStream_t stream, int tensor_type, float* dst, co
     const bool old_thirty_two = !eight && rows <= 64 && kb % 8 == 0 && groups32 >= gemv_compute_units() * 5 / 8 && groups32 <= bound;
     // Column groups: where the plan's sums are its own, for every form of the call (the bits of a pair's halves); elsewhere they are the
     // older kernels' and the faster one takes the call (us, Q4_0, K = 4096): one column group and three and more win (6144 columns
-    // 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8, 32000 29.8 -> 26.6), two on up to 32 rows lose to batch32_mfma_kernel where that can
-    // run (14336 columns 16.4 against 17.1, a pair of 6144 15.2 against 15.9).  A slice that K fills to less than three quarters is a
+    // 12.0 -> 10.7, a pair of 14336 27.9 -> 24.8, 32000 29.8 -> 26.6), two on up to 32 rows lose (14336 columns 16.4 against 17.1, a pair
+    // of 6144 15.2 against 15.9, 24 rows, K = 3072 x 9216 15.1 against 15.7).  Several on a slice that K fills to less than three quarters are a
     // loss of its own, which only more than 48 rows make up for (K = 2304 x 12290 columns, 40 rows 21.2 against 22.2; 64 rows x 32000
-    // columns 49.1 -> 39.2).  Q8_0 wins with one column group (K = 2048 x 8192 columns 9.8 -> 9.2; pairs of 5632 11.7 against 12.6).
+    // columns 49.1 -> 39.2).  Q8_0 wins with one column group and such a K (K = 2048 x 8192 columns 9.8 -> 9.2; pairs of 5632 11.7 against
+    // 12.6; 17 rows, K = 1280 x 8192 8.7 against 9.0).
     const bool adds = both_plain && apart(dst) && (!weight_b_prepared || apart(dst_b));
     BatchGroupsPlan plan;
-    const bool column_groups = !eight && bound_set != 0 &&
-                               batch_groups_plan(tensor_type, rows, in_dim, out_dim, weight_b_prepared != nullptr, adds, &plan) &&
+    const bool planned = !eight && bound_set != 0 && batch_groups_plan(tensor_type, rows, in_dim, out_dim, weight_b_prepared != nullptr, adds, &plan);
+    const bool filled = planned && 4 * kb >= 3 * plan.share_blocks;
+    const bool column_groups = planned &&
                                (rows > 64 ? batch_mfma_column_groups(tensor_type, rows, in_dim, out_dim)
-                                          : plan.own_sums || plan.column_groups == 1 ||
-                                                (tensor_type == 2 && (plan.parts == 4 || 4 * kb >= 3 * plan.share_blocks || rows > 48) &&
-                                                 (plan.column_groups > 2 || rows > 32 || !old_thirty_two)));
+                                          : plan.own_sums || (plan.column_groups == 1 && (tensor_type == 2 || filled)) ||
+                                                (tensor_type == 2 && (plan.parts == 4 || filled || rows > 48) && (plan.column_groups > 2 || rows > 32)));
     const bool thirty_two = old_thirty_two && !column_groups;
     if (column_groups) {
         real_shares = plan.shares;

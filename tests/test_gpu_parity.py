@@ -276,7 +276,7 @@ def test_prefill_keeps_small_activations(fmt, rows, in_dim, out_dim):
 @pytest.mark.parametrize("rows,in_dim,out_dim,bias", [
     (77, 2048, 2048, False), (96, 2048, 5632, False), (65, 3584, 2001, False),  # a run a wavefront on one group of columns, on several; two
     (96, 4096, 6145, False), (66, 4096, 1000, True), (80, 4096, 1000, False),   # ... on several, two apart, two K shares
-    (70, 14336, 1000, False), (90, 14336, 1000, True),                          # four a wavefront
+    (70, 14336, 1000, False), (90, 14336, 1000, True),                          # (the GEMM)
     (65, 768, 513, False), (96, 1024, 33001, False)])                           # four wavefronts on K
 def test_short_prompts_keep_small_activations(rows, in_dim, out_dim, bias):
     """65 to 96 rows of Q4_0: rows scaled by powers of two give the same bits scaled, from scale products just above 2^-126 (as
@@ -330,7 +330,7 @@ def short_chain_sums(dots: np.ndarray, products: np.ndarray, shares: int, wavefr
 
 @pytest.mark.parametrize("rows,in_dim,out_dim,shares,wavefronts", [
     (77, 4096, 2048, 1, 8), (65, 3584, 2559, 1, 8), (96, 2304, 1500, 1, 8),  # two runs, one group of columns (a pair: two)
-    (70, 6144, 700, 2, 8), (66, 4352, 1000, 2, 8), (80, 8192, 1344, 2, 8),   # ... on two K shares
+    (70, 6144, 700, 2, 8), (66, 4352, 1000, 2, 8), (80, 8192, 1279, 2, 8),   # ... on two K shares
     (77, 2048, 2730, 1, 4), (96, 1792, 8201, 1, 4),                          # ... of four wavefronts, several groups
     (77, 2048, 2048, 1, 8), (65, 768, 513, 1, 4)])                           # one run
 def test_short_prompts_add_up_in_short_chains(rows, in_dim, out_dim, shares, wavefronts):
