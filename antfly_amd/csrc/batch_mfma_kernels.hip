@@ -1427,7 +1427,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
     // A chain of additions is at most sixteen blocks long.  Runs of four stages put the first half's sums down in the
     // wavefront's own part of the room below.
     constexpr bool kPutDown = kHalves == 4;
-    static_assert(!kPutDown || kOne, "the room is free for the one column group only");
+    static_assert(!kPutDown || (kOne && !kAgain), "the room is free for the one column group only");
     constexpr int kSums = kApart ? kHalves : 1;
     // ... and where a run's sums are added up by themselves, four: even and odd blocks apart.
     constexpr bool kOdd = kHalves == 1 || kChains > 0;
@@ -1656,7 +1656,6 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             }
             if (kAgain && kApart && p % kPairs == kPairs - 1 && small_scales) form_again(cg, p / kPairs, p / kPairs + 1, acc[p / kPairs]);
             if (kPutDown && p == kSteps / 2 - 1) {
-                if (kAgain && small_scales) form_again(cg, 0, kHalves / 2, acc[0]);
                 store_sums(0);
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[0][v] = 0.0f;
@@ -1667,7 +1666,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
                 count_up(1);
             }
         }
-        if (kAgain && !kApart && small_scales) form_again(cg, kPutDown ? kHalves / 2 : 0, kHalves, acc[0]);
+        if (kAgain && !kApart && small_scales) form_again(cg, 0, kHalves, acc[0]);
         if (kPutDown) {
 #pragma unroll
             for (int v = 0; v < kLive; ++v) acc[0][v] = red[(wave * kLive + v) * 64 + lane] + acc[0][v];
@@ -1848,8 +1847,19 @@ struct BatchGroupsPlan {
     int row_groups, column_groups, parts, halves, shares, share_blocks;
     int chains;  // kChains
     bool own_sums;  // the sums are not formed in the older kernels' order
-    long grid;  // workgroups
 };
+
+// Whether the column-group kernel exists for a cut: those that batch_groups_plan makes.  Q8_0 of up to 16 rows is the eight-row kernel's
+// where K is whole runs, its two runs take one column group, on few columns 33 rows and more; four runs take 33 to 64 rows and one group;
+// beyond 64 rows a chain of two runs is left on several groups of eight wavefronts' K alone.
+constexpr bool batch_groups_exist(int type, int rows_to, bool sixteen_rows, int halves, int parts, int chains, bool one) {
+    if (type == 8 && (rows_to == 96 || sixteen_rows || chains == 1 || halves == 4)) return false;
+    if (type == 8 && !one && (halves == 2 || (parts == 8 && rows_to == 32))) return false;
+    if (halves == 4) return rows_to == 64 && parts == 8 && chains == 0 && one;
+    if (chains == 2) return halves == 2 && parts == 8 && one && (type == 2 || rows_to == 64);
+    if (chains == 1) return halves == 2 && rows_to == 96;
+    return halves == 1 || rows_to != 96 || (parts == 8 && !one);
+}
 
 template <int kType, int kHalves, int kParts, int kChains>
 hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
@@ -1868,16 +1878,16 @@ hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, c
     auto launch_for = [&](auto live, auto rows_to, int at) {
         constexpr int kLive = decltype(live)::value, kRows = decltype(rows_to)::value;
         constexpr int lds = BatchGroups<kType, kLive, kHalves, kParts>::kLdsBytes;
-        if (plan.column_groups == 1) return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, true>, lds, &lds_limit[at]);
-        if constexpr (kHalves == 4 || kChains == 2) return hipErrorInvalidValue;  // (not among the plans)
-        else return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, false>, lds, &lds_limit[at + 1]);
-    };
-    if constexpr (kChains == 1) {
-        if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
+        if (plan.column_groups == 1) {
+            if constexpr (batch_groups_exist(kType, kRows, kLive == 8, kHalves, kParts, kChains, true))
+                return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, true>, lds, &lds_limit[at]);
+        } else {
+            if constexpr (batch_groups_exist(kType, kRows, kLive == 8, kHalves, kParts, kChains, false))
+                return launch(batch_groups_mfma_kernel<kType, kLive, kHalves, kParts, kChains, kRows, false>, lds, &lds_limit[at + 1]);
+        }
         return hipErrorInvalidValue;  // (not among the plans)
-    }
-    if constexpr (kType == 2)
-        if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
+    };
+    if (rows > 64) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 96>{}, 6);
     if (rows > 32) return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 64>{}, 0);
     if (rows <= 16) return launch_for(std::integral_constant<int, 8>{}, std::integral_constant<int, 32>{}, 2);
     return launch_for(std::integral_constant<int, 16>{}, std::integral_constant<int, 32>{}, 4);
@@ -1887,20 +1897,15 @@ template <int kType>
 hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, const uint32_t* qa, const float* sa, const uint8_t* weight, int rows,
                             int in_dim, int out_dim, const BatchGroupsPlan& plan, const Epilogue& ep, const BmSecond& second, bool accumulate) {
 #define AFHIP_BMG(H, P, CHAINS) bm_launch_groups_of<kType, H, P, CHAINS>(stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, plan, ep, second, accumulate)
-    if (plan.chains == 2) return plan.halves == 2 && plan.parts == 8 ? AFHIP_BMG(2, 8, 2) : hipErrorInvalidValue;
-    if (plan.chains == 1) {
-        if constexpr (kType == 2)
-            if (plan.halves == 2) return plan.parts == 8 ? AFHIP_BMG(2, 8, 1) : AFHIP_BMG(2, 4, 1);
-        return hipErrorInvalidValue;
-    }
-    switch (plan.parts * 10 + plan.halves) {
-        case 81: return AFHIP_BMG(1, 8, 0);
-        case 82: return AFHIP_BMG(2, 8, 0);
-        case 84:  // (Q4_0 alone)
-            if constexpr (kType == 2) return AFHIP_BMG(4, 8, 0);
-            else return hipErrorInvalidValue;
-        case 41: return AFHIP_BMG(1, 4, 0);
-        case 42: return AFHIP_BMG(2, 4, 0);
+    switch (plan.parts * 100 + plan.halves * 10 + plan.chains) {
+        case 810: return AFHIP_BMG(1, 8, 0);
+        case 820: return AFHIP_BMG(2, 8, 0);
+        case 821: return AFHIP_BMG(2, 8, 1);
+        case 822: return AFHIP_BMG(2, 8, 2);
+        case 840: return AFHIP_BMG(4, 8, 0);
+        case 410: return AFHIP_BMG(1, 4, 0);
+        case 420: return AFHIP_BMG(2, 4, 0);
+        case 421: return AFHIP_BMG(2, 4, 1);
         default: return hipErrorInvalidValue;
     }
 #undef AFHIP_BMG
@@ -1975,7 +1980,7 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
         if (p.shares > 1) p.share_blocks = ((kb + p.shares - 1) / p.shares + stage_blocks - 1) / stage_blocks * stage_blocks;
     }
     p.column_groups = p.chains == 2 || p.halves == 4 ? 1 : static_cast<int>(groups_for(pair ? 2 : 1));
-    p.grid = grid(p.column_groups, pair ? 2 : 1);
+    if (!batch_groups_exist(tensor_type, rows > 64 ? 96 : (rows > 32 ? 64 : 32), rows <= 16, p.halves, p.parts, p.chains, p.column_groups == 1)) return false;
     *plan = p;
     return true;
 }
