@@ -1724,14 +1724,6 @@ static size_t bm8_lds_bytes(int tensor_type, int column_groups, int halves = 2) 
     const int share_blocks = (tensor_type == 2 ? BmFormat<2>::kShareBlocks : BmFormat<8>::kShareBlocks) / 2 * halves;
     return kBmLdsBytes + (column_groups >= 3 || halves > 2 ? 16 * column_groups * (share_blocks / 8) * 16 : 0);
 }
-// (raising a kernel's limit is sticky: once per instantiation)
-template <typename Kernel>
-static hipError_t bm_allow_large_lds(Kernel kernel, size_t lds, std::atomic<size_t>* limit) {
-    if (lds <= limit->load(std::memory_order_acquire)) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e == hipSuccess) limit->store(160 * 1024, std::memory_order_release);
-    return e;
-}
 
 constexpr bool bm8_can_quantize(int tensor_type, int halves, int groups) { return groups == 1 && halves <= (tensor_type == 2 ? 2 : 4); }
 
@@ -1743,9 +1735,9 @@ hipError_t bm_launch8(hipStream_t stream, float* dst, float* partial, const uint
     const dim3 grid(static_cast<unsigned>((out_dim + cols - 1) / cols), static_cast<unsigned>(shares), second.weight ? 2u : 1u), block(kBmThreads);
     if (accumulate || shares == 1) partial = nullptr;
     const size_t lds = bm8_lds_bytes(kType, kCG, kHalves);
-    static std::atomic<size_t> lds_limit[4] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
-    auto launch = [&](auto kernel, std::atomic<size_t>* limit) {
-        if (hipError_t e = bm_allow_large_lds(kernel, lds, limit); e != hipSuccess) return e;
+    static LdsLimit lds_limit[4];
+    auto launch = [&](auto kernel, LdsLimit* limit) {
+        if (hipError_t e = allow_lds(kernel, lds, limit); e != hipSuccess) return e;
         hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, partial, qa, sa, weight, rows, in_dim, out_dim, share_blocks, cols,
                            accumulate ? 1 : 0, ep, second);
         return hipGetLastError();
@@ -1868,9 +1860,9 @@ hipError_t bm_launch_groups_of(hipStream_t stream, float* dst, float* partial, c
     const dim3 grid(static_cast<unsigned>(plan.row_groups == 1 ? col_tiles : (col_tiles + 7) / 8 * 8 * plan.row_groups), static_cast<unsigned>(plan.shares),
                     second.weight ? 2u : 1u),
         block(kBmThreads);
-    static std::atomic<size_t> lds_limit[8] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
-    auto launch = [&](auto kernel, int lds, std::atomic<size_t>* limit) {
-        if (hipError_t e = bm_allow_large_lds(kernel, lds, limit); e != hipSuccess) return e;
+    static LdsLimit lds_limit[8];
+    auto launch = [&](auto kernel, int lds, LdsLimit* limit) {
+        if (hipError_t e = allow_lds(kernel, lds, limit); e != hipSuccess) return e;
         hipLaunchKernelGGL(kernel, grid, block, lds, stream, dst, plan.shares > 1 && !accumulate ? partial : nullptr, qa, sa, weight, rows, in_dim,
                            out_dim, plan.share_blocks, plan.row_groups, plan.column_groups, ep, second, accumulate ? 1 : 0);
         return hipGetLastError();
@@ -2237,8 +2229,8 @@ hipError_t launch_batch8_timeline(hipStream_t stream, uint32_t* stamps, size_t s
                        static_cast<float*>(nullptr), static_cast<float*>(nullptr), 0);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     int share_blocks = (kb + BmFormat<2>::kWaveBlocks - 1) / BmFormat<2>::kWaveBlocks * BmFormat<2>::kWaveBlocks;
-    static std::atomic<size_t> lds_limit{64 * 1024};
-    if (hipError_t e = bm_allow_large_lds(batch8_mfma_kernel<2, 4, true>, bm8_lds_bytes(2, 4), &lds_limit); e != hipSuccess) return e;
+    static LdsLimit lds_limit;
+    if (hipError_t e = allow_lds(batch8_mfma_kernel<2, 4, true>, bm8_lds_bytes(2, 4), &lds_limit); e != hipSuccess) return e;
     hipLaunchKernelGGL((batch8_mfma_kernel<2, 4, true>), dim3(static_cast<unsigned>(groups), 1, 1), dim3(kBmThreads), bm8_lds_bytes(2, 4), stream,
                        reinterpret_cast<float*>(stamps), static_cast<float*>(nullptr), qa, sa, weight_prepared, rows, in_dim, out_dim, share_blocks,
                        cols, 0, Epilogue{}, BmSecond{nullptr, nullptr, Epilogue{}});

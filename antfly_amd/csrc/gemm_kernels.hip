@@ -46,7 +46,6 @@
 // lane % 32, so stores are 128 bytes contiguous along n.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 #include <cstdlib>
 #include <type_traits>
 
@@ -604,14 +603,8 @@ hipError_t launch_wide_tile(hipStream_t stream, float* dst, const int8_t* qx, co
     // per-lane load offsets are 32-bit, relative to the workgroup's first row
     if (static_cast<long long>(S::kTM > S::kTN ? S::kTM : S::kTN) * in_dim > 0x7fffffffLL) return hipErrorInvalidValue;
     auto kernel = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false, false, false, kPerM, kPerN>;
-    static std::atomic<bool> attr_done{false};
-    if (!attr_done.load(std::memory_order_acquire)) {
-        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               S::kLdsBytes);
-            e != hipSuccess)
-            return e;
-        attr_done.store(true, std::memory_order_release);
-    }
+    static LdsLimit lds_limit;
+    if (hipError_t e = allow_lds(kernel, S::kLdsBytes, &lds_limit); e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), 1, second.dst ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, stream, dst,
                        nullptr, qx, sx, weight, rows, in_dim, out_dim, m_tiles, n_tiles, in_dim / 32, nullptr, ep, second);
     return hipGetLastError();
@@ -638,21 +631,10 @@ hipError_t launch_tile(hipStream_t stream, float* dst, int* dots, const int8_t* 
     auto kernel_f32 = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false>;
     auto kernel_shares = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, false, true>;
     auto kernel_dots = gemm_i8_kernel<kType, kWavesM, kWavesN, kSplit, true>;
-    // more than 64 KB of LDS has to be asked for once per kernel
-    static std::atomic<bool> attr_done{false};
-    const hipError_t attr = attr_done.load(std::memory_order_acquire) ? hipSuccess : [&]() {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel_f32),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, S::kLdsBytes);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel_shares), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                S::kLdsBytes);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel_dots), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                S::kLdsBytes);
-        if (e == hipSuccess) attr_done.store(true, std::memory_order_release);  // a failure is not remembered: the next call tries again
-        return e;
-    }();
-    if (attr != hipSuccess) return attr;
+    static LdsLimit lds_limit[3];
+    if (hipError_t e = allow_lds(kernel_f32, S::kLdsBytes, &lds_limit[0]); e != hipSuccess) return e;
+    if (hipError_t e = allow_lds(kernel_shares, S::kLdsBytes, &lds_limit[1]); e != hipSuccess) return e;
+    if (hipError_t e = allow_lds(kernel_dots, S::kLdsBytes, &lds_limit[2]); e != hipSuccess) return e;
     if (dots)
         hipLaunchKernelGGL(kernel_dots, g, b, S::kLdsBytes, stream, dst, dots, qx, sx, weight, rows, in_dim, out_dim,
                            m_tiles, n_tiles, share_blocks, sums, ep, second);

@@ -25,7 +25,6 @@
 //     stay in registers across passes.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 #include <type_traits>
 
 #include "device_common.h"
@@ -374,14 +373,6 @@ __global__ __launch_bounds__(1024) void gemv_batch_kernel(
     if (kRows > kFirst) run_pass(std::integral_constant<int, kFirst>{}, std::integral_constant<int, (kRows > kFirst ? kRows - kFirst : 1)>{});
 }
 
-template <typename Kernel>
-hipError_t allow_lds(Kernel kernel, size_t lds, std::atomic<size_t>* limit) {
-    if (lds <= limit->load(std::memory_order_acquire)) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e == hipSuccess) limit->store(160 * 1024, std::memory_order_release);
-    return e;
-}
-
 template <int kType, int kRows, bool kDots>
 hipError_t launch_rows(hipStream_t stream, float* dst_a, float* dst_b, int* dots, const float* input, const uint8_t* weight_a,
                        const uint8_t* weight_b, int in_dim, int out_dim, float* partial, const Epilogue& ep_a, const Epilogue& ep_b) {
@@ -396,7 +387,7 @@ hipError_t launch_rows(hipStream_t stream, float* dst_a, float* dst_b, int* dots
     const size_t lds = ready_counter ? static_cast<size_t>(kRows) * (kQRowBytes + kSliceBlocks * 8 + kRawRowBytes) + 16
                                      : static_cast<size_t>(kRows) * kRawRowBytes;
     auto kernel = gemv_batch_kernel<kType, kRows, kDots>;
-    static std::atomic<size_t> lds_limit{64 * 1024};
+    static LdsLimit lds_limit;
     if (hipError_t e = allow_lds(kernel, lds, &lds_limit); e != hipSuccess) return e;
     const size_t tile_off = tile_scales_offset(kType, static_cast<size_t>(out_dim) * kb);
     if ((tile_off >> 4) > 0xFFFFFFFFull) return hipErrorInvalidValue;

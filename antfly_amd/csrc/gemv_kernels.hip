@@ -28,7 +28,6 @@
 //   * a launch may serve two matrices of the same shape that share X (GemvTargets).
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 
 #include "device_common.h"
 #include "gemv_common.h"
@@ -756,17 +755,6 @@ int workgroup_waves(int requested_threads, int max_threads, int slices, int grou
     return best;
 }
 
-// Raising the dynamic-LDS limit is sticky per kernel: done once per kernel, outside
-// any stream capture a caller may open later.
-template <typename Kernel>
-hipError_t allow_large_lds(Kernel kernel, size_t lds, std::atomic<size_t>* limit) {
-    if (lds <= limit->load(std::memory_order_acquire)) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       160 * 1024);
-    if (e == hipSuccess) limit->store(160 * 1024, std::memory_order_release);  // (two host threads may both get here: the call is idempotent)
-    return e;
-}
-
 // Whether a fused launch waits for its quantizing wavefronts through the LDS counter (kGemvReadyCounter) instead of a
 // barrier: only when some wavefront does not quantize, and for one row only when it is long (measured: a gain from
 // K = 6144 on, a small loss on one row of 4096 values, whose two quantizers are done before the barrier matters).
@@ -829,8 +817,8 @@ hipError_t launch_fused(hipStream_t stream, const GemvTargets& tg0, int* dots, c
                                  : gemv_fused_kernel<kType, kRows, kCols, kDots, kArgmax, false, 0, 1>;
         }
     }
-    static std::atomic<size_t> lds_limit[6] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
-    if (hipError_t e = allow_large_lds(kernel, lds, &lds_limit[(compact ? 1 : 0) + 2 * defer]); e != hipSuccess) return e;
+    static LdsLimit lds_limit[6];
+    if (hipError_t e = allow_lds(kernel, lds, &lds_limit[(compact ? 1 : 0) + 2 * defer]); e != hipSuccess) return e;
     const int grid = (groups + groups_per_wg - 1) / groups_per_wg;
     if (key_count) *key_count = grid;
     // one round of workgroups: the wavefronts of a unit enter its load queue one after the other
@@ -860,8 +848,8 @@ hipError_t launch_rows(hipStream_t stream, const GemvTargets& tg0, int* dots, co
     const int groups_per_wg = waves / slices;
     const size_t lds = gemv_fused_lds_bytes(rows, in_dim);
     auto kernel = gemv_rows_kernel<kType, kCols, kDots>;
-    static std::atomic<size_t> lds_limit{64 * 1024};
-    if (hipError_t e = allow_large_lds(kernel, lds, &lds_limit); e != hipSuccess) return e;
+    static LdsLimit lds_limit;
+    if (hipError_t e = allow_lds(kernel, lds, &lds_limit); e != hipSuccess) return e;
     const int grid = (groups + groups_per_wg - 1) / groups_per_wg;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * 64), lds, stream, tg, dots,
                        reinterpret_cast<const int4*>(pre.q), pre.scale, pre.sum, rows, in_dim, out_dim, slices);
@@ -935,8 +923,8 @@ hipError_t launch_gemv_probe_rows(hipStream_t stream, int probe, float* dst, con
         if (waves_out) *waves_out = waves;
         if (stamps_bytes < static_cast<size_t>(grid) * waves * 32 || slices > 255 || groups_per_wg > 255) return hipErrorInvalidValue;
         auto kernel = gemv_fused_kernel<2, kRows, kCols, false, false, false, kProbeTimeline>;
-        static std::atomic<size_t> long_lds_limit{64 * 1024};
-        if (hipError_t e = allow_large_lds(kernel, lds, &long_lds_limit); e != hipSuccess) return e;
+        static LdsLimit long_lds_limit;
+        if (hipError_t e = allow_lds(kernel, lds, &long_lds_limit); e != hipSuccess) return e;
         const uint32_t shape = static_cast<uint32_t>(slices) | static_cast<uint32_t>(groups_per_wg) << 8 |
                                (grid <= compute_units() ? 1u << 16 : 0u) | (ready_counter ? kGemvReadyCounter : 0u);
         const GemvExtras extras{reinterpret_cast<int*>(stamps), nullptr, Epilogue{}, Epilogue{}};
@@ -957,12 +945,11 @@ hipError_t launch_gemv_probe_rows(hipStream_t stream, int probe, float* dst, con
     if (probe == kProbeTimeline && (stamps == nullptr || stamps_bytes < static_cast<size_t>(grid) * waves * 32)) return hipErrorInvalidValue;
     const GemvExtras extras{reinterpret_cast<int*>(stamps), nullptr, Epilogue{}, Epilogue{}};
     const size_t lds = gemv_fused_lds_bytes(kRows, in_dim) + (ready_counter ? ready_counter_lds_bytes(x_blocks) : 0);
-    static std::atomic<size_t> lds_limit[9] = {{64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024},
-                                               {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}, {64 * 1024}};
+    static LdsLimit lds_limit[9];
 #define AFHIP_PROBE(P)                                                                                                  \
     case P: {                                                                                                           \
         auto kernel = gemv_fused_kernel<2, kRows, kCols, false, false, true, P, (kRows >= 4 ? 2 : 0)>;                  \
-        if (hipError_t e = allow_large_lds(kernel, lds, &lds_limit[P]); e != hipSuccess) return e;                      \
+        if (hipError_t e = allow_lds(kernel, lds, &lds_limit[P]); e != hipSuccess) return e;                      \
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(64, waves), lds, stream, weight_prepared,                           \
                            static_cast<const uint8_t*>(nullptr), input, dst, static_cast<float*>(nullptr),              \
                            static_cast<uint32_t>(tile_off >> 4), in_dim / 32, out_dim, shape, extras);                  \

@@ -34,7 +34,6 @@
 // is a multiple of 32.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 
 #include <stdint.h>
 
@@ -1754,14 +1753,9 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
                 if (half_tiles) k8 = steps <= 1 ? gemv_q4k_i8_kernel<1, 1, 1024, false, true> : gemv_q4k_i8_kernel<1, 2, 1024, false, true>;
             }
             const size_t lds8 = q4k_i8_lds_bytes(rows, in_dim, waves);
-            static std::atomic<bool> large_lds8[13] = {};
+            static LdsLimit lds_limit8[13];
             const int limit8 = half_tiles ? variant + 6 : (half_sums ? 12 : variant);
-            if (lds8 > 64 * 1024 && !large_lds8[limit8]) {
-                if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k8), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-                    e != hipSuccess)
-                    return e;
-                large_lds8[limit8] = true;
-            }
+            if (hipError_t e = allow_lds(k8, lds8, &lds_limit8[limit8]); e != hipSuccess) return e;
             if (two_shares) {
                 const int count = rows * out_dim;
                 hipLaunchKernelGGL(q4k_zero_results_kernel, dim3((count + 1023) / 1024), dim3(256), 0, stream, dst,
@@ -1801,14 +1795,8 @@ hipError_t launch_q4k_mfma_rows(hipStream_t stream, float* dst, const float* x, 
             break;
     }
     if (kernel == nullptr) return hipErrorInvalidValue;
-    static std::atomic<bool> large_lds[12] = {};  // raising the limit is sticky per kernel: once, outside any stream capture opened later
-    if (lds > 64 * 1024 && !large_lds[variant + (own_slice ? 6 : 0)]) {
-        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               160 * 1024);
-            e != hipSuccess)
-            return e;
-        large_lds[variant + (own_slice ? 6 : 0)] = true;
-    }
+    static LdsLimit lds_limit[12];
+    if (hipError_t e = allow_lds(kernel, lds, &lds_limit[variant + (own_slice ? 6 : 0)]); e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * 64), lds, stream, dst, x, weight, rows, in_dim, out_dim, slices,
                        sb_per_slice, ep);
     return hipGetLastError();
@@ -2011,13 +1999,8 @@ hipError_t launch_fp6_tile(const Q4kGemmCall& q) {
     const long long grid = (static_cast<long long>(n_groups) * m_groups + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     auto kernel = gemm_q4k_fp6_kernel<kWaves, kR, kC, kOcc>;
-    static std::atomic<bool> attr_done{false};
-    if (S::kLdsBytes > 64 * 1024 && !attr_done.load(std::memory_order_acquire)) {
-        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLdsBytes);
-            e != hipSuccess)
-            return e;
-        attr_done.store(true, std::memory_order_release);
-    }
+    static LdsLimit lds_limit;
+    if (hipError_t e = allow_lds(kernel, S::kLdsBytes, &lds_limit); e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), q.shares, q.second ? 2 : 1), dim3(S::kThreads), S::kLdsBytes, q.stream, q.dst,
                        q.digits, q.sums, q.weight, q.rows, q.in_dim, q.out_dim, m_groups, n_groups, 8, q.sb_per_split, q.partial, q.first_to_dst ? 1 : 0, q.ep,
                        q.second ? *q.second : Q4kSecond{nullptr, nullptr, Epilogue{}}, q.x);

@@ -5,7 +5,15 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "lds_limit.h"
+
 namespace afhip {
+
+template <typename Kernel>
+hipError_t allow_lds(Kernel kernel, size_t lds, LdsLimit* limit) {
+    return limit->raise(lds, hipSuccess, [] { int d; return hipGetDevice(&d) == hipSuccess ? d : -1; },
+                        [&] { return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
+}
 
 // What the kernel that writes Y does to each total before storing it: + bias[o], then the
 // activation, then + residual[r][o] -- the engine's linear / linearRelu / linearQuickGelu /

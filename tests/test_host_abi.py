@@ -4,6 +4,7 @@ validation) behaves like the reference's.  No kernel is launched."""
 import ctypes as C
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -283,3 +284,31 @@ def test_session_wiring_patches_are_well_formed_and_apply():
             hunks += 1
         assert hunks >= 1, name
         assert added and any(re.search(r"hip|Hip", t) for t in added), name
+
+
+def test_lds_limit_is_raised_once_on_each_device(tmp_path):
+    """The record of a kernel's raised LDS limit (csrc/lds_limit.h), on the host: small launches ask for nothing, a device is asked
+    once, another one of its own, a failure is tried again, devices past the record every time."""
+    source = tmp_path / "lds_limit_test.cpp"
+    source.write_text('''#include <cstdio>
+#include "lds_limit.h"
+int main() {
+    afhip::LdsLimit limit;
+    int asked = 0, current = 0, answer = 0;
+    auto call = [&](size_t lds) { return limit.raise(lds, 0, [&] { return current; }, [&] { ++asked; return answer; }); };
+    const struct { int device, answer; size_t lds; int want_status, want_asked; } steps[] = {
+        {0, 0, 64 * 1024, 0, 0}, {0, 7, 65 * 1024, 7, 1}, {0, 0, 65 * 1024, 0, 2}, {0, 0, 160 * 1024, 0, 2}, {1, 0, 65 * 1024, 0, 3},
+        {1, 0, 65 * 1024, 0, 3}, {0, 0, 65 * 1024, 0, 3}, {63, 0, 65 * 1024, 0, 4}, {63, 0, 65 * 1024, 0, 4}, {64, 0, 65 * 1024, 0, 5},
+        {64, 0, 65 * 1024, 0, 6}, {-1, 0, 65 * 1024, 0, 7}, {-1, 0, 65 * 1024, 0, 8}};
+    for (const auto& s : steps) {
+        current = s.device, answer = s.answer;
+        const int status = call(s.lds);
+        if (status != s.want_status || asked != s.want_asked) return std::printf("device %d lds %zu: status %d, asked %d\\\\n", s.device, s.lds, status, asked), 1;
+    }
+    return 0;
+}
+''')
+    binary = tmp_path / "lds_limit_test"
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "antfly_amd", "csrc"), str(source), "-o", str(binary)], check=True)
+    done = subprocess.run([str(binary)], capture_output=True, text=True)
+    assert done.returncode == 0, done.stdout
