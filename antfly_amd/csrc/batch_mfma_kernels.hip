@@ -40,8 +40,8 @@
 //     staged weight requests, one workgroup per compute unit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
-
 #include <cstdlib>
 #include <type_traits>
 
@@ -1933,15 +1933,16 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     p.row_groups = (rows + 31) / 32;
     const long columns = (out_dim + 31) / 32;
     const bool few = 2 * columns * p.row_groups <= units;
-    // one workgroup a compute unit: each takes as many column groups as that needs
+    // One workgroup a compute unit: each takes as many column groups as that needs.  A launch takes the tiles of `groups` groups of columns
+    // (of eight XCDs each where there are row groups) for every row group, K share and matrix.
+    auto wide = [&] { return 8 / p.parts; };
     auto grid = [&](long groups, int matrices) {
-        const long wide = 8 / p.parts, tiles = (columns + groups * wide - 1) / (groups * wide);
+        const long tiles = (columns + groups * wide() - 1) / (groups * wide());
         return (p.row_groups == 1 ? tiles : (tiles + 7) / 8 * 8) * matrices * p.row_groups * static_cast<long>(p.shares);
     };
-    auto groups_for = [&](int matrices) {
-        long groups = 1;
-        while (grid(groups, matrices) > units && groups < columns) ++groups;
-        return groups;
+    auto groups_for = [&](int matrices) {  // the fewest whose grid is no more than the units, or all columns
+        const long each = static_cast<long>(matrices) * p.row_groups * p.shares, most = p.row_groups == 1 ? units / each : units / (8 * each) * 8;
+        return most == 0 ? columns : std::min(columns, (columns + most * wide() - 1) / (most * wide()));
     };
     p.parts = 8;
     p.shares = 1;
