@@ -128,9 +128,10 @@ static long batch_mfma_min_rows() {
 // faster than the decode kernels (the rules below).
 static bool batch_mfma_preferred(int tensor_type, size_t rows, size_t in_dim, size_t out_dim, bool pair) {
     const long forced = batch_mfma_min_rows();
-    // Up to 64 rows everywhere; 65 .. 96 of Q4_0 (beside batch_mfma_column_groups, whose kernel is the better one on its shapes) where the GEMM's grid of 32 x 64 tiles passes one workgroup a compute unit (on
-    // one it takes 15.5 us at K = 4096 x 4608 columns) and this kernel's 32-column tiles need few rounds.  It takes 17 us for every
-    // unit's worth of workgroups whatever K up to a share of 128 blocks, so K has to be near that (this kernel / the GEMM, 65 rows):
+    // Up to 64 rows everywhere; 65 .. 96 of Q4_0 where the GEMM's grid of 32 x 64 tiles passes one workgroup a compute unit (on one it
+    // takes 15.5 us at K = 4096 x 4608 columns) and this kernel's 32-column tiles need few rounds (the column-group kernel's shapes are
+    // batch_mfma_column_groups').  It takes 17 us for every unit's worth of workgroups whatever K up to a share of 128 blocks, so K has
+    // to be near that (this kernel / the GEMM, 65 rows):
     //  * one share and one round, K over 3072: 3104 x 6144 columns 19.2 / 20.2, 4096 x 8192 19.5 / 20.7; 3072 x 6144 18.1 / 17.0
     //    and, with a second share, 4352 x 6144 29.1 / 23.6, 6144 x 6144 33.4 / 27.0 go to the GEMM
     //  * a pair, one launch here and two of the GEMM, also in three rounds: 4096 x 11008 50.2 / 56.1, 4096 x 12288 50.8 / 56.5

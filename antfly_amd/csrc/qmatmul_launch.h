@@ -186,17 +186,17 @@ hipError_t launch_linear_q4k_q8k(hipStream_t stream, float* dst, const void* wor
 bool linear_q4k_q8k_shares_launch(bool tiled, size_t rows, size_t in_dim);
 // One, two or four rows on the tile-major layout at K <= 3072: the quantizer runs inside the matmul launch
 // (same bits as the two launches; `workspace` is not touched).
-// ... of more than nine rows, small calls: the quantizer inside the matmul launch, up to three matrices; bit for bit what
-// launch_quantize_q8k and launch_linear_q4k_q8k give.  X and the results must not overlap.
-bool linear_q4k_q8k_rows_fuses_quantizer(size_t rows, size_t in_dim, size_t out_dim, int matrices);
-hipError_t launch_linear_q4k_q8k_fused_rows(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
-                                            int out_dim, const Epilogue& ep, float* dst_b = nullptr, const uint8_t* weight_b = nullptr,
-                                            const Epilogue& ep_b = Epilogue(), float* dst_c = nullptr, const uint8_t* weight_c = nullptr,
-                                            const Epilogue& ep_c = Epilogue());
 bool linear_q4k_q8k_fuses_quantizer(bool tiled, size_t rows, size_t in_dim);
 hipError_t launch_linear_q4k_q8k_fused(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
                                        int out_dim, const Epilogue& ep, float* dst_b = nullptr, const uint8_t* weight_b = nullptr,
                                        const Epilogue& ep_b = Epilogue{});  // (dst_b / weight_b: a second matrix in the same launch)
+// More than nine rows, small calls: the quantizer inside the matmul launch too, up to three matrices; bit for bit what launch_quantize_q8k
+// and launch_linear_q4k_q8k give.  X and the results must not overlap.
+bool linear_q4k_q8k_rows_fuses_quantizer(size_t rows, size_t in_dim, size_t out_dim, int matrices);
+hipError_t launch_linear_q4k_q8k_fused_rows(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
+                                            int out_dim, const Epilogue& ep, float* dst_b = nullptr, const uint8_t* weight_b = nullptr,
+                                            const Epilogue& ep_b = Epilogue{}, float* dst_c = nullptr, const uint8_t* weight_c = nullptr,
+                                            const Epilogue& ep_c = Epilogue{});
 hipError_t launch_gemv_q4k(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
                            int out_dim, const Epilogue& ep = Epilogue{});
 hipError_t launch_dequantize_q4k_rows(hipStream_t stream, float* dst, const uint8_t* weight, const long long* ids,
