@@ -654,8 +654,10 @@ def test_column_groups_of_the_thirty_two_row_kernel(fmt, rows, in_dim, out_dim, 
         xd, y = G.to_dev(x), torch.full((rows * out_dim,), float("nan"), dtype=torch.float32, device=G.DEV)
         least = (rows * in_dim + 255) // 256 * 256 + rows * (in_dim // 32) * 8
         assert least < ws.numel()
+        ws[least:] = 0xA5  # what is not lent (the column-group kernel's operands, of whole row groups, reach into it)
         kernels.launchLinearF32(G.stream(), fmt, PREP, G.buf(y), G.buf(xd), G.buf(wd[0]), rows, in_dim, out_dim, G.buf(ws[:least]))
         torch.cuda.synchronize()
+        assert bool((ws[least:] == 0xA5).all())
         assert G.max_rel_err(y.cpu().numpy().reshape(rows, out_dim), single[0].reshape(rows, out_dim).astype(np.float64)) <= TIGHT
     ref = O.linear_no_bias(fmt, x, w[-1], rows, in_dim, out_dim, workers=8)
     assert G.max_rel_err(got[-1], ref.astype(np.float64)) <= TIGHT
