@@ -1050,14 +1050,17 @@ hipError_t launch_linear_q4k_q8k_fused(hipStream_t stream, float* dst, const flo
     return hipGetLastError();
 }
 
-// Whether the matrix-core form quantizes in the matmul launch: up to eight wavefronts a compute unit, two on a SIMD.  Past that the
-// repeated quantizing costs more than its launch (us, fused / two launches; wavefronts a unit): 64 x 2048 x 2048 (8) 6.7 / 8.5, 514 x 512 x
-// 512 (4.1) 7.3 / 8.6, but 197 x 768 x 3072 (14.6) 11.8 / 10.7, 154 x 1536 x 1536 (11) 10.8 / 8.8, 514 x 768 x 3072 (37) 24.4 / 15.2.
+// Whether the matrix-core form quantizes in the matmul launch: up to eight wavefronts a compute unit, two on a SIMD, and as whole workgroups
+// of up to eight.  Past that the repeated quantizing costs more than its launch (us, fused / two launches; wavefronts a unit): 64 x 2048 x
+// 2048 (8) 6.7 / 8.5, 514 x 512 x 512 (4.1) 7.3 / 8.6, but 197 x 768 x 3072 (14.6) 11.8 / 10.7, 154 x 1536 x 1536 (11) 10.8 / 8.8, 514 x 768 x
+// 3072 (37) 24.4 / 15.2; of six wavefronts a unit holds one workgroup, of three two: 77 x 1536 x 2048 (7.5 in 320 workgroups) 11.0 / 8.8,
+// 77 x 768 x 4096 (7.5 in 640) 9.3 / 8.75, but a pair of 64 x 1536 x 1024 (6 in 256) 7.7 / 8.85.
 constexpr size_t kQ8kFusedWaves = 8;
 bool linear_q4k_q8k_rows_fuses_quantizer(size_t rows, size_t in_dim, size_t out_dim, int matrices) {
-    const size_t groups = (rows + kQ8kFusedRows - 1) / kQ8kFusedRows, tiles = (out_dim + 31) / 32;
-    return linear_q4k_q8k_shares_launch(true, rows, in_dim) && groups <= 65535 &&
-           groups * tiles * static_cast<size_t>(matrices) * (in_dim / kQ4kBlockValues) <= kQ8kFusedWaves * static_cast<size_t>(gemv_compute_units());
+    const size_t groups = (rows + kQ8kFusedRows - 1) / kQ8kFusedRows, tiles = (out_dim + 31) / 32, units = static_cast<size_t>(gemv_compute_units());
+    const size_t kb = in_dim / kQ4kBlockValues, workgroups = groups * tiles * static_cast<size_t>(matrices);
+    if (!linear_q4k_q8k_shares_launch(true, rows, in_dim) || groups > 65535) return false;
+    return kb > kQ8kFusedWaves ? workgroups * kb <= kQ8kFusedWaves * units : workgroups <= kQ8kFusedWaves / kb * units;
 }
 
 hipError_t launch_linear_q4k_q8k_fused_rows(hipStream_t stream, float* dst, const float* x, const uint8_t* weight, int rows, int in_dim,
