@@ -1842,12 +1842,12 @@ struct BatchGroupsPlan {
 };
 
 // Whether the column-group kernel exists for a cut: those that batch_groups_plan makes.  Q8_0 of up to 16 rows is the eight-row kernel's
-// where K is whole runs, its two runs take one column group, on few columns 33 rows and more; four runs take 33 to 64 rows and one group;
+// where K is whole runs, its two runs take one column group, on few columns 33 rows and more; four runs take 25 to 64 rows and one group;
 // beyond 64 rows a chain of two runs is left on several groups of eight wavefronts' K alone.
 constexpr bool batch_groups_exist(int type, int rows_to, bool sixteen_rows, int halves, int parts, int chains, bool one) {
     if (type == 8 && (rows_to == 96 || sixteen_rows || chains == 1 || halves == 4)) return false;
     if (type == 8 && !one && (halves == 2 || (parts == 8 && rows_to == 32))) return false;
-    if (halves == 4) return rows_to == 64 && parts == 8 && chains == 0 && one;
+    if (halves == 4) return rows_to != 96 && !sixteen_rows && parts == 8 && chains == 0 && one;
     if (chains == 2) return halves == 2 && parts == 8 && one && (type == 2 || rows_to == 64);
     if (chains == 1) return halves == 2 && rows_to == 96;
     return halves == 1 || rows_to != 96 || (parts == 8 && !one);
@@ -1913,10 +1913,11 @@ hipError_t bm_launch_groups(hipStream_t stream, float* dst, float* partial, cons
 //   * Two shares of two runs add a reduce launch to an op with an epilogue and take twice the workgroups: on 32 rows only where a pair is one
 //     round too (K = 5632: 2048 columns 10.9 -> 10.5, but a pair of 4096 14.6 against 16.8), beyond 64 where one matrix is (1344 columns with
 //     a bias 14.7 against 17.1).
-//   * Four runs a share on 33 to 64 rows and few columns only (a pair in one round: 48 rows, K = 14336 x 1024 columns 18.6 -> 16.3, with a bias
-//     18.9 -> 18.5, 2048 columns 19.4 -> 17.9, but a pair 29.6 against 31.1).  On 32 rows the older kernels' K shares are better, most of all
-//     for an op with an epilogue (14336 x 1024 14.1 against 16.1, with a bias 14.3 against 18.5; 14336 x 4096 19.1 -> 18.3, but with a bias
-//     19.3 against 21.3), beyond 64 the GEMM's (11008 x 512 15.1 against 16.2, with a bias 15.5 against 18.8).
+//   * Four runs a share on few columns: 25 to 32 rows of more than three eighths of the units' where K fills two shares (K = 14336 x 4096 columns
+//     19.1 -> 18.3 .. 18.9 and a pair 34.2 -> 32.4, with the smaller error of shorter chains; an op with an epilogue pays its reduce launch,
+//     19.3 against 21.1), 33 to 64 rows where a pair is one round (48 rows, 14336 x 1024 18.6 -> 16.3, with a bias 18.9 -> 18.5; 2048
+//     columns 19.4 -> 17.9, but a pair 29.6 against 31.1).  Elsewhere the older kernels' K shares are better (32 rows, 14336 x 1024 14.1
+//     against 16.1, a pair of 9216 x 4096 27.2 / 29.6), beyond 64 rows the GEMM's (11008 x 512 15.1 against 16.2, with a bias 15.5 / 18.8).
 //   * Beyond 64 rows, where the other route is the GEMM, which shares K out on one group of columns: a wavefront's two runs go into chains
 //     of even and odd blocks, and K shares are equal.  Error against the GEMM's, a chain of sixteen in brackets: 77 x 4096 x 2048 0.89
 //     (1.01), 96 x 2304 x 1500 0.95 (1.14), 66 x 4352 x 1024 0.95 (1.13), 77 x 2048 x 8192 0.87 (1.00); 10.28 -> 10.33, 9.78 -> 9.91, 10.7 ->
@@ -1965,7 +1966,9 @@ bool batch_groups_plan(int tensor_type, int rows, int in_dim, int out_dim, bool 
     p.shares = (kb + p.share_blocks - 1) / p.share_blocks;
     p.own_sums = few || p.halves != 2;  // (up to 64 rows)
     if (p.shares == 2 && p.halves == 2 && (p.row_groups == 1 ? grid(1, 2) : (p.row_groups == 3 ? grid(1, 1) : 0)) > units) return false;
-    if (p.halves == 4 && (!few || tensor_type == 8 || p.row_groups != 2 || grid(1, 2) > units)) return false;
+    const bool four_runs = p.row_groups == 1 ? rows > 24 && 8 * columns > 3 * units && p.shares == 2 && 8 * kb >= 7 * p.shares * 4 * run
+                                             : p.row_groups == 2 && grid(1, 2) <= units;
+    if (p.halves == 4 && (!few || tensor_type == 8 || !four_runs)) return false;
     if (tensor_type == 8 && few && runs > 1 && (p.row_groups == 1 || 4 * p.row_groups * columns > units)) return false;
     if (tensor_type == 8 && !few && p.halves == 1 && p.parts == 8 && p.row_groups == 1) return false;
     if (rows > 64 && p.halves == 2 && p.chains == 0 && (p.parts == 4 || groups_for(1) == 1)) {
