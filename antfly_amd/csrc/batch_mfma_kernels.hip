@@ -1518,7 +1518,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
         const int l = side_tid * kPer & 63, v = side_tid * kPer >> 6;
         const int m = row0 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3);
         const int n = n_first + cg * B::kGroupCols + side * 32 + (l & 31);
-        if (plain && n + kPer <= out_dim) {
+        // The frequent ways first, their code straight behind the sums': behind the epilogue's, a pass of 32 rows through eight layers (64
+        // launches of different kernels) took 502 us instead of 496, though each kernel by itself took the same time
+        if (__builtin_expect(plain && n + kPer <= out_dim, 1)) {
             if (m < rows) {
                 float* const to = dst + static_cast<size_t>(m) * out_dim + n;
 #pragma unroll
@@ -1526,9 +1528,15 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
             }
             return;
         }
+        if (__builtin_expect(accumulate, 1)) {  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
+#pragma unroll
+            for (int k = 0; k < kPer; ++k)
+                if (m < rows && n + k < out_dim) unsafeAtomicAdd(dst + static_cast<size_t>(m) * out_dim + n + k, total[k]);
+            return;
+        }
         // finish_output for neighbouring columns together, the activations out of the way: one column after the other it took 0.7 us of a small
         // call (Q8_0 17 x 256 x 512 with a bias 6.86 -> 6.16, without 5.7; Q4_0 48 x 4096 x 8192 with a bias 17.2 -> 16.65)
-        if (partial == nullptr && !accumulate) {
+        if (__builtin_expect(partial == nullptr, 0)) {
             if (ep.bias != nullptr) {
 #pragma unroll
                 for (int k = 0; k < kPer; ++k) total[k] += ep.bias[min(n + k, out_dim - 1)];
@@ -1545,16 +1553,14 @@ __global__ __launch_bounds__(kBmThreads, 2) void batch_groups_mfma_kernel(float*
         }
         if (m >= rows) return;
         float* const to = (partial != nullptr ? partial + static_cast<size_t>(blockIdx.y) * rows * out_dim : dst) + static_cast<size_t>(m) * out_dim + n;
-        if (!accumulate && n + kPer <= out_dim) {
+        if (n + kPer <= out_dim) {
 #pragma unroll
             for (int k = 0; k < kPer; ++k) to[k] = total[k];
             return;
         }
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            if (n + k >= out_dim) break;
-            if (accumulate) unsafeAtomicAdd(to + k, total[k]);  // (two K shares, no epilogue, the result cleared beforehand: see batch8_mfma_kernel)
-            else to[k] = total[k];
+            if (n + k < out_dim) to[k] = total[k];
         }
     };
 
