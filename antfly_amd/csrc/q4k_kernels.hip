@@ -828,7 +828,7 @@ __global__ __launch_bounds__(768) void linear_q4k_q8k_mfma_kernel(float* __restr
 // Sixteen rows and not 32: the quantizer's vector work (560 instructions a wavefront) is what the launch waits for, and small calls have
 // compute units to spare for it.  us a call as a graph node, against the two launches: 77 x 768 x 768 8.1 -> 5.3, 77 x 768 x 3072 8.6 ->
 // 7.4, 77 x 3072 x 768 10.3 -> 8.5, 50 x 512 x 2048 8.0 -> 5.5, 64 x 2048 x 2048 8.5 -> 6.7; an encoder's layers (77 rows, launched one by
-// one, where a launch costs the host 3.6 us) 168 -> 126 a pass.
+// one, where a launch costs the host 3.6 us) 191 -> 137 a pass.
 constexpr int kQ8kFusedRows = 16;
 constexpr int kQ8kStageRow = kQ4kBlockValues + 16;                       // bytes: sixteen rows' fragments in different banks
 constexpr int kQ8kStageBytes = kQ8kFusedRows * kQ8kStageRow;             // of a wavefront, its sums in the same place afterwards
