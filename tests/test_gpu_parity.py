@@ -277,7 +277,7 @@ def test_prefill_keeps_small_activations(fmt, rows, in_dim, out_dim):
     (77, 2048, 2048, False), (96, 2048, 5632, False), (65, 3584, 2001, False),  # a run a wavefront on one group of columns, on several; two
     (96, 4096, 6145, False), (66, 4096, 1000, True), (80, 4096, 1000, False),   # ... on several, two apart, two K shares
     (70, 14336, 1000, False), (90, 14336, 1000, True),                          # (the GEMM)
-    (65, 768, 513, False), (96, 1024, 33001, False)])                           # four wavefronts on K
+    (65, 768, 513, False), (96, 1024, 33001, False), (70, 1792, 9001, False)])  # four wavefronts on K: one run, two
 def test_short_prompts_keep_small_activations(rows, in_dim, out_dim, bias):
     """65 to 96 rows of Q4_0: rows scaled by powers of two give the same bits scaled, from scale products just above 2^-126 (as
     test_prefill_keeps_small_activations) to activations of 2^100, and rows of one call do not feel each other.  Rows around 2^87
@@ -300,7 +300,10 @@ def test_short_prompts_keep_small_activations(rows, in_dim, out_dim, bias):
         y, got = (G.linear_bias(Q4, PREP, each, wd, np.zeros(out_dim, np.float32), rows, in_dim, out_dim) for each in (x, scaled))
     else:
         y, got = (G.linear(Q4, PREP, each, wd, rows, in_dim, out_dim) for each in (x, scaled))
-    assert np.array_equal(got, (y.astype(np.float64) * factor[:, None]).astype(np.float32))
+    want = (y.astype(np.float64) * factor[:, None]).astype(np.float32)
+    assert np.array_equal(got, want)
+    for half in G.linear_pair(Q4, PREP, scaled, wd, wd, rows, in_dim, out_dim):
+        assert np.array_equal(half, want)
 
 
 def short_chain_sums(dots: np.ndarray, products: np.ndarray, shares: int, wavefronts: int) -> np.ndarray:
